@@ -13,7 +13,7 @@ residual 1e-10 with V(2,2) multicolour-SSOR GMG preconditioning FGMRES(30):
               there; the finest level keeps SSOR).  The networks are trained
               once before the timed steps; training time is reported
               separately, not part of the step;
-  * learned_fp16s : learned with the finest level's SSOR colour launches
+  * learned_fp16s : learned with the finest level's SSOR launches
               on row-scaled FP16 copies of the values (reported alongside;
               the metric's value is the learned form with FP32 storage).
 After the timed forms the networks are trained again on other seeds of the
@@ -43,12 +43,10 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0      # MI355X HBM3E, GB/s
 FP64_PEAK_TFLOPS = 78.6    # MI355X FP64 (vector = MFMA), TFLOP/s
 BF16_PEAK_TFLOPS = 2500.0  # MI355X dense BF16 MFMA, TFLOP/s
-# HBM bytes per dispatch at 64^3 Q2 from rocprofv3 FETCH_SIZE x 2.000 +
-# WRITE_SIZE x 1.000 passes over tests/cpp/kernel_probe (the factors make the
-# counters of a 1 GiB device copy read 1 GiB each), in
-# profiles/k_rows_ssor_spmv_fp32_q2_64_hbm_traffic.md:
-TRAFFIC_SSOR_LAUNCH = 30_917_171  # k_rows<float,3,1>, one colour launch (average over the sweeps)
-TRAFFIC_SPMV = 561_289_188  # k_rows<float,0,1>
+# HBM bytes per dispatch at 64^3 Q2 from hardware counters (None: not counted
+# for the current kernels)
+TRAFFIC_SSOR_LAUNCH = None  # k_line_sweep<float, float, 2>, one line group (average over the sweeps)
+TRAFFIC_SPMV = None  # k_line_rows<float, 2, 0>
 
 
 def cpu_info():
@@ -397,26 +395,26 @@ def main():
     # column indices; x counted once per launch, every launch gathers from
     # all of it):
     #   SpMV:                 stored values s_v + x (N s_v) + y of the active rows
-    #   SSOR colour launch:   the colour's values + x (N s_v) + f read and x
-    #                         written for the colour's rows; one launch = one
-    #                         of the 54 colour applications of a sweep (the
-    #                         27 colours forward and backward)
+    #   SSOR group launch:    the group's values + x (N s_v) + f read and x
+    #                         written for the group's rows; one launch = one of
+    #                         the 9 line groups (3 colours each), forward or
+    #                         backward
     # Durations are those of the single dispatches (events recorded by the
     # dispatch, pmx_time_kernel 10 / 11), not of back-to-back launch sequences.
     nvals = int(d[6])
     nact = int(d[1])
-    ncol = int(d[7])
+    ngrp = int(round(int(d[7]) ** (2 / 3)))  # line groups: colours per axis squared
     kern = {}
     roof = {}
     for prec, sv in ((1, 4), (0, 8)):
         ms_spmv = S.time_kernel(11, -1, prec, reps=20)
         ms_col = S.time_kernel(10, -1, prec, reps=4)
         b_spmv = nvals * sv + N * sv + nact * sv
-        b_col = nvals * sv / ncol + N * sv + 2 * nact * sv / ncol
+        b_col = nvals * sv / ngrp + N * sv + 2 * nact * sv / ngrp
         roof[prec] = {"spmv_ms": ms_spmv, "spmv_bytes": b_spmv, "col_ms": ms_col, "col_bytes": b_col}
-    # calibration of the colour launch on the same level and with the same
+    # calibration of the group launch on the same level and with the same
     # dispatch events: a dispatch that does nothing (its workgroup counts) and
-    # a plain streaming read of the colour's FP32 values alone
+    # a plain streaming read of a group's share of the FP32 values alone
     cal = {"empty_dispatch_ms": S.time_kernel(12, -1, 1, reps=4),
            "stream_read_values_ms": S.time_kernel(13, -1, 1, reps=4)}
     kern["ssor_sweep_fp32_ms"] = S.time_kernel(3, -1, 1, reps=10)
@@ -523,12 +521,12 @@ def main():
         "fallbacks": {f: res[f]["fallbacks"] for f in res},
         "final_rel_residual": {f: res[f]["rel_res"] for f in res},
         "kernels_ms": {"spmv_fp32_dispatch": round(r32["spmv_ms"], 4), "spmv_fp64_dispatch": round(roof[0]["spmv_ms"], 4),
-                       "ssor_colour_fp32_dispatch": round(r32["col_ms"], 4),
-                       "ssor_colour_fp64_dispatch": round(roof[0]["col_ms"], 4),
+                       "ssor_group_fp32_dispatch": round(r32["col_ms"], 4),
+                       "ssor_group_fp64_dispatch": round(roof[0]["col_ms"], 4),
                        **{k: round(v, 4) for k, v in kern.items()}},
-        # the dominant kernel of the timed solve: the colour launches of the
+        # the dominant kernel of the timed solve: the line-group launches of the
         # finest level's FP32 SSOR sweeps
-        "roofline": {"bound": "hbm", "kernel": "k_rows<float,3,1> (one SSOR colour launch, finest level)",
+        "roofline": {"bound": "hbm", "kernel": "k_line_sweep<float,float,2> (one SSOR group launch, finest level)",
                      "achieved": round(col_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(col_gbs / HBM_PEAK_GBS, 4), "traffic": TRAFFIC_SSOR_LAUNCH,
                      "algorithmic_bytes": int(r32["col_bytes"]), "dispatch_ms": round(r32["col_ms"], 5),
@@ -536,7 +534,7 @@ def main():
                                      "stream_read_of_the_values_ms": round(cal["stream_read_values_ms"], 5),
                                      "launch_over_stream_read": round(r32["col_ms"] / cal["stream_read_values_ms"],
                                                                       3)}},
-        "roofline_spmv": {"bound": "hbm", "kernel": "k_rows<float,0,1> (stencil SpMV, finest level)",
+        "roofline_spmv": {"bound": "hbm", "kernel": "k_line_rows<float,2,0> (stencil SpMV, finest level)",
                           "achieved": round(spmv_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                           "frac": round(spmv_gbs / HBM_PEAK_GBS, 4), "traffic": TRAFFIC_SPMV,
                           "algorithmic_bytes": int(r32["spmv_bytes"]), "dispatch_ms": round(r32["spmv_ms"], 5),

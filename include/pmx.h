@@ -69,7 +69,8 @@ int pmx_system_create(pmx_ctx *ctx, int nref0, int nlev, int order, pmx_system *
 int pmx_system_destroy(pmx_system *sys);
 /* dims[0]=N_DegreesOfFreedom [1]=ActiveBound [2]=N_Cells [3]=N_Entries of the
  * CSR structure [4]=N_BaseFunct [5]=lattice points per direction
- * [6]=stored stencil values [7]=smoother colours */
+ * [6]=stencil entries of the interior rows, the rows of a residue class
+ * (mod 2 for Q1, 6 for Q2) rounded up to a multiple of 16 [7]=smoother colours */
 int pmx_system_dims(pmx_system *sys, int level, long long *dims);
 
 /* TFESpace3D::GetBeginIndex / GetGlobalNumbers (include/FE/FESpace3D.h),
@@ -171,7 +172,7 @@ int pmx_csr_matvec(pmx_ctx *ctx, int n, const int *rowptr, const int *kcol, cons
  *  [14] BiCGStab flexible branch (1 = v = A y)
  *  [15] precision: 0 FP64 throughout, 1 FP32 operator/MG/Krylov vectors
  *       inside an FP64 defect correction, 2 = 1 plus the learned post-smoother;
- *       3 / 4 = 1 / 2 with the SOR/SSOR sweeps that run launch per colour
+ *       3 / 4 = 1 / 2 with the launched SOR/SSOR sweeps
  *       reading row-scaled FP16 values (a_ij / a_ii, saturated to the finite
  *       FP16 range) and 1 / a_ii in FP32: half the value bytes of the sweeps,
  *       which only precondition (defects, transfers and Krylov vectors keep
@@ -277,12 +278,13 @@ int pmx_tcd_restore_massmat(pmx_system *sys);
  * timed with two events around the `reps` repetitions (ms per repetition).
  * 10 and 11 give the average duration of a single dispatch, from events
  * recorded by the dispatch itself (hipExtLaunchKernelGGL), without the gaps
- * between dispatches: 10 one colour launch of an SSOR sweep (launch per
- * colour), 11 one SpMV; calibration of 10 on the same level, also per
- * dispatch: 12 a dispatch that does nothing with the workgroup count of each
- * colour launch, 13 a plain streaming read of each colour's stored values in
- * the precision's storage.  precision 0 FP64, 1 FP32, 3 FP32 with the
- * SOR/SSOR colour launches on row-scaled FP16 values (opt[15] = 3).  out: ms. */
+ * between dispatches: 10 one launch of an SSOR sweep (a line group: the
+ * colours of equal (y, z) residues), 11 one SpMV; calibration of 10 on the
+ * same level, also per dispatch: 12 a dispatch that does nothing with the
+ * workgroup count of each group launch, 13 a plain streaming read of a group's
+ * share of the stored values in the precision's storage.  precision 0 FP64,
+ * 1 FP32, 3 FP32 with the launched SOR/SSOR sweeps on row-scaled FP16 values
+ * (opt[15] = 3).  out: ms. */
 int pmx_time_kernel(pmx_system *sys, int kernel, int level, int precision, int reps, double *ms);
 
 /* ---- learned post-smoother (no counterpart in the reference; it replaces

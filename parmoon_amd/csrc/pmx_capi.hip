@@ -47,9 +47,9 @@ struct DevBuf {
     check(hipMalloc(&p, sizeof(T) * m), "hipMalloc");
     n = m;
   }
-  // alloc, and a fresh allocation starts zeroed (stream-ordered): the
-  // padding rows of the last value slice of a class are never written by
-  // the assembly and stay zero
+  // alloc, and a fresh allocation starts zeroed (stream-ordered): the values
+  // of the boundary node that completes a line's last row pair are never
+  // written by the assembly and stay zero
   void alloc_zeroed(size_t m, hipStream_t st) {
     if (m == n && p) return;
     alloc(m);
@@ -72,7 +72,7 @@ struct Ctx {
 // per-precision work vectors of one level
 template <typename T>
 struct Vecs {
-  DevBuf<T> val;                      // CSS values in this precision
+  DevBuf<T> val;                      // values (line layout) in this precision
   DevBuf<T> x, f, d, aux;             // MG level vectors
   DevBuf<T> sold, sdef;               // step length control: u and f - A u before the pre-smoothing
 };
@@ -81,11 +81,7 @@ struct Level {
   Layout L;
   Numbering Nb;
   DevLayout D;
-  DevBuf<int> boundary, segidx;
-  DevBuf<DevSegment> segs;
-  DevBuf<BlockInfo> blocks_all, blocks_colour;
-  DevBuf<RowBlock> rows_all, rows_colour;  // the same with the class records inline
-  DevBuf<int> colour_off, colour_seg;
+  DevBuf<int> boundary;
   DevBuf<int> lat2dof, dof2lat, rowptr, kcol;
   DevBuf<double> val2;                // second matrix (SUPG K)
   DevBuf<double> mass;                // time stepping: mass matrix M
@@ -222,91 +218,16 @@ static void setup_level(System &Y, Level &lv, int nref) {
     Nb.have_csr = false;
   }
   DevLayout &D = lv.D;
-  D.order = L.order; D.n = L.n; D.M = L.M; D.S = L.S;
-  D.N = L.N; D.nvals = L.nvals; D.nactive = L.nactive;
+  D.order = L.order; D.n = L.n; D.M = L.M;
+  while ((2 << D.lg) < L.M - 1) D.lg++;
+  D.N = L.N; D.nvals = L.nstored; D.nactive = L.nactive;
   D.ncolours = L.ncolours;
-  std::vector<DevSegment> ds(L.segs.size());
-  for (size_t i = 0; i < L.segs.size(); i++) {
-    const Segment &s = L.segs[i];
-    ds[i] = DevSegment{s.x0, s.y0, s.z0, s.cx, s.cy, s.cz, s.ex, s.ey, s.ez, s.ns, s.dslot, L.S, s.count, s.voff};
-  }
-  lv.segs.upload(ds.data(), ds.size(), st);
-  std::vector<int> sidx(L.S * L.S * L.S, -1);
-  for (size_t i = 0; i < L.segs.size(); i++) {
-    const Segment &s = L.segs[i];
-    sidx[s.rx + L.S * (s.ry + L.S * s.rz)] = (int)i;
-  }
-  lv.segidx.upload(sidx.data(), sidx.size(), st);
-  // Launch order of the blocks: sorted by the lattice position of their first
-  // row (z, then y) across residue classes, in every list.  A launch's blocks
-  // are split into 8 contiguous chunks, one per XCD (xcd_remap), so each XCD
-  // works on one z-slab: the x values its rows gather (the slab plus two
-  // planes either side) stay in that XCD's L2 instead of every XCD streaming
-  // the whole vector once per class, and the rows sharing a cell are
-  // assembled close in time.  Rows of one list are independent, so the order
-  // changes no result.
-  auto key = [&](const BlockInfo &b) {
-    const Segment &sg = L.segs[b.seg];
-    const int64_t t = b.base / sg.cx;
-    const int64_t y = sg.y0 + (int64_t)L.S * (t % sg.cy), z = sg.z0 + (int64_t)L.S * (t / sg.cy);
-    return std::make_tuple(z, y, b.seg, b.base);
-  };
-  auto spatial = [&](std::vector<BlockInfo> v) {
-    std::stable_sort(v.begin(), v.end(), [&](const BlockInfo &a, const BlockInfo &b) { return key(a) < key(b); });
-    return v;
-  };
-  auto inline_records = [&](const std::vector<BlockInfo> &v) {
-    std::vector<RowBlock> r(v.size());
-    for (size_t i = 0; i < v.size(); i++) r[i] = RowBlock{ds[v[i].seg], v[i].base, 0};
-    return r;
-  };
-  {
-    const std::vector<BlockInfo> ba = spatial(L.blocks_all);
-    lv.blocks_all.upload(ba.data(), ba.size(), st);
-    const std::vector<RowBlock> ra = inline_records(ba);
-    lv.rows_all.upload(ra.data(), ra.size(), st);
-  }
-  std::vector<BlockInfo> bc;
-  D.colour_off.assign(L.ncolours + 1, 0);
-  for (int c = 0; c < L.ncolours; c++) {
-    D.colour_off[c] = (int)bc.size();
-    const std::vector<BlockInfo> bs = spatial(L.blocks_colour[c]);
-    bc.insert(bc.end(), bs.begin(), bs.end());
-  }
-  D.colour_off[L.ncolours] = (int)bc.size();
-  lv.blocks_colour.upload(bc.data(), bc.size(), st);
-  {
-    const std::vector<RowBlock> rc = inline_records(bc);
-    lv.rows_colour.upload(rc.data(), rc.size(), st);
-  }
-  lv.colour_off.upload(D.colour_off.data(), D.colour_off.size(), st);
-  {
-    // segments are stored colour-major: colour c owns segments cs[c] .. cs[c+1]-1
-    std::vector<int> cs(L.ncolours + 1, 0);
-    std::vector<int64_t> rows(L.ncolours, 0);
-    for (size_t i = 0; i < L.segs.size(); i++) {
-      const int c = L.segs[i].colour;
-      if (i > 0 && c < L.segs[i - 1].colour) throw std::logic_error("segments not colour-major");
-      cs[c + 1]++;
-      rows[c] += L.segs[i].count;
-    }
-    for (int c = 0; c < L.ncolours; c++) cs[c + 1] += cs[c];
-    lv.colour_seg.upload(cs.data(), cs.size(), st);
-    D.colour_seg_dev = lv.colour_seg.p;
-    D.max_colour_rows = *std::max_element(rows.begin(), rows.end());
-    D.nsegs = (int)L.segs.size();
-  }
+  D.max_colour_rows = L.max_colour_rows;
   lv.boundary.upload(L.boundary.data(), L.boundary.size(), st);
   D.boundary = lv.boundary.p; D.nboundary = (int)L.boundary.size();
-  D.segs = lv.segs.p; D.segidx = lv.segidx.p;
-  D.blocks_all = lv.blocks_all.p; D.nblocks_all = (int)L.blocks_all.size();
-  D.blocks_colour = lv.blocks_colour.p;
-  D.rows_all = lv.rows_all.p;
-  D.rows_colour = lv.rows_colour.p;
-  D.colour_off_dev = lv.colour_off.p;
 
   lv.rhs.alloc(L.N);
-  lv.v64.val.alloc_zeroed(L.nvals, st);
+  lv.v64.val.alloc_zeroed(L.nstored, st);
   for (auto *b : {&lv.v64.x, &lv.v64.f, &lv.v64.d, &lv.v64.aux}) b->alloc(L.N);
 }
 
@@ -409,14 +330,14 @@ static void coarse_inverse(System &Y, Level &lv) {
   // the inverse of the values it was built from is still valid when the
   // coarsest operator has not changed bit for bit (time steps with
   // time-independent coefficients re-assemble the same matrix)
-  const int64_t nv = lv.L.nvals;
+  const int64_t nv = lv.L.nstored;
   lv.flag.alloc(1);
   if (lv.ainv_n == nI && lv.ainv_src.p && bits_equal(lv.v64.val.p, lv.ainv_src.p, nv, lv.flag.p, st)) return;
   lv.aug.alloc((size_t)nI * (nI + N));
   lv.piv.alloc(nI);
   lv.ainv.alloc((size_t)nI * N);
   lv.ainv_n = 0;
-  coarse_inverse_dense(lv.D, lv.v64.val.p, lv.cidx.p, nI, lv.aug.p, lv.piv.p, lv.ainv.p, st);
+  coarse_inverse_dense(lv.D, lv.v64.val.p, lv.iidx.p, lv.cidx.p, nI, lv.aug.p, lv.piv.p, lv.ainv.p, st);
   lv.ainv_src.alloc(nv);
   copy<double>(lv.ainv_src.p, lv.v64.val.p, nv, st);
   check(hipStreamSynchronize(st), "coarse inverse");
@@ -436,13 +357,13 @@ static void ensure_val32(System &Y) {
     if (lv.have_val32) continue;
     if (!lv.v32.val.p) {
       Y.invalidate_graphs();
-      lv.v32.val.alloc(lv.L.nvals);
+      lv.v32.val.alloc(lv.L.nstored);
       for (auto *b : {&lv.v32.x, &lv.v32.f, &lv.v32.d, &lv.v32.aux}) b->alloc(lv.L.N);
       // the defect's Dirichlet entries are read by the learned step with zero
       // weights only (dinv and A c vanish there), so they just have to be finite
       fill<float>(lv.v32.d.p, 0.0f, lv.L.N, Y.ctx->st);
     }
-    convert<float, double>(lv.v32.val.p, lv.v64.val.p, lv.L.nvals, Y.ctx->st);
+    convert<float, double>(lv.v32.val.p, lv.v64.val.p, lv.L.nstored, Y.ctx->st);
     lv.have_val32 = true;
   }
 }
@@ -455,7 +376,7 @@ static void ensure_val16(System &Y) {
     if (lv.have_val16) continue;
     if (!lv.val16.p) {
       Y.invalidate_graphs();
-      lv.val16.alloc(lv.L.nvals);
+      lv.val16.alloc(lv.L.nstored);  // (scaled_values writes every entry)
       lv.sdinv.alloc(lv.L.N);
       fill<float>(lv.sdinv.p, 0.0f, lv.L.N, Y.ctx->st);
     }
@@ -500,34 +421,29 @@ static void level_smooth(System &Y, Level &lv, int kind, double omega, int sweep
   // through the one CU and is slower there than launch per colour
   const int64_t wg_default = sizeof(T) == 4 ? kSweepWgRows : 0;
   const int64_t wg_limit = Y.opt[21] == 0 ? wg_default : (int64_t)Y.opt[21];
-  for (int s = 0; s < sweeps; s++) {
-    if (kind == 1) {
+  if (kind == 1) {
+    for (int s = 0; s < sweeps; s++) {
       copy<T>(v.aux.p, v.x.p, lv.L.N, st);
       boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
-      css_apply<T>(lv.D, 2, v.val.p, v.aux.p, v.f.p, v.x.p, omega, -1, st);
-    } else if (lv.D.max_colour_rows <= wg_limit && sweep_wg_fits(lv.D, sizeof(T))) {
-      sweep_wg<T>(lv.D, v.val.p, v.x.p, v.f.p, omega, kind == 3 ? 1 : 0, st);
-    } else {
-      // with omega = 1 a colour right after itself (the turn of an SSOR sweep,
-      // the start of the next one) reproduces its rows bit for bit and is skipped
-      const bool skip = kind == 3 && omega == 1.0;
-      // Dirichlet rows x = f (no sweep changes them afterwards)
-      if (s == 0) boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
-      auto colour = [&](int c) {
-        if constexpr (std::is_same<T, float>::value) {
-          if (Y.half_smoother) {
-            if (!lv.have_val16) throw std::logic_error("level_smooth: FP16 smoother values missing");
-            css_sor_scaled(lv.D, lv.val16.p, lv.sdinv.p, v.x.p, v.f.p, omega, c, st);
-            return;
-          }
-        }
-        css_apply<T>(lv.D, 3, v.val.p, v.x.p, v.f.p, v.x.p, omega, c, st);
-      };
-      for (int c = (skip && s > 0) ? 1 : 0; c < lv.L.ncolours; c++) colour(c);
-      if (kind == 3)
-        for (int c = lv.L.ncolours - (skip ? 2 : 1); c >= 0; c--) colour(c);
+      rows_apply<T>(lv.D, 2, v.val.p, v.aux.p, v.f.p, v.x.p, omega, st);
+    }
+    return;
+  }
+  if (sweeps < 1) return;
+  if (lv.D.max_colour_rows <= wg_limit && sweep_wg_fits(lv.D, sizeof(T))) {
+    for (int s = 0; s < sweeps; s++) sweep_wg<T>(lv.D, v.val.p, v.x.p, v.f.p, omega, kind == 3 ? 1 : 0, st);
+    return;
+  }
+  // Dirichlet rows x = f (no sweep changes them afterwards)
+  boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
+  if constexpr (std::is_same<T, float>::value) {
+    if (Y.half_smoother) {
+      if (!lv.have_val16) throw std::logic_error("level_smooth: FP16 smoother values missing");
+      sor_sweeps_scaled(lv.D, lv.val16.p, lv.sdinv.p, v.x.p, v.f.p, omega, kind == 3, sweeps, st);
+      return;
     }
   }
+  sor_sweeps<T>(lv.D, v.val.p, v.x.p, v.f.p, omega, kind == 3, sweeps, st);
 }
 // Learned post-smoothing of one level (replaces the post-sweeps of
 // TMGLevel3D; no counterpart in the reference): with d = f - A x and
@@ -548,7 +464,7 @@ static void learned_post(System &Y, Level &lv, LearnedNet &net, bool fresh = tru
   if (fresh && !x_zero) {
     // defect of the interior rows; its Dirichlet entries meet zero weights
     // below (dinv = 0 there, A c = 0 there) and are finite (zero or f - x)
-    css_apply<float>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, -1, st);
+    rows_apply<float>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, st);
   }
   // the network's first layer builds its input from the features, u = D^-1 d
   // and the partials of ||u||^2
@@ -561,7 +477,7 @@ static void learned_post(System &Y, Level &lv, LearnedNet &net, bool fresh = tru
     in.part = part + 2 * kRedBlocks;
   }
   net_forward_correction(net, lv.L.M, sc, sq, lv.lc.p, st, &in);
-  css_apply<float>(lv.D, 0, v.val.p, lv.lc.p, nullptr, lv.lac.p, 0.0, -1, st);  // Dirichlet entries stay 0
+  rows_apply<float>(lv.D, 0, v.val.p, lv.lc.p, nullptr, lv.lac.p, 0.0, st);  // Dirichlet entries stay 0
   if (carry)
     learned_update_carry(d0, v.d.p, lv.lac.p, lv.lc.p, v.x.p, lv.dinv.p, lv.lc.p, N, part, part + 2 * kRedBlocks,
                          st);
@@ -601,7 +517,7 @@ static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
     } else if (cs >= 1 && cs <= 3 && sweep_wg_fits(lv.D, sizeof(T))) {
       // sweeps until the defect is reduced by SC_COARSE_RED_FACTOR_SCALAR
       // (opt[11]) or SC_COARSE_MAXIT_SCALAR (opt[10]) sweeps were made
-      coarse_wg<T>(lv.D, v.val.p, v.x.p, v.f.p, o[8], cs, std::max(1, (int)o[10]), o[11], v.d.p, v.aux.p, st);
+      coarse_wg<T>(lv.D, v.val.p, v.x.p, v.f.p, o[8], cs, std::max(1, (int)o[10]), o[11], v.aux.p, st);
     } else {
       level_smooth<T>(Y, lv, cs == 17 ? 3 : cs, o[8], std::max(1, (int)o[10]));
     }
@@ -616,7 +532,7 @@ static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
   if (slc) {
     if (!v.sold.p || !v.sdef.p) throw std::logic_error("step length control buffers missing");
     copy<T>(v.sold.p, v.x.p, lv.L.N, st);
-    css_apply<T>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.sdef.p, 0.0, -1, st);
+    rows_apply<T>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.sdef.p, 0.0, st);
     boundary<T>(lv.D, 1, v.sdef.p, v.x.p, v.f.p, st);
   }
   bool pre_done = false;
@@ -629,7 +545,7 @@ static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
   }
   if (!pre_done) {
     level_smooth<T>(Y, lv, kind, o[8], (int)o[6]);
-    css_apply<T>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, -1, st);
+    rows_apply<T>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, st);
   }
   // the defect's Dirichlet entries are not set: the restriction to an
   // interior coarse node reads interior fine nodes only (taps 2y-3..2y+3 and
@@ -660,7 +576,7 @@ static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
     // e = u - uold, y = A e, omega = (def, y) / (y, y), u = uold + omega e
     double *num = Y.ctx->part.p + 3 * kRedBlocks + 16;
     axpy_diff<T>(v.aux.p, v.x.p, v.sold.p, lv.L.N, st);
-    css_apply<T>(lv.D, 0, v.val.p, v.aux.p, nullptr, v.d.p, 0.0, -1, st);
+    rows_apply<T>(lv.D, 0, v.val.p, v.aux.p, nullptr, v.d.p, 0.0, st);
     boundary<T>(lv.D, 0, v.d.p, v.aux.p, nullptr, st);
     dot<T>(v.sdef.p, v.d.p, lv.L.N, Y.ctx->part.p, num, 0, st);
     dot<T>(v.d.p, v.d.p, lv.L.N, Y.ctx->part.p, num + 1, 0, st);
@@ -738,7 +654,7 @@ static void fine_matvec(System &Y, const T *x, T *y) {
       return;
     }
   }
-  css_apply<T>(lv.D, 0, vecs<T>(lv).val.p, x, nullptr, y, 0.0, -1, Y.ctx->st);
+  rows_apply<T>(lv.D, 0, vecs<T>(lv).val.p, x, nullptr, y, 0.0, Y.ctx->st);
   boundary<T>(lv.D, 0, y, x, nullptr, Y.ctx->st);
 }
 template <typename T>
@@ -750,7 +666,7 @@ static void fine_defect(System &Y, const T *x, const T *b, T *r) {
       return;
     }
   }
-  css_apply<T>(lv.D, 1, vecs<T>(lv).val.p, x, b, r, 0.0, -1, Y.ctx->st);
+  rows_apply<T>(lv.D, 1, vecs<T>(lv).val.p, x, b, r, 0.0, Y.ctx->st);
   boundary<T>(lv.D, 1, r, x, b, Y.ctx->st);
 }
 
@@ -954,8 +870,8 @@ static int krylov(System &Y, T *x, const T *b, int maxit, double rmin, double re
 // the level's transposed FP32 values for learned_res_step (from the current
 // FP32 values; call after they change)
 static void learned_transpose(System &Y, Level &lv) {
-  lv.valT.alloc(lv.L.nvals);
-  css_transpose_values(lv.D, lv.v32.val.p, lv.valT.p, Y.ctx->st);
+  lv.valT.alloc(lv.L.nstored);
+  transpose_values(lv.D, lv.v32.val.p, lv.valT.p, Y.ctx->st);
 }
 static void learned_res_step(System &Y, Level &lv, LearnedNet &net, const float *u, float *loss_dev) {
   hipStream_t st = Y.ctx->st;
@@ -965,9 +881,9 @@ static void learned_res_step(System &Y, Level &lv, LearnedNet &net, const float 
   learned_build_input(net, u, nullptr, 1.0, lv.feat.p, lv.L.N, st);
   net_forward_act(net, M, true, st);
   learned_mask(net.out, M, lv.lc.p, st);
-  css_apply<float>(lv.D, 0, v.val.p, lv.lc.p, nullptr, lv.lac.p, 0.0, -1, st);  // Dirichlet entries stay 0
+  rows_apply<float>(lv.D, 0, v.val.p, lv.lc.p, nullptr, lv.lac.p, 0.0, st);  // Dirichlet entries stay 0
   learned_res_loss(net, M, u, lv.dinv.p, lv.lac.p, v.aux.p, st);
-  css_transpose(lv.D, lv.valT.p, v.aux.p, v.d.p, st);
+  transpose_apply(lv.D, lv.valT.p, v.aux.p, v.d.p, st);
   net_backward_from(net, M, v.d.p, st);
   learned_loss_sum(net, loss_dev, st);
 }
@@ -1045,7 +961,7 @@ static void learned_train(System &Y, const double *to, double *ti) {
         fill<float>(v.f.p, 0.0f, N, st);
       }
       mg_cycle<float>(Y, L - j, false);
-      css_apply<float>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, -1, st);
+      rows_apply<float>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, st);
       boundary<float>(lv.D, 1, v.d.p, v.x.p, v.f.p, st);
       learned_input(lv.dinv.p, v.d.p, lv.lc.p, N, st);
       dot<float>(lv.lc.p, lv.lc.p, N, Y.ctx->part.p, Y.lscal.p, 1, st);
@@ -1610,7 +1526,7 @@ static void system_assemble(System &Y, const double *prm, const HostCallbacks *c
       assemble(lv.D, Y.prm.p, Y.example, form, Y.qref.p, nq, Y.tab.p, Y.qpbuf.p, nullptr, nullptr, nullptr,
                lv.rhs.p, st, cb != nullptr, Y.qpbuf.p + Y.qp_tab_off, cell_corners(Y, lv));
     } else {
-      if (Y.two_matrices) lv.val2.alloc_zeroed(lv.L.nvals, st);
+      if (Y.two_matrices) lv.val2.alloc_zeroed(lv.L.nstored, st);
       assemble(lv.D, Y.prm.p, Y.example, form, Y.qref.p, nq, Y.tab.p, Y.qpbuf.p, cell_buffer(Y), lv.v64.val.p,
                Y.two_matrices ? lv.val2.p : nullptr, lv.rhs.p, st, cb != nullptr, Y.qpbuf.p + Y.qp_tab_off,
                cell_corners(Y, lv));
@@ -1687,9 +1603,9 @@ static void assemble_into(System &Y, const double *prm, bool mass) {
   const int nq = Y.nq;
   for (auto &lp : Y.lev) {
     Level &lv = *lp;
-    if (mass) lv.mass.alloc_zeroed(lv.L.nvals, st);
-    else lv.stiff.alloc_zeroed(lv.L.nvals, st);
-    if (Y.two_matrices) lv.val2.alloc_zeroed(lv.L.nvals, st);
+    if (mass) lv.mass.alloc_zeroed(lv.L.nstored, st);
+    else lv.stiff.alloc_zeroed(lv.L.nstored, st);
+    if (Y.two_matrices) lv.val2.alloc_zeroed(lv.L.nstored, st);
     assemble(lv.D, Y.prm.p, Y.example, Y.form, Y.qref.p, nq, Y.tab.p, Y.qpbuf.p, cell_buffer(Y),
              mass ? lv.mass.p : lv.stiff.p, Y.two_matrices ? lv.val2.p : nullptr, lv.rhs.p, st, false,
              Y.qpbuf.p + Y.qp_tab_off, cell_corners(Y, lv));
@@ -1759,15 +1675,15 @@ static void tcd_systmat(System &Y) {
   Level &lv = *Y.lev.back();
   const int64_t N = lv.L.N;
   const bool supg = Y.two_matrices;
-  css_apply<double>(lv.D, 0, lv.mass.p, Y.oldsol.p, nullptr, Y.tmp1.p, 0.0, -1, st);
-  css_apply<double>(lv.D, 0, lv.stiff.p, Y.oldsol.p, nullptr, Y.tmp2.p, 0.0, -1, st);
-  if (supg) css_apply<double>(lv.D, 0, lv.val2.p, Y.oldsol.p, nullptr, Y.tmp3.p, 0.0, -1, st);
+  rows_apply<double>(lv.D, 0, lv.mass.p, Y.oldsol.p, nullptr, Y.tmp1.p, 0.0, st);
+  rows_apply<double>(lv.D, 0, lv.stiff.p, Y.oldsol.p, nullptr, Y.tmp2.p, 0.0, st);
+  if (supg) rows_apply<double>(lv.D, 0, lv.val2.p, Y.oldsol.p, nullptr, Y.tmp3.p, 0.0, st);
   tcd_rhs(lv.D, Y.oldrhs.p, lv.rhs.p, Y.tmp1.p, Y.tmp2.p, supg ? Y.tmp3.p : nullptr, tau * th3, tau * th4,
           tau * th2, Y.b.p, st);
   for (auto &lp : Y.lev) {
     Level &l = *lp;
     // the FP32 copy (once the FP32 forms have allocated it) in the same pass
-    system_matrix(l.v64.val.p, l.v32.val.p, l.mass.p, supg ? l.val2.p : nullptr, l.stiff.p, tau * th1, l.L.nvals,
+    system_matrix(l.v64.val.p, l.v32.val.p, l.mass.p, supg ? l.val2.p : nullptr, l.stiff.p, tau * th1, l.L.nstored,
                   st);
     l.have_val32 = l.v32.val.p != nullptr;
     l.have_val16 = false;
@@ -1840,15 +1756,15 @@ int pmx_matrix_entries(pmx_system *sys, int level, int which, double *entries) {
     out.alloc(csr_nnz(lv.L));
     if (which == 4) {
       ensure_val32(Y);
-      css_to_csr<float>(lv.D, lv.rowptr.p, lv.kcol.p, lv.dof2lat.p, lv.L.nactive, lv.v32.val.p, out.p, Y.ctx->st);
+      values_to_csr<float>(lv.D, lv.rowptr.p, lv.kcol.p, lv.dof2lat.p, lv.L.nactive, lv.v32.val.p, out.p, Y.ctx->st);
     } else if (which == 5) {
       ensure_val16(Y);
-      css_to_csr<_Float16>(lv.D, lv.rowptr.p, lv.kcol.p, lv.dof2lat.p, lv.L.nactive, lv.val16.p, out.p,
+      values_to_csr<_Float16>(lv.D, lv.rowptr.p, lv.kcol.p, lv.dof2lat.p, lv.L.nactive, lv.val16.p, out.p,
                            Y.ctx->st);
     } else {
       const double *src = which == 0 ? lv.v64.val.p : which == 1 ? lv.val2.p : which == 2 ? lv.mass.p : lv.stiff.p;
       if (!src) throw std::logic_error("that matrix has not been assembled");
-      css_to_csr<double>(lv.D, lv.rowptr.p, lv.kcol.p, lv.dof2lat.p, lv.L.nactive, src, out.p, Y.ctx->st);
+      values_to_csr<double>(lv.D, lv.rowptr.p, lv.kcol.p, lv.dof2lat.p, lv.L.nactive, src, out.p, Y.ctx->st);
     }
     check(hipMemcpyAsync(entries, out.p, sizeof(double) * out.n, hipMemcpyDeviceToHost, Y.ctx->st), "d2h");
     check(hipStreamSynchronize(Y.ctx->st), "sync");
@@ -1874,7 +1790,7 @@ int pmx_level_set_entries(pmx_system *sys, int level, int n, const int *rowptr, 
     hipStream_t st = Y.ctx->st;
     DevBuf<double> in;
     in.upload(entries, lv.Nb.kcol.size(), st);
-    csr_to_css(lv.D, lv.rowptr.p, lv.kcol.p, lv.dof2lat.p, lv.L.nactive, in.p, lv.v64.val.p, st);
+    csr_to_values(lv.D, lv.rowptr.p, lv.kcol.p, lv.dof2lat.p, lv.L.nactive, in.p, lv.v64.val.p, st);
     lv.have_val32 = false;
     lv.have_val16 = false;
     lv.have_dinv = false;
@@ -1898,13 +1814,13 @@ int pmx_matvec(pmx_system *sys, int level, int precision, const double *x, doubl
     hipStream_t st = Y.ctx->st;
     if (precision == 0) {
       to_lattice<double>(Y, lv, x, lv.v64.aux.p);
-      css_apply<double>(lv.D, 0, lv.v64.val.p, lv.v64.aux.p, nullptr, lv.v64.d.p, 0.0, -1, st);
+      rows_apply<double>(lv.D, 0, lv.v64.val.p, lv.v64.aux.p, nullptr, lv.v64.d.p, 0.0, st);
       boundary<double>(lv.D, 0, lv.v64.d.p, lv.v64.aux.p, nullptr, st);
       from_lattice<double>(Y, lv, lv.v64.d.p, y);
     } else {
       ensure_val32(Y);
       to_lattice<float>(Y, lv, x, lv.v32.aux.p);
-      css_apply<float>(lv.D, 0, lv.v32.val.p, lv.v32.aux.p, nullptr, lv.v32.d.p, 0.0, -1, st);
+      rows_apply<float>(lv.D, 0, lv.v32.val.p, lv.v32.aux.p, nullptr, lv.v32.d.p, 0.0, st);
       boundary<float>(lv.D, 0, lv.v32.d.p, lv.v32.aux.p, nullptr, st);
       from_lattice<float>(Y, lv, lv.v32.d.p, y);
     }
@@ -1918,7 +1834,7 @@ int pmx_defect(pmx_system *sys, int level, const double *x, const double *b, dou
     hipStream_t st = Y.ctx->st;
     to_lattice<double>(Y, lv, x, lv.v64.aux.p);
     to_lattice<double>(Y, lv, b, lv.v64.f.p);
-    css_apply<double>(lv.D, 1, lv.v64.val.p, lv.v64.aux.p, lv.v64.f.p, lv.v64.d.p, 0.0, -1, st);
+    rows_apply<double>(lv.D, 1, lv.v64.val.p, lv.v64.aux.p, lv.v64.f.p, lv.v64.d.p, 0.0, st);
     boundary<double>(lv.D, 1, lv.v64.d.p, lv.v64.aux.p, lv.v64.f.p, st);
     double *nr = Y.ctx->part.p + 3 * kRedBlocks;
     dot<double>(lv.v64.d.p, lv.v64.d.p, lv.L.N, Y.ctx->part.p, nr, 1, st);
@@ -1936,7 +1852,7 @@ int pmx_defect_noalloc(pmx_system *sys, int level, const double *x, const double
       throw std::invalid_argument("pmx_defect_noalloc: the level has more than 8,388,608 rows (the scratch limit)");
     double *part = noalloc_scratch(*Y.ctx);
     hipStream_t st = Y.ctx->st;
-    css_apply<double>(lv.D, 1, lv.v64.val.p, x, b, r, 0.0, -1, st);
+    rows_apply<double>(lv.D, 1, lv.v64.val.p, x, b, r, 0.0, st);
     boundary<double>(lv.D, 1, r, x, b, st);
     dot_chunked(r, r, lv.L.N, part, res, 1, st);
     check(hipGetLastError(), "pmx_defect_noalloc launch");
@@ -2127,8 +2043,8 @@ int pmx_time_kernel(pmx_system *sys, int kernel, int level, int precision, int r
       if (precision == 0) {
         Vecs<double> &v = lv.v64;
         switch (kernel) {
-          case 0: css_apply<double>(lv.D, 0, v.val.p, v.x.p, nullptr, v.d.p, 0.0, -1, st); break;
-          case 1: css_apply<double>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, -1, st); break;
+          case 0: rows_apply<double>(lv.D, 0, v.val.p, v.x.p, nullptr, v.d.p, 0.0, st); break;
+          case 1: rows_apply<double>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, st); break;
           case 2: level_smooth<double>(Y, lv, 1, 0.8, 1); break;
           case 3: level_smooth<double>(Y, lv, 3, 1.0, 1); break;
           case 4: assemble(lv.D, Y.prm.p, Y.example, Y.form, Y.qref.p, Y.nq, Y.tab.p, Y.qpbuf.p, cell_buffer(Y), v.val.p, Y.two_matrices ? lv.val2.p : nullptr, lv.rhs.p, st, false, Y.qpbuf.p + Y.qp_tab_off, cell_corners(Y, lv)); break;
@@ -2140,8 +2056,8 @@ int pmx_time_kernel(pmx_system *sys, int kernel, int level, int precision, int r
       } else {
         Vecs<float> &v = lv.v32;
         switch (kernel) {
-          case 0: css_apply<float>(lv.D, 0, v.val.p, v.x.p, nullptr, v.d.p, 0.0, -1, st); break;
-          case 1: css_apply<float>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, -1, st); break;
+          case 0: rows_apply<float>(lv.D, 0, v.val.p, v.x.p, nullptr, v.d.p, 0.0, st); break;
+          case 1: rows_apply<float>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, st); break;
           case 2: level_smooth<float>(Y, lv, 1, 0.8, 1); break;
           case 3: level_smooth<float>(Y, lv, 3, 1.0, 1); break;
           case 5: if (li > 0) prolongate<float>(Y.lev[li - 1]->D, lv.D, Y.lev[li - 1]->v32.x.p, v.aux.p, st); break;
@@ -2155,15 +2071,15 @@ int pmx_time_kernel(pmx_system *sys, int kernel, int level, int precision, int r
     };
     if (kernel == 10 || kernel == 11) {
       // durations of the individual dispatches (not the gaps between them):
-      // 10 the colour launches of SSOR sweeps (launch per colour forced), 11 SpMV
+      // 10 the group launches of SSOR sweeps (launches forced), 11 SpMV
       Y.opt[21] = -1;
       auto run = [&]() {
         if (kernel == 10) {
           if (precision) level_smooth<float>(Y, lv, 3, 1.0, 1);
           else level_smooth<double>(Y, lv, 3, 1.0, 1);
         } else {
-          if (precision) css_apply<float>(lv.D, 0, lv.v32.val.p, lv.v32.x.p, nullptr, lv.v32.d.p, 0.0, -1, st);
-          else css_apply<double>(lv.D, 0, lv.v64.val.p, lv.v64.x.p, nullptr, lv.v64.d.p, 0.0, -1, st);
+          if (precision) rows_apply<float>(lv.D, 0, lv.v32.val.p, lv.v32.x.p, nullptr, lv.v32.d.p, 0.0, st);
+          else rows_apply<double>(lv.D, 0, lv.v64.val.p, lv.v64.x.p, nullptr, lv.v64.d.p, 0.0, st);
         }
       };
       run();
@@ -2184,24 +2100,19 @@ int pmx_time_kernel(pmx_system *sys, int kernel, int level, int precision, int r
     }
     if (kernel == 12 || kernel == 13) {
       // calibration of kind 10 on the same level: 12 a dispatch that does
-      // nothing with the workgroup count of each colour launch; 13 a plain
-      // streaming read of each colour's stored values (FP64, FP32 or the FP16
-      // smoother values), one dispatch per colour; average per dispatch
-      std::vector<int64_t> lo(lv.L.ncolours, -1), hi(lv.L.ncolours, 0);
-      for (const Segment &g : lv.L.segs) {
-        const int64_t len = (g.count + kSlice - 1) / kSlice * kSlice * g.ns;
-        if (lo[g.colour] < 0 || g.voff < lo[g.colour]) lo[g.colour] = g.voff;
-        hi[g.colour] = std::max(hi[g.colour], g.voff + len);
-      }
+      // nothing with the workgroup count of each group launch; 13 a plain
+      // streaming read of a group's share of the stored values (FP64, FP32 or
+      // the FP16 smoother values), one dispatch per group; average per dispatch
+      const int groups = lv.D.order == 2 ? 9 : 4;
       const size_t es = Y.half_smoother ? 2 : (precision ? 4 : 8);
       const char *base = Y.half_smoother ? (const char *)lv.val16.p
                                          : (precision ? (const char *)lv.v32.val.p : (const char *)lv.v64.val.p);
       float *sink = lv.v32.aux.p ? lv.v32.aux.p : (float *)lv.v64.aux.p;
+      const int64_t share = (int64_t)lv.L.nstored * (int64_t)es / groups / 16 * 16;
       auto run = [&]() {
-        for (int c = 0; c < lv.L.ncolours; c++) {
-          if (lo[c] < 0) continue;
-          if (kernel == 12) empty_dispatch(lv.D.colour_off[c + 1] - lv.D.colour_off[c], st);
-          else stream_read(base + lo[c] * es, (hi[c] - lo[c]) * (int64_t)es, sink, st);
+        for (int c = 0; c < groups; c++) {
+          if (kernel == 12) empty_dispatch(lv.D, c, st);
+          else stream_read(base + c * share, share, sink, st);
         }
       };
       run();

@@ -7,18 +7,26 @@
 // (ConstructSpace) is only used at the boundary: `lat2dof`/`dof2lat` permute
 // between the two.
 //
-// Operators are stored "colour-sliced stencil" (CSS): the active (interior)
-// lattice nodes are split into residue classes modulo S (S = 2 for Q1, 6 for
-// Q2).  A class has one smoother colour (coordinates mod 2 resp. mod 3) and
-// one stencil shape (Q2: extent 2 along an even coordinate, 1 along an odd
-// one), so a class is a strided sub-lattice whose rows all have the same
-// column offsets.  Inside a class the rows are cut into slices of 16 and a
-// slice stores its values slot-major:
-//   val[seg.voff + (idx/16)*(16*ns) + slot*16 + idx%16]
-// so the wavefront that owns 16 rows with 4 lanes per row reads 4
-// consecutive slots of 16 rows = 256 contiguous bytes (FP32) per load, and no
-// column indices are stored.  Dirichlet rows (lattice boundary) are identity
-// and not stored.
+// Operators are stored in the "line layout".  Interior rows are paired along x
+// (rows 2m + 1 and 2m + 2, m < P = (M - 1) / 2: an odd and an even node; the
+// last even one is the boundary node x = M - 1, whose values are zero), and a
+// pair's entries are grouped by the lattice line (y + dy, z + dz) of their
+// columns.  A line (y, z) stores its groups one after another, a group holds
+// VL = 3 + (2 order + 1) slots (the odd row's 3 entries, dx = -1 .. 1, then
+// the even row's, dx = -order .. order), and slot s of pair m is at
+//   val[((group_base(P, y, z) + k) * VL + s) * P + m]
+// so that every load of the P lanes of a line is contiguous and no column
+// index is stored.  A group's run of x values (5 for Q2, 4 for Q1) serves both
+// rows of the pair.  The groups of a line whose own lines come before it in
+// the sweep order are stored first (k < nlo), then the line itself, then the
+// others, so a half sweep streams one contiguous part of each line.
+//
+// Sweep order.  The multicolour smoother takes the colours of (x, y, z) mod C
+// (C = 2 for Q1, 3 for Q2) with x fastest.  Lines with equal (y mod C, z mod C)
+// do not couple, so all of them are swept in one launch, each by its own
+// workgroup, which takes the x colours of its line one after another: C^2
+// launches for the C^3 colours, in the same order of updates.
+// Dirichlet rows (lattice boundary) are identity and not stored.
 #pragma once
 #include <cstdint>
 #include <string>
@@ -27,50 +35,60 @@
 namespace pmx {
 
 constexpr int kBlock = 256;       // threads per workgroup of the operator kernels
-constexpr int kRowsPerBlock = 64; // rows per entry of the block tables (and per row-kernel workgroup)
-// workgroup of the single-workgroup sweep: FP64 rows need twice the
-// registers for their loads in flight, so half the lanes
-template <typename T> constexpr int sweep_threads() { return sizeof(T) == 8 ? 512 : 1024; }
-constexpr int kMaxSegs = 216;        // residue classes of a level: at most 6^3
-constexpr int kMaxColours = 27;
+constexpr int kRowsPerBlock = 64; // rows per workgroup of the one-thread-per-row kernels
 constexpr int64_t kSweepLdsBytes = 48 * 1024;  // largest x staged in LDS by the single-workgroup sweep
 constexpr int kSweepWgRows = 512;    // default: single-workgroup sweep up to this many rows per colour
-#ifndef PMX_SLICE
-#define PMX_SLICE 16
-#endif
-constexpr int kSlice = PMX_SLICE;  // rows per value slice (see Layout)
+constexpr int kSplits = 4;           // partial sums of a row: group k belongs to partial k mod 4
 constexpr int kRedBlocks = 1024;  // partial sums of the deterministic reductions
 
+#if defined(__HIPCC__)
+#define PMX_HD __host__ __device__
+#else
+#define PMX_HD
+#endif
+
+// arithmetic of the line layout for order O (1: Q1, 2: Q2)
+template <int O> struct Lines {
+  static constexpr int C = O == 2 ? 3 : 2;       // colours per axis
+  static constexpr int S = O == 2 ? 6 : 2;       // period of the line structure (extent and colour)
+  static constexpr int VL = 3 + 2 * O + 1;       // slots of a row pair per group
+  static constexpr int kMaxGroups = O == 2 ? 25 : 9;
+  // half extent of the stencil along an axis at lattice coordinate t
+  PMX_HD static constexpr int ext(int t) { return O == 2 && (t & 1) == 0 ? 2 : 1; }
+  PMX_HD static constexpr int width(int t) { return 2 * ext(t) + 1; }
+  // sum of the widths of coordinates 1 .. t - 1
+  PMX_HD static constexpr int width_sum(int t) {
+    return O == 2 ? 8 * ((t - 1) >> 1) + (((t - 1) & 1) ? 3 : 0) : 3 * (t - 1);
+  }
+  PMX_HD static constexpr int width_total(int P) { return width_sum(2 * P); }
+  // groups stored before line (y, z)
+  PMX_HD static constexpr int64_t group_base(int P, int y, int z) {
+    return (int64_t)width_sum(z) * width_total(P) + width(z) * width_sum(y);
+  }
+  // slot of column offset dx in row x of a pair
+  PMX_HD static constexpr int slot(int x, int dx) { return (x & 1) ? dx + 1 : 3 + dx + O; }
+  PMX_HD static constexpr int64_t values(int P) {
+    return (int64_t)width_total(P) * width_total(P) * VL * P;
+  }
+};
+
+// the lines of a launch (see unit_lines in pmx_lines.hpp)
+struct LineSet {
+  int y0, ys, nc;  // y classes y0 + c ys, c < nc
+  int z0, zs;      // planes z0 + zs kz
+  int upz;         // units per plane
+};
+
+// residue class of interior nodes mod (2 for Q1, 6 for Q2): one smoother
+// colour and one stencil shape
 struct Segment {
-  int rx, ry, rz;     // residues mod S
+  int rx, ry, rz;     // residues
   int x0, y0, z0;     // first interior lattice coordinate of the class
   int cx, cy, cz;     // node counts per direction
   int ex, ey, ez;     // stencil half extents
   int colour;
-  int ns;             // slots = (2ex+1)(2ey+1)(2ez+1)
-  int dslot;          // slot of offset (0,0,0)
+  int ns;             // entries per row (2ex+1)(2ey+1)(2ez+1)
   int64_t count;      // cx*cy*cz
-  int64_t voff;       // offset of the class in the value array
-};
-
-// device-side copy of a segment (plain struct, kernel argument via array)
-struct DevSegment {
-  int x0, y0, z0, cx, cy, cz;
-  int ex, ey, ez, ns, dslot, stride;
-  int64_t count, voff;
-};
-
-// one entry per launched block: which segment and the first node index
-struct BlockInfo {
-  int seg;
-  int base;
-};
-
-// a block entry of the row kernels with its class record inline, so that a
-// workgroup finds its rows with one load instead of two dependent ones
-struct RowBlock {
-  DevSegment s;
-  int base, pad;
 };
 
 struct Layout {
@@ -79,10 +97,11 @@ struct Layout {
   int64_t nactive = 0;      // interior nodes
   int ncolours = 8;
   std::vector<Segment> segs;
-  int64_t nvals = 0;        // total stored stencil values
-  // block tables: all segments (spmv) and per colour (smoothers)
-  std::vector<BlockInfo> blocks_all;
-  std::vector<std::vector<BlockInfo>> blocks_colour;
+  // entries of the interior rows with the rows of each class rounded up to a
+  // multiple of 16 (reported by pmx_system_dims)
+  int64_t nvals = 0;
+  int64_t nstored = 0;      // values of the line layout
+  int64_t max_colour_rows = 0;
   std::vector<int> boundary;  // lattice indices of Dirichlet nodes
 };
 

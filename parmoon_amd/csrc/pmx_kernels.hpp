@@ -1,10 +1,6 @@
 // pmx_kernels.hpp -- HIP kernels of libpmx (gfx950).
 //
-// All operator kernels work on lattice-ordered vectors and the colour-sliced
-// stencil (CSS) value layout described in pmx_internal.hpp.  One thread owns
-// one lattice node; a wavefront covers 64 consecutive nodes of one residue
-// class, so stencil values are read fully coalesced and every wavefront
-// follows the same stencil shape (no divergence).
+// Vectors are lattice ordered; the matrix kernels are in pmx_lines.hip.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -14,31 +10,6 @@
 
 namespace pmx {
 
-
-// MI355X dispatches consecutive workgroups round-robin over its 8 XCDs.  Remap
-// so that each XCD works on one contiguous slice of the block table: the
-// neighbouring nodes whose x values a block gathers then stay in that XCD's L2.
-__device__ __forceinline__ int xcd_remap(int bid, int G) {
-  const int X = 8;
-  const int q = G / X, r = G % X, xcd = bid % X, k = bid / X;
-  return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + k;
-}
-
-// first value of row idx of a class (slot stride kSlice)
-__device__ __forceinline__ int64_t vbase(const DevSegment &s, int idx) {
-  return s.voff + (int64_t)(idx / kSlice) * ((int64_t)s.ns * kSlice) + (idx % kSlice);
-}
-// The row-scaled FP16 smoother values are stored with the slots of a row in
-// groups of eight: inside a slice of kSlice rows, group o holds, row by row,
-// the row's slots 8o .. 8o+7 (16 contiguous bytes per row, a last group of
-// ns mod 8 slots likewise), so a row's values arrive in 16-byte loads.  The
-// slice sizes are those of the FP32 values.
-__device__ __forceinline__ int64_t v16slice(const DevSegment &s, int idx) {
-  return s.voff + (int64_t)(idx / kSlice) * ((int64_t)s.ns * kSlice);
-}
-__host__ __device__ constexpr int v16off(int ns, int r, int slot) {
-  return (slot >> 3) * 8 * kSlice + r * ((slot >> 3) < (ns >> 3) ? 8 : (ns & 7)) + (slot & 7);
-}
 
 // ---------------------------------------------------------------- BLAS-1
 template <typename T>

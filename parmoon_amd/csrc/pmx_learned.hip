@@ -16,6 +16,7 @@
 
 #include "pmx_kernels.hpp"
 #include "pmx_learned.hpp"
+#include "pmx_lines.hpp"
 #include "pmx_ops.hpp"
 
 namespace pmx {
@@ -692,16 +693,13 @@ void net_adam(LearnedNet &net, float lr, hipStream_t st, float gscale) {
 }
 
 // ------------------------------------------------------------------ use as a smoother
-__global__ void k_diag_inv(const BlockInfo *__restrict__ blocks, const DevSegment *__restrict__ segs, int M,
-                           const float *__restrict__ val, float *__restrict__ dinv) {
-  const BlockInfo bi = blocks[blockIdx.x];
-  const DevSegment s = segs[bi.seg];
-  const int idx = bi.base + threadIdx.x;
-  if (idx >= s.count) return;
-  const int i = idx % s.cx, t = idx / s.cx, j = t % s.cy, k = t / s.cy;
-  const int p = (s.x0 + s.stride * i) + M * ((s.y0 + s.stride * j) + M * (s.z0 + s.stride * k));
-  const int64_t vb = s.voff + (int64_t)(idx / kSlice) * ((int64_t)s.ns * kSlice) + (idx % kSlice);
-  dinv[p] = 1.0f / val[vb + (int64_t)s.dslot * kSlice];
+// (one thread per interior row: blockIdx.y = z - 1, blockIdx.x covers a plane)
+template <int O>
+__global__ void k_diag_inv(int M, const float *__restrict__ val, float *__restrict__ dinv) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, m2 = M - 2;
+  if (t >= m2 * m2) return;
+  const int x = 1 + t % m2, y = 1 + t / m2, z = 1 + blockIdx.y;
+  dinv[x + (int64_t)M * (y + (int64_t)M * z)] = 1.0f / val[value_index<O>((M - 1) / 2, x, y, z, 0, 0, 0)];
 }
 __global__ void k_learned_input(const float *__restrict__ dinv, const float *__restrict__ d, float *__restrict__ u,
                                 int64_t n) {
@@ -757,27 +755,23 @@ __global__ void k_build_input(const float *__restrict__ u, const double *__restr
   }
 }
 // the six nearest couplings of every interior row, divided by its diagonal
-__global__ void k_features(const BlockInfo *__restrict__ blocks, const DevSegment *__restrict__ segs, int M,
-                           const float *__restrict__ val, uint16_t *__restrict__ feat) {
-  const BlockInfo bi = blocks[blockIdx.x];
-  const DevSegment s = segs[bi.seg];
-  const int idx = bi.base + threadIdx.x;
-  if (idx >= s.count) return;
-  const int i = idx % s.cx, t = idx / s.cx, j = t % s.cy, k = t / s.cy;
-  const int64_t p = (s.x0 + s.stride * i) + (int64_t)M * ((s.y0 + s.stride * j) + (int64_t)M * (s.z0 + s.stride * k));
-  const int64_t vb = s.voff + (int64_t)(idx / kSlice) * ((int64_t)s.ns * kSlice) + (idx % kSlice);
-  const int wx = 2 * s.ex + 1, wy = 2 * s.ey + 1;
-  auto slot = [&](int dx, int dy, int dz) { return (dx + s.ex) + wx * ((dy + s.ey) + wy * (dz + s.ez)); };
-  const float dinv = 1.0f / val[vb + (int64_t)s.dslot * kSlice];
+template <int O>
+__global__ void k_features(int M, const float *__restrict__ val, uint16_t *__restrict__ feat) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, m2 = M - 2, P = (M - 1) / 2;
+  if (t >= m2 * m2) return;
+  const int x = 1 + t % m2, y = 1 + t / m2, z = 1 + blockIdx.y;
+  const int64_t p = x + (int64_t)M * (y + (int64_t)M * z);
+  auto a = [&](int dx, int dy, int dz) { return val[value_index<O>(P, x, y, z, dx, dy, dz)]; };
+  const float dinv = 1.0f / a(0, 0, 0);
   const int off[6][3] = {{1, 0, 0}, {-1, 0, 0}, {0, 1, 0}, {0, -1, 0}, {0, 0, 1}, {0, 0, -1}};
-  const int ext[3] = {s.ex, s.ey, s.ez};
+  const int ext[3] = {Lines<O>::ext(x), Lines<O>::ext(y), Lines<O>::ext(z)};
   uint16_t f[16] = {0};
 #pragma unroll
   for (int q = 0; q < 6; q++) {
-    f[1 + q] = f2bf(val[vb + (int64_t)slot(off[q][0], off[q][1], off[q][2]) * kSlice] * dinv);
+    f[1 + q] = f2bf(a(off[q][0], off[q][1], off[q][2]) * dinv);
     const int axis = q >> 1;
     if (ext[axis] >= 2)
-      f[7 + q] = f2bf(val[vb + (int64_t)slot(2 * off[q][0], 2 * off[q][1], 2 * off[q][2]) * kSlice] * dinv);
+      f[7 + q] = f2bf(a(2 * off[q][0], 2 * off[q][1], 2 * off[q][2]) * dinv);
   }
   u16x8 v0, v1;
 #pragma unroll
@@ -865,10 +859,14 @@ __global__ void k_learned_random(float *__restrict__ xv, int M, uint32_t seed) {
 
 static unsigned grid_for(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 4096); }
 
+static dim3 interior_grid(int M) {
+  return dim3((unsigned)(((M - 2) * (M - 2) + kRowsPerBlock - 1) / kRowsPerBlock), (unsigned)(M - 2));
+}
 void learned_diag_inv(const DevLayout &D, const float *val, float *dinv, hipStream_t st) {
   fill<float>(dinv, 0.f, D.N, st);
-  hipLaunchKernelGGL(k_diag_inv, dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st, D.blocks_all, D.segs, D.M, val,
-                     dinv);
+  const dim3 g = interior_grid(D.M);
+  if (D.order == 2) hipLaunchKernelGGL(k_diag_inv<2>, g, dim3(kRowsPerBlock), 0, st, D.M, val, dinv);
+  else hipLaunchKernelGGL(k_diag_inv<1>, g, dim3(kRowsPerBlock), 0, st, D.M, val, dinv);
 }
 void learned_input(const float *dinv, const float *d, float *u, int64_t n, hipStream_t st) {
   hipLaunchKernelGGL(k_learned_input, dim3(grid_for(n)), dim3(256), 0, st, dinv, d, u, n);
@@ -900,8 +898,9 @@ void learned_build_input(LearnedNet &net, const float *u, const double *nrm, dou
 }
 void learned_features(const DevLayout &D, const float *val, uint16_t *feat, hipStream_t st) {
   fill<uint16_t>(feat, (uint16_t)0, D.N * kNetIn, st);
-  hipLaunchKernelGGL(k_features, dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st, D.blocks_all, D.segs, D.M, val,
-                     feat);
+  const dim3 g = interior_grid(D.M);
+  if (D.order == 2) hipLaunchKernelGGL(k_features<2>, g, dim3(kRowsPerBlock), 0, st, D.M, val, feat);
+  else hipLaunchKernelGGL(k_features<1>, g, dim3(kRowsPerBlock), 0, st, D.M, val, feat);
 }
 void learned_random(float *x, int M, uint32_t seed, hipStream_t st) {
   hipLaunchKernelGGL(k_learned_random, dim3(grid_for((int64_t)M * M * M)), dim3(256), 0, st, x, M, seed);
@@ -941,54 +940,33 @@ __global__ __launch_bounds__(256) void k_res_loss(int M, const float *__restrict
 }
 // y_j = sum over interior rows i of a_ij g_i, for interior j (0 on the boundary):
 // The transpose of the stored stencil operator restricted to interior rows,
-// stored in the same CSS layout: slot d of row j holds a_{j+d, j}, the entry
-// at offset -d of the interior row j + d (0 where j + d is not an interior
-// row or its stencil box lacks -d).  The FE pattern is structurally
-// symmetric, so every such entry has its slot in row j's box.  A workgroup
-// takes 64 rows j of one residue class, so the class of every neighbour row
-// j + d, its stencil shape, the slot of -d and the shift of the
-// class-lattice indices are the same across the workgroup (scalar work, S a
-// compile-time constant); per lane only the neighbour's row index and the
-// bounds remain.
-template <int E, int S>
-__global__ __launch_bounds__(kRowsPerBlock) void k_css_transpose_values(const BlockInfo *__restrict__ blocks,
-                                                                        const DevSegment *__restrict__ segs,
-                                                                        const int *__restrict__ segidx,
-                                                                        const float *__restrict__ val,
-                                                                        float *__restrict__ valT) {
-  const BlockInfo bi = blocks[blockIdx.x];
-  const DevSegment sj = segs[bi.seg];
-  const int idx = bi.base + threadIdx.x;
-  if (idx >= sj.count) return;
-  const int rx = sj.x0 % S, ry = sj.y0 % S, rz = sj.z0 % S;
-  const int i = idx % sj.cx, t = idx / sj.cx, j = t % sj.cy, k = t / sj.cy;
-  const int64_t vbj = sj.voff + (int64_t)(idx / kSlice) * ((int64_t)sj.ns * kSlice) + (idx % kSlice);
+// stored in the same layout: the entry of row j at offset d holds
+// a_{j+d, j}, the entry at offset -d of the interior row j + d (0 where j + d
+// is a Dirichlet node).  The FE pattern is structurally symmetric, so every
+// such entry has its slot in row j's box.  One thread per row pair of a line
+// and group, so that the stores are contiguous along the line.
+template <int O>
+__global__ __launch_bounds__(kBlock) void k_transpose_values(int lg, const float *__restrict__ val,
+                                                             float *__restrict__ valT) {
+  using L = Lines<O>;
+  const int P = 1 << lg, M = 2 * P + 1;
+  const int64_t id = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  const int m = (int)(id & (P - 1));
+  const int ln = (int)(id >> lg);
+  if (ln >= (M - 2) * (M - 2)) return;
+  const int y = 1 + ln % (M - 2), z = 1 + ln / (M - 2);
+  const GroupTable<O> &g = group_table<O>();
+  const int c = line_class<O>(y, z), k = blockIdx.y;
+  if (k >= g.ng[c]) return;
+  const int dy = (g.off[c][k] & 15) - 8, dz = (g.off[c][k] >> 4) - 8;
+  const bool in = y + dy > 0 && y + dy < M - 1 && z + dz > 0 && z + dz < M - 1;
+  float *o = valT + line_values<float, O>(P, L::group_base(P, y, z), m) + (int64_t)k * (L::VL * P);
 #pragma unroll
-  for (int dz = -E; dz <= E; dz++)
-#pragma unroll
-    for (int dy = -E; dy <= E; dy++)
-#pragma unroll
-      for (int dx = -E; dx <= E; dx++) {
-        if (dx < -sj.ex || dx > sj.ex || dy < -sj.ey || dy > sj.ey || dz < -sj.ez || dz > sj.ez) continue;
-        const int slot_j = (dx + sj.ex) + (2 * sj.ex + 1) * ((dy + sj.ey) + (2 * sj.ey + 1) * (dz + sj.ez));
-        float v = 0.f;
-        const int si = segidx[((rx + dx + S) % S) + S * (((ry + dy + S) % S) + S * ((rz + dz + S) % S))];
-        if (si >= 0) {
-          const DevSegment s = segs[si];
-          if (dx >= -s.ex && dx <= s.ex && dy >= -s.ey && dy <= s.ey && dz >= -s.ez && dz <= s.ez) {
-            const int slot = (-dx + s.ex) + (2 * s.ex + 1) * ((-dy + s.ey) + (2 * s.ey + 1) * (-dz + s.ez));
-            // class-lattice index of j + d in the neighbour's class (exact division)
-            const int ti = i + (sj.x0 + dx - s.x0) / S, tj = j + (sj.y0 + dy - s.y0) / S,
-                      tk = k + (sj.z0 + dz - s.z0) / S;
-            if (ti >= 0 && ti < s.cx && tj >= 0 && tj < s.cy && tk >= 0 && tk < s.cz) {
-              const int ri = ti + s.cx * (tj + s.cy * tk);
-              v = val[s.voff + (int64_t)(ri / kSlice) * ((int64_t)s.ns * kSlice) + (ri % kSlice) +
-                      (int64_t)slot * kSlice];
-            }
-          }
-        }
-        valT[vbj + (int64_t)slot_j * kSlice] = v;
-      }
+  for (int s = 0; s < L::VL; s++) {
+    const int x = s < 3 ? 2 * m + 1 : 2 * m + 2, dx = s < 3 ? s - 1 : s - 3 - O;
+    const bool use = in && x < M - 1 && x + dx > 0 && x + dx < M - 1;
+    o[s * P] = use ? val[value_index<O>(P, x + dx, y + dy, z + dz, -dx, -dy, -dz)] : 0.f;
+  }
 }
 
 void learned_mask(const float *in, int M, float *out, hipStream_t st) {
@@ -1003,17 +981,16 @@ void learned_res_loss(LearnedNet &net, int M, const float *u, const float *dinv,
 void learned_loss_sum(LearnedNet &net, float *loss_dev, hipStream_t st) {
   hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(kBlock), 0, st, net.lpart, kLossBlocks, loss_dev);
 }
-void css_transpose_values(const DevLayout &D, const float *val, float *valT, hipStream_t st) {
-  if (D.S != (D.order == 2 ? 6 : 2)) throw std::logic_error("css_transpose_values: unexpected residue modulus");
+void transpose_values(const DevLayout &D, const float *val, float *valT, hipStream_t st) {
+  const int64_t n = (int64_t)(D.M - 2) * (D.M - 2) << D.lg;
+  const unsigned g = (unsigned)((n + kBlock - 1) / kBlock);
   if (D.order == 2)
-    hipLaunchKernelGGL((k_css_transpose_values<2, 6>), dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st,
-                       D.blocks_all, D.segs, D.segidx, val, valT);
+    hipLaunchKernelGGL(k_transpose_values<2>, dim3(g, Lines<2>::kMaxGroups), dim3(kBlock), 0, st, D.lg, val, valT);
   else
-    hipLaunchKernelGGL((k_css_transpose_values<1, 2>), dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st,
-                       D.blocks_all, D.segs, D.segidx, val, valT);
+    hipLaunchKernelGGL(k_transpose_values<1>, dim3(g, Lines<1>::kMaxGroups), dim3(kBlock), 0, st, D.lg, val, valT);
 }
-void css_transpose(const DevLayout &D, const float *valT, const float *g, float *y, hipStream_t st) {
-  css_apply<float>(D, 0, valT, g, nullptr, y, 0.0, -1, st);
+void transpose_apply(const DevLayout &D, const float *valT, const float *g, float *y, hipStream_t st) {
+  rows_apply<float>(D, 0, valT, g, nullptr, y, 0.0, st);
   boundary<float>(D, 3, y, nullptr, nullptr, st);  // y = 0 on the boundary nodes
 }
 

@@ -43,7 +43,7 @@ int node_colour(const Layout &L, int x, int y, int z) {
   return (x % 2) + 2 * (y % 2) + 4 * (z % 2);
 }
 
-void build_layout(Layout &L, int nref, int order, int block) {
+void build_layout(Layout &L, int nref, int order, int) {
   if (order != 1 && order != 2) throw std::invalid_argument("order must be 1 or 2");
   if (nref < 1 || nref > 10) throw std::invalid_argument("nref out of range");
   L.nref = nref;
@@ -59,6 +59,7 @@ void build_layout(Layout &L, int nref, int order, int block) {
   const int S = L.S, M = L.M;
   auto first = [&](int r) { return r >= 1 ? r : S; };
   auto cnt = [&](int x0) { return x0 <= M - 2 ? (M - 2 - x0) / S + 1 : 0; };
+  std::vector<int64_t> rows(L.ncolours, 0);
   // classes ordered by colour, then by residue
   for (int col = 0; col < L.ncolours; col++)
     for (int rz = 0; rz < S; rz++)
@@ -80,20 +81,13 @@ void build_layout(Layout &L, int nref, int order, int block) {
           }
           s.colour = col;
           s.ns = (2 * s.ex + 1) * (2 * s.ey + 1) * (2 * s.ez + 1);
-          s.dslot = s.ex + (2 * s.ex + 1) * (s.ey + (2 * s.ey + 1) * s.ez);
-          s.voff = L.nvals;
-          L.nvals += ((s.count + kSlice - 1) / kSlice) * kSlice * s.ns;
+          L.nvals += (s.count + 15) / 16 * 16 * s.ns;
+          rows[col] += s.count;
           L.segs.push_back(s);
         }
-  L.blocks_all.clear();
-  L.blocks_colour.assign(L.ncolours, {});
-  for (int si = 0; si < (int)L.segs.size(); si++) {
-    const Segment &s = L.segs[si];
-    for (int64_t b = 0; b < s.count; b += block) {
-      L.blocks_all.push_back({si, (int)b});
-      L.blocks_colour[s.colour].push_back({si, (int)b});
-    }
-  }
+  L.max_colour_rows = *std::max_element(rows.begin(), rows.end());
+  const int P = (L.M - 1) / 2;
+  L.nstored = order == 2 ? Lines<2>::values(P) : Lines<1>::values(P);
   L.boundary.clear();
   for (int z = 0; z < M; z++)
     for (int y = 0; y < M; y++)

@@ -1,7 +1,6 @@
 // pmx_ops.hip -- operator, transfer, assembly and Krylov kernels (gfx950) and
 // their stream-ordered launchers.
 #include <hip/hip_runtime.h>
-#include <hip/hip_ext.h>
 
 #include <cmath>
 #include <cstdlib>
@@ -12,6 +11,7 @@
 
 #include "pmx_functors.hpp"
 #include "pmx_kernels.hpp"
+#include "pmx_lines.hpp"
 #include "pmx_ops.hpp"
 
 namespace pmx {
@@ -22,349 +22,6 @@ __global__ __launch_bounds__(kBlock) void k_reduce_final(const double *__restric
   for (int i = threadIdx.x; i < np; i += kBlock) s += part[i];
   s = block_sum<double>(s);
   if (threadIdx.x == 0) out[0] = do_sqrt ? sqrt(s) : s;
-}
-
-// ============================================================ stencil rows
-// One matrix row is handled by R lanes (R = row_lanes of the level): lane
-// `part` accumulates groups of slots part, part+R, ... and a shuffle
-// reduction combines them.  Modes:
-// 0: y = A x                          (MatVect, Blas2.C:86-118)
-// 1: y = f - A x                      (ScalarDefect, Blas2.C:37-83)
-// 2: y = (1-w) x + w (f - A_off x)/d  (TMGLevel3D::Jacobi, MGLevel3D.C:469-563), x = old iterate
-// 3: x = w ((f - A_off x)/d - x) + x  (TMGLevel3D::SOR, MGLevel3D.C:280-361) in place, one colour
-// 4: mode 3 on row-scaled values: val holds a_ij / a_ii (the diagonal slot
-//    unused), dinv the lattice vector 1 / a_ii: x = w (f dinv - W_off x - x) + x
-template <typename T> struct Acc { using type = T; };
-
-// W consecutive lattice values starting at q (the x-run of one (dy, dz) group
-// of a stencil row) in as few loads as the element alignment allows:
-// one 16-byte load plus one element for W = 5 floats, 8 + 4 bytes for W = 3.
-template <typename T, int W>
-__device__ __forceinline__ void load_run(const T *q, T (&r)[W]) {
-  if constexpr (sizeof(T) == 4 && W == 5) {
-    float4 a;
-    __builtin_memcpy(&a, q, 16);
-    r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w; r[4] = q[4];
-  } else if constexpr (sizeof(T) == 4 && W == 3) {
-    float2 a;
-    __builtin_memcpy(&a, q, 8);
-    r[0] = a.x; r[1] = a.y; r[2] = q[2];
-  } else if constexpr (sizeof(T) == 8 && W == 5) {
-    double2 a, b;
-    __builtin_memcpy(&a, q, 16);
-    __builtin_memcpy(&b, q + 2, 16);
-    r[0] = a.x; r[1] = a.y; r[2] = b.x; r[3] = b.y; r[4] = q[4];
-  } else if constexpr (sizeof(T) == 8 && W == 3) {
-    double2 a;
-    __builtin_memcpy(&a, q, 16);
-    r[0] = a.x; r[1] = a.y; r[2] = q[2];
-  } else {
-#pragma unroll
-    for (int k = 0; k < W; k++) r[k] = q[k];
-  }
-}
-
-// The slots of a row are grouped by (dy, dz); the WX slots of a group read
-// WX consecutive x values, fetched as one run (XL: x lives in LDS and is read
-// element by element).  Lane `part` of the R lanes takes groups part,
-// part+R, ...  The diagonal, f and the old x of the row are loaded up front
-// by all R lanes, so their latency overlaps the stencil loads.
-template <typename T, int EX, int EY, int EZ, int R, int MODE, bool XL = false, typename V = T>
-__device__ __forceinline__ void row_split(const DevSegment &s, int idx, int part, int M,
-                                          const V *__restrict__ val, const T *x, const T *__restrict__ f, T *y,
-                                          double omega, const float *__restrict__ dinv = nullptr) {
-  using A = typename Acc<T>::type;
-  constexpr int WX = 2 * EX + 1, WY = 2 * EY + 1, WZ = 2 * EZ + 1, NG = WY * WZ;
-  constexpr int DS = EX + WX * (EY + WY * EZ), DG = DS / WX;
-  const int i = idx % s.cx;
-  const int t = idx / s.cx;
-  const int j = t % s.cy, k = t / s.cy;
-  const int p = (s.x0 + s.stride * i) + M * ((s.y0 + s.stride * j) + M * (s.z0 + s.stride * k));
-  constexpr int NS = WX * WY * WZ;
-  // MODE 4: the FP16 values' slice and the row within it (v16off layout)
-  const V *v = MODE == 4 ? val + v16slice(s, idx) : val + vbase(s, idx);
-  const int rs = idx % kSlice;
-  A fp = 0, diag = 1, told = 0;
-  if constexpr (MODE >= 1) fp = (A)f[p];
-  if constexpr (MODE == 4) {
-    fp *= (A)dinv[p];
-    told = (A)x[p];
-  } else if constexpr (MODE >= 2) {
-    diag = (A)v[DS * kSlice];
-    told = (A)x[p];
-  }
-  // Loads and FMAs are unconditional (a lane past the last group re-reads the
-  // last group with zero weights, the diagonal gets a zero weight in the
-  // smoothers), so that a wavefront issues all loads before its first FMA
-  // instead of one round trip per group.
-  A acc = 0;
-#pragma unroll
-  for (int m = 0; m < (NG + R - 1) / R; m++) {
-    const int g0 = part + R * m;
-    const bool ok = g0 < NG;
-    const int g = ok ? g0 : NG - 1;
-    const int dy = g % WY - EY, dz = g / WY - EZ;
-    const T *q = x + (p - EX + M * (dy + M * dz));
-    T xr[WX];
-    V vr[WX];
-    if constexpr (XL) {
-#pragma unroll
-      for (int e = 0; e < WX; e++) xr[e] = q[e];
-    } else {
-      load_run<T, WX>(q, xr);
-    }
-#pragma unroll
-    for (int e = 0; e < WX; e++) {
-      if constexpr (MODE == 4) vr[e] = v[v16off(NS, rs, g * WX + e)];
-      else vr[e] = v[(g * WX + e) * kSlice];
-    }
-#pragma unroll
-    for (int e = 0; e < WX; e++) {
-      const bool use = ok && !(MODE >= 2 && e == EX && g == DG);
-      acc += (use ? (A)vr[e] : (A)0) * (A)xr[e];
-    }
-  }
-#pragma unroll
-  for (int o = R / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, R);
-  if (part != 0) return;
-  if (MODE == 0) y[p] = (T)acc;
-  else if (MODE == 1) y[p] = (T)(fp - acc);
-  else if (MODE == 2) y[p] = (T)((1 - (A)omega) * told + (A)omega * (fp - acc) / diag);
-  // SOR: the Gauss-Seidel value itself when omega = 1, so that a colour
-  // applied twice in a row gives the same bits (the neighbours it reads are
-  // unchanged) and sweeps may skip such a repeat (diag = 1 in mode 4)
-  else if (omega == 1.0) y[p] = (T)((fp - acc) / diag);
-  else y[p] = (T)((A)omega * ((fp - acc) / diag - told) + told);
-}
-
-// R lanes per row, kRowsPerBlock rows per workgroup; with one lane per row
-// the compiler is held to 128 registers so that 4 waves share a SIMD.
-template <typename T, int MODE, int R>
-__global__ __launch_bounds__(kRowsPerBlock * R, R == 1 ? 4 : 1) void k_rows(const RowBlock *__restrict__ rows, int M,
-                                                 const T *__restrict__ val, const T *x, const T *__restrict__ f,
-                                                 T *y, double omega) {
-  const RowBlock &rb = rows[xcd_remap(blockIdx.x, gridDim.x)];
-  const DevSegment s = rb.s;
-  const int idx = rb.base + threadIdx.x / R;
-  const int part = threadIdx.x % R;
-  if (idx >= s.count) return;  // the R lanes of a row leave together
-#define PMX_ROW(EX, EY, EZ) row_split<T, EX, EY, EZ, R, MODE>(s, idx, part, M, val, x, f, y, omega)
-  switch (s.ex * 100 + s.ey * 10 + s.ez) {
-    case 111: PMX_ROW(1, 1, 1); break;
-    case 211: PMX_ROW(2, 1, 1); break;
-    case 121: PMX_ROW(1, 2, 1); break;
-    case 221: PMX_ROW(2, 2, 1); break;
-    case 112: PMX_ROW(1, 1, 2); break;
-    case 212: PMX_ROW(2, 1, 2); break;
-    case 122: PMX_ROW(1, 2, 2); break;
-    default: PMX_ROW(2, 2, 2); break;
-  }
-#undef PMX_ROW
-}
-
-// Mode 4 (SOR of one colour on row-scaled FP16 values, FP32 vectors), laid
-// out as k_rows.
-template <int R>
-__global__ __launch_bounds__(kRowsPerBlock * R, R == 1 ? 4 : 1) void k_sor_scaled(
-    const RowBlock *__restrict__ rows, int M, const _Float16 *__restrict__ val, const float *__restrict__ dinv,
-    float *x, const float *__restrict__ f, double omega) {
-  const RowBlock &rb = rows[xcd_remap(blockIdx.x, gridDim.x)];
-  const DevSegment s = rb.s;
-  const int idx = rb.base + threadIdx.x / R;
-  const int part = threadIdx.x % R;
-  if (idx >= s.count) return;
-#define PMX_ROW(EX, EY, EZ) row_split<float, EX, EY, EZ, R, 4, false, _Float16>(s, idx, part, M, val, x, f, x, omega, dinv)
-  switch (s.ex * 100 + s.ey * 10 + s.ez) {
-    case 111: PMX_ROW(1, 1, 1); break;
-    case 211: PMX_ROW(2, 1, 1); break;
-    case 121: PMX_ROW(1, 2, 1); break;
-    case 221: PMX_ROW(2, 2, 1); break;
-    case 112: PMX_ROW(1, 1, 2); break;
-    case 212: PMX_ROW(2, 1, 2); break;
-    case 122: PMX_ROW(1, 2, 2); break;
-    default: PMX_ROW(2, 2, 2); break;
-  }
-#undef PMX_ROW
-}
-
-// Row-scaled FP16 copy of the FP32 stencil values for mode 4: slot k of an
-// active row holds a_k / a_diag rounded to FP16 (saturated at +-65504, the
-// largest finite FP16 value), and dinv[p] = 1 / a_diag in FP32.  One thread
-// per row.
-__global__ __launch_bounds__(kRowsPerBlock) void k_scaled_values(const BlockInfo *__restrict__ blocks,
-                                                                 const DevSegment *__restrict__ segs, int M,
-                                                                 const float *__restrict__ val,
-                                                                 _Float16 *__restrict__ val16,
-                                                                 float *__restrict__ dinv) {
-  const BlockInfo bi = blocks[blockIdx.x];
-  const DevSegment s = segs[bi.seg];
-  const int idx = bi.base + threadIdx.x;
-  if (idx >= s.count) return;
-  const int i = idx % s.cx, t = idx / s.cx;
-  const int j = t % s.cy, k = t / s.cy;
-  const int p = (s.x0 + s.stride * i) + M * ((s.y0 + s.stride * j) + M * (s.z0 + s.stride * k));
-  const int64_t vb = vbase(s, idx);
-  const float d = val[vb + (int64_t)s.dslot * kSlice];
-  const float r = 1.0f / d;
-  dinv[p] = r;
-  const int64_t sb = v16slice(s, idx);
-  for (int q = 0; q < s.ns; q++) {
-    const float w = val[vb + (int64_t)q * kSlice] * r;
-    val16[sb + v16off(s.ns, idx % kSlice, q)] = (_Float16)fminf(fmaxf(w, -65504.0f), 65504.0f);
-  }
-}
-
-// The rows of colour c of a level staged in LDS (segment table lseg, colour
-// ranges lcs, each segment's first row in its colour lrow0, rows per colour
-// lrows), R lanes per row, computed by row_split in mode MODE with x in LDS.
-template <typename T, int R, int MODE, int NT>
-__device__ __forceinline__ void wg_colour_rows(const DevSegment *lseg, const int *lcs, const int *lrow0,
-                                               const int *lrows, int c, int M, const T *__restrict__ val,
-                                               const T *lx, const T *__restrict__ f, T *y, double omega) {
-  const int part = threadIdx.x % R;
-  const int s0 = lcs[c], s1 = lcs[c + 1], n = lrows[c];
-  // the R lanes of a row share r, so they run the same trip count
-  for (int r = threadIdx.x / R; r < n; r += NT / R) {
-    int si = s0;
-    while (si + 1 < s1 && r >= lrow0[si + 1]) si++;
-    const DevSegment s = lseg[si];
-    const int idx = r - lrow0[si];
-#define PMX_ROW(EX, EY, EZ) row_split<T, EX, EY, EZ, R, MODE, true>(s, idx, part, M, val, lx, f, y, omega)
-    switch (s.ex * 100 + s.ey * 10 + s.ez) {
-      case 111: PMX_ROW(1, 1, 1); break;
-      case 211: PMX_ROW(2, 1, 1); break;
-      case 121: PMX_ROW(1, 2, 1); break;
-      case 221: PMX_ROW(2, 2, 1); break;
-      case 112: PMX_ROW(1, 1, 2); break;
-      case 212: PMX_ROW(2, 1, 2); break;
-      case 122: PMX_ROW(1, 2, 2); break;
-      default: PMX_ROW(2, 2, 2); break;
-    }
-#undef PMX_ROW
-  }
-}
-// stage the segment table, colour ranges and row offsets, and x with
-// Dirichlet rows x = f, in LDS
-template <typename T, int NT>
-__device__ __forceinline__ void wg_stage(const DevSegment *__restrict__ segs, int nseg,
-                                         const int *__restrict__ colour_seg, int ncol, int N, const T *x,
-                                         const T *__restrict__ f, const int *__restrict__ bnd, int nb,
-                                         DevSegment *lseg, int *lcs, int *lrow0, int *lrows, T *lx) {
-  for (int i = threadIdx.x; i < nseg; i += NT) lseg[i] = segs[i];
-  for (int i = threadIdx.x; i <= ncol; i += NT) lcs[i] = colour_seg[i];
-  for (int i = threadIdx.x; i < N; i += NT) lx[i] = x[i];
-  __syncthreads();
-  for (int i = threadIdx.x; i < nb; i += NT) lx[bnd[i]] = f[bnd[i]];
-  for (int c = threadIdx.x; c < ncol; c += NT) {
-    int n = 0;
-    for (int si = lcs[c]; si < lcs[c + 1]; si++) {
-      lrow0[si] = n;
-      n += (int)lseg[si].count;
-    }
-    lrows[c] = n;
-  }
-  __syncthreads();
-}
-
-// A whole SOR (ssor = 0) or SSOR (ssor = 1) sweep of a small level in one
-// workgroup: the level's x is copied into LDS (Dirichlet rows x = f), the
-// colours run one after another (backwards again for SSOR) with a workgroup
-// barrier between them, and x is copied back.  The rows of a colour are
-// enumerated across its residue classes, R lanes per row as in k_rows, and
-// each row is computed by row_split, so the iterate is bit-identical to the
-// launch-per-colour sweep.  On a level whose colours have a few hundred rows
-// this replaces 2 x 27 launch latencies per SSOR sweep by barriers, and the
-// x round trips through memory by LDS accesses.
-template <typename T, int R>
-__global__ __launch_bounds__(sweep_threads<T>()) void k_sweep_wg(const DevSegment *__restrict__ segs, int nseg,
-                                                            const int *__restrict__ colour_seg, int ncol, int M,
-                                                            const T *__restrict__ val, T *x,
-                                                            const T *__restrict__ f, double omega, int ssor,
-                                                            const int *__restrict__ bnd, int nb) {
-  constexpr int NT = sweep_threads<T>();
-  extern __shared__ __align__(16) unsigned char sweep_lds[];
-  T *lx = reinterpret_cast<T *>(sweep_lds);
-  __shared__ DevSegment lseg[kMaxSegs];
-  __shared__ int lcs[kMaxColours + 1];
-  __shared__ int lrow0[kMaxSegs + 1];
-  __shared__ int lrows[kMaxColours];
-  const int N = M * M * M;
-  wg_stage<T, NT>(segs, nseg, colour_seg, ncol, N, x, f, bnd, nb, lseg, lcs, lrow0, lrows, lx);
-  const int nsteps = ssor ? 2 * ncol : ncol;
-  for (int step = 0; step < nsteps; step++) {
-    const int c = step < ncol ? step : 2 * ncol - 1 - step;
-    wg_colour_rows<T, R, 3, NT>(lseg, lcs, lrow0, lrows, c, M, val, lx, f, lx, omega);
-    __syncthreads();
-  }
-  for (int i = threadIdx.x; i < N; i += NT) x[i] = lx[i];
-}
-
-// ||f - A x|| of the LDS iterate over all rows (Dirichlet rows: 0), the
-// same value in every thread.  d: global scratch of N entries whose
-// Dirichlet entries hold 0.
-template <typename T, int R, int NT>
-__device__ double wg_defect_norm(const DevSegment *lseg, const int *lcs, const int *lrow0, const int *lrows,
-                                 int ncol, int M, const T *__restrict__ val, const T *lx, const T *__restrict__ f,
-                                 T *d, double *lred) {
-  const int N = M * M * M;
-  for (int c = 0; c < ncol; c++) wg_colour_rows<T, R, 1, NT>(lseg, lcs, lrow0, lrows, c, M, val, lx, f, d, 0.0);
-  __syncthreads();
-  double s = 0;
-  for (int i = threadIdx.x; i < N; i += NT) s += (double)d[i] * (double)d[i];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-  if (threadIdx.x % 64 == 0) lred[threadIdx.x / 64] = s;
-  __syncthreads();
-  double t = 0;
-  for (int w = 0; w < NT / 64; w++) t += lred[w];
-  __syncthreads();
-  return sqrt(t);
-}
-// The coarse-level loop of TMultiGrid3D::Smooth(CoarseSmooth)
-// (MultiGrid3D.C:225-337) in one workgroup: res = ||f - A x||, then while
-// res > red * res_0 and fewer than maxit sweeps: one Jacobi (kind 1, omega
-// damped), SOR (2) or SSOR (3) sweep and res again.  The sweeps compute each
-// row as the launched sweeps do (bit-identical iterates); d and xj are
-// global scratch of N entries (defect, Jacobi output).
-template <typename T, int R>
-__global__ __launch_bounds__(sweep_threads<T>()) void k_coarse_wg(const DevSegment *__restrict__ segs, int nseg,
-                                                             const int *__restrict__ colour_seg, int ncol, int M,
-                                                             const T *__restrict__ val, T *x,
-                                                             const T *__restrict__ f, double omega, int kind,
-                                                             int maxit, double red, const int *__restrict__ bnd,
-                                                             int nb, T *d, T *xj) {
-  constexpr int NT = sweep_threads<T>();
-  extern __shared__ __align__(16) unsigned char sweep_lds[];
-  T *lx = reinterpret_cast<T *>(sweep_lds);
-  __shared__ DevSegment lseg[kMaxSegs];
-  __shared__ int lcs[kMaxColours + 1];
-  __shared__ int lrow0[kMaxSegs + 1];
-  __shared__ int lrows[kMaxColours];
-  __shared__ double lred[NT / 64];
-  const int N = M * M * M;
-  for (int i = threadIdx.x; i < nb; i += NT) {
-    d[bnd[i]] = T(0);
-    xj[bnd[i]] = f[bnd[i]];
-  }
-  wg_stage<T, NT>(segs, nseg, colour_seg, ncol, N, x, f, bnd, nb, lseg, lcs, lrow0, lrows, lx);
-  double res = wg_defect_norm<T, R, NT>(lseg, lcs, lrow0, lrows, ncol, M, val, lx, f, d, lred);
-  const double reduction = red * res;
-  for (int it = 0; res > reduction && it < maxit; it++) {
-    if (kind == 1) {
-      for (int c = 0; c < ncol; c++) wg_colour_rows<T, R, 2, NT>(lseg, lcs, lrow0, lrows, c, M, val, lx, f, xj, omega);
-      __syncthreads();
-      for (int i = threadIdx.x; i < N; i += NT) lx[i] = xj[i];
-      __syncthreads();
-    } else {
-      const int nsteps = kind == 3 ? 2 * ncol : ncol;
-      for (int step = 0; step < nsteps; step++) {
-        const int c = step < ncol ? step : 2 * ncol - 1 - step;
-        wg_colour_rows<T, R, 3, NT>(lseg, lcs, lrow0, lrows, c, M, val, lx, f, lx, omega);
-        __syncthreads();
-      }
-    }
-    res = wg_defect_norm<T, R, NT>(lseg, lcs, lrow0, lrows, ncol, M, val, lx, f, d, lred);
-  }
-  for (int i = threadIdx.x; i < N; i += NT) x[i] = lx[i];
 }
 
 // flag = 1 if a and b differ in any bit (all writers store the same value)
@@ -738,7 +395,7 @@ __host__ __device__ inline bool coeffs_inline(int example) {
 // loops are uniform across the wavefront and the basis tables are read with
 // scalar loads; TWO selects the second matrix of the SUPG TCD form.
 template <int ORDER, int EX, int EY, int EZ, bool TWO, bool INL, bool RONLY>
-__device__ __forceinline__ void assemble_row(const DevSegment &s, int idx, int M, int n, int nq, int form,
+__device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int n, int nq, int form,
                                              const double *__restrict__ prm, const double *__restrict__ qref,
                                              const double *__restrict__ qp, const double *__restrict__ tab,
                                              double *__restrict__ val, double *__restrict__ val2,
@@ -747,15 +404,15 @@ __device__ __forceinline__ void assemble_row(const DevSegment &s, int idx, int M
   constexpr int NCY = (ORDER == 2 && EY == 1) ? 1 : 2;
   constexpr int NCZ = (ORDER == 2 && EZ == 1) ? 1 : 2;
   constexpr int K = ORDER + 1, NB = K * K * K;
-  const int i = idx % s.cx;
-  const int t = idx / s.cx;
-  const int j = t % s.cy, k = t / s.cy;
-  const int px = s.x0 + s.stride * i, py = s.y0 + s.stride * j, pz = s.z0 + s.stride * k;
   const int p = px + M * (py + M * pz);
   const double g = 2.0 * n;  // reference -> physical derivative factor 2/h
-  double *v = val + vbase(s, idx);
-  double *v2 = TWO ? val2 + vbase(s, idx) : nullptr;
-  constexpr int cnt = kSlice;
+  // the row's entries: group position of (dy, dz), slot of dx
+  const int P = (M - 1) / 2;
+  const int64_t v0 = line_values<double, ORDER>(P, Lines<ORDER>::group_base(P, py, pz), (px - 1) >> 1);
+  const int *pos = group_table<ORDER>().pos[__builtin_amdgcn_readfirstlane(line_class<ORDER>(py, pz))];
+  auto at = [&](int dx, int dy, int dz) {
+    return v0 + (int64_t)(pos[(dy + 2) + 5 * (dz + 2)] * Lines<ORDER>::VL + Lines<ORDER>::slot(px, dx)) * P;
+  };
   double frhs = 0;
   // Q1 rows of the one-matrix forms (27 slots) are accumulated in registers
   // over the 8 cells (loops unrolled, every slot a compile-time index) and
@@ -849,40 +506,63 @@ __device__ __forceinline__ void assemble_row(const DevSegment &s, int idx, int M
             // Q1: the first of the row's cells (in loop order) that meets
             // the slot, (max(0, dx), max(0, dy), max(0, dz)), stores; the
             // later ones add, so the values need no clearing beforehand
-            v[slot * cnt] = acc[b];
-            if (TWO) v2[slot * cnt] = acc2[b];
+            val[at(dx, dy, dz)] = acc[b];
+            if (TWO) val2[at(dx, dy, dz)] = acc2[b];
           } else {
-            v[slot * cnt] += acc[b];
-            if (TWO) v2[slot * cnt] += acc2[b];
+            val[at(dx, dy, dz)] += acc[b];
+            if (TWO) val2[at(dx, dy, dz)] += acc2[b];
           }
         }
       }
   if constexpr (REG && !RONLY) {
 #pragma unroll
-    for (int q = 0; q < 27; q++) v[q * cnt] = racc[q];
+    for (int q = 0; q < 27; q++) val[at(q % 3 - 1, (q / 3) % 3 - 1, q / 9 - 1)] = racc[q];
   }
   rhs[p] = frhs;
 }
 
+// Rows of the one-thread-per-row assembly kernels: 64 row pairs of a unit's
+// lines (unit_lines), the odd rows in one workgroup and the even rows in the
+// next, so that a wavefront's rows have one stencil shape and its stores of a
+// slot are contiguous.  False: no row.
+template <int O>
+__device__ __forceinline__ bool unit_row(const LineSet &set, int M, int lg, int *px, int *py, int *pz) {
+  const int b = xcd_remap(blockIdx.x, gridDim.x), P = 1 << lg, segs = lg > 6 ? P / 64 : 1;
+  const int part = b % (2 * segs);
+  const UnitLines u = unit_lines<O>(set, M, lg, b / (2 * segs));
+  const int t = threadIdx.x + 64 * (part >> 1), m = t & (P - 1);
+  *px = 2 * m + 1 + (part & 1);
+  *py = u.y0 + Lines<O>::S * (t >> lg);
+  *pz = u.z;
+  return *py <= M - 2 && *px <= M - 2;
+}
+// the same shape for the whole wavefront
+template <int O> __device__ __forceinline__ int unit_shape(int lg, const LineSet &set, int M) {
+  const int b = xcd_remap(blockIdx.x, gridDim.x), segs = lg > 6 ? (1 << lg) / 64 : 1;
+  const UnitLines u = unit_lines<O>(set, M, lg, b / (2 * segs));
+  return __builtin_amdgcn_readfirstlane(Lines<O>::ext(1 + (b & 1)) * 100 + Lines<O>::ext(u.y0) * 10 + Lines<O>::ext(u.z));
+}
+static unsigned row_blocks(const DevLayout &D, int units) {
+  return (unsigned)units * 2 * (D.lg > 6 ? (1u << D.lg) / 64 : 1);
+}
+
 template <int ORDER, bool TWO, bool INL, bool RONLY>
-__global__ __launch_bounds__(kRowsPerBlock) void k_assemble(const BlockInfo *__restrict__ blocks,
-                                                     const DevSegment *__restrict__ segs, int M, int n, int nq,
+__global__ __launch_bounds__(kRowsPerBlock) void k_assemble(LineSet set, int lg, int M, int n, int nq,
                                                      const double *__restrict__ prm, const double *__restrict__ qref,
                                                      const double *__restrict__ qp, const double *__restrict__ tab,
                                                      double *__restrict__ val, double *__restrict__ val2,
                                                      double *__restrict__ rhs) {
-  const BlockInfo bi = blocks[xcd_remap(blockIdx.x, gridDim.x)];
-  const DevSegment s = segs[bi.seg];
-  const int idx = bi.base + threadIdx.x;
-  if (idx >= s.count) return;
+  int px, py, pz;
+  const bool ok = unit_row<ORDER>(set, M, lg, &px, &py, &pz);
+  const int code = unit_shape<ORDER>(lg, set, M);
+  if (!ok) return;
   const int form = (int)prm[PMX_PRM_FORM];
 #define PMX_AROW(O, EX, EY, EZ) \
-  assemble_row<O, EX, EY, EZ, TWO, INL, RONLY>(s, idx, M, n, nq, form, prm, qref, qp, tab, val, val2, rhs)
+  assemble_row<O, EX, EY, EZ, TWO, INL, RONLY>(px, py, pz, M, n, nq, form, prm, qref, qp, tab, val, val2, rhs)
   if (ORDER == 1) {
     PMX_AROW(1, 1, 1, 1);
     return;
   }
-  const int code = s.ex * 100 + s.ey * 10 + s.ez;
   switch (code) {
     case 111: PMX_AROW(2, 1, 1, 1); break;
     case 211: PMX_AROW(2, 2, 1, 1); break;
@@ -914,49 +594,41 @@ __global__ void k_boundary_rhs(const int *__restrict__ bnd, int nbd, int M, cons
 }
 
 // ============================================================ CSR export
-// entries in the reference CSR (sorted rows, Dirichlet rows = 1) from CSS values
-template <typename T>
-__global__ void k_css_to_csr(const int *__restrict__ rowptr, const int *__restrict__ kcol,
-                             const int *__restrict__ dof2lat, int64_t N, int64_t active, int M, int S,
-                             const int *__restrict__ segidx, const DevSegment *__restrict__ segs,
-                             const T *__restrict__ val, double *__restrict__ out) {
+// entries in the reference CSR (sorted rows, Dirichlet rows = 1) from the
+// line layout's values (FP16: the row-scaled smoother values)
+template <typename T, int O>
+__global__ void k_values_to_csr(const int *__restrict__ rowptr, const int *__restrict__ kcol,
+                                const int *__restrict__ dof2lat, int64_t N, int64_t active, int M,
+                                const T *__restrict__ val, double *__restrict__ out) {
   const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (r >= N) return;
-  const int b = rowptr[r], e = rowptr[r + 1];
+  const int b = rowptr[r], e = rowptr[r + 1], P = (M - 1) / 2;
   if (r >= active) { out[b] = 1.0; return; }
   const int p = dof2lat[r];
   const int x = p % M, y = (p / M) % M, z = p / (M * M);
-  const DevSegment s = segs[segidx[(x % S) + S * ((y % S) + S * (z % S))]];
-  const int idx = ((x - s.x0) / s.stride) + s.cx * (((y - s.y0) / s.stride) + s.cy * ((z - s.z0) / s.stride));
   for (int n = b; n < e; n++) {
     const int q = dof2lat[kcol[n]];
     const int dx = q % M - x, dy = (q / M) % M - y, dz = q / (M * M) - z;
-    const int slot = (dx + s.ex) + (2 * s.ex + 1) * ((dy + s.ey) + (2 * s.ey + 1) * (dz + s.ez));
-    if constexpr (std::is_same<T, _Float16>::value)
-      out[n] = (double)val[v16slice(s, idx) + v16off(s.ns, idx % kSlice, slot)];
-    else
-      out[n] = (double)val[vbase(s, idx) + (int64_t)slot * kSlice];
+    if constexpr (sizeof(T) == 2) out[n] = (double)val[value_index16<O>(P, x, y, z, dx, dy, dz)];
+    else out[n] = (double)val[value_index<O>(P, x, y, z, dx, dy, dz)];
   }
 }
 
-// The inverse of k_css_to_csr for the active rows: the entries of a CSR
-// matrix with the level's pattern (reference numbering) into the CSS values.
-__global__ void k_csr_to_css(const int *__restrict__ rowptr, const int *__restrict__ kcol,
-                             const int *__restrict__ dof2lat, int64_t active, int M, int S,
-                             const int *__restrict__ segidx, const DevSegment *__restrict__ segs,
-                             const double *__restrict__ in, double *__restrict__ val) {
+// The inverse of k_values_to_csr for the active rows: the entries of a CSR
+// matrix with the level's pattern (reference numbering) into the line layout.
+template <int O>
+__global__ void k_csr_to_values(const int *__restrict__ rowptr, const int *__restrict__ kcol,
+                                const int *__restrict__ dof2lat, int64_t active, int M,
+                                const double *__restrict__ in, double *__restrict__ val) {
   const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (r >= active) return;
-  const int b = rowptr[r], e = rowptr[r + 1];
+  const int b = rowptr[r], e = rowptr[r + 1], P = (M - 1) / 2;
   const int p = dof2lat[r];
   const int x = p % M, y = (p / M) % M, z = p / (M * M);
-  const DevSegment s = segs[segidx[(x % S) + S * ((y % S) + S * (z % S))]];
-  const int idx = ((x - s.x0) / s.stride) + s.cx * (((y - s.y0) / s.stride) + s.cy * ((z - s.z0) / s.stride));
   for (int n = b; n < e; n++) {
     const int q = dof2lat[kcol[n]];
     const int dx = q % M - x, dy = (q / M) % M - y, dz = q / (M * M) - z;
-    const int slot = (dx + s.ex) + (2 * s.ex + 1) * ((dy + s.ey) + (2 * s.ey + 1) * (dz + s.ez));
-    val[vbase(s, idx) + (int64_t)slot * kSlice] = in[n];
+    val[value_index<O>(P, x, y, z, dx, dy, dz)] = in[n];
   }
 }
 
@@ -1005,25 +677,21 @@ __global__ __launch_bounds__(kBlock) void k_gemv_coarse(int nI, int N, const dou
 // ============================================================ coarse inverse
 // Augmented [A_II | R] (n_I x (n_I + N), row-major), R[i][p] = 1 for the
 // interior node p of row i, -a(i, p) for Dirichlet columns p.
-__global__ void k_css_to_aug(const BlockInfo *__restrict__ blocks, const DevSegment *__restrict__ segs, int M,
-                             const int *__restrict__ cidx, int nI, const double *__restrict__ val,
-                             double *__restrict__ aug, int64_t ld) {
-  const BlockInfo bi = blocks[blockIdx.x];
-  const DevSegment s = segs[bi.seg];
-  const int idx = bi.base + threadIdx.x;
-  if (idx >= s.count) return;
-  const int i = idx % s.cx, t = idx / s.cx, j = t % s.cy, k = t / s.cy;
-  const int x = s.x0 + s.stride * i, y = s.y0 + s.stride * j, z = s.z0 + s.stride * k;
-  const int p = x + M * (y + M * z);
-  const int r = cidx[p];
+template <int O>
+__global__ void k_values_to_aug(int M, const int *__restrict__ iidx, const int *__restrict__ cidx, int nI,
+                                const double *__restrict__ val, double *__restrict__ aug, int64_t ld) {
+  using L = Lines<O>;
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= nI) return;
+  const int p = iidx[r], x = p % M, y = (p / M) % M, z = p / (M * M), P = (M - 1) / 2;
   double *row = aug + (int64_t)r * ld;
   row[nI + p] = 1.0;
-  int slot = 0;
-  for (int dz = -s.ez; dz <= s.ez; dz++)
-    for (int dy = -s.ey; dy <= s.ey; dy++)
-      for (int dx = -s.ex; dx <= s.ex; dx++, slot++) {
+  const int ex = L::ext(x), ey = L::ext(y), ez = L::ext(z);
+  for (int dz = -ez; dz <= ez; dz++)
+    for (int dy = -ey; dy <= ey; dy++)
+      for (int dx = -ex; dx <= ex; dx++) {
         const int q = (x + dx) + M * ((y + dy) + M * (z + dz));
-        const double v = val[vbase(s, idx) + (int64_t)slot * kSlice];
+        const double v = val[value_index<O>(P, x, y, z, dx, dy, dz)];
         const int cq = cidx[q];
         if (cq >= 0) row[cq] = v;
         else row[nI + q] = -v;
@@ -1338,173 +1006,6 @@ void mgs_arnoldi(T *w, const T *V, int64_t n, int k1, double *h, T *vnext, doubl
   hipLaunchKernelGGL(k_norm_scale<T>, dim3(g), dim3(kBlock), 0, st, w, pa, g, h + k1, vnext, n);
 }
 
-// Per-dispatch timing of the row kernels: while a timer is installed on the
-// calling thread, css_apply launches through hipExtLaunchKernelGGL with a
-// start and a stop event of the timer around each dispatch (the events take
-// the dispatch's own begin and end, not the gaps between dispatches).
-static thread_local DispatchTimer *g_timer = nullptr;
-void set_dispatch_timer(DispatchTimer *t) { g_timer = t; }
-double DispatchTimer::total_ms() const {
-  double s = 0;
-  for (int k = 0; k < used; k++) {
-    float ms = 0;
-    check(hipEventElapsedTime(&ms, ev[2 * k], ev[2 * k + 1]), "dispatch timer");
-    s += ms;
-  }
-  return s;
-}
-DispatchTimer::~DispatchTimer() {
-  for (hipEvent_t e : ev) (void)hipEventDestroy(e);
-}
-static void timer_events(hipEvent_t *e0, hipEvent_t *e1) {
-  DispatchTimer &t = *g_timer;
-  if (2 * t.used + 1 >= (int)t.ev.size()) {
-    for (int k = 0; k < 2; k++) {
-      hipEvent_t e;
-      check(hipEventCreate(&e), "event");
-      t.ev.push_back(e);
-    }
-  }
-  *e0 = t.ev[2 * t.used];
-  *e1 = t.ev[2 * t.used + 1];
-  t.used++;
-}
-
-template <typename T>
-void css_apply(const DevLayout &D, int mode, const T *val, const T *x, const T *f, T *y, double omega, int colour,
-               hipStream_t st) {
-  const RowBlock *blk = colour < 0 ? D.rows_all : D.rows_colour + D.colour_off[colour];
-  const int nblk = colour < 0 ? D.nblocks_all : D.colour_off[colour + 1] - D.colour_off[colour];
-  if (nblk == 0) return;
-#define PMX_ROWS(MODE, R)                                                                                      \
-  if (g_timer) {                                                                                               \
-    hipEvent_t e0, e1;                                                                                         \
-    timer_events(&e0, &e1);                                                                                    \
-    hipExtLaunchKernelGGL((k_rows<T, MODE, R>), dim3(nblk), dim3(kRowsPerBlock * R), 0, st, e0, e1, 0, blk, D.M,  \
-                          val, x, f, y, omega);                                                                \
-  } else                                                                                                       \
-    hipLaunchKernelGGL((k_rows<T, MODE, R>), dim3(nblk), dim3(kRowsPerBlock * R), 0, st, blk, D.M, val, x, f, y,  \
-                       omega)
-#define PMX_ROWS_R(MODE)                                                                                       \
-  switch (row_lanes(D)) {                                                                                      \
-    case 1: PMX_ROWS(MODE, 1); break;                                                                          \
-    case 2: PMX_ROWS(MODE, 2); break;                                                                          \
-    default: PMX_ROWS(MODE, 4); break;                                                                         \
-  }
-  switch (mode) {
-    case 0: PMX_ROWS_R(0); break;
-    case 1: PMX_ROWS_R(1); break;
-    case 2: PMX_ROWS_R(2); break;
-    default: PMX_ROWS_R(3); break;
-  }
-#undef PMX_ROWS_R
-#undef PMX_ROWS
-}
-void css_sor_scaled(const DevLayout &D, const _Float16 *val16, const float *dinv, float *x, const float *f,
-                    double omega, int colour, hipStream_t st) {
-  const RowBlock *blk = D.rows_colour + D.colour_off[colour];
-  const int nblk = D.colour_off[colour + 1] - D.colour_off[colour];
-  if (nblk == 0) return;
-#define PMX_ROWS(R)                                                                                            \
-  if (g_timer) {                                                                                               \
-    hipEvent_t e0, e1;                                                                                         \
-    timer_events(&e0, &e1);                                                                                    \
-    hipExtLaunchKernelGGL((k_sor_scaled<R>), dim3(nblk), dim3(kRowsPerBlock * R), 0, st, e0, e1, 0, blk, D.M,     \
-                          val16, dinv, x, f, omega);                                                           \
-  } else                                                                                                       \
-    hipLaunchKernelGGL((k_sor_scaled<R>), dim3(nblk), dim3(kRowsPerBlock * R), 0, st, blk, D.M, val16, dinv, x,  \
-                       f, omega)
-#ifdef PMX_SCALED_LANES
-  const int lanes = PMX_SCALED_LANES;  // a fixed lane count (tuning builds)
-#else
-  const int lanes = row_lanes(D);
-#endif
-  switch (lanes) {
-    case 1: PMX_ROWS(1); break;
-    case 2: PMX_ROWS(2); break;
-    default: PMX_ROWS(4); break;
-  }
-#undef PMX_ROWS
-}
-// Calibration kernels of the dispatch measurements: a dispatch that does
-// nothing, and a plain streaming read (16 bytes per load, two loads per lane)
-// whose sum reaches memory only in a case that never occurs.
-__global__ void k_empty_dispatch() {}
-__global__ __launch_bounds__(256) void k_stream_read(const float4 *__restrict__ a, int64_t n4,
-                                                     float *__restrict__ sink) {
-  const int64_t i = (int64_t)blockIdx.x * 512 + threadIdx.x;
-  float s = 0.f;
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    if (i + 256 * k < n4) {
-      const float4 v = a[i + 256 * k];
-      s += v.x + v.y + v.z + v.w;
-    }
-  }
-  if (s == -1234567.0f) sink[0] = s;
-}
-void empty_dispatch(int blocks, hipStream_t st) {
-  if (blocks < 1) return;
-  if (g_timer) {
-    hipEvent_t e0, e1;
-    timer_events(&e0, &e1);
-    hipExtLaunchKernelGGL(k_empty_dispatch, dim3(blocks), dim3(kRowsPerBlock), 0, st, e0, e1, 0);
-  } else {
-    hipLaunchKernelGGL(k_empty_dispatch, dim3(blocks), dim3(kRowsPerBlock), 0, st);
-  }
-}
-void stream_read(const void *p, int64_t bytes, float *sink, hipStream_t st) {
-  const int64_t n4 = bytes / 16;
-  if (n4 < 1) return;
-  if ((reinterpret_cast<uintptr_t>(p) & 15) != 0) throw std::invalid_argument("stream_read: 16-byte alignment");
-  const unsigned g = (unsigned)((n4 + 511) / 512);
-  const float4 *a = static_cast<const float4 *>(p);
-  if (g_timer) {
-    hipEvent_t e0, e1;
-    timer_events(&e0, &e1);
-    hipExtLaunchKernelGGL(k_stream_read, dim3(g), dim3(256), 0, st, e0, e1, 0, a, n4, sink);
-  } else {
-    hipLaunchKernelGGL(k_stream_read, dim3(g), dim3(256), 0, st, a, n4, sink);
-  }
-}
-void scaled_values(const DevLayout &D, const float *val, _Float16 *val16, float *dinv, hipStream_t st) {
-  if (D.nblocks_all == 0) return;
-  hipLaunchKernelGGL(k_scaled_values, dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st, D.blocks_all, D.segs, D.M,
-                     val, val16, dinv);
-}
-template <typename T>
-void sweep_wg(const DevLayout &D, const T *val, T *x, const T *f, double omega, int ssor, hipStream_t st) {
-  if (D.nsegs > kMaxSegs || D.ncolours > kMaxColours) throw std::logic_error("sweep_wg: segment table too large");
-  if (!sweep_wg_fits(D, sizeof(T))) throw std::logic_error("sweep_wg: level does not fit in LDS");
-  const size_t lds = (size_t)D.N * sizeof(T);
-#define PMX_SWEEP(R)                                                                                            \
-  hipLaunchKernelGGL((k_sweep_wg<T, R>), dim3(1), dim3(sweep_threads<T>()), lds, st, D.segs, D.nsegs,             \
-                     D.colour_seg_dev, D.ncolours, D.M, val, x, f, omega, ssor, D.boundary, D.nboundary)
-  switch (row_lanes(D)) {
-    case 1: PMX_SWEEP(1); break;
-    case 2: PMX_SWEEP(2); break;
-    default: PMX_SWEEP(4); break;
-  }
-#undef PMX_SWEEP
-}
-template <typename T>
-void coarse_wg(const DevLayout &D, const T *val, T *x, const T *f, double omega, int kind, int maxit, double red,
-               T *d, T *xj, hipStream_t st) {
-  if (D.nsegs > kMaxSegs || D.ncolours > kMaxColours) throw std::logic_error("coarse_wg: segment table too large");
-  if (!sweep_wg_fits(D, sizeof(T))) throw std::logic_error("coarse_wg: level does not fit in LDS");
-  if (kind < 1 || kind > 3) throw std::invalid_argument("coarse_wg: smoother must be 1, 2 or 3");
-  const size_t lds = (size_t)D.N * sizeof(T);
-#define PMX_COARSE(R)                                                                                           \
-  hipLaunchKernelGGL((k_coarse_wg<T, R>), dim3(1), dim3(sweep_threads<T>()), lds, st, D.segs, D.nsegs,           \
-                     D.colour_seg_dev, D.ncolours, D.M, val, x, f, omega, kind, maxit, red, D.boundary,          \
-                     D.nboundary, d, xj)
-  switch (row_lanes(D)) {
-    case 1: PMX_COARSE(1); break;
-    case 2: PMX_COARSE(2); break;
-    default: PMX_COARSE(4); break;
-  }
-#undef PMX_COARSE
-}
 template <typename T>
 void boundary(const DevLayout &D, int mode, T *y, const T *x, const T *f, hipStream_t st) {
   const int g = (D.nboundary + kBlock - 1) / kBlock;
@@ -1546,14 +1047,15 @@ void gemv_coarse(int nI, int N, const double *W, const int *iidx, const T *x, T 
   const unsigned g = (unsigned)((nI * 64 + kBlock - 1) / kBlock);
   hipLaunchKernelGGL(k_gemv_coarse<T>, dim3(g), dim3(kBlock), 0, st, nI, N, W, iidx, x, y);
 }
-void coarse_inverse_dense(const DevLayout &D, const double *val, const int *cidx, int nI, double *aug, int *piv,
-                          double *W, hipStream_t st) {
+void coarse_inverse_dense(const DevLayout &D, const double *val, const int *iidx, const int *cidx, int nI, double *aug,
+                          int *piv, double *W, hipStream_t st) {
   if (nI > 8192) throw std::invalid_argument("coarse inverse: too many interior nodes");
   const int N = (int)D.N;
   const int64_t ld = nI + (int64_t)N;
   fill<double>(aug, 0.0, nI * ld, st);
-  hipLaunchKernelGGL(k_css_to_aug, dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st, D.blocks_all, D.segs, D.M, cidx,
-                     nI, val, aug, ld);
+  const dim3 ga((unsigned)((nI + 63) / 64));
+  if (D.order == 2) hipLaunchKernelGGL(k_values_to_aug<2>, ga, dim3(64), 0, st, D.M, iidx, cidx, nI, val, aug, ld);
+  else hipLaunchKernelGGL(k_values_to_aug<1>, ga, dim3(64), 0, st, D.M, iidx, cidx, nI, val, aug, ld);
   const unsigned g = (unsigned)((nI + 3) / 4);
   for (int c = 0; c < nI; c++) hipLaunchKernelGGL(k_gj_step, dim3(g), dim3(256), 0, st, aug, nI, ld, c, piv);
   hipLaunchKernelGGL(k_gj_finish, dim3((unsigned)(((int64_t)nI * N + 255) / 256)), dim3(256), 0, st, aug, nI, N, ld,
@@ -1574,17 +1076,23 @@ void csr_defect(int n, const int *rp, const int *kc, const T *val, const T *x, c
   const int g = (int)(((int64_t)n * 16 + kBlock - 1) / kBlock);
   hipLaunchKernelGGL(k_csr_spmv<T>, dim3(g), dim3(kBlock), 0, st, n, rp, kc, val, x, r, b);
 }
-void csr_to_css(const DevLayout &D, const int *rowptr, const int *kcol, const int *dof2lat, int64_t active,
-                const double *in, double *val, hipStream_t st) {
+void csr_to_values(const DevLayout &D, const int *rowptr, const int *kcol, const int *dof2lat, int64_t active,
+                   const double *in, double *val, hipStream_t st) {
   if (active == 0) return;
-  hipLaunchKernelGGL(k_csr_to_css, dim3((unsigned)((active + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, rowptr,
-                     kcol, dof2lat, active, D.M, D.S, D.segidx, D.segs, in, val);
+  const dim3 g((unsigned)((active + kBlock - 1) / kBlock));
+  if (D.order == 2)
+    hipLaunchKernelGGL(k_csr_to_values<2>, g, dim3(kBlock), 0, st, rowptr, kcol, dof2lat, active, D.M, in, val);
+  else
+    hipLaunchKernelGGL(k_csr_to_values<1>, g, dim3(kBlock), 0, st, rowptr, kcol, dof2lat, active, D.M, in, val);
 }
 template <typename T>
-void css_to_csr(const DevLayout &D, const int *rowptr, const int *kcol, const int *dof2lat, int64_t active,
-                const T *val, double *out, hipStream_t st) {
-  hipLaunchKernelGGL(k_css_to_csr<T>, dim3((unsigned)((D.N + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, rowptr,
-                     kcol, dof2lat, D.N, active, D.M, D.S, D.segidx, D.segs, val, out);
+void values_to_csr(const DevLayout &D, const int *rowptr, const int *kcol, const int *dof2lat, int64_t active,
+                   const T *val, double *out, hipStream_t st) {
+  const dim3 g((unsigned)((D.N + kBlock - 1) / kBlock));
+  if (D.order == 2)
+    hipLaunchKernelGGL((k_values_to_csr<T, 2>), g, dim3(kBlock), 0, st, rowptr, kcol, dof2lat, D.N, active, D.M, val, out);
+  else
+    hipLaunchKernelGGL((k_values_to_csr<T, 1>), g, dim3(kBlock), 0, st, rowptr, kcol, dof2lat, D.N, active, D.M, val, out);
 }
 
 // ---- Q2 one-matrix forms on MFMA: local matrices per cell, then a row gather.
@@ -1741,64 +1249,89 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_mfma(int n, int nq, int f
 // the slot of every cell entry are compile-time constants: along an axis
 // with extent 2 (even lattice coordinate, a vertex plane) the node is local
 // coordinate 2 - 2 i of cell i, along an axis with extent 1 local coordinate 1.
+// A wavefront's 64 rows lie in consecutive cells of one x-line of cells (or,
+// P < 64, of several lines 3 cells apart in y), so it fetches each incident
+// cell's 64 local rows of 224 bytes together, 14 lanes per row, through LDS
+// (rows padded to 29 doubles), the next cell's while it adds the current one.
+// Bound by HBM: 64^3 Q2 reads the 1.6 GB cell buffer and writes 1.05 GB of
+// values in 0.6 ms; a row per lane straight from memory, 14 loads that each
+// touch 64 cache lines, took 0.77 - 1.1 ms.
+constexpr int kKcPad = kKcRow + 1;
 template <int EX, int EY, int EZ>
-__device__ __forceinline__ void assemble_row_kc(const DevSegment &s, int idx, int M, int n,
-                                                const double *__restrict__ kc, double *__restrict__ val,
+__device__ __forceinline__ void assemble_row_kc(double (*sh)[64 * kKcPad], bool ok, int px, int py, int pz, int lg, int M,
+                                                int n, const double *__restrict__ kc, double *__restrict__ val,
                                                 double *__restrict__ rhs) {
-  constexpr int NCX = EX == 1 ? 1 : 2, NCY = EY == 1 ? 1 : 2, NCZ = EZ == 1 ? 1 : 2;
+  constexpr int NCX = EX == 1 ? 1 : 2, NCY = EY == 1 ? 1 : 2, NCZ = EZ == 1 ? 1 : 2, NC = NCX * NCY * NCZ;
   constexpr int WX = 2 * EX + 1, WY = 2 * EY + 1, WZ = 2 * EZ + 1, NS = WX * WY * WZ;
-  const int i = idx % s.cx, t = idx / s.cx;
-  const int j = t % s.cy, k = t / s.cy;
-  const int px = s.x0 + s.stride * i, py = s.y0 + s.stride * j, pz = s.z0 + s.stride * k;
-  double *v = val + vbase(s, idx);
+  constexpr int PIECES = kKcRow / 2;
+  const int lane = threadIdx.x;
+  const int P = 1 << lg;
+  // row r of the wavefront: local row a(cell) of the cell c0 + (r & (P-1)) + 3 n (r >> lg)
+  const int x0 = __builtin_amdgcn_readfirstlane(px), y0 = __builtin_amdgcn_readfirstlane(py),
+            z0 = __builtin_amdgcn_readfirstlane(pz);
+  const int64_t last = (int64_t)n * n * n - 1;
+  double2 part[PIECES];
+  auto fetch = [&](int i) {
+    const int ix = i % NCX, iy = (i / NCX) % NCY, iz = i / (NCX * NCY);
+    const int ax = EX == 1 ? 1 : 2 - 2 * ix, ay = EY == 1 ? 1 : 2 - 2 * iy, az = EZ == 1 ? 1 : 2 - 2 * iz;
+    const int a = ax + 3 * (ay + 3 * az);
+    const int64_t c0 = ((x0 - 1) / 2 + ix) + (int64_t)n * (((y0 - 1) / 2 + iy) + (int64_t)n * ((z0 - 1) / 2 + iz));
+#pragma unroll
+    for (int e = 0; e < PIECES; e++) {
+      const int id = lane + 64 * e, r = id / PIECES, q = id % PIECES;
+      int64_t cell = c0 + (lg >= 6 ? r : (r & (P - 1)) + 3 * n * (r >> lg));
+      cell = cell < last ? cell : last;  // rows past the lattice (not stored)
+      part[e] = reinterpret_cast<const double2 *>(kc + (cell * 27 + a) * kKcRow)[q];
+    }
+  };
+  const int *pos = group_table<2>().pos[__builtin_amdgcn_readfirstlane(line_class<2>(py, pz))];
+  double *v = val + line_values<double, 2>(P, Lines<2>::group_base(P, py, pz), (px - 1) >> 1);
   double frhs = 0;
   double acc[NS];
 #pragma unroll
   for (int q = 0; q < NS; q++) acc[q] = 0.0;
-  const int cx0 = (px - 1) / 2, cy0 = (py - 1) / 2, cz0 = (pz - 1) / 2;
+  fetch(0);
 #pragma unroll
-  for (int iz = 0; iz < NCZ; iz++)
+  for (int i = 0; i < NC; i++) {
+    double *buf = sh[i & 1];
 #pragma unroll
-    for (int iy = 0; iy < NCY; iy++)
+    for (int e = 0; e < PIECES; e++) {
+      const int id = lane + 64 * e, r = id / PIECES, q = id % PIECES;
+      buf[r * kKcPad + 2 * q] = part[e].x;
+      buf[r * kKcPad + 2 * q + 1] = part[e].y;
+    }
+    if (i + 1 < NC) fetch(i + 1);
+    __syncthreads();  // one wavefront
+    const int ix = i % NCX, iy = (i / NCX) % NCY, iz = i / (NCX * NCY);
+    const int ax = EX == 1 ? 1 : 2 - 2 * ix, ay = EY == 1 ? 1 : 2 - 2 * iy, az = EZ == 1 ? 1 : 2 - 2 * iz;
+    const double *row = buf + lane * kKcPad;
 #pragma unroll
-      for (int ix = 0; ix < NCX; ix++) {
-        const int ax = EX == 1 ? 1 : 2 - 2 * ix, ay = EY == 1 ? 1 : 2 - 2 * iy, az = EZ == 1 ? 1 : 2 - 2 * iz;
-        const int a = ax + 3 * (ay + 3 * az);
-        const int64_t cell = (cx0 + ix) + (int64_t)n * ((cy0 + iy) + (int64_t)n * (cz0 + iz));
-        const double2 *Kr = reinterpret_cast<const double2 *>(kc + (cell * 27 + a) * kKcRow);
-        double row[kKcRow];
+    for (int b = 0; b < 27; b++) {
+      const int dx = b % 3 - ax, dy = (b / 3) % 3 - ay, dz = b / 9 - az;
+      acc[(dx + EX) + WX * ((dy + EY) + WY * (dz + EZ))] += row[b];
+    }
+    frhs += row[27];
 #pragma unroll
-        for (int e = 0; e < kKcRow / 2; e++) {
-          const double2 u = Kr[e];
-          row[2 * e] = u.x;
-          row[2 * e + 1] = u.y;
-        }
-#pragma unroll
-        for (int b = 0; b < 27; b++) {
-          const int dx = b % 3 - ax, dy = (b / 3) % 3 - ay, dz = b / 9 - az;
-          acc[(dx + EX) + WX * ((dy + EY) + WY * (dz + EZ))] += row[b];
-        }
-        frhs += row[27];
-#pragma unroll
-        for (int q = 0; q < NS; q++) {
-          const int dx = q % WX - EX, dy = (q / WX) % WY - EY, dz = q / (WX * WY) - EZ;
-          const int lx = (NCX == 2 && dx >= 0) ? 1 : 0, ly = (NCY == 2 && dy >= 0) ? 1 : 0,
-                    lz = (NCZ == 2 && dz >= 0) ? 1 : 0;
-          if (lx == ix && ly == iy && lz == iz) v[q * kSlice] = acc[q];
-        }
-      }
-  rhs[px + M * (py + M * pz)] = frhs;
+    for (int q = 0; q < NS; q++) {
+      const int dx = q % WX - EX, dy = (q / WX) % WY - EY, dz = q / (WX * WY) - EZ;
+      const int lx = (NCX == 2 && dx >= 0) ? 1 : 0, ly = (NCY == 2 && dy >= 0) ? 1 : 0,
+                lz = (NCZ == 2 && dz >= 0) ? 1 : 0;
+      if (lx == ix && ly == iy && lz == iz && ok)
+        v[(int64_t)(pos[(dy + 2) + 5 * (dz + 2)] * Lines<2>::VL + (EX == 1 ? dx + 1 : dx + 5)) * P] = acc[q];
+    }
+  }
+  if (ok) rhs[px + M * (py + M * pz)] = frhs;
 }
-__global__ __launch_bounds__(kRowsPerBlock) void k_assemble_kc(const BlockInfo *__restrict__ blocks,
-                                                               const DevSegment *__restrict__ segs, int M, int n,
+__global__ __launch_bounds__(kRowsPerBlock) void k_assemble_kc(LineSet set, int lg, int M, int n,
                                                                const double *__restrict__ kc,
                                                                double *__restrict__ val, double *__restrict__ rhs) {
-  const BlockInfo bi = blocks[xcd_remap(blockIdx.x, gridDim.x)];
-  const DevSegment s = segs[bi.seg];
-  const int idx = bi.base + threadIdx.x;
-  if (idx >= s.count) return;
-#define PMX_KROW(EX, EY, EZ) assemble_row_kc<EX, EY, EZ>(s, idx, M, n, kc, val, rhs)
-  switch (s.ex * 100 + s.ey * 10 + s.ez) {
+  static_assert(kRowsPerBlock == 64, "one wavefront");
+  __shared__ double sh[2][64 * kKcPad];
+  int px, py, pz;
+  const bool ok = unit_row<2>(set, M, lg, &px, &py, &pz);
+  const int code = unit_shape<2>(lg, set, M);
+#define PMX_KROW(EX, EY, EZ) assemble_row_kc<EX, EY, EZ>(sh, ok, px, py, pz, lg, M, n, kc, val, rhs)
+  switch (code) {
     case 111: PMX_KROW(1, 1, 1); break;
     case 211: PMX_KROW(2, 1, 1); break;
     case 121: PMX_KROW(1, 2, 1); break;
@@ -1816,6 +1349,9 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
               bool qp_given, double *ftab, const uint8_t *corner) {
   const int64_t ncells = (int64_t)D.n * D.n * D.n;
   const int64_t ncq = ncells * nq;
+  int units;
+  const LineSet set = all_lines(D, &units);
+  const dim3 gr(row_blocks(D, units));
   // with the per-cell frame codes (CELL_MEASURE 4) the coefficients go
   // through the qp records, which carry the cell's first-point size
   const bool inl = !qp_given && coeffs_inline(example) && !corner;
@@ -1854,8 +1390,7 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
   if (form == PMX_FORM_RHS || form == PMX_FORM_RHS_SUPG) {
     // right-hand-side forms (no local matrices): the matrices are left as they are
 #define PMX_RHS(O, IN)                                                                                     \
-  hipLaunchKernelGGL((k_assemble<O, false, IN, true>), dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st,        \
-                     D.blocks_all, D.segs, D.M, D.n, nq, prm_dev, qref, qsrc, tab, nullptr, nullptr, rhs)
+  hipLaunchKernelGGL((k_assemble<O, false, IN, true>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq, prm_dev, qref, qsrc, tab, nullptr, nullptr, rhs)
     if (D.order == 1) {
       if (inl) PMX_RHS(1, true);
       else PMX_RHS(1, false);
@@ -1885,8 +1420,7 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
       else PMX_CELL(false, false);
     }
 #undef PMX_CELL
-    hipLaunchKernelGGL(k_assemble_kc, dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st, D.blocks_all, D.segs, D.M, D.n,
-                       kc, val, rhs);
+    hipLaunchKernelGGL(k_assemble_kc, gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, kc, val, rhs);
     hipLaunchKernelGGL(k_boundary_rhs, dim3((D.nboundary + kBlock - 1) / kBlock), dim3(kBlock), 0, st, D.boundary,
                        D.nboundary, D.M, prm_dev, rhs);
     return;
@@ -1899,9 +1433,7 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
     if (val2) check(hipMemsetAsync(val2, 0, sizeof(double) * D.nvals, st), "memset val2");
   }
 #define PMX_ASM(O, TW, IN)                                                                                   \
-  hipLaunchKernelGGL((k_assemble<O, TW, IN, false>), dim3(D.nblocks_all), dim3(kRowsPerBlock), 0, st,             \
-                     D.blocks_all,                                                                                \
-                     D.segs, D.M, D.n, nq, prm_dev, qref, qsrc, tab, val, val2, rhs)
+  hipLaunchKernelGGL((k_assemble<O, TW, IN, false>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq, prm_dev, qref, qsrc, tab, val, val2, rhs)
 #define PMX_ASM2(O, TW) \
   do {                   \
     if (inl) PMX_ASM(O, TW, true); \
@@ -2069,23 +1601,18 @@ void set_scalar(double *dst, const double *src, double scale, hipStream_t st) {
   template void mgs_arnoldi<T>(T *, const T *, int64_t, int, double *, T *, double *, hipStream_t);         \
   template void axpy_diff<T>(T *, const T *, const T *, int64_t, hipStream_t);                              \
   template void step_length_update<T>(T *, const T *, const double *, double, int64_t, hipStream_t);        \
-  template void css_apply<T>(const DevLayout &, int, const T *, const T *, const T *, T *, double, int,     \
-                             hipStream_t);                                                                  \
   template void boundary<T>(const DevLayout &, int, T *, const T *, const T *, hipStream_t);                \
-  template void sweep_wg<T>(const DevLayout &, const T *, T *, const T *, double, int, hipStream_t);          \
-  template void coarse_wg<T>(const DevLayout &, const T *, T *, const T *, double, int, int, double, T *, T *, \
-                             hipStream_t);                                                                  \
   template void prolongate<T>(const DevLayout &, const DevLayout &, const T *, T *, hipStream_t);           \
   template void prolongate_add<T>(const DevLayout &, const DevLayout &, const T *, T *, double, hipStream_t); \
   template void restrict_<T>(const DevLayout &, const DevLayout &, T *, const T *, hipStream_t, bool);      \
   template void gemv_coarse<T>(int, int, const double *, const int *, const T *, T *, hipStream_t);         \
   template void csr_spmv<T>(int, const int *, const int *, const T *, const T *, T *, hipStream_t);         \
   template void csr_defect<T>(int, const int *, const int *, const T *, const T *, const T *, T *, hipStream_t); \
-  template void css_to_csr<T>(const DevLayout &, const int *, const int *, const int *, int64_t, const T *, \
+  template void values_to_csr<T>(const DevLayout &, const int *, const int *, const int *, int64_t, const T *, \
                               double *, hipStream_t);
 PMX_INST(double)
 PMX_INST(float)
-template void css_to_csr<_Float16>(const DevLayout &, const int *, const int *, const int *, int64_t,
+template void values_to_csr<_Float16>(const DevLayout &, const int *, const int *, const int *, int64_t,
                                    const _Float16 *, double *, hipStream_t);
 template void fill<uint16_t>(uint16_t *, uint16_t, int64_t, hipStream_t);
 template void fill<int>(int *, int, int64_t, hipStream_t);

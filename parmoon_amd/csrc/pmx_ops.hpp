@@ -12,22 +12,12 @@ namespace pmx {
 
 // device mirror of a Layout
 struct DevLayout {
-  int order = 1, n = 0, M = 0, S = 2;
+  int order = 1, n = 0, M = 0;
+  int lg = 0;  // log2 of the row pairs per line, (M - 1) / 2
   int64_t N = 0, nvals = 0, nactive = 0;
   int nboundary = 0;
   int *boundary = nullptr;
-  DevSegment *segs = nullptr;
-  int *segidx = nullptr;  // residue class (rx + S(ry + S rz)) -> segment, -1 if empty
-  BlockInfo *blocks_all = nullptr;  // all rows, spatial order (z, y of the first row)
-  int nblocks_all = 0;
-  BlockInfo *blocks_colour = nullptr;
-  const RowBlock *rows_all = nullptr;     // blocks_all with the class records inline (row kernels)
-  const RowBlock *rows_colour = nullptr;  // blocks_colour likewise
-  std::vector<int> colour_off;  // host: block offsets per colour
-  int *colour_off_dev = nullptr;  // the same on the device
-  int *colour_seg_dev = nullptr;  // first segment of each colour (segments are colour-major), ncolours + 1
   int64_t max_colour_rows = 0;    // rows of the largest colour
-  int nsegs = 0;                  // residue classes with rows
   int ncolours = 0;
 };
 
@@ -52,15 +42,15 @@ struct DispatchTimer {
   DispatchTimer &operator=(const DispatchTimer &) = delete;
   ~DispatchTimer();
 };
-// while installed (non-null), the row kernels of css_apply record each
-// dispatch between two events of the timer; nullptr uninstalls
+// while installed (non-null), the launched row kernels record each dispatch
+// between two events of the timer; nullptr uninstalls
 void set_dispatch_timer(DispatchTimer *t);
 
 // calibration of the dispatch measurements (both honour the dispatch timer):
-// a dispatch of `blocks` workgroups that does nothing, and a plain streaming
-// read of `bytes` bytes at p (16-byte aligned; sink: one float, written never
-// in practice)
-void empty_dispatch(int blocks, hipStream_t st);
+// a dispatch that does nothing with the workgroups of a line group's launch,
+// and a plain streaming read of `bytes` bytes at p (16-byte aligned; sink: one
+// float, written never in practice)
+void empty_dispatch(const DevLayout &D, int group, hipStream_t st);
 void stream_read(const void *p, int64_t bytes, float *sink, hipStream_t st);
 
 template <typename T> void fill(T *x, T v, int64_t n, hipStream_t st);
@@ -91,10 +81,22 @@ void step_length_update(T *u, const T *uold, const double *num_nom, double param
 template <typename T>
 void mgs_arnoldi(T *w, const T *V, int64_t n, int k1, double *h, T *vnext, double *part, hipStream_t st);
 
-// mode 0 spmv, 1 defect, 2 jacobi (x = old iterate, y = new), 3 sor (in place on y); colour -1 = all classes
+// mode 0 product, 1 defect, 2 Jacobi (x = old iterate, y = new) over the
+// interior rows (Dirichlet rows: boundary)
 template <typename T>
-void css_apply(const DevLayout &D, int mode, const T *val, const T *x, const T *f, T *y, double omega, int colour,
-               hipStream_t st);
+void rows_apply(const DevLayout &D, int mode, const T *val, const T *x, const T *f, T *y, double omega,
+                hipStream_t st);
+// n SOR (forward) or SSOR sweeps in colour order, one launch per line group;
+// the Dirichlet entries of x are left as they are
+template <typename T>
+void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, double omega, bool ssor, int n, hipStream_t st);
+// the same on the row-scaled FP16 values and the FP32 1/diag of scaled_values
+void sor_sweeps_scaled(const DevLayout &D, const _Float16 *val16, const float *dinv, float *x, const float *f,
+                       double omega, bool ssor, int n, hipStream_t st);
+// the lines of a launch over all interior lines / over a line group, and its
+// number of units
+LineSet all_lines(const DevLayout &D, int *units);
+LineSet group_lines(const DevLayout &D, int g, int *units);
 // out = {||u - u_h||_L2, |u - u_h|_H1} of the lattice function u (FP64) against
 // the example's exact solution with the rule of qref/tab (part: 2 kRedBlocks)
 void fe_errors(const DevLayout &D, const double *prm_dev, const double *qref, const double *tab, int nq,
@@ -104,20 +106,6 @@ bool bits_equal(const double *a, const double *b, int64_t n, int *flag, hipStrea
 // whole SOR (ssor 0) / SSOR (ssor 1) sweep with Dirichlet rows x = f, one
 // workgroup with the level's x in LDS (levels with M^3 * s <= kSweepLdsBytes)
 inline bool sweep_wg_fits(const DevLayout &D, size_t s) { return (int64_t)D.N * (int64_t)s <= kSweepLdsBytes; }
-// Lanes per row of the row kernels on a level (the same for every kernel and
-// precision of the level, so the single-workgroup and the launch-per-colour
-// sweeps compute each row alike): 4 where a colour has at most kSweepWgRows
-// rows (few rows: more lanes per row shorten the load chain of each), 1 from
-// 2^20 active rows on (one lane per row touches the fewest cache lines per
-// gathered x run), 2 between.
-inline int row_lanes(const DevLayout &D) {
-  if (D.max_colour_rows <= kSweepWgRows) return 4;
-  return D.nactive >= (int64_t(1) << 20) ? 1 : 2;
-}
-// one SOR colour (mode 4 of k_rows) on the row-scaled FP16 values and the
-// FP32 1/diag of scaled_values; x in place
-void css_sor_scaled(const DevLayout &D, const _Float16 *val16, const float *dinv, float *x, const float *f,
-                    double omega, int colour, hipStream_t st);
 // the row-scaled FP16 copy of the FP32 stencil values (a_ij / a_ii,
 // saturated to the finite FP16 range) and dinv = 1 / a_ii on the active rows
 void scaled_values(const DevLayout &D, const float *val, _Float16 *val16, float *dinv, hipStream_t st);
@@ -126,10 +114,10 @@ void sweep_wg(const DevLayout &D, const T *val, T *x, const T *f, double omega, 
 // the coarse-level smoothing loop of TMultiGrid3D (MultiGrid3D.C:225-337) in
 // one workgroup (levels with sweep_wg_fits): sweeps of kind 1 Jacobi, 2 SOR,
 // 3 SSOR while ||f - A x|| > red ||f - A x_0|| and fewer than maxit were
-// made; d, xj: scratch of D.N entries
+// made; xj: scratch of D.N entries
 template <typename T>
 void coarse_wg(const DevLayout &D, const T *val, T *x, const T *f, double omega, int kind, int maxit, double red,
-               T *d, T *xj, hipStream_t st);
+               T *xj, hipStream_t st);
 // Dirichlet rows: mode 0 y=x, 1 y=f-x, 2 y=f, 3 y=0
 template <typename T> void boundary(const DevLayout &D, int mode, T *y, const T *x, const T *f, hipStream_t st);
 template <typename T>
@@ -148,20 +136,20 @@ template <typename T>
 void gemv_coarse(int nI, int N, const double *W, const int *iidx, const T *x, T *y, hipStream_t st);
 // W of the level by Gauss-Jordan with partial pivoting (cidx: lattice node ->
 // interior row or -1; aug: n_I x (n_I + N) workspace; piv: n_I ints)
-void coarse_inverse_dense(const DevLayout &D, const double *val, const int *cidx, int nI, double *aug, int *piv,
-                          double *W, hipStream_t st);
+void coarse_inverse_dense(const DevLayout &D, const double *val, const int *iidx, const int *cidx, int nI, double *aug,
+                          int *piv, double *W, hipStream_t st);
 template <typename T, typename U> void gather(T *out, const U *in, const int *map, int64_t n, hipStream_t st);
 template <typename T>
 void csr_spmv(int n, const int *rp, const int *kc, const T *val, const T *x, T *y, hipStream_t st);
 // r = b - A x on a CSR matrix
 template <typename T>
 void csr_defect(int n, const int *rp, const int *kc, const T *val, const T *x, const T *b, T *r, hipStream_t st);
-// CSR entries with the level's pattern (reference numbering) into the CSS
-// values of the active rows (the inverse of css_to_csr there)
-void csr_to_css(const DevLayout &D, const int *rowptr, const int *kcol, const int *dof2lat, int64_t active,
+// CSR entries with the level's pattern (reference numbering) into the line
+// layout's values of the active rows (the inverse of values_to_csr there)
+void csr_to_values(const DevLayout &D, const int *rowptr, const int *kcol, const int *dof2lat, int64_t active,
                 const double *in, double *val, hipStream_t st);
 template <typename T>
-void css_to_csr(const DevLayout &D, const int *rowptr, const int *kcol, const int *dof2lat, int64_t active,
+void values_to_csr(const DevLayout &D, const int *rowptr, const int *kcol, const int *dof2lat, int64_t active,
                 const T *val, double *out, hipStream_t st);
 // example: prm[PMX_PRM_EXAMPLE] (selects evaluating the coefficients inline or
 // through the quadrature-point buffer); form: prm[PMX_PRM_FORM]; kc: cell
