@@ -74,6 +74,7 @@ template <typename T>
 struct Vecs {
   DevBuf<T> val;                      // values (line layout) in this precision
   DevBuf<T> x, f, d, aux;             // MG level vectors
+  DevBuf<T> psum;                     // half sums of the SSOR sweeps (sor_sweeps)
   DevBuf<T> sold, sdef;               // step length control: u and f - A u before the pre-smoothing
 };
 
@@ -147,6 +148,7 @@ struct System {
     bool valid = false;
     int prec = 0;
     double key[16] = {0};
+    bool upper = false;  // the cycle leaves the upper sums of its result
     hipGraphExec_t exec = nullptr;
   };
   Graph graphs[2];
@@ -170,6 +172,7 @@ struct System {
   // values (opt[15] = 3 / 4)
   bool half_smoother = false;
   DevBuf<double> lscal;               // norm, (d, Ac), (Ac, Ac)
+  DevBuf<int> bnd_set;                // start_zero / start_boundary
   ~System() {
     for (auto &n : nets) n.release();
     for (auto &g : graphs)
@@ -228,7 +231,7 @@ static void setup_level(System &Y, Level &lv, int nref) {
 
   lv.rhs.alloc(L.N);
   lv.v64.val.alloc_zeroed(L.nstored, st);
-  for (auto *b : {&lv.v64.x, &lv.v64.f, &lv.v64.d, &lv.v64.aux}) b->alloc(L.N);
+  for (auto *b : {&lv.v64.x, &lv.v64.f, &lv.v64.d, &lv.v64.aux, &lv.v64.psum}) b->alloc(L.N);
 }
 
 // Gauss rules of src/QuadFormulas/QuadFormulaHexa.C:70-146 and Q1/Q2 Lagrange
@@ -358,7 +361,7 @@ static void ensure_val32(System &Y) {
     if (!lv.v32.val.p) {
       Y.invalidate_graphs();
       lv.v32.val.alloc(lv.L.nstored);
-      for (auto *b : {&lv.v32.x, &lv.v32.f, &lv.v32.d, &lv.v32.aux}) b->alloc(lv.L.N);
+      for (auto *b : {&lv.v32.x, &lv.v32.f, &lv.v32.d, &lv.v32.aux, &lv.v32.psum}) b->alloc(lv.L.N);
       // the defect's Dirichlet entries are read by the learned step with zero
       // weights only (dinv and A c vanish there), so they just have to be finite
       fill<float>(lv.v32.d.p, 0.0f, lv.L.N, Y.ctx->st);
@@ -412,8 +415,13 @@ static void ensure_learned(System &Y) {
 }
 
 // ------------------------------------------------------------- multigrid
+// What is known of a level's x when its smoothing starts: nothing; zero in the
+// interior (x = f on the Dirichlet nodes, Y.bnd_set tells if those are zero);
+// zero everywhere, and f zero on the Dirichlet nodes.
+enum { kStartAny = 0, kStartInteriorZero = 1, kStartZero = 2 };
+// `sweeps` sweeps on v.x; true: v.psum holds the upper sums of the result
 template <typename T>
-static void level_smooth(System &Y, Level &lv, int kind, double omega, int sweeps) {
+static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweeps, int start = kStartAny) {
   hipStream_t st = Y.ctx->st;
   Vecs<T> &v = vecs<T>(lv);
   // levels whose largest colour has at most this many rows sweep in one
@@ -427,23 +435,26 @@ static void level_smooth(System &Y, Level &lv, int kind, double omega, int sweep
       boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
       rows_apply<T>(lv.D, 2, v.val.p, v.aux.p, v.f.p, v.x.p, omega, st);
     }
-    return;
+    return false;
   }
-  if (sweeps < 1) return;
+  if (sweeps < 1) return false;
   if (lv.D.max_colour_rows <= wg_limit && sweep_wg_fits(lv.D, sizeof(T))) {
     for (int s = 0; s < sweeps; s++) sweep_wg<T>(lv.D, v.val.p, v.x.p, v.f.p, omega, kind == 3 ? 1 : 0, st);
-    return;
+    return false;
   }
   // Dirichlet rows x = f (no sweep changes them afterwards)
-  boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
+  if (start == kStartAny) boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
+  const int *bs = start == kStartInteriorZero ? Y.bnd_set.p : nullptr;
   if constexpr (std::is_same<T, float>::value) {
     if (Y.half_smoother) {
       if (!lv.have_val16) throw std::logic_error("level_smooth: FP16 smoother values missing");
-      sor_sweeps_scaled(lv.D, lv.val16.p, lv.sdinv.p, v.x.p, v.f.p, omega, kind == 3, sweeps, st);
-      return;
+      sor_sweeps_scaled(lv.D, lv.val16.p, lv.sdinv.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps,
+                        start != kStartAny, bs, st);
+      return false;
     }
   }
-  sor_sweeps<T>(lv.D, v.val.p, v.x.p, v.f.p, omega, kind == 3, sweeps, st);
+  sor_sweeps<T>(lv.D, v.val.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps, start != kStartAny, bs, st);
+  return kind == 3;
 }
 // Learned post-smoothing of one level (replaces the post-sweeps of
 // TMGLevel3D; no counterpart in the reference): with d = f - A x and
@@ -499,9 +510,10 @@ static bool learned_level(const System &Y, int i) {
   const int n = (int)Y.lev.size();
   return Y.learn_active && i >= n - Y.learned_levels && i < n - Y.learned_skip;
 }
+// start: what is known of level i's x on entry (kStartZero: the first visit
+// after the Reset).  True: v.psum holds the upper sums of the level's result.
 template <typename T>
-// x_zero: x of level i is 0 on entry (the first visit after the Reset)
-static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
+static bool mg_cycle(System &Y, int i, bool post = true, int start = kStartAny) {
   hipStream_t st = Y.ctx->st;
   const double *o = Y.opt;
   Level &lv = *Y.lev[i];
@@ -521,7 +533,7 @@ static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
     } else {
       level_smooth<T>(Y, lv, cs == 17 ? 3 : cs, o[8], std::max(1, (int)o[10]));
     }
-    return;
+    return false;
   }
   Level &cl = *Y.lev[i - 1];
   Vecs<T> &cv = vecs<T>(cl);
@@ -535,29 +547,28 @@ static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
     rows_apply<T>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.sdef.p, 0.0, st);
     boundary<T>(lv.D, 1, v.sdef.p, v.x.p, v.f.p, st);
   }
-  bool pre_done = false;
+  bool pre_done = false, upper = false;
   if constexpr (std::is_same<T, float>::value) {
     if (Y.learned_pre && learned_level(Y, i)) {
       // the steps leave the defect of their last update in v.d
-      learned_smooth(Y, lv, Y.nets[i], std::max(1, (int)o[20]), true, x_zero);
+      learned_smooth(Y, lv, Y.nets[i], std::max(1, (int)o[20]), true, start == kStartZero);
       pre_done = true;
     }
   }
   if (!pre_done) {
-    level_smooth<T>(Y, lv, kind, o[8], (int)o[6]);
-    rows_apply<T>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, st);
+    const bool u = level_smooth<T>(Y, lv, kind, o[8], (int)o[6], start);
+    rows_apply<T>(lv.D, 1, v.val.p, v.x.p, v.f.p, v.d.p, 0.0, st, u ? v.psum.p : nullptr);
   }
   // the defect's Dirichlet entries are not set: the restriction to an
   // interior coarse node reads interior fine nodes only (taps 2y-3..2y+3 and
   // 2y-1..2y+1 with 1 <= y <= Mc-2), and the coarse surface is set to 0
-  // (CorrectDefect)
-  restrict_<T>(cl.D, lv.D, cv.f.p, v.d.p, st, true);
-  fill<T>(cv.x.p, (T)0, cl.L.N, st);                   // Reset
+  // (CorrectDefect); the coarse x is set to 0 (Reset)
+  restrict_<T>(cl.D, lv.D, cv.f.p, v.d.p, st, cv.x.p);
   // the first visit of the coarse level starts from its Reset (x = 0); the
   // learned pre-smoothing there takes d = f (restrict_ with zero_surface
   // leaves the coarse f zero on the Dirichlet surface, so the Dirichlet
   // entries of that defect are the ones A x = 0 would give)
-  for (int j = 0; j < Y.rec[i]; j++) mg_cycle<T>(Y, i - 1, true, j == 0 && Y.x_zero_shortcut);
+  for (int j = 0; j < Y.rec[i]; j++) mg_cycle<T>(Y, i - 1, true, j == 0 && Y.x_zero_shortcut ? kStartZero : kStartAny);
   if ((int)o[12] < 1) Y.rec[i] = 1;
   // prolongation, CorrectNodes and x += SC_GMG_DAMP e
   prolongate_add<T>(cl.D, lv.D, cv.x.p, v.x.p, o[13], st);
@@ -569,7 +580,7 @@ static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
         post_done = true;
       }
     }
-    if (!post_done) level_smooth<T>(Y, lv, kind, o[8], (int)o[7]);
+    if (!post_done) upper = level_smooth<T>(Y, lv, kind, o[8], (int)o[7]);
   }
   if (slc) {
     // TMGLevel3D::StepLengthControl (MGLevel3D.C:908-960), MultiGrid3D.C:671-679:
@@ -581,7 +592,9 @@ static void mg_cycle(System &Y, int i, bool post = true, bool x_zero = false) {
     dot<T>(v.sdef.p, v.d.p, lv.L.N, Y.ctx->part.p, num, 0, st);
     dot<T>(v.d.p, v.d.p, lv.L.N, Y.ctx->part.p, num + 1, 0, st);
     step_length_update<T>(v.x.p, v.sold.p, num, o[8], lv.L.N, st);
+    upper = false;
   }
+  return upper;
 }
 // TMultiGrid3D::SetRecursion (MultiGrid3D.C:697-725): gamma cycles per level
 static void set_recursion(System &Y) {
@@ -590,27 +603,27 @@ static void set_recursion(System &Y) {
   Y.rec.assign(Y.lev.size() + 1, 1);
   for (int k = 2; k <= L; k++) Y.rec[k] = gam > 0 ? gam : 2;
 }
-// one MG cycle on the finest level's f -> x (zero start, SetDirichletNodes)
+// one MG cycle on the finest level's f -> x (zero start, SetDirichletNodes);
+// x = 0 and *Y.bnd_set = 0 on entry
 template <typename T>
-static void mg_cycle_from_zero(System &Y) {
-  hipStream_t st = Y.ctx->st;
+static bool mg_cycle_from_zero(System &Y) {
   const int L = (int)Y.lev.size() - 1;
   Level &lv = *Y.lev[L];
   Vecs<T> &v = vecs<T>(lv);
-  fill<T>(v.x.p, (T)0, lv.L.N, st);
-  boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);  // SetDirichletNodes
+  start_boundary<T>(lv.D, v.x.p, v.f.p, Y.bnd_set.p, Y.ctx->st);  // SetDirichletNodes
   set_recursion(Y);
-  mg_cycle<T>(Y, L);
+  return mg_cycle<T>(Y, L, true, kStartInteriorZero);
 }
 // z = MG(v): TMultiGridScaIte::Iterate with zero start (MultiGridScaIte.C:89-130).
-// The cycle (about a thousand kernels for 5 Q2 levels) is captured once into a
-// HIP graph and replayed, so the GPU is not left waiting on launches.
+// The cycle is captured once into a HIP graph and replayed, so the GPU is not
+// left waiting on launches.  True: the finest level's psum holds the upper
+// sums of z.
 template <typename T>
-static void mg_prec(System &Y, T *z, const T *vin) {
+static bool mg_prec(System &Y, T *z, const T *vin) {
   hipStream_t st = Y.ctx->st;
   Level &lv = *Y.lev.back();
   Vecs<T> &v = vecs<T>(lv);
-  copy<T>(v.f.p, vin, lv.L.N, st);
+  start_zero<T>(v.f.p, v.x.p, vin, Y.bnd_set.p, lv.L.N, st);
   const int pi = std::is_same<T, double>::value ? 0 : 1;
   System::Graph &g = Y.graphs[pi];
   double key[16];
@@ -623,13 +636,14 @@ static void mg_prec(System &Y, T *z, const T *vin) {
   key[13] = learned ? Y.learned_pre : 0;
   key[14] = Y.slc;
   key[15] = pi == 1 && Y.half_smoother ? 1 : 0;
+  bool upper;
   if (Y.use_graphs) {
     if (!g.valid || std::memcmp(key, g.key, sizeof(key)) != 0) {
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
       g.exec = nullptr;
       hipGraph_t graph;
       check(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "begin capture");
-      mg_cycle_from_zero<T>(Y);
+      g.upper = mg_cycle_from_zero<T>(Y);
       check(hipStreamEndCapture(st, &graph), "end capture");
       check(hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0), "graph instantiate");
       (void)hipGraphDestroy(graph);
@@ -637,16 +651,19 @@ static void mg_prec(System &Y, T *z, const T *vin) {
       g.valid = true;
     }
     check(hipGraphLaunch(g.exec, st), "graph launch");
+    upper = g.upper;
   } else {
-    mg_cycle_from_zero<T>(Y);
+    upper = mg_cycle_from_zero<T>(Y);
   }
   copy<T>(z, v.x.p, lv.L.N, st);
+  return upper;
 }
 
 // y = A x on the finest level (stencil + Dirichlet identity rows); in FP64
 // the caller's CSR matrix instead while pmx_iterate runs
+// (upper: x is the result that mg_prec has just left, with its upper sums)
 template <typename T>
-static void fine_matvec(System &Y, const T *x, T *y) {
+static void fine_matvec(System &Y, const T *x, T *y, bool upper = false) {
   Level &lv = *Y.lev.back();
   if constexpr (std::is_same<T, double>::value) {
     if (Y.use_ucsr) {
@@ -654,7 +671,7 @@ static void fine_matvec(System &Y, const T *x, T *y) {
       return;
     }
   }
-  rows_apply<T>(lv.D, 0, vecs<T>(lv).val.p, x, nullptr, y, 0.0, Y.ctx->st);
+  rows_apply<T>(lv.D, 0, vecs<T>(lv).val.p, x, nullptr, y, 0.0, Y.ctx->st, upper ? vecs<T>(lv).psum.p : nullptr);
   boundary<T>(lv.D, 0, y, x, nullptr, Y.ctx->st);
 }
 template <typename T>
@@ -709,8 +726,8 @@ static int fgmres(System &Y, T *x, const T *b, int m, int maxit, double rmin, do
     int i;
     for (i = 0; i < m && j <= maxit; i++, j++) {
       T *vi = V + (size_t)i * N, *zi = Z + (size_t)i * N;
-      mg_prec<T>(Y, zi, vi);
-      fine_matvec<T>(Y, zi, w);
+      const bool upper = mg_prec<T>(Y, zi, vi);
+      fine_matvec<T>(Y, zi, w, upper);
       mgs_arnoldi<T>(w, V, N, i + 1, H + (size_t)i * ld, V + (size_t)(i + 1) * N, part, st);
       givens(H, cs, sn, s, i, ld, res, st);
       const double r_prev = r;
@@ -818,8 +835,8 @@ static int bicgstab(System &Y, T *x, const T *b, int maxit, double rmin, double 
       check(hipMemcpyAsync(p, t, sizeof(T) * N, hipMemcpyDeviceToDevice, st), "copy");
     }
     rho_last = rho;
-    mg_prec<T>(Y, yv, p);
-    if (flexible) fine_matvec<T>(Y, yv, v);
+    bool upper = mg_prec<T>(Y, yv, p);
+    if (flexible) fine_matvec<T>(Y, yv, v, upper);
     else check(hipMemcpyAsync(v, yv, sizeof(T) * N, hipMemcpyDeviceToDevice, st), "copy");
     dot<T>(rt, v, N, part, sc + 1, 0, st);
     double delta = read_scalar(Y, sc + 1);
@@ -830,8 +847,8 @@ static int bicgstab(System &Y, T *x, const T *b, int maxit, double rmin, double 
     dot<T>(r, r, N, part, sc + 2, 1, st);
     dn = read_scalar(Y, sc + 2);
     if (dn < dn0 * red || dn < rmin) break;
-    mg_prec<T>(Y, yv, r);
-    if (flexible) fine_matvec<T>(Y, yv, t);
+    upper = mg_prec<T>(Y, yv, r);
+    if (flexible) fine_matvec<T>(Y, yv, t, upper);
     else check(hipMemcpyAsync(t, yv, sizeof(T) * N, hipMemcpyDeviceToDevice, st), "copy");
     dot<T>(t, t, N, part, sc + 3, 0, st);
     double tt = read_scalar(Y, sc + 3);
@@ -1369,6 +1386,7 @@ int pmx_system_create(pmx_ctx *ctx, int nref0, int nlev, int order, pmx_system *
       const Level &f = *Y.lev.back();
       Y.sol.alloc(f.L.N);
       Y.b.alloc(f.L.N);
+      Y.bnd_set.alloc(1);
       check(hipStreamSynchronize(ctx->c.st), "sync");
     } catch (...) {
       delete h;

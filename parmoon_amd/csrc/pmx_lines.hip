@@ -68,10 +68,13 @@ template <int O> __device__ __forceinline__ int run_split(int m, int P) { return
 // MODE 0: y = A x (MatVect, Blas2.C:86-118)
 // MODE 1: y = f - A x (ScalarDefect, Blas2.C:37-83)
 // MODE 2: y = (1-w) x + w (f - A_off x)/d (TMGLevel3D::Jacobi, MGLevel3D.C:469-563)
-template <typename T, int O, int MODE>
+// HALF (modes 0, 1): the sums over the groups after the lines are those that
+// the last backward sweep left in psum (x has not changed since), so only the
+// first half of the values is read.  64^3 Q2 FP32: 100 -> 53 us.
+template <typename T, int O, int MODE, bool HALF>
 __global__ __launch_bounds__(512) void k_line_rows(LineSet set, int lg, const T *__restrict__ val,
                                                    const T *__restrict__ x, const T *__restrict__ f,
-                                                   T *__restrict__ y, double omega) {
+                                                   T *__restrict__ y, double omega, const T *__restrict__ psum) {
   using L = Lines<O>;
   __shared__ PairSums<T> red[kSplits - 1][128];
   const int P = 1 << lg, M = 2 * P + 1, ul = lg < 6 ? 6 : lg;
@@ -84,8 +87,12 @@ __global__ __launch_bounds__(512) void k_line_rows(LineSet set, int lg, const T 
   const int nlo = g.nlo[c], ng = g.ng[c], d3 = run_split<O>(m, P);
   const T *v = val + line_values<T, O>(P, L::group_base(P, ly, u.z), m);
   const int p0 = M * (ly + M * u.z) + 2 * m;
-  T own[L::VL], xr[5], fo = 0, fe = 0;
+  T own[L::VL], xr[5], fo = 0, fe = 0, ho = 0, he = 0;
   if (w == 0) {
+    if (HALF) {
+      ho = psum[p0 + 1];
+      he = psum[p0 + 2];
+    }
     load_group<T, O>(v + (int64_t)nlo * (L::VL * P), P, own);
     load_run<T, 3>(x + p0, xr);
     load_run<T, O == 2 ? 2 : 1>(x + p0 + d3, xr + 3);
@@ -94,12 +101,16 @@ __global__ __launch_bounds__(512) void k_line_rows(LineSet set, int lg, const T 
       fe = f[p0 + 2];
     }
   }
-  PairSums<T> s = pair_sums<T, T, O, 2>(v, x + p0, g.off[c], nlo, ng, true, true, w, P, M, d3);
+  PairSums<T> s = pair_sums<T, T, O, 2>(v, x + p0, g.off[c], nlo, ng, true, !HALF, w, P, M, d3);
   if (w) red[w - 1][t] = s;
   __syncthreads();
   if (w || !ok) return;
 #pragma unroll
   for (int q = 0; q < kSplits - 1; q++) add_partial(s, red[q][t]);
+  if (HALF) {
+    s.hi_o = ho;
+    s.hi_e = he;
+  }
   T ro = own_odd<T, T, O>(own, xr, s.lo_o + s.hi_o), re = own_even<T, T, O>(own, xr, s.lo_e + s.hi_e);
   const T xo = xr[1], xe = xr[2];
   if (MODE == 2) {
@@ -166,13 +177,27 @@ __device__ __forceinline__ void line_steps(T *l, const V *own, const PairRow<T> 
 
 // One line group of a sweep; V = _Float16: row-scaled values a_ij / a_ii with
 // dinv = 1 / a_ii (x = w (f dinv - W_off x - x) + x).
+//
+// Half sums.  In a forward sweep the lines before a row's line already hold
+// their new x; the backward sweep reaches the row before it changes them, so
+// the row's sum over them is the same (and likewise the sums over the lines
+// after it from a backward to the next forward sweep).  The sums are kept in
+// psum: a backward launch reads only the values after its lines, a following
+// forward launch only those before them, and n symmetric sweeps read the
+// matrix n + 1/2 times (n when x starts at zero) instead of 2n.
 // Bound by the launch (about 4 us whatever its size) plus the values from HBM:
-// 64^3 Q2 FP32 15.9 us per group of 58 MB.  A launch per colour, 3 C^2 of
-// them, took 8.7 us each (26 us for the rows of a group).
+// 64^3 Q2 FP32 15.9 us per group of 58 MB with all values, 10 us with half of
+// them.  A launch per colour, 3 C^2 of them, took 8.7 us each (26 us for the
+// rows of a group).
+enum {
+  kSumLo = 1, kSumHi = 2,                         // sums to compute
+  kSumKept = 4,                                   // the other one is in psum (else it is 0)
+  kKeepLo = 16, kKeepHi = 32, kKeepZero = 48,     // what to leave in psum
+};
 template <typename T, typename V, int O>
-__global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq, const V *__restrict__ val,
-                                                    const float *__restrict__ dinv, T *x, const T *__restrict__ f,
-                                                    double omega) {
+__global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq, int sums, const V *__restrict__ val,
+                                                    T *x, const T *__restrict__ f, T *__restrict__ psum, double omega,
+                                                    const int *__restrict__ bnd_set, const float *__restrict__ dinv) {
   using L = Lines<O>;
   constexpr bool kScaled = sizeof(V) == 2;
   __shared__ PairSums<T> red[kSplits - 1][128];
@@ -189,8 +214,15 @@ __global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq
   const int p0 = M * (ly + M * u.z) + 2 * m;
   V own[L::VL];
   PairRow<T> r{0, 0, 0, 0, 1, 1};
-  T *l = lx + (t >> lg) * (2 * P + 2);
+  T *l = lx + (t >> lg) * (2 * P + 2), ko = 0, ke = 0;
+  // a start from zero has no sums over the lines after a row, unless the
+  // boundary values are not zero
+  const bool lo = sums & kSumLo, hi = (sums & kSumHi) || (bnd_set && *bnd_set != 0);
   if (w == 0) {
+    if (sums & kSumKept) {
+      ko = psum[p0 + 1];
+      ke = psum[p0 + 2];
+    }
     load_group<V, O>(v + (int64_t)nlo * (L::VL * P), P, own);
     r.fo = f[p0 + 1];
     r.fe = f[p0 + 2];
@@ -205,7 +237,7 @@ __global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq
     l[2 * m + 2] = x[p0 + 2];
     if (m == 0) l[0] = x[p0];
   }
-  PairSums<T> s = pair_sums<T, V, O, 2>(v, x + p0, g.off[c], nlo, ng, true, true, w, P, M, d3);
+  PairSums<T> s = pair_sums<T, V, O, 2>(v, x + p0, g.off[c], nlo, ng, lo, hi, w, P, M, d3);
   if (w) red[w - 1][t] = s;
   __syncthreads();
   const bool wide = P > 64;
@@ -213,13 +245,27 @@ __global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq
   if (w == 0) {
 #pragma unroll
     for (int q = 0; q < kSplits - 1; q++) add_partial(s, red[q][t]);
+    if (sums & kSumKept) {
+      if (lo) {
+        s.hi_o = ko;
+        s.hi_e = ke;
+      } else {
+        s.lo_o = ko;
+        s.lo_e = ke;
+      }
+    }
     r.so = s.lo_o + s.hi_o;
     r.se = s.lo_e + s.hi_e;
   }
   line_steps<T, V, O>(l, own, r, m, P, seq, omega, w == 0, wide);
   if (w || !ok) return;
+  const int keep = sums & kKeepZero;
   x[p0 + 1] = l[2 * m + 1];
-  if (m < P - 1) x[p0 + 2] = l[2 * m + 2];
+  if (keep) psum[p0 + 1] = keep == kKeepLo ? s.lo_o : keep == kKeepHi ? s.hi_o : T(0);
+  if (m < P - 1) {
+    x[p0 + 2] = l[2 * m + 2];
+    if (keep) psum[p0 + 2] = keep == kKeepLo ? s.lo_e : keep == kKeepHi ? s.hi_e : T(0);
+  }
 }
 
 // ============================================================ one workgroup
@@ -494,15 +540,21 @@ static unsigned unit_threads(const DevLayout &D) { return (unsigned)kSplits * st
 
 template <typename T>
 void rows_apply(const DevLayout &D, int mode, const T *val, const T *x, const T *f, T *y, double omega,
-                hipStream_t st) {
+                hipStream_t st, const T *psum) {
   int units;
   const LineSet s = all_lines(D, &units);
-#define PMX_ROWS(O, MODE) launch(k_line_rows<T, O, MODE>, (unsigned)units, unit_threads(D), st, s, D.lg, val, x, f, y, omega)
-#define PMX_ROWS_M(O)               \
-  switch (mode) {                   \
-    case 0: PMX_ROWS(O, 0); break;  \
-    case 1: PMX_ROWS(O, 1); break;  \
-    default: PMX_ROWS(O, 2); break; \
+#define PMX_ROWS(O, MODE, HALF) \
+  launch(k_line_rows<T, O, MODE, HALF>, (unsigned)units, unit_threads(D), st, s, D.lg, val, x, f, y, omega, psum)
+#define PMX_ROWS_M(O)                      \
+  if (psum) {                              \
+    if (mode == 0) PMX_ROWS(O, 0, true);   \
+    else PMX_ROWS(O, 1, true);             \
+  } else {                                 \
+    switch (mode) {                        \
+      case 0: PMX_ROWS(O, 0, false); break;  \
+      case 1: PMX_ROWS(O, 1, false); break;  \
+      default: PMX_ROWS(O, 2, false); break; \
+    }                                      \
   }
   if (D.order == 2) {
     PMX_ROWS_M(2)
@@ -514,36 +566,51 @@ void rows_apply(const DevLayout &D, int mode, const T *val, const T *x, const T 
 }
 
 template <typename T, typename V>
-static void sweep_group(const DevLayout &D, int g, int seq, const V *val, const float *dinv, T *x, const T *f,
-                        double omega, hipStream_t st) {
+static void sweep_group(const DevLayout &D, int g, int seq, int sums, const V *val, const float *dinv, T *x, const T *f,
+                        T *psum, double omega, const int *bnd_set, hipStream_t st) {
   int units;
   const LineSet s = group_lines(D, g, &units);
   if (D.order == 2)
-    launch(k_line_sweep<T, V, 2>, (unsigned)units, unit_threads(D), st, s, D.lg, seq, val, dinv, x, f, omega);
+    launch(k_line_sweep<T, V, 2>, (unsigned)units, unit_threads(D), st, s, D.lg, seq, sums, val, x, f, psum, omega,
+           bnd_set, dinv);
   else
-    launch(k_line_sweep<T, V, 1>, (unsigned)units, unit_threads(D), st, s, D.lg, seq, val, dinv, x, f, omega);
+    launch(k_line_sweep<T, V, 1>, (unsigned)units, unit_threads(D), st, s, D.lg, seq, sums, val, x, f, psum, omega,
+           bnd_set, dinv);
 }
 template <typename T, typename V>
-static void sweeps(const DevLayout &D, const V *val, const float *dinv, T *x, const T *f, double omega, bool ssor,
-                   int n, hipStream_t st) {
+static void sweeps(const DevLayout &D, const V *val, const float *dinv, T *x, const T *f, T *psum, double omega,
+                   bool ssor, int n, bool zero, const int *bnd_set, hipStream_t st) {
   const int G = D.order == 2 ? 9 : 4;
   for (int s = 0; s < n; s++) {
+    const bool start = s == 0 && zero;
+    const int *bs = start ? bnd_set : nullptr;
     // the last group turns a symmetric sweep around, the first one the next
-    // sweep: both directions of its lines in one launch
-    for (int g = ssor && s > 0 ? 1 : 0; g < G; g++)
-      sweep_group<T, V>(D, g, ssor && g == G - 1 ? kForwardBackward : kForward, val, dinv, x, f, omega, st);
-    if (ssor)
-      for (int g = G - 2; g >= 0; g--)
-        sweep_group<T, V>(D, g, g == 0 && s + 1 < n ? kBackwardForward : kBackward, val, dinv, x, f, omega, st);
+    // sweep: both directions of its lines in one launch (the last group has no
+    // lines after it, the first one none before it: their kept sum is zero)
+    for (int g = ssor && s > 0 ? 1 : 0; g < G; g++) {
+      const bool turn = ssor && g == G - 1;
+      int sums = kSumLo;
+      if (s > 0 && ssor) sums |= kSumKept;
+      else if (!start) sums |= kSumHi;
+      if (ssor) sums |= turn ? kKeepZero : kKeepLo;
+      sweep_group<T, V>(D, g, turn ? kForwardBackward : kForward, sums, val, dinv, x, f, psum, omega, bs, st);
+    }
+    if (!ssor) continue;
+    for (int g = G - 2; g >= 0; g--) {
+      const bool turn = g == 0 && s + 1 < n;
+      sweep_group<T, V>(D, g, turn ? kBackwardForward : kBackward, kSumHi | kSumKept | (turn ? kKeepZero : kKeepHi), val,
+                        dinv, x, f, psum, omega, nullptr, st);
+    }
   }
 }
 template <typename T>
-void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, double omega, bool ssor, int n, hipStream_t st) {
-  sweeps<T, T>(D, val, nullptr, x, f, omega, ssor, n, st);
+void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n, bool zero,
+                const int *bnd_set, hipStream_t st) {
+  sweeps<T, T>(D, val, nullptr, x, f, psum, omega, ssor, n, zero, bnd_set, st);
 }
 void sor_sweeps_scaled(const DevLayout &D, const _Float16 *val16, const float *dinv, float *x, const float *f,
-                       double omega, bool ssor, int n, hipStream_t st) {
-  sweeps<float, _Float16>(D, val16, dinv, x, f, omega, ssor, n, st);
+                       float *psum, double omega, bool ssor, int n, bool zero, const int *bnd_set, hipStream_t st) {
+  sweeps<float, _Float16>(D, val16, dinv, x, f, psum, omega, ssor, n, zero, bnd_set, st);
 }
 void scaled_values(const DevLayout &D, const float *val, _Float16 *val16, float *dinv, hipStream_t st) {
   int units;
@@ -607,8 +674,10 @@ void stream_read(const void *p, int64_t bytes, float *sink, hipStream_t st) {
 }
 
 #define PMX_INST(T)                                                                                              \
-  template void rows_apply<T>(const DevLayout &, int, const T *, const T *, const T *, T *, double, hipStream_t); \
-  template void sor_sweeps<T>(const DevLayout &, const T *, T *, const T *, double, bool, int, hipStream_t);      \
+  template void rows_apply<T>(const DevLayout &, int, const T *, const T *, const T *, T *, double, hipStream_t,  \
+                              const T *);                                                                        \
+  template void sor_sweeps<T>(const DevLayout &, const T *, T *, const T *, T *, double, bool, int, bool,        \
+                              const int *, hipStream_t);                                                         \
   template void sweep_wg<T>(const DevLayout &, const T *, T *, const T *, double, int, hipStream_t);              \
   template void coarse_wg<T>(const DevLayout &, const T *, T *, const T *, double, int, int, double, T *, hipStream_t);
 PMX_INST(double)

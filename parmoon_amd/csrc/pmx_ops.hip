@@ -135,10 +135,10 @@ __global__ __launch_bounds__(kBlock) void k_prolong(const T *__restrict__ xc, T 
     xf[id] = s;
   }
 }
-// zero_surface: 0 on the coarse lattice surface (CorrectDefect fused)
+// xc: 0 on the coarse lattice surface and xc = 0 (CorrectDefect and Reset fused)
 template <typename T, int ORDER>
 __global__ __launch_bounds__(kBlock) void k_restrict(T *__restrict__ rc, const T *__restrict__ rf, int Mc, int Mf,
-                                                     int zero_surface) {
+                                                     T *__restrict__ xc) {
   constexpr int R = TransferTaps<ORDER>::R;
   const unsigned id = blockIdx.x * kBlock + threadIdx.x;
   const unsigned Nc = (unsigned)Mc * Mc * Mc;
@@ -163,7 +163,8 @@ __global__ __launch_bounds__(kBlock) void k_restrict(T *__restrict__ rc, const T
         s += (wz[c] != 0.0 && wy[b] != 0.0 && wx[a] != 0.0) ? t : T(0);
       }
     }
-  if (zero_surface && (x == 0 || y == 0 || z == 0 || x == Mc - 1 || y == Mc - 1 || z == Mc - 1)) s = 0;
+  if (xc) xc[id] = T(0);
+  if (xc && (x == 0 || y == 0 || z == 0 || x == Mc - 1 || y == Mc - 1 || z == Mc - 1)) s = 0;
   rc[id] = s;
 }
 
@@ -884,6 +885,36 @@ void dot(const T *x, const T *y, int64_t n, double *part, double *out, int do_sq
   hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, st, part, g, out, do_sqrt);
 }
 
+// ------------------------------------------------------- start of a cycle
+template <typename T>
+__global__ void k_start_zero(T *__restrict__ f, T *__restrict__ x, const T *__restrict__ v, int *__restrict__ bnd_set,
+                             int64_t n) {
+  const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i0 == 0) *bnd_set = 0;
+  for (int64_t i = i0; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    f[i] = v[i];
+    x[i] = T(0);
+  }
+}
+template <typename T>
+__global__ void k_start_boundary(const int *__restrict__ bnd, int nb, T *__restrict__ x, const T *__restrict__ f,
+                                 int *__restrict__ bnd_set) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nb) return;
+  const T v = f[bnd[i]];
+  x[bnd[i]] = v;
+  if (v != T(0)) *bnd_set = 1;  // (every writer stores the same value; NaN counts)
+}
+template <typename T>
+void start_zero(T *f, T *x, const T *v, int *bnd_set, int64_t n, hipStream_t st) {
+  hipLaunchKernelGGL(k_start_zero<T>, dim3(grid_for(n)), dim3(kBlock), 0, st, f, x, v, bnd_set, n);
+}
+template <typename T>
+void start_boundary(const DevLayout &D, T *x, const T *f, int *bnd_set, hipStream_t st) {
+  hipLaunchKernelGGL(k_start_boundary<T>, dim3((D.nboundary + kBlock - 1) / kBlock), dim3(kBlock), 0, st, D.boundary,
+                     D.nboundary, x, f, bnd_set);
+}
+
 // ------------------------------------------------------- step length control
 template <typename T>
 __global__ void k_diff(T *__restrict__ e, const T *__restrict__ u, const T *__restrict__ uold, int64_t n) {
@@ -1033,14 +1064,12 @@ void prolongate_add(const DevLayout &C, const DevLayout &F, const T *xc, T *xf, 
     hipLaunchKernelGGL((k_prolong<T, 1, 1>), dim3(grid_for(F.N)), dim3(kBlock), 0, st, xc, xf, C.M, F.M, damp);
 }
 template <typename T>
-void restrict_(const DevLayout &C, const DevLayout &F, T *rc, const T *rf, hipStream_t st, bool zero_surface) {
+void restrict_(const DevLayout &C, const DevLayout &F, T *rc, const T *rf, hipStream_t st, T *xc) {
   if (F.N >= (int64_t(1) << 31)) throw std::runtime_error("restrict: lattice too large for 32-bit indices");
   if (F.order == 2)
-    hipLaunchKernelGGL((k_restrict<T, 2>), dim3(grid_for(C.N)), dim3(kBlock), 0, st, rc, rf, C.M, F.M,
-                       (int)zero_surface);
+    hipLaunchKernelGGL((k_restrict<T, 2>), dim3(grid_for(C.N)), dim3(kBlock), 0, st, rc, rf, C.M, F.M, xc);
   else
-    hipLaunchKernelGGL((k_restrict<T, 1>), dim3(grid_for(C.N)), dim3(kBlock), 0, st, rc, rf, C.M, F.M,
-                       (int)zero_surface);
+    hipLaunchKernelGGL((k_restrict<T, 1>), dim3(grid_for(C.N)), dim3(kBlock), 0, st, rc, rf, C.M, F.M, xc);
 }
 template <typename T>
 void gemv_coarse(int nI, int N, const double *W, const int *iidx, const T *x, T *y, hipStream_t st) {
@@ -1604,7 +1633,9 @@ void set_scalar(double *dst, const double *src, double scale, hipStream_t st) {
   template void boundary<T>(const DevLayout &, int, T *, const T *, const T *, hipStream_t);                \
   template void prolongate<T>(const DevLayout &, const DevLayout &, const T *, T *, hipStream_t);           \
   template void prolongate_add<T>(const DevLayout &, const DevLayout &, const T *, T *, double, hipStream_t); \
-  template void restrict_<T>(const DevLayout &, const DevLayout &, T *, const T *, hipStream_t, bool);      \
+  template void restrict_<T>(const DevLayout &, const DevLayout &, T *, const T *, hipStream_t, T *);       \
+  template void start_zero<T>(T *, T *, const T *, int *, int64_t, hipStream_t);                            \
+  template void start_boundary<T>(const DevLayout &, T *, const T *, int *, hipStream_t);                    \
   template void gemv_coarse<T>(int, int, const double *, const int *, const T *, T *, hipStream_t);         \
   template void csr_spmv<T>(int, const int *, const int *, const T *, const T *, T *, hipStream_t);         \
   template void csr_defect<T>(int, const int *, const int *, const T *, const T *, const T *, T *, hipStream_t); \

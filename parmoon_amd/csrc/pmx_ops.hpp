@@ -82,17 +82,23 @@ template <typename T>
 void mgs_arnoldi(T *w, const T *V, int64_t n, int k1, double *h, T *vnext, double *part, hipStream_t st);
 
 // mode 0 product, 1 defect, 2 Jacobi (x = old iterate, y = new) over the
-// interior rows (Dirichlet rows: boundary)
+// interior rows (Dirichlet rows: boundary); psum (modes 0, 1): the upper sums
+// that sor_sweeps left for this x, which halves the values read
 template <typename T>
 void rows_apply(const DevLayout &D, int mode, const T *val, const T *x, const T *f, T *y, double omega,
-                hipStream_t st);
+                hipStream_t st, const T *psum = nullptr);
 // n SOR (forward) or SSOR sweeps in colour order, one launch per line group;
-// the Dirichlet entries of x are left as they are
+// the Dirichlet entries of x are left as they are.  psum (SSOR): N entries of
+// scratch that hold the upper sums of the result's rows afterwards.  zero: the
+// interior of x is zero (its contribution is not read); bnd_set (optional,
+// with zero): a device flag that is not 0 if the boundary of x is not zero.
 template <typename T>
-void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, double omega, bool ssor, int n, hipStream_t st);
+void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n, bool zero,
+                const int *bnd_set, hipStream_t st);
 // the same on the row-scaled FP16 values and the FP32 1/diag of scaled_values
+// (psum: sums of the scaled values)
 void sor_sweeps_scaled(const DevLayout &D, const _Float16 *val16, const float *dinv, float *x, const float *f,
-                       double omega, bool ssor, int n, hipStream_t st);
+                       float *psum, double omega, bool ssor, int n, bool zero, const int *bnd_set, hipStream_t st);
 // the lines of a launch over all interior lines / over a line group, and its
 // number of units
 LineSet all_lines(const DevLayout &D, int *units);
@@ -127,9 +133,14 @@ void prolongate(const DevLayout &C, const DevLayout &F, const T *xc, T *xf, hipS
 // (the Dirichlet nodes of a layout are its lattice surface)
 template <typename T>
 void prolongate_add(const DevLayout &C, const DevLayout &F, const T *xc, T *xf, double damp, hipStream_t st);
-// zero_surface: the coarse Dirichlet entries are set to 0 (CorrectDefect)
+// xc: the cycle's restriction, which also sets the coarse Dirichlet entries
+// to 0 (CorrectDefect) and the coarse iterate xc to 0 (Reset)
 template <typename T>
-void restrict_(const DevLayout &C, const DevLayout &F, T *rc, const T *rf, hipStream_t st, bool zero_surface = false);
+void restrict_(const DevLayout &C, const DevLayout &F, T *rc, const T *rf, hipStream_t st, T *xc = nullptr);
+// the start of a cycle from zero: f = v, x = 0, *bnd_set = 0; then
+// start_boundary: x = f on the Dirichlet nodes, *bnd_set = 1 if any is not 0
+template <typename T> void start_zero(T *f, T *x, const T *v, int *bnd_set, int64_t n, hipStream_t st);
+template <typename T> void start_boundary(const DevLayout &D, T *x, const T *f, int *bnd_set, hipStream_t st);
 // coarsest-level solve: y_I = W x with W = A_II^-1 [I, -A_IB] (n_I x N, lattice
 // columns; iidx: interior row -> lattice node); y_B = x_B is set separately
 template <typename T>
