@@ -183,9 +183,9 @@ int pmx_csr_matvec(pmx_ctx *ctx, int n, const int *rowptr, const int *kcol, cons
  *  [19] precision 2: number of finest levels with the learned post-smoother
  *       (0 = the levels it was trained for)
  *  [20] precision 2: learned steps per post-smoothing (default 1)
- *  [21] SOR/SSOR sweeps of levels whose largest colour has at most this many
- *       rows run in one workgroup (same iterate, fewer launches); 0 = 512 in
- *       FP32 and never in FP64, < 0 = never
+ *  [21] SOR/SSOR sweeps of small levels (at most 17^3 lattice nodes) whose
+ *       largest colour has at most this many rows run plane by plane (same
+ *       iterate, fewer launches); 0 = all of them, < 0 = never
  *  [22] precision 2: the finest [22] of the [19] levels keep the plain smoother
  *  [23] precision 2: 1 = the learned steps also replace the pre-smoothing
  * info (out, 8 doubles): [0] iterations (Krylov steps summed) [1] final FP64

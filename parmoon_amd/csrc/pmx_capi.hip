@@ -83,6 +83,7 @@ struct Level {
   Numbering Nb;
   DevLayout D;
   DevBuf<int> boundary;
+  DevBuf<int2> pairs;                 // row pairs by line group (small levels)
   DevBuf<int> lat2dof, dof2lat, rowptr, kcol;
   DevBuf<double> val2;                // second matrix (SUPG K)
   DevBuf<double> mass;                // time stepping: mass matrix M
@@ -228,6 +229,12 @@ static void setup_level(System &Y, Level &lv, int nref) {
   D.max_colour_rows = L.max_colour_rows;
   lv.boundary.upload(L.boundary.data(), L.boundary.size(), st);
   D.boundary = lv.boundary.p; D.nboundary = (int)L.boundary.size();
+  if (L.M >= 3 && D.lg <= 4) {
+    D.pair_tiles = pair_tiles(L);
+    lv.pairs.alloc(pair_table_size(D));
+    pair_table(D, lv.pairs.p, st);
+    D.pairs = lv.pairs.p;
+  }
 
   lv.rhs.alloc(L.N);
   lv.v64.val.alloc_zeroed(L.nstored, st);
@@ -366,7 +373,7 @@ static void ensure_val32(System &Y) {
       // weights only (dinv and A c vanish there), so they just have to be finite
       fill<float>(lv.v32.d.p, 0.0f, lv.L.N, Y.ctx->st);
     }
-    convert<float, double>(lv.v32.val.p, lv.v64.val.p, lv.L.nstored, Y.ctx->st);
+    values32(lv.D, lv.v64.val.p, lv.v32.val.p, Y.ctx->st);
     lv.have_val32 = true;
   }
 }
@@ -424,11 +431,9 @@ template <typename T>
 static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweeps, int start = kStartAny) {
   hipStream_t st = Y.ctx->st;
   Vecs<T> &v = vecs<T>(lv);
-  // levels whose largest colour has at most this many rows sweep in one
-  // workgroup; by default FP32 only: an FP64 sweep moves twice the bytes
-  // through the one CU and is slower there than launch per colour
-  const int64_t wg_default = sizeof(T) == 4 ? kSweepWgRows : 0;
-  const int64_t wg_limit = Y.opt[21] == 0 ? wg_default : (int64_t)Y.opt[21];
+  // small levels sweep by planes, with FP32 values also where the larger ones
+  // take FP16 values (there is no traffic to save); opt[21] as in pmx.h
+  const bool planes = plane_sweeps_fit(lv.D) && (Y.opt[21] == 0 || lv.D.max_colour_rows <= (int64_t)Y.opt[21]);
   if (kind == 1) {
     for (int s = 0; s < sweeps; s++) {
       copy<T>(v.aux.p, v.x.p, lv.L.N, st);
@@ -438,22 +443,18 @@ static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweep
     return false;
   }
   if (sweeps < 1) return false;
-  if (lv.D.max_colour_rows <= wg_limit && sweep_wg_fits(lv.D, sizeof(T))) {
-    for (int s = 0; s < sweeps; s++) sweep_wg<T>(lv.D, v.val.p, v.x.p, v.f.p, omega, kind == 3 ? 1 : 0, st);
-    return false;
-  }
   // Dirichlet rows x = f (no sweep changes them afterwards)
   if (start == kStartAny) boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
   const int *bs = start == kStartInteriorZero ? Y.bnd_set.p : nullptr;
   if constexpr (std::is_same<T, float>::value) {
-    if (Y.half_smoother) {
+    if (Y.half_smoother && !planes) {
       if (!lv.have_val16) throw std::logic_error("level_smooth: FP16 smoother values missing");
       sor_sweeps_scaled(lv.D, lv.val16.p, lv.sdinv.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps,
                         start != kStartAny, bs, st);
       return false;
     }
   }
-  sor_sweeps<T>(lv.D, v.val.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps, start != kStartAny, bs, st);
+  sor_sweeps<T>(lv.D, v.val.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps, start != kStartAny, bs, planes, st);
   return kind == 3;
 }
 // Learned post-smoothing of one level (replaces the post-sweeps of
@@ -1701,8 +1702,7 @@ static void tcd_systmat(System &Y) {
   for (auto &lp : Y.lev) {
     Level &l = *lp;
     // the FP32 copy (once the FP32 forms have allocated it) in the same pass
-    system_matrix(l.v64.val.p, l.v32.val.p, l.mass.p, supg ? l.val2.p : nullptr, l.stiff.p, tau * th1, l.L.nstored,
-                  st);
+    system_matrix(l.D, l.v64.val.p, l.v32.val.p, l.mass.p, supg ? l.val2.p : nullptr, l.stiff.p, tau * th1, st);
     l.have_val32 = l.v32.val.p != nullptr;
     l.have_val16 = false;
     l.have_dinv = false;

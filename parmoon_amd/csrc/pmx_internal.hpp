@@ -12,12 +12,14 @@
 // last even one is the boundary node x = M - 1, whose values are zero), and a
 // pair's entries are grouped by the lattice line (y + dy, z + dz) of their
 // columns.  A line (y, z) stores its groups one after another, a group holds
-// VL = 3 + (2 order + 1) slots (the odd row's 3 entries, dx = -1 .. 1, then
-// the even row's, dx = -order .. order), and slot s of pair m is at
-//   val[((group_base(P, y, z) + k) * VL + s) * P + m]
-// so that every load of the P lanes of a line is contiguous and no column
-// index is stored.  A group's run of x values (5 for Q2, 4 for Q1) serves both
-// rows of the pair.  The groups of a line whose own lines come before it in
+// VL = 3 + (2 order + 1) slots per pair (the odd row's 3 entries, dx = -1 .. 1,
+// then the even row's, dx = -order .. order) in chunks of 16 bytes (2 FP64, 4
+// FP32, 8 FP16 slots; the last chunk holds the rest), chunk after chunk:
+//   val[(group_base(P, y, z) + k) * VL * P + Slots<V, order>::at(P, m, s)]
+// so that the P lanes of a line load contiguous 16-byte chunks and no column
+// index is stored.  (One slot per load costs the same on long lines, but on
+// the 8 pairs of a 17^3 line each load touches 8 lines for 32 bytes of each.)
+// A group's run of x values (5 for Q2, 4 for Q1) serves both rows of the pair.  The groups of a line whose own lines come before it in
 // the sweep order are stored first (k < nlo), then the line itself, then the
 // others, so a half sweep streams one contiguous part of each line.
 //
@@ -36,8 +38,7 @@ namespace pmx {
 
 constexpr int kBlock = 256;       // threads per workgroup of the operator kernels
 constexpr int kRowsPerBlock = 64; // rows per workgroup of the one-thread-per-row kernels
-constexpr int64_t kSweepLdsBytes = 48 * 1024;  // largest x staged in LDS by the single-workgroup sweep
-constexpr int kSweepWgRows = 512;    // default: single-workgroup sweep up to this many rows per colour
+constexpr int64_t kSweepLdsBytes = 48 * 1024;  // largest x staged in LDS by the single-workgroup kernel
 constexpr int kSplits = 4;           // partial sums of a row: group k belongs to partial k mod 4
 constexpr int kRedBlocks = 1024;  // partial sums of the deterministic reductions
 
@@ -69,6 +70,15 @@ template <int O> struct Lines {
   PMX_HD static constexpr int slot(int x, int dx) { return (x & 1) ? dx + 1 : 3 + dx + O; }
   PMX_HD static constexpr int64_t values(int P) {
     return (int64_t)width_total(P) * width_total(P) * VL * P;
+  }
+};
+
+// position of slot s of pair m in a group of values of type V
+template <typename V, int O> struct Slots {
+  static constexpr int VL = Lines<O>::VL, W = 16 / (int)sizeof(V);  // slots per chunk
+  PMX_HD static constexpr int width(int c) { return VL - c < W ? VL - c : W; }  // of the chunk at slot c
+  PMX_HD static constexpr int at(int P, int m, int s) {
+    return (s / W) * W * P + m * width(s / W * W) + s % W;
   }
 };
 

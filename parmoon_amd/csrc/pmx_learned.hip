@@ -699,7 +699,7 @@ __global__ void k_diag_inv(int M, const float *__restrict__ val, float *__restri
   const int t = blockIdx.x * blockDim.x + threadIdx.x, m2 = M - 2;
   if (t >= m2 * m2) return;
   const int x = 1 + t % m2, y = 1 + t / m2, z = 1 + blockIdx.y;
-  dinv[x + (int64_t)M * (y + (int64_t)M * z)] = 1.0f / val[value_index<O>((M - 1) / 2, x, y, z, 0, 0, 0)];
+  dinv[x + (int64_t)M * (y + (int64_t)M * z)] = 1.0f / val[value_index<float, O>((M - 1) / 2, x, y, z, 0, 0, 0)];
 }
 __global__ void k_learned_input(const float *__restrict__ dinv, const float *__restrict__ d, float *__restrict__ u,
                                 int64_t n) {
@@ -761,7 +761,7 @@ __global__ void k_features(int M, const float *__restrict__ val, uint16_t *__res
   if (t >= m2 * m2) return;
   const int x = 1 + t % m2, y = 1 + t / m2, z = 1 + blockIdx.y;
   const int64_t p = x + (int64_t)M * (y + (int64_t)M * z);
-  auto a = [&](int dx, int dy, int dz) { return val[value_index<O>(P, x, y, z, dx, dy, dz)]; };
+  auto a = [&](int dx, int dy, int dz) { return val[value_index<float, O>(P, x, y, z, dx, dy, dz)]; };
   const float dinv = 1.0f / a(0, 0, 0);
   const int off[6][3] = {{1, 0, 0}, {-1, 0, 0}, {0, 1, 0}, {0, -1, 0}, {0, 0, 1}, {0, 0, -1}};
   const int ext[3] = {Lines<O>::ext(x), Lines<O>::ext(y), Lines<O>::ext(z)};
@@ -955,17 +955,17 @@ __global__ __launch_bounds__(kBlock) void k_transpose_values(int lg, const float
   const int ln = (int)(id >> lg);
   if (ln >= (M - 2) * (M - 2)) return;
   const int y = 1 + ln % (M - 2), z = 1 + ln / (M - 2);
-  const GroupTable<O> &g = group_table<O>();
-  const int c = line_class<O>(y, z), k = blockIdx.y;
-  if (k >= g.ng[c]) return;
-  const int dy = (g.off[c][k] & 15) - 8, dz = (g.off[c][k] >> 4) - 8;
+  const GroupOrder<O> g(y, z);
+  const int k = blockIdx.y;
+  if (k >= g.groups()) return;
+  const int off = g.line(k, 16) + 16 * 2 + 2, dy = (off & 15) - 2, dz = (off >> 4) - 2;
   const bool in = y + dy > 0 && y + dy < M - 1 && z + dz > 0 && z + dz < M - 1;
-  float *o = valT + line_values<float, O>(P, L::group_base(P, y, z), m) + (int64_t)k * (L::VL * P);
+  float *o = valT + line_values<O>(P, y, z) + (int64_t)k * (L::VL * P);
 #pragma unroll
   for (int s = 0; s < L::VL; s++) {
     const int x = s < 3 ? 2 * m + 1 : 2 * m + 2, dx = s < 3 ? s - 1 : s - 3 - O;
     const bool use = in && x < M - 1 && x + dx > 0 && x + dx < M - 1;
-    o[s * P] = use ? val[value_index<O>(P, x + dx, y + dy, z + dz, -dx, -dy, -dz)] : 0.f;
+    o[Slots<float, O>::at(P, m, s)] = use ? val[value_index<float, O>(P, x + dx, y + dy, z + dz, -dx, -dy, -dz)] : 0.f;
   }
 }
 

@@ -35,11 +35,12 @@ template <typename T> struct PairSums {
 };
 // this unit's partial sums: lo / hi select the parts
 template <typename T, typename V, int O, int U>
-__device__ __forceinline__ PairSums<T> pair_sums(const V *v, const T *x, const int *off, int nlo, int ng, bool lo,
-                                                 bool hi, int w, int P, int M, int d3) {
+__device__ __forceinline__ PairSums<T> pair_sums(const V *v, const T *x, const GroupOrder<O> &g, bool lo, bool hi, int w,
+                                                 int P, int M, int m, int d3) {
+  const int nlo = g.before();
   PairSums<T> s{0, 0, 0, 0};
-  if (lo) add_groups<T, V, O, U>(v, x, off, w, nlo, kSplits, P, M, d3, s.lo_o, s.lo_e);
-  if (hi) add_groups<T, V, O, U>(v, x, off, nlo + 1 + w, ng, kSplits, P, M, d3, s.hi_o, s.hi_e);
+  if (lo) add_groups<T, V, O, U>(v, x, g, w, nlo, kSplits, P, M, m, d3, s.lo_o, s.lo_e);
+  if (hi) add_groups<T, V, O, U>(v, x, g, nlo + 1 + w, g.groups(), kSplits, P, M, m, d3, s.hi_o, s.hi_e);
   return s;
 }
 template <typename T> __device__ __forceinline__ void add_partial(PairSums<T> &s, const PairSums<T> &p) {
@@ -82,10 +83,10 @@ __global__ __launch_bounds__(512) void k_line_rows(LineSet set, int lg, const T 
   const UnitLines u = unit_lines<O>(set, M, lg, xcd_remap(blockIdx.x, gridDim.x));
   const int m = t & (P - 1), yy = u.y0 + L::S * (t >> lg);
   const bool ok = yy <= M - 2;
-  const int ly = ok ? yy : u.y0, c = line_class<O>(u.y0, u.z);
-  const GroupTable<O> &g = group_table<O>();
-  const int nlo = g.nlo[c], ng = g.ng[c], d3 = run_split<O>(m, P);
-  const T *v = val + line_values<T, O>(P, L::group_base(P, ly, u.z), m);
+  const int ly = ok ? yy : u.y0;
+  const GroupOrder<O> g(u.y0, u.z);
+  const int nlo = g.before(), d3 = run_split<O>(m, P);
+  const T *v = val + line_values<O>(P, ly, u.z);
   const int p0 = M * (ly + M * u.z) + 2 * m;
   T own[L::VL], xr[5], fo = 0, fe = 0, ho = 0, he = 0;
   if (w == 0) {
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(512) void k_line_rows(LineSet set, int lg, const T 
       ho = psum[p0 + 1];
       he = psum[p0 + 2];
     }
-    load_group<T, O>(v + (int64_t)nlo * (L::VL * P), P, own);
+    load_group<T, O>(v + (int64_t)nlo * (L::VL * P), P, m, own);
     load_run<T, 3>(x + p0, xr);
     load_run<T, O == 2 ? 2 : 1>(x + p0 + d3, xr + 3);
     if (MODE >= 1) {
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(512) void k_line_rows(LineSet set, int lg, const T 
       fe = f[p0 + 2];
     }
   }
-  PairSums<T> s = pair_sums<T, T, O, 2>(v, x + p0, g.off[c], nlo, ng, true, !HALF, w, P, M, d3);
+  PairSums<T> s = pair_sums<T, T, O, 2>(v, x + p0, g, true, !HALF, w, P, M, m, d3);
   if (w) red[w - 1][t] = s;
   __syncthreads();
   if (w || !ok) return;
@@ -131,30 +132,89 @@ __global__ __launch_bounds__(512) void k_line_rows(LineSet set, int lg, const T 
 
 // ============================================================ line sweeps
 // x = w ((f - A_off x)/d - x) + x (TMGLevel3D::SOR, MGLevel3D.C:280-361) for
-// the rows of a line, colour by colour.  l: the line's x in LDS (coordinate
-// 0 .. 2P).  The lanes of a line belong to one wavefront (P <= 64: LDS
-// operations of a wavefront complete in order) or to one workgroup (P = 128).
+// the rows of a line, colour by colour.  A lane holds the x of its pair; the
+// neighbours' values come by wavefront shifts (a line's lanes are consecutive
+// and, for P <= 64, in one wavefront; for P = 128 through LDS).
 enum { kForward = 0, kBackward = 1, kForwardBackward = 2, kBackwardForward = 3 };
 template <typename T> struct PairRow {
-  T fo, fe, so, se, dio, die;  // right-hand side, sums of the other lines, diagonals
+  T fo, fe, so, se;      // right-hand side, sums of the other lines
+  T dio, die, rio, rie;  // diagonals and their reciprocals
 };
+// a / d from r = 1 / d: the quotient with its remainder added back, the last
+// step of a division, so that the chain of a line's colours does not wait for
+// the reciprocals
+template <typename T> __device__ __forceinline__ T quotient(T a, T d, T r) {
+  const T q = a * r;
+  return fma(fma(-q, d, a), r, q);
+}
+// v of the lane before (DPP wave_shr:1) / after (wave_shl:1); 0 past the ends
+template <int CTRL> __device__ __forceinline__ float wave_shift(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ double wave_shift(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+constexpr int kWaveShr1 = 0x138, kWaveShl1 = 0x130;
+// number of colour steps of a sequence, and the colour of step i.  At a turn
+// the repeated colour reproduces its rows bit for bit when omega is 1 (the
+// neighbours it reads are unchanged) and is skipped.
+template <int C> __device__ __forceinline__ int colour_steps(int seq, int skip) { return seq < 2 ? C : 2 * C - skip; }
+template <int C> __device__ __forceinline__ int colour_of_step(int i, int seq, int skip) {
+  const int c = i < C ? i : 2 * C - 1 - skip - i;
+  return seq == kBackward || seq == kBackwardForward ? C - 1 - c : c;
+}
+// P <= 64.  x[0 .. 2] of the pair: coordinate 2m (used of the line's first
+// pair only: the boundary value), 2m + 1, 2m + 2; every lane of the wavefront
+// calls it.
 template <typename T, typename V, int O>
-__device__ __forceinline__ void line_steps(T *l, const V *own, const PairRow<T> &r, int m, int P, int seq, double omega,
-                                           bool active, bool wide) {
+__device__ __forceinline__ void line_steps(T *x, const V *own, const PairRow<T> &r, int m, int P, int seq,
+                                           double omega) {
+  constexpr int C = Lines<O>::C;
+  const int co = (2 * m + 1) % C, ce = m < P - 1 ? (2 * m + 2) % C : C;
+  const int skip = omega == 1.0 ? 1 : 0, n = colour_steps<C>(seq, skip);
+  const T w = (T)omega;
+  // the entries beyond the line's last node are zero (the even row of the last
+  // pair is the boundary node): whatever the shifts bring meets weight 0
+  const T a0 = (T)own[0], a2 = (T)own[2], b0 = (T)own[3], b1 = O == 2 ? (T)own[4] : (T)own[3];
+  for (int i = 0; i < n; i++) {
+    const int c = colour_of_step<C>(i, seq, skip);
+    // (by all lanes: a shift reads nothing from a lane that is switched off)
+    const T before = wave_shift<kWaveShr1>(x[2]), left = m == 0 ? x[0] : before;
+    const T right = wave_shift<kWaveShl1>(x[1]), far = O == 2 ? wave_shift<kWaveShl1>(x[2]) : T(0);
+    const bool odd = c == co;
+    T s = odd ? r.so : r.se;
+    if (O == 2) {
+      // odd row: columns 2m, 2m + 2; even row: 2m, 2m + 1, 2m + 3, 2m + 4
+      s = fma(odd ? a0 : b0, left, s);
+      s = fma(odd ? a2 : b1, odd ? x[2] : x[1], s);
+      T e = fma((T)own[6], right, s);
+      e = fma((T)own[7], far, e);
+      s = odd ? s : e;
+    } else {
+      // odd row: columns 2m, 2m + 2; even row: 2m + 1, 2m + 3
+      s = fma(odd ? a0 : b0, odd ? left : x[1], s);
+      s = fma(odd ? a2 : (T)own[5], odd ? x[2] : right, s);
+    }
+    const T gs = quotient((odd ? r.fo : r.fe) - s, odd ? r.dio : r.die, odd ? r.rio : r.rie);
+    const T old = odd ? x[1] : x[2], nx = skip ? gs : w * (gs - old) + old;
+    if (odd) x[1] = nx;
+    if (c == ce) x[2] = nx;
+  }
+}
+// P = 128: l is the line's x in LDS (coordinate 0 .. 2P), every thread of the
+// workgroup calls it, `active` in those that hold the line's pairs
+template <typename T, typename V, int O>
+__device__ __forceinline__ void line_steps_wide(T *l, const V *own, const PairRow<T> &r, int m, int P, int seq,
+                                                double omega, bool active) {
   constexpr int C = Lines<O>::C;
   const int co = (2 * m + 1) % C, ce = (2 * m + 2) % C;
-  // at a turn the repeated colour reproduces its rows bit for bit when omega
-  // is 1 (the neighbours it reads are unchanged) and is skipped
-  const int skip = omega == 1.0 ? 1 : 0, n = seq < 2 ? C : 2 * C - skip;
+  const int skip = omega == 1.0 ? 1 : 0, n = colour_steps<C>(seq, skip);
   for (int i = 0; i < n; i++) {
-    int c = i < C ? i : 2 * C - 1 - skip - i;
-    if (seq == kBackward || seq == kBackwardForward) c = C - 1 - c;
-    if (wide) {
-      __syncthreads();
-    } else {
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
+    const int c = colour_of_step<C>(i, seq, skip);
+    __syncthreads();
     if (!active) continue;
     const bool odd = c == co;
     if (odd || (c == ce && m < P - 1)) {
@@ -163,12 +223,12 @@ __device__ __forceinline__ void line_steps(T *l, const V *own, const PairRow<T> 
 #pragma unroll
       for (int e = 0; e < 3; e++) x[e] = q[e];
       if (odd) {
-        const T gs = (r.fo - own_odd<T, V, O>(own, x, r.so)) / r.dio;
+        const T gs = quotient(r.fo - own_odd<T, V, O>(own, x, r.so), r.dio, r.rio);
         q[1] = skip ? gs : (T)omega * (gs - x[1]) + x[1];
       } else {
         x[3] = q[3];
         if (O == 2) x[4] = q[4];
-        const T gs = (r.fe - own_even<T, V, O>(own, x, r.se)) / r.die;
+        const T gs = quotient(r.fe - own_even<T, V, O>(own, x, r.se), r.die, r.rie);
         q[2] = skip ? gs : (T)omega * (gs - x[2]) + x[2];
       }
     }
@@ -201,20 +261,20 @@ __global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq
   using L = Lines<O>;
   constexpr bool kScaled = sizeof(V) == 2;
   __shared__ PairSums<T> red[kSplits - 1][128];
-  __shared__ T lx[264];
+  __shared__ T lx[258];  // P = 128: the line
   const int P = 1 << lg, M = 2 * P + 1, ul = lg < 6 ? 6 : lg;
   const int t = threadIdx.x & ((1 << ul) - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> ul);
   const UnitLines u = unit_lines<O>(set, M, lg, xcd_remap(blockIdx.x, gridDim.x));
   const int m = t & (P - 1), yy = u.y0 + L::S * (t >> lg);
   const bool ok = yy <= M - 2;
-  const int ly = ok ? yy : u.y0, c = line_class<O>(u.y0, u.z);
-  const GroupTable<O> &g = group_table<O>();
-  const int nlo = g.nlo[c], ng = g.ng[c], d3 = run_split<O>(m, P);
-  const V *v = val + line_values<V, O>(P, L::group_base(P, ly, u.z), m);
+  const int ly = ok ? yy : u.y0;
+  const GroupOrder<O> g(u.y0, u.z);
+  const int nlo = g.before(), d3 = run_split<O>(m, P);
+  const V *v = val + line_values<O>(P, ly, u.z);
   const int p0 = M * (ly + M * u.z) + 2 * m;
   V own[L::VL];
-  PairRow<T> r{0, 0, 0, 0, 1, 1};
-  T *l = lx + (t >> lg) * (2 * P + 2), ko = 0, ke = 0;
+  PairRow<T> r{0, 0, 0, 0, 1, 1, 1, 1};
+  T xp[3] = {0, 0, 0}, ko = 0, ke = 0;
   // a start from zero has no sums over the lines after a row, unless the
   // boundary values are not zero
   const bool lo = sums & kSumLo, hi = (sums & kSumHi) || (bnd_set && *bnd_set != 0);
@@ -223,7 +283,7 @@ __global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq
       ko = psum[p0 + 1];
       ke = psum[p0 + 2];
     }
-    load_group<V, O>(v + (int64_t)nlo * (L::VL * P), P, own);
+    load_group<V, O>(v + (int64_t)nlo * (L::VL * P), P, m, own);
     r.fo = f[p0 + 1];
     r.fe = f[p0 + 2];
     if constexpr (kScaled) {
@@ -232,12 +292,12 @@ __global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq
     } else {
       r.dio = (T)own[1];
       r.die = (T)own[3 + O];
+      r.rio = T(1) / r.dio;
+      r.rie = T(1) / r.die;
     }
-    l[2 * m + 1] = x[p0 + 1];
-    l[2 * m + 2] = x[p0 + 2];
-    if (m == 0) l[0] = x[p0];
+    load_run<T, 3>(x + p0, xp);
   }
-  PairSums<T> s = pair_sums<T, V, O, 2>(v, x + p0, g.off[c], nlo, ng, lo, hi, w, P, M, d3);
+  PairSums<T> s = pair_sums<T, V, O, 2>(v, x + p0, g, lo, hi, w, P, M, m, d3);
   if (w) red[w - 1][t] = s;
   __syncthreads();
   const bool wide = P > 64;
@@ -257,141 +317,763 @@ __global__ __launch_bounds__(512) void k_line_sweep(LineSet set, int lg, int seq
     r.so = s.lo_o + s.hi_o;
     r.se = s.lo_e + s.hi_e;
   }
-  line_steps<T, V, O>(l, own, r, m, P, seq, omega, w == 0, wide);
+  if (wide) {
+    if (w == 0) {
+      lx[2 * m + 1] = xp[1];
+      lx[2 * m + 2] = xp[2];
+      if (m == 0) lx[0] = xp[0];
+    }
+    line_steps_wide<T, V, O>(lx, own, r, m, P, seq, omega, w == 0);
+    xp[1] = lx[2 * m + 1];
+    xp[2] = lx[2 * m + 2];
+  } else {
+    line_steps<T, V, O>(xp, own, r, m, P, seq, omega);
+  }
   if (w || !ok) return;
   const int keep = sums & kKeepZero;
-  x[p0 + 1] = l[2 * m + 1];
+  x[p0 + 1] = xp[1];
   if (keep) psum[p0 + 1] = keep == kKeepLo ? s.lo_o : keep == kKeepHi ? s.hi_o : T(0);
   if (m < P - 1) {
-    x[p0 + 2] = l[2 * m + 2];
+    x[p0 + 2] = xp[2];
     if (keep) psum[p0 + 2] = keep == kKeepLo ? s.lo_e : keep == kKeepHi ? s.hi_e : T(0);
   }
 }
 
 // ============================================================ one workgroup
-// A whole sweep of a small level in one workgroup: the level's x is in LDS,
-// the line groups follow each other with workgroup barriers.  A lane's row
-// pair may belong to any line of the group (its class and group table are the
-// lane's own), 4 x 64 pairs at a time with kSplits wavefronts each.
-constexpr int kWgThreads = 1024, kWgSlots = kWgThreads / 64 / kSplits;
-template <int O> struct WgTables {
-  int off[Lines<O>::S * Lines<O>::S][Lines<O>::kMaxGroups];
+// Steps of small levels in one workgroup: x is in LDS, a step takes the row
+// pairs of a line group, 64 per slot of kSplits wavefronts at a time ("tile"),
+// and the steps follow each other with workgroup barriers.
+//
+// Bound by the instructions and the chain of a tile (16 wavefronts share 4
+// SIMDs), not by bandwidth:
+//  * where a lane's pair lies and which groups it has does not change from
+//    visit to visit and comes from a table (PairEntry), one load ahead;
+//  * the values of a tile do not depend on x and are loaded while the tile
+//    before it is combined and swept (the barriers wait for LDS only);
+//  * a lane issues the same loads as the others: an offset past the end of the
+//    buffer descriptor loads zero.  (With branches around them the compiler
+//    merges the registers of loads in flight by copies, and waits for them.)
+// 17^3 Q2 FP32: 3.3 us per group step; loading the values inside the step took
+// 5.2 us, a launch per group takes 4.5 us.
+template <typename T, int O> struct Wg {
+  static constexpr int kThreads = 1024, kSlots = kThreads / 64 / kSplits, kTile = 64 * kSlots;
+  static constexpr int kGroups = Lines<O>::C * Lines<O>::C;
+  static constexpr int kParts = O == 2 && sizeof(T) == 4 ? 3 : 2;  // groups of a row per split and batch
+  static constexpr int kOffsets = O == 2 ? Lines<2>::S * Lines<2>::S * Lines<2>::kMaxGroups : 0;
+  // LDS of a slot: the partial sums of its splits, a row pair's own group and
+  // the reciprocals of its diagonals
+  static constexpr int kRow = Lines<O>::VL + 2;
+  static constexpr size_t kSlotBytes = 64 * ((kSplits - 1) * sizeof(PairSums<T>) + kRow * sizeof(T));
+  static constexpr size_t kRedBytes = kSlots * kSlotBytes + 2 * kOffsets;
 };
-template <int O> __device__ __forceinline__ void wg_tables(WgTables<O> &s) {
-  constexpr int n = Lines<O>::S * Lines<O>::S * Lines<O>::kMaxGroups;
-  const int *src = &group_table<O>().off[0][0];
-  for (int i = threadIdx.x; i < n; i += kWgThreads) (&s.off[0][0])[i] = src[i];
+static_assert(Wg<float, 2>::kTile == kPairTile, "tile of the pair table");
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
-// Runs fn(pair sums, line, lane data) for the pairs of the lines y = y0 + ys j,
-// z = z0 + zs k of the level; every thread of the workgroup calls it.
-struct WgPair {
-  int m, p0, c;       // pair, lattice index of coordinate 2m, class
-  int64_t base;       // groups stored before the line
-  bool ok;
-};
-template <typename T, int O, class F>
-__device__ __forceinline__ void wg_lines(const WgTables<O> &tb, PairSums<T> (*red)[kSplits - 1][64], int lg, int y0,
-                                         int ys, int z0, int zs, const T *__restrict__ val, const T *lx, bool lo,
-                                         bool hi, F fn) {
+// Entry q of group g at (g tiles + q / kPairTile) kPairTile + q % kPairTile:
+//   x: lattice index of coordinate 2m (20 bits), m (6 bits), last pair of its
+//      line, no pair (the entry completes a tile)
+//   y: groups stored before the line (16 bits), groups before it in the sweep
+//      (5), all its groups (5), class of the line (6)
+template <int O>
+__global__ __launch_bounds__(kPairTile) void k_pair_table(int lg, int tiles, int2 *__restrict__ out) {
   using L = Lines<O>;
-  const int P = 1 << lg, M = 2 * P + 1;
-  if (y0 > M - 2 || z0 > M - 2) return;
-  const int ny = (M - 2 - y0) / ys + 1, nz = (M - 2 - z0) / zs + 1, np = ny * nz * P;
+  const int P = 1 << lg, M = 2 * P + 1, g = blockIdx.x / tiles, q = (blockIdx.x % tiles) * kPairTile + threadIdx.x;
+  const int yr = g % L::C, zr = g / L::C, y0 = yr ? yr : L::C, z0 = zr ? zr : L::C;
+  const int ny = y0 <= M - 2 ? (M - 2 - y0) / L::C + 1 : 0, nz = z0 <= M - 2 ? (M - 2 - z0) / L::C + 1 : 0;
+  const bool ok = q < (ny * nz << lg);
+  const int ln = ok ? q >> lg : 0, y = ny && nz ? y0 + L::C * (ln % ny) : 1, z = ny && nz ? z0 + L::C * (ln / ny) : 1;
+  const int m = q & (P - 1);
+  const GroupOrder<O> o(y, z);
+  int2 e;
+  e.x = (M * (y + M * z) + 2 * m) | m << 20 | (m == P - 1 ? 1 << 26 : 0) | (ok ? 0 : 1 << 27);
+  e.y = (int)((unsigned)L::group_base(P, y, z) | (unsigned)o.before() << 16 | (unsigned)o.groups() << 21 |
+              (unsigned)(y % L::S + L::S * (z % L::S)) << 26);
+  out[blockIdx.x * kPairTile + threadIdx.x] = e;
+}
+struct WgPair {
+  int m, p0;  // pair, lattice index of coordinate 2m
+  bool last, ok;
+  unsigned line;  // PairEntry y
+  __device__ __forceinline__ explicit WgPair(int2 e)
+      : m((e.x >> 20) & 63), p0(e.x & 0xfffff), last(e.x & 1 << 26), ok(!(e.x & 1 << 27)), line((unsigned)e.y) {}
+  __device__ __forceinline__ int base() const { return (int)(line & 0xffff); }
+  __device__ __forceinline__ int before() const { return (int)(line >> 16 & 31); }
+  __device__ __forceinline__ int groups() const { return (int)(line >> 21 & 31); }
+  __device__ __forceinline__ int cls() const { return (int)(line >> 26); }
+};
+// What a step needs of a level; plane: of one plane of it, x in LDS from the
+// first plane that the rows touch
+template <typename T> struct WgLevel {
+  const T *val;
+  const int2 *pairs;
+  int lg, tiles;
+};
+struct WgStep {
+  int g, seq, sums;  // line group, of a sweep: direction and sums (k_line_sweep)
+};
+// the line offsets (dy + M dz) M of the groups of every class (Q2; the lines
+// of a Q1 group are of one class): behind the pairs, and a copy in LDS
+template <int O> __global__ void k_group_offsets(int lg, short *__restrict__ out) {
+  using L = Lines<O>;
+  const int M = 2 * (1 << lg) + 1, c = blockIdx.x, k = threadIdx.x;
+  const GroupOrder<O> o(c % L::S + L::S, c / L::S + L::S);
+  out[c * L::kMaxGroups + k] = k < o.groups() ? (short)(o.line(k, M) * M) : (short)0;
+}
+template <typename T, int O> __device__ __forceinline__ void wg_offsets(const WgLevel<T> &lv, short *tab) {
+  constexpr int n = Wg<T, O>::kOffsets;
+  const int *src = reinterpret_cast<const int *>(lv.pairs + Wg<T, O>::kGroups * lv.tiles * kPairTile);
+  static_assert(n % 2 == 0, "whole words");
+  for (int i = threadIdx.x; i < n / 2; i += blockDim.x) reinterpret_cast<int *>(tab)[i] = src[i];
+}
+constexpr int kNoOffset = 0x40000000;
+__device__ __forceinline__ int2 pair_entry(__amdgpu_buffer_rsrc_t pairs, int off) {
+  const auto u = __builtin_amdgcn_raw_buffer_load_b64(pairs, off, 0, 0);
+  int2 e;
+  __builtin_memcpy(&e, &u, 8);
+  return e;
+}
+template <typename T> struct LevelBuffer {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ LevelBuffer(const T *p, int64_t n)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(p), 0, (int)(n * (int64_t)sizeof(T)), 0x00020000)) {}
+  // N consecutive elements at off (bytes, per lane) + base (bytes, uniform)
+  template <int N> __device__ __forceinline__ void at(int off, int base, T *out) const {
+    if constexpr (N * sizeof(T) == 16) {
+      const auto u = __builtin_amdgcn_raw_buffer_load_b128(r, off, base, 0);
+      __builtin_memcpy(out, &u, 16);
+    } else {
+      static_assert(N * sizeof(T) == 8, "8 or 16 bytes");
+      const auto u = __builtin_amdgcn_raw_buffer_load_b64(r, off, base, 0);
+      __builtin_memcpy(out, &u, 8);
+    }
+  }
+  __device__ __forceinline__ T one(int off) const {
+    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+  }
+  // a group's values for pair m; off: the group (bytes), or none
+  template <int O> __device__ __forceinline__ void group(int off, int P, int m, T *out) const {
+    using S = Slots<T, O>;
+    constexpr int ES = sizeof(T);
+    at<S::width(0)>(off + m * (S::width(0) * ES), 0, out);
+    if constexpr (S::VL > S::W) at<S::width(S::W)>(off + m * (S::width(S::W) * ES), S::W * P * ES, out + S::W);
+    if constexpr (S::VL > 2 * S::W)
+      at<S::width(2 * S::W)>(off + m * (S::width(2 * S::W) * ES), 2 * S::W * P * ES, out + 2 * S::W);
+    if constexpr (S::VL > 3 * S::W)
+      at<S::width(3 * S::W)>(off + m * (S::width(3 * S::W) * ES), 3 * S::W * P * ES, out + 3 * S::W);
+    static_assert(S::VL <= 4 * S::W, "at most four chunks");
+  }
+};
+// LDS of wg_run: sums, rows, group offsets
+template <typename T, int O> struct WgLds {
+  PairSums<T> *red;
+  T *rows;
+  short *tab;
+  __device__ __forceinline__ WgLds(unsigned char *p, int slots)
+      : red(reinterpret_cast<PairSums<T> *>(p)), rows(reinterpret_cast<T *>(red + slots * (kSplits - 1) * 64)),
+        tab(reinterpret_cast<short *>(rows + slots * Wg<T, O>::kRow * 64)) {}
+  __device__ __forceinline__ T *end() const { return reinterpret_cast<T *>(tab + Wg<T, O>::kOffsets); }
+};
+// Runs the steps of an iterator (bool next(WgStep &)): for every tile the pair
+// sums of the parts in step.sums, then fn(step, pair, sums, own values and
+// reciprocals of the diagonals, pre) with pre = before_sums(step, pair) in the
+// wavefronts of split 0, and a barrier after it.  lx: x in LDS, at its lattice
+// indices.  A tile's groups come in batches of kSplits * kParts, the next one
+// in flight while one is added.  The own group is loaded by split 1, which
+// hands it over with the sums (split 0 still uses the one of the tile before).
+template <typename T, int O, class It, class Pre, class F>
+__device__ __forceinline__ void wg_run(const WgLds<T, O> &lds, const WgLevel<T> &lv, const T *lx, It it,
+                                       Pre before_sums, F fn) {
+  using L = Lines<O>;
+  using W = Wg<T, O>;
+  constexpr int VL = L::VL, NX = O == 2 ? 5 : 4, NP = W::kParts, ES = sizeof(T), B = kSplits * NP;
+  const int P = 1 << lv.lg, M = 2 * P + 1;
   const int t = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slot = wave / kSplits, w = wave % kSplits;
-  const GroupTable<O> &g = group_table<O>();
-  for (int q0 = 0; q0 < np; q0 += 64 * kWgSlots) {
-    const int q = q0 + 64 * slot + t, qc = q < np ? q : np - 1;
-    const int ln = qc >> lg, kz = ln / ny;
-    const int y = y0 + ys * (ln - kz * ny), z = z0 + zs * kz;
-    WgPair pr;
-    pr.ok = q < np;
-    pr.m = qc & (P - 1);
-    pr.c = line_class<O>(y, z);
-    pr.base = L::group_base(P, y, z);
-    pr.p0 = M * (y + M * z) + 2 * pr.m;
-    const T *v = val + line_values<T, O>(P, pr.base, pr.m);
-    const int nlo = g.nlo[pr.c], ng = g.ng[pr.c];
-    T own[L::VL];
-    if (w == 0) load_group<T, O>(v + (int64_t)nlo * (L::VL * P), P, own);
-    PairSums<T> s = pair_sums<T, T, O, 2>(v, lx + pr.p0, tb.off[pr.c], nlo, ng, lo, hi, w, P, M, run_split<O>(pr.m, P));
-    if (w) red[slot][w - 1][t] = s;
-    __syncthreads();
-    if (w == 0) {
-#pragma unroll
-      for (int k = 0; k < kSplits - 1; k++) add_partial(s, red[slot][k][t]);
-      fn(pr, s, own);
+  const LevelBuffer<T> buf(lv.val, L::values(P));
+  struct At {
+    WgStep st;
+    int tile, nlo, n;  // batches of the lower part, of both
+    __device__ __forceinline__ void start() {
+      // (lines of extent 2 have the most groups)
+      const int zr = O == 2 ? (st.g * 11) >> 5 : st.g >> 1, yr = st.g - L::C * zr;
+      const int lo = O == 2 ? 10 * zr + 2 * yr : 6 * zr + 2 * yr, hi = L::kMaxGroups - 1 - lo;
+      tile = 0;
+      nlo = (st.sums & kSumLo) ? (lo + B - 1) / B : 0;
+      n = nlo + ((st.sums & kSumHi) ? (hi + B - 1) / B : 0);
+      if (n == 0) n = 1;
     }
-    __syncthreads();
+    __device__ __forceinline__ bool next(It &it, int tiles) {
+      if (++tile < tiles) return true;
+      if (!it.next(st)) return false;
+      start();
+      return true;
+    }
+  };
+  const __amdgpu_buffer_rsrc_t pbuf = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int2 *>(lv.pairs), 0, W::kGroups * lv.tiles * kPairTile * (int)sizeof(int2), 0x00020000);
+  auto entry = [&](const At &a, bool any) {
+    return pair_entry(pbuf, any ? ((a.st.g * lv.tiles + a.tile) * kPairTile + 64 * slot + t) * 8 : kNoOffset);
+  };
+  // line offset of group k of the lane's pair (class of the line group for Q1)
+  auto line_offset = [&](const At &a, const WgPair &pr, int k) {
+    if constexpr (O == 2) {
+      return (int)lds.tab[pr.cls() * L::kMaxGroups + k];
+    } else {
+      const GroupOrder<1> o((a.st.g & 1) + 2, (a.st.g >> 1) + 2);
+      return o.line(k, M) * M;
+    }
+  };
+  // the groups k0, k0 + kSplits, .. < k1 of a batch for this split
+  auto range = [&](const At &a, int batch, const WgPair &pr, int &k0, int &k1) {
+    if (batch < a.nlo) {
+      k0 = w + B * batch;
+      k1 = pr.before();
+    } else {
+      k0 = pr.before() + 1 + w + B * (batch - a.nlo);
+      k1 = (a.st.sums & kSumHi) ? pr.groups() : 0;
+    }
+    if (!pr.ok) k1 = 0;
+  };
+  T v[NP][VL], own[VL];
+  // a batch, with the last one the own group
+  auto load = [&](const At &a, int batch, const WgPair &pr, bool any) {
+    int k0, k1;
+    range(a, batch, pr, k0, k1);
+    if (!any) k1 = 0;
+    const int off = (pr.base() + k0) * (VL * P * ES);
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+      buf.template group<O>(k0 + kSplits * i < k1 ? off + i * (kSplits * VL * P * ES) : kNoOffset, P, pr.m, v[i]);
+    buf.template group<O>(
+        any && w == 1 && batch + 1 == a.n ? (pr.base() + pr.before()) * (VL * P * ES) : kNoOffset, P, pr.m, own);
+  };
+  PairSums<T> s{0, 0, 0, 0};
+  // a batch's part of the split's sums, in the order of k
+  auto add = [&](const At &a, int batch, const WgPair &pr) {
+    const int d3 = pr.last ? (O == 2 ? 1 : 2) : 3;
+    const bool lo = batch < a.nlo;
+    int k0, k1;
+    range(a, batch, pr, k0, k1);
+    T ao = lo ? s.lo_o : s.hi_o, ae = lo ? s.lo_e : s.hi_e;
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      const int k = k0 + kSplits * i;
+      const T *q = lx + pr.p0 + line_offset(a, pr, k < L::kMaxGroups ? k : 0);
+      if (k >= k1) q = lx + pr.p0;  // (values 0)
+      T r[NX];
+#pragma unroll
+      for (int e = 0; e < 3; e++) r[e] = q[e];
+#pragma unroll
+      for (int e = 3; e < NX; e++) r[e] = q[d3 + e - 3];
+#pragma unroll
+      for (int e = 0; e < 3; e++) ao = fma(v[i][e], r[e], ao);
+#pragma unroll
+      for (int e = 0; e < 2 * O + 1; e++) ae = fma(v[i][3 + e], r[e + 2 - O], ae);
+    }
+    if (lo) {
+      s.lo_o = ao;
+      s.lo_e = ae;
+    } else {
+      s.hi_o = ao;
+      s.hi_e = ae;
+    }
+  };
+  At cur;
+  if (!it.next(cur.st)) return;
+  cur.start();
+  WgPair pr(entry(cur, true));
+  load(cur, 0, pr, true);
+  while (true) {
+    At nxt = cur;
+    const bool go = nxt.next(it, lv.tiles);
+    const int2 en = entry(nxt, go);
+    for (int b = 0; b + 1 < cur.n; b++) {
+      add(cur, b, pr);
+      load(cur, b + 1, pr, true);
+    }
+    add(cur, cur.n - 1, pr);
+    if (w) lds.red[(slot * (kSplits - 1) + w - 1) * 64 + t] = s;
+    if (w == 1) {
+      T *o = lds.rows + slot * (W::kRow * 64) + t;
+#pragma unroll
+      for (int e = 0; e < VL; e++) o[64 * e] = own[e];
+      o[64 * VL] = T(1) / own[1];
+      o[64 * VL + 64] = T(1) / own[3 + O];
+    }
+    const WgPair mine = pr;
+    pr = WgPair(en);
+    load(nxt, 0, pr, go);
+    if (w == 0) {
+      const auto pre = before_sums(cur.st, mine);
+      lds_barrier();
+      T row[W::kRow];
+      const T *o = lds.rows + slot * (W::kRow * 64) + t;
+#pragma unroll
+      for (int e = 0; e < W::kRow; e++) row[e] = o[64 * e];
+#pragma unroll
+      for (int k = 0; k < kSplits - 1; k++) add_partial(s, lds.red[(slot * (kSplits - 1) + k) * 64 + t]);
+      fn(cur.st, mine, s, row, pre);
+    } else {
+      lds_barrier();
+    }
+    lds_barrier();
+    if (!go) return;
+    cur = nxt;
+    s = PairSums<T>{0, 0, 0, 0};
   }
+}
+// The rows of a sweep step; f, psum: lattice vectors
+template <typename T> struct WgSweepRow {
+  PairRow<T> r;
+  T x[3], ko, ke;
+};
+template <typename T, int O>
+__device__ __forceinline__ WgSweepRow<T> wg_sweep_row(const WgStep &st, const WgPair &pr, const T *lx, const T *f,
+                                                      const T *psum) {
+  const int p = pr.p0;
+  const bool kept = st.sums & kSumKept;
+  return WgSweepRow<T>{{f[p + 1], f[p + 2], T(0), T(0), T(0), T(0), T(0), T(0)},
+                       {lx[p], lx[p + 1], lx[p + 2]},
+                       kept ? psum[p + 1] : T(0),
+                       kept ? psum[p + 2] : T(0)};
 }
 template <typename T, int O>
-__device__ __forceinline__ void wg_sweep(const WgTables<O> &tb, PairSums<T> (*red)[kSplits - 1][64], int lg,
-                                         const T *__restrict__ val, T *lx, const T *__restrict__ f, double omega,
-                                         bool ssor) {
-  using L = Lines<O>;
-  constexpr int G = L::C * L::C;
-  const int P = 1 << lg;
-  for (int i = 0; i < (ssor ? 2 * G - 1 : G); i++) {
-    const int gi = i < G ? i : 2 * G - 2 - i;
-    const int seq = i >= G ? kBackward : (ssor && i == G - 1) ? kForwardBackward : kForward;
-    const int yr = gi % L::C, zr = gi / L::C;
-    wg_lines<T, O>(tb, red, lg, yr ? yr : L::C, L::C, zr ? zr : L::C, L::C, val, lx, true, true,
-                   [&](const WgPair &pr, const PairSums<T> &s, const T *own) {
-                     const PairRow<T> r{f[pr.p0 + 1], f[pr.p0 + 2], s.lo_o + s.hi_o, s.lo_e + s.hi_e, own[1], own[3 + O]};
-                     line_steps<T, T, O>(lx + pr.p0 - 2 * pr.m, own, r, pr.m, P, seq, omega, pr.ok, false);
-                   });
+__device__ __forceinline__ void wg_sweep_pair(const WgStep &st, const WgPair &pr, PairSums<T> s, const T *own,
+                                              WgSweepRow<T> row, T *lx, T *psum, int P, double omega) {
+  const int po = pr.p0 + 1, pe = pr.p0 + 2;
+  if (st.sums & kSumKept) {
+    if (st.sums & kSumLo) {
+      s.hi_o = row.ko;
+      s.hi_e = row.ke;
+    } else {
+      s.lo_o = row.ko;
+      s.lo_e = row.ke;
+    }
+  }
+  row.r.so = s.lo_o + s.hi_o;
+  row.r.se = s.lo_e + s.hi_e;
+  row.r.dio = own[1];
+  row.r.die = own[3 + O];
+  row.r.rio = own[Lines<O>::VL];
+  row.r.rie = own[Lines<O>::VL + 1];
+  line_steps<T, T, O>(row.x, own, row.r, pr.m, P, st.seq, omega);
+  if (!pr.ok) return;
+  const int keep = st.sums & kKeepZero;
+  lx[po] = row.x[1];
+  if (keep) psum[po] = keep == kKeepLo ? s.lo_o : keep == kKeepHi ? s.hi_o : T(0);
+  if (!pr.last) {
+    lx[pe] = row.x[2];
+    if (keep) psum[pe] = keep == kKeepLo ? s.lo_e : keep == kKeepHi ? s.hi_e : T(0);
   }
 }
-// the level's x, Dirichlet rows x = f
-template <typename T>
+// The steps of n SOR / SSOR sweeps over the line groups (the launches of sweeps())
+template <int O> struct WgSweeps {
+  int n;
+  bool ssor, zero;
+  int s = 0, j = -1;  // sweep, position in it (forward 0 .. G-1, backward G .. 2G-2)
+  __host__ __device__ bool next(WgStep &st) {
+    constexpr int G = Lines<O>::C * Lines<O>::C;
+    if (++j == (ssor ? 2 * G - 1 : G)) {
+      s++;
+      j = ssor ? 1 : 0;  // (the turn at group 0 belongs to the sweep before)
+    }
+    if (s >= n) return false;
+    st.g = j;
+    if (!ssor) {
+      st.seq = kForward;
+      st.sums = kSumLo | (zero && s == 0 ? 0 : kSumHi);
+    } else if (j < G) {
+      const bool turn = j == G - 1;
+      st.seq = turn ? kForwardBackward : kForward;
+      st.sums = kSumLo | (s > 0 ? kSumKept : zero ? 0 : kSumHi) | (turn ? kKeepZero : kKeepLo);
+    } else {
+      st.g = 2 * G - 2 - j;
+      const bool turn = st.g == 0 && s + 1 < n;
+      st.seq = turn ? kBackwardForward : kBackward;
+      st.sums = kSumHi | kSumKept | (turn ? kKeepZero : kKeepHi);
+    }
+    return true;
+  }
+};
+// every row once, in the order of the groups
+template <int O> struct WgAll {
+  int sums;
+  int g = -1;
+  __device__ __forceinline__ bool next(WgStep &st) {
+    st = WgStep{++g, 0, sums};
+    return g < Lines<O>::C * Lines<O>::C;
+  }
+};
+template <typename T, int O>
+__device__ __forceinline__ void wg_sweeps(const WgLds<T, O> &lds, const WgLevel<T> &lv, T *lx, const T *f, T *psum,
+                                          double omega, bool ssor, int n, bool zero) {
+  wg_run<T, O>(
+      lds, lv, lx, WgSweeps<O>{n, ssor, zero},
+      [&](const WgStep &st, const WgPair &pr) { return wg_sweep_row<T, O>(st, pr, lx, f, psum); },
+      [&](const WgStep &st, const WgPair &pr, const PairSums<T> &s, const T *own, const WgSweepRow<T> &row) {
+        wg_sweep_pair<T, O>(st, pr, s, own, row, lx, psum, 1 << lv.lg, omega);
+      });
+}
+struct WgNothing {};
+// the two rows' sums of a pair over all other entries
+template <typename T, int O>
+__device__ __forceinline__ void wg_off_diagonal(const WgPair &pr, const PairSums<T> &s, const T *own, const T *lx,
+                                                T &ro, T &re) {
+  const T *x = lx + pr.p0;
+  const int d3 = pr.last ? (O == 2 ? 1 : 2) : 3;
+  T xe[5] = {x[0], x[1], x[2], x[d3], O == 2 ? x[d3 + 1] : T(0)};
+  ro = own_odd<T, T, O>(own, xe, s.lo_o + s.hi_o);
+  re = own_even<T, T, O>(own, xe, s.lo_e + s.hi_e);
+}
+// fn(pair, odd, even): f - A x of every row pair; half: psum holds the upper sums
+template <typename T, int O, class F>
+__device__ __forceinline__ void wg_defect(const WgLds<T, O> &lds, const WgLevel<T> &lv, const T *lx, const T *f, const T *psum,
+                                          bool half, F fn) {
+  wg_run<T, O>(
+      lds, lv, lx, WgAll<O>{half ? kSumLo : kSumLo | kSumHi},
+      [](const WgStep &, const WgPair &) { return WgNothing{}; },
+      [&](const WgStep &, const WgPair &pr, PairSums<T> s, const T *own, WgNothing) {
+        if (half) {
+          s.hi_o = psum[pr.p0 + 1];
+          s.hi_e = psum[pr.p0 + 2];
+        }
+        T ro, re;
+        wg_off_diagonal<T, O>(pr, s, own, lx, ro, re);
+        fn(pr, f[pr.p0 + 1] - fma(own[1], lx[pr.p0 + 1], ro), f[pr.p0 + 2] - fma(own[3 + O], lx[pr.p0 + 2], re));
+      });
+}
+// one damped Jacobi sweep; xn: lattice vector for the new interior values
+template <typename T, int O>
+__device__ __forceinline__ void wg_jacobi(const WgLds<T, O> &lds, const WgLevel<T> &lv, T *lx, const T *f, T *xn,
+                                          double omega) {
+  const int M = 2 * (1 << lv.lg) + 1;
+  const T a = (T)omega;
+  wg_run<T, O>(
+      lds, lv, lx, WgAll<O>{kSumLo | kSumHi}, [](const WgStep &, const WgPair &) { return WgNothing{}; },
+      [&](const WgStep &, const WgPair &pr, const PairSums<T> &s, const T *own, WgNothing) {
+        T ro, re;
+        wg_off_diagonal<T, O>(pr, s, own, lx, ro, re);
+        if (!pr.ok) return;
+        xn[pr.p0 + 1] = (1 - a) * lx[pr.p0 + 1] + a * (f[pr.p0 + 1] - ro) / own[1];
+        if (!pr.last) xn[pr.p0 + 2] = (1 - a) * lx[pr.p0 + 2] + a * (f[pr.p0 + 2] - re) / own[3 + O];
+      });
+  __syncthreads();
+  for (int i = threadIdx.x; i < M * M * M; i += Wg<T, O>::kThreads) {
+    const int px = i % M, py = (i / M) % M, pz = i / (M * M);
+    if (px > 0 && py > 0 && pz > 0 && px < M - 1 && py < M - 1 && pz < M - 1) lx[i] = xn[i];
+  }
+  __syncthreads();
+}
+// the level's x with the Dirichlet rows x = f
+template <typename T, int NT>
 __device__ __forceinline__ void wg_stage(T *lx, const T *x, const T *__restrict__ f, int N, const int *__restrict__ bnd,
                                          int nb) {
-  for (int i = threadIdx.x; i < N; i += kWgThreads) lx[i] = x[i];
+  for (int i = threadIdx.x; i < N; i += NT) lx[i] = x[i];
   __syncthreads();
-  for (int i = threadIdx.x; i < nb; i += kWgThreads) lx[bnd[i]] = f[bnd[i]];
+  for (int i = threadIdx.x; i < nb; i += NT) lx[bnd[i]] = f[bnd[i]];
   __syncthreads();
 }
+// ============================================================ plane sweeps
+// Sweeps of small levels with a workgroup per plane: planes of one colour do
+// not couple, so the C (at a turn 2C - 1) line groups of a plane follow each
+// other in LDS, and a launch does the steps of a plane colour instead of one
+// line group.
+//
+// On top of the launch a step is a chain: sums, barrier, the colours of the
+// lines, barrier.  Wavefronts 0 .. kSplits - 1 take the splits of the sums
+// and load the values of the next step while the last wavefront goes through
+// the colours; that one has loaded the lines' own groups by then.  The pairs of
+// a plane's line group fit one wavefront (M <= 17).  An SSOR sweep at 17^3,
+// FP32 / FP64: Q2 39 / 49 us (5 launches), Q1 16 / 17 us (3); a launch per line
+// group 74 / 77 us (17 launches), 23 / 24 us (7); all of it in one workgroup
+// 59 / 98 and 32 / 37 us.  (Splits that sweep as well, with the loads before
+// the colours: 46 / 57 us.)
+template <typename T, int O> struct Plane {
+  static constexpr int C = Lines<O>::C, VL = Lines<O>::VL;
+  static constexpr int kThreads = 64 * (kSplits + 1), kPlanes = 2 * O + 1;
+  static constexpr int kParts = O == 2 ? 6 : 2;  // groups of a part per split
+  static constexpr int kLoads = O == 2 ? 5 : 3;  // elements of x per thread and round
+  static size_t lds_bytes(int M) {
+    return 64 * kSplits * sizeof(PairSums<T>) + 2 * Wg<T, O>::kOffsets + sizeof(T) * (kPlanes + 2) * M * M;
+  }
+};
+// A step in 12 bits: line group, direction, sums
+__host__ __device__ inline unsigned plane_step(const WgStep &s) {
+  return (unsigned)(s.g | s.seq << 4 | s.sums << 6);
+}
+template <int O> struct PlaneStep {
+  int g, seq, sums;
+  __device__ __forceinline__ explicit PlaneStep(uint64_t code)
+      : g((int)(code & 15)), seq((int)(code >> 4 & 3)), sums((int)(code >> 6 & 63)) {}
+  __device__ __forceinline__ int zr() const { return O == 2 ? (g * 11) >> 5 : g >> 1; }
+  __device__ __forceinline__ int yr() const { return g - Lines<O>::C * zr(); }
+  // groups before a line of extent O, the most of the step
+  __device__ __forceinline__ int lower() const { return O == 2 ? 10 * zr() + 2 * yr() : 6 * zr() + 2 * yr(); }
+};
 template <typename T, int O>
-__global__ __launch_bounds__(kWgThreads) void k_sweep_wg(int lg, const T *__restrict__ val, T *x,
-                                                         const T *__restrict__ f, double omega, int ssor,
-                                                         const int *__restrict__ bnd, int nb) {
-  extern __shared__ __align__(16) unsigned char sweep_lds[];
-  T *lx = reinterpret_cast<T *>(sweep_lds);
-  __shared__ WgTables<O> tb;
-  __shared__ PairSums<T> red[kWgSlots][kSplits - 1][64];
-  const int M = 2 * (1 << lg) + 1, N = M * M * M;
-  wg_tables<O>(tb);
-  wg_stage(lx, x, f, N, bnd, nb);
-  wg_sweep<T, O>(tb, red, lg, val, lx, f, omega, ssor != 0);
-  for (int i = threadIdx.x; i < N; i += kWgThreads) x[i] = lx[i];
+__global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel<T> lv, int z0, uint64_t steps,
+                                                                         uint64_t upper, T *x,
+                                                                         const T *__restrict__ f, T *psum, double omega,
+                                                                         const int *__restrict__ bnd_set) {
+  using L = Lines<O>;
+  using Q = Plane<T, O>;
+  extern __shared__ __align__(16) unsigned char wg_lds[];
+  constexpr int C = Q::C, VL = L::VL, NP = Q::kParts, NX = O == 2 ? 5 : 4, ES = sizeof(T), H = NP > 2 ? NP / 2 : NP;
+  const int P = 1 << lv.lg, M = 2 * P + 1, MM = M * M, z = z0 + C * (int)blockIdx.x;
+  const int t = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  PairSums<T> *red = reinterpret_cast<PairSums<T> *>(wg_lds);
+  short *tab = reinterpret_cast<short *>(red + 64 * kSplits);
+  // x of the planes that the rows touch, the plane's f and kept sums; positions
+  // are relative to the first of those planes
+  T *lx = reinterpret_cast<T *>(tab + Wg<T, O>::kOffsets), *lf = lx + (Q::kPlanes - O) * MM, *lp = lf + MM;
+  // (a start from zero has upper sums where the boundary values are not zero)
+  if (bnd_set && *bnd_set) steps |= upper;
+  const LevelBuffer<T> buf(lv.val, L::values(P));
+  const __amdgpu_buffer_rsrc_t pbuf = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int2 *>(lv.pairs), 0, Wg<T, O>::kGroups * lv.tiles * kPairTile * (int)sizeof(int2), 0x00020000);
+  // the lane's pair in each of the plane's line groups (of the lanes past the
+  // last line a pair that exists, for its position)
+  int2 e[C];
+  {
+    const int zr = z % C;
+#pragma unroll
+    for (int yr = 0; yr < C; yr++) {
+      const int n = ((M - 2 - (yr ? yr : C)) / C + 1) << lv.lg;
+      e[yr] = pair_entry(pbuf, (((yr + C * zr) * lv.tiles) * kPairTile + (z - (zr ? zr : C)) / C * n + (t < n ? t : 0)) * 8);
+    }
+  }
+  const LevelBuffer<T> bx(x, (int64_t)M * MM), bf(f, (int64_t)M * MM), bp(psum, (int64_t)M * MM);
+  const LevelBuffer<float> bo(reinterpret_cast<const float *>(lv.pairs + Wg<T, O>::kGroups * lv.tiles * kPairTile),
+                              Wg<T, O>::kOffsets / 2);  // (words of two)
+  const bool kept = psum != nullptr;
+  T vx[Q::kLoads], vf, vp;
+  float vo[2];
+  auto x_loads = [&](int i0) {
+    const int x0 = (z - O) * MM;
+#pragma unroll
+    for (int u = 0; u < Q::kLoads; u++) {
+      const int i = i0 + u * Q::kThreads;
+      // (elements outside the lattice load zero: they are not read)
+      vx[u] = bx.one(i < Q::kPlanes * MM && x0 + i >= 0 ? (x0 + i) * ES : kNoOffset);
+    }
+  };
+  auto x_stores = [&](int i0) {
+#pragma unroll
+    for (int u = 0; u < Q::kLoads; u++) {
+      const int i = i0 + u * Q::kThreads;
+      if (i < Q::kPlanes * MM) lx[i] = vx[u];
+    }
+  };
+  x_loads(threadIdx.x);
+  {
+    const int i = threadIdx.x, off = i < MM ? (z * MM + i) * ES : kNoOffset;
+    vf = bf.one(off);
+    vp = bp.one(kept ? off : kNoOffset);
+    if (Wg<T, O>::kOffsets) {
+      vo[0] = bo.one(4 * i);
+      vo[1] = bo.one(4 * (i + Q::kThreads));
+    }
+  }
+#pragma unroll
+  for (int yr = 0; yr < C; yr++) {
+    e[yr].x -= (z - O) * MM;
+    if (t >= ((M - 2 - (yr ? yr : C)) / C + 1) << lv.lg) e[yr].x |= 1 << 27;
+  }
+  auto stage = [&] {
+    x_stores(threadIdx.x);
+    if ((int)threadIdx.x < MM) {
+      lf[O * MM + threadIdx.x] = vf;
+      lp[O * MM + threadIdx.x] = vp;
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int i = (int)threadIdx.x + u * Q::kThreads;
+      if (i < Wg<T, O>::kOffsets / 2) reinterpret_cast<float *>(tab)[i] = vo[u];
+    }
+    static_assert(Wg<T, O>::kOffsets / 2 <= 2 * Q::kThreads, "offsets per thread");
+    for (int i = threadIdx.x + Q::kLoads * Q::kThreads; i < Q::kPlanes * MM; i += Q::kLoads * Q::kThreads) {
+      x_loads(i);
+      x_stores(i);
+    }
+    for (int i = threadIdx.x + Q::kThreads; i < MM; i += Q::kThreads) {
+      lf[O * MM + i] = bf.one((z * MM + i) * ES);
+      lp[O * MM + i] = bp.one(kept ? (z * MM + i) * ES : kNoOffset);
+    }
+  };
+  auto pair_of = [&](const PlaneStep<O> &s) {
+    int2 r = e[0];
+#pragma unroll
+    for (int yr = 1; yr < C; yr++)
+      if (s.yr() == yr) r = e[yr];
+    return WgPair(r);
+  };
+  if (w < kSplits) {
+    PlaneStep<O> s(steps);
+    WgPair pr = pair_of(s);
+    T v[NP][VL];
+    int at[NP];  // x of the groups
+    // the values of one part; the second half of them only where a row of the
+    // step has so many groups
+    auto many = [&](bool lo) { return NP > 2 && (lo ? s.lower() : L::kMaxGroups - 1 - s.lower()) > kSplits * H; };
+    auto load = [&](bool lo) {
+      const int k0 = lo ? w : pr.before() + 1 + w, k1 = !pr.ok ? 0 : lo ? pr.before() : pr.groups();
+      const int off = (pr.base() + k0) * (VL * P * ES);
+      auto one = [&](int i) {
+        buf.template group<O>(k0 + kSplits * i < k1 ? off + i * (kSplits * VL * P * ES) : kNoOffset, P, pr.m, v[i]);
+      };
+#pragma unroll
+      for (int i = 0; i < H; i++) one(i);
+      if (many(lo)) {
+#pragma unroll
+        for (int i = H; i < NP; i++) one(i);
+      }
+    };
+    auto positions = [&](bool lo) {
+      const int k0 = lo ? w : pr.before() + 1 + w, k1 = lo ? pr.before() : pr.groups();
+      const GroupOrder<1> o((s.g & 1) + 2, (s.g >> 1) + 2);
+#pragma unroll
+      for (int i = 0; i < NP; i++) {
+        const int k = k0 + kSplits * i;
+        int d;
+        if constexpr (O == 2) d = tab[pr.cls() * L::kMaxGroups + (k < k1 ? k : 0)];
+        else d = o.line(k < k1 ? k : 0, M) * M;
+        at[i] = pr.p0 + (k < k1 ? d : 0);  // (past the last group values 0)
+      }
+    };
+    T so, se;
+    auto add = [&](bool lo) {
+      const int d3 = pr.last ? (O == 2 ? 1 : 2) : 3;
+      so = se = 0;
+      auto one = [&](int i) {
+        const T *q = lx + at[i];
+        T r[NX];
+#pragma unroll
+        for (int c = 0; c < 3; c++) r[c] = q[c];
+#pragma unroll
+        for (int c = 3; c < NX; c++) r[c] = q[d3 + c - 3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) so = fma(v[i][c], r[c], so);
+#pragma unroll
+        for (int c = 0; c < 2 * O + 1; c++) se = fma(v[i][3 + c], r[c + 2 - O], se);
+      };
+#pragma unroll
+      for (int i = 0; i < H; i++) one(i);
+      if (many(lo)) {
+#pragma unroll
+        for (int i = H; i < NP; i++) one(i);
+      }
+    };
+    load(s.sums & kSumLo);
+    stage();
+    __syncthreads();
+    positions(s.sums & kSumLo);
+    while (true) {
+      PairSums<T> p{0, 0, 0, 0};
+      if (s.sums & kSumLo) {
+        add(true);
+        p.lo_o = so;
+        p.lo_e = se;
+        if (s.sums & kSumHi) {
+          load(false);
+          positions(false);
+        }
+      }
+      if (s.sums & kSumHi) {
+        add(false);
+        p.hi_o = so;
+        p.hi_e = se;
+      }
+      red[64 * w + t] = p;
+      lds_barrier();
+      steps >>= 12;
+      if (steps) {
+        s = PlaneStep<O>(steps);
+        pr = pair_of(s);
+        load(s.sums & kSumLo);
+        positions(s.sums & kSumLo);
+      }
+      lds_barrier();
+      if (!steps) break;
+    }
+  } else {
+    PlaneStep<O> s(steps);
+    WgPair pr = pair_of(s);
+    auto load = [&](const WgPair &q, bool any, T *own) {
+      buf.template group<O>(any && q.ok ? (q.base() + q.before()) * (VL * P * ES) : kNoOffset, P, q.m, own);
+    };
+    T own[VL], next[VL];
+    load(pr, true, own);
+    stage();
+    __syncthreads();
+    while (true) {
+      steps >>= 12;
+      const PlaneStep<O> sn(steps);
+      const WgPair pn = pair_of(sn);
+      load(pn, steps != 0, next);
+      const int p = pr.p0;
+      PairRow<T> r{lf[p + 1], lf[p + 2], T(0), T(0), own[1], own[3 + O], T(1) / own[1], T(1) / own[3 + O]};
+      T xp[3] = {lx[p], lx[p + 1], lx[p + 2]};
+      const T ko = lp[p + 1], ke = lp[p + 2];
+      lds_barrier();
+      PairSums<T> u = red[t];
+#pragma unroll
+      for (int k = 1; k < kSplits; k++) add_partial(u, red[64 * k + t]);
+      if (s.sums & kSumKept) {
+        if (s.sums & kSumLo) {
+          u.hi_o = ko;
+          u.hi_e = ke;
+        } else {
+          u.lo_o = ko;
+          u.lo_e = ke;
+        }
+      }
+      r.so = u.lo_o + u.hi_o;
+      r.se = u.lo_e + u.hi_e;
+      line_steps<T, T, O>(xp, own, r, pr.m, P, s.seq, omega);
+      const int keep = s.sums & kKeepZero;
+      if (pr.ok) {
+        lx[p + 1] = xp[1];
+        if (keep) lp[p + 1] = keep == kKeepLo ? u.lo_o : keep == kKeepHi ? u.hi_o : T(0);
+        if (!pr.last) {
+          lx[p + 2] = xp[2];
+          if (keep) lp[p + 2] = keep == kKeepLo ? u.lo_e : keep == kKeepHi ? u.hi_e : T(0);
+        }
+      }
+      lds_barrier();
+      if (!steps) break;
+      s = sn;
+      pr = pn;
+#pragma unroll
+      for (int c = 0; c < VL; c++) own[c] = next[c];
+    }
+  }
+  for (int i = threadIdx.x; i < MM; i += Q::kThreads) {
+    const int px = i % M, py = i / M;
+    if (px < 1 || py < 1 || px > M - 2 || py > M - 2) continue;
+    x[z * MM + i] = lx[O * MM + i];
+    if (kept) psum[z * MM + i] = lp[O * MM + i];
+  }
 }
-
 // ||f - A x|| of the LDS iterate over all rows (Dirichlet rows: 0), the same
 // value in every thread
 template <typename T, int O>
-__device__ double wg_defect_norm(const WgTables<O> &tb, PairSums<T> (*red)[kSplits - 1][64], int lg,
-                                 const T *__restrict__ val, const T *lx, const T *__restrict__ f, double *lred) {
-  const int P = 1 << lg;
+__device__ double wg_defect_norm(const WgLds<T, O> &lds, const WgLevel<T> &lv, const T *lx, const T *f, double *lred) {
+  constexpr int NT = Wg<T, O>::kThreads;
   double sum = 0;
-  wg_lines<T, O>(tb, red, lg, 1, 1, 1, 1, val, lx, true, true,
-                 [&](const WgPair &pr, const PairSums<T> &s, const T *own) {
-                   if (!pr.ok) return;
-                   const T *x = lx + pr.p0;
-                   T ro = own_odd<T, T, O>(own, x, s.lo_o + s.hi_o);
-                   const T d = f[pr.p0 + 1] - fma(own[1], x[1], ro);
-                   sum += (double)d * (double)d;
-                   if (pr.m < P - 1) {
-                     T re = own_even<T, T, O>(own, x, s.lo_e + s.hi_e);
-                     const T e = f[pr.p0 + 2] - fma(own[3 + O], x[2], re);
-                     sum += (double)e * (double)e;
-                   }
-                 });
+  wg_defect<T, O>(lds, lv, lx, f, nullptr, false, [&](const WgPair &pr, T d, T e) {
+    if (!pr.ok) return;
+    sum += (double)d * (double)d;
+    if (!pr.last) sum += (double)e * (double)e;
+  });
   for (int o = 32; o > 0; o >>= 1) sum += __shfl_down(sum, o, 64);
   if (threadIdx.x % 64 == 0) lred[threadIdx.x / 64] = sum;
   __syncthreads();
   double t = 0;
-  for (int w = 0; w < kWgThreads / 64; w++) t += lred[w];
+  for (int w = 0; w < NT / 64; w++) t += lred[w];
   __syncthreads();
   return sqrt(t);
 }
@@ -400,47 +1082,29 @@ __device__ double wg_defect_norm(const WgTables<O> &tb, PairSums<T> (*red)[kSpli
 // res > red * res_0 and fewer than maxit sweeps: one Jacobi (kind 1, omega
 // damped), SOR (2) or SSOR (3) sweep and res again.  The sweeps compute each
 // row as the launched sweeps do (bit-identical iterates); xj: global scratch
-// of N entries (Jacobi output).
+// of N entries (Jacobi output, kept sums).
 template <typename T, int O>
-__global__ __launch_bounds__(kWgThreads) void k_coarse_wg(int lg, const T *__restrict__ val, T *x,
-                                                          const T *__restrict__ f, double omega, int kind, int maxit,
-                                                          double red_factor, const int *__restrict__ bnd, int nb,
-                                                          T *xj) {
-  extern __shared__ __align__(16) unsigned char sweep_lds[];
-  T *lx = reinterpret_cast<T *>(sweep_lds);
-  __shared__ WgTables<O> tb;
-  __shared__ PairSums<T> red[kWgSlots][kSplits - 1][64];
-  __shared__ double lred[kWgThreads / 64];
-  const int P = 1 << lg, M = 2 * P + 1, N = M * M * M;
-  wg_tables<O>(tb);
-  for (int i = threadIdx.x; i < nb; i += kWgThreads) xj[bnd[i]] = f[bnd[i]];
-  wg_stage(lx, x, f, N, bnd, nb);
-  double res = wg_defect_norm<T, O>(tb, red, lg, val, lx, f, lred);
+__global__ __launch_bounds__((Wg<T, O>::kThreads)) void k_coarse_wg(WgLevel<T> lv, T *x,
+                                                                    const T *__restrict__ f, double omega, int kind,
+                                                                    int maxit, double red_factor,
+                                                                    const int *__restrict__ bnd, int nb, T *xj) {
+  extern __shared__ __align__(16) unsigned char wg_lds[];
+  const WgLds<T, O> lds(wg_lds, Wg<T, O>::kSlots);
+  T *lx = lds.end();
+  __shared__ double lred[Wg<T, O>::kThreads / 64];
+  const int M = 2 * (1 << lv.lg) + 1, N = M * M * M;
+  wg_offsets<T, O>(lv, lds.tab);
+  wg_stage<T, Wg<T, O>::kThreads>(lx, x, f, N, bnd, nb);
+  double res = wg_defect_norm<T, O>(lds, lv, lx, f, lred);
   const double reduction = red_factor * res;
   for (int it = 0; res > reduction && it < maxit; it++) {
-    if (kind == 1) {
-      const T a = (T)omega;
-      wg_lines<T, O>(tb, red, lg, 1, 1, 1, 1, val, lx, true, true,
-                     [&](const WgPair &pr, const PairSums<T> &s, const T *own) {
-                       if (!pr.ok) return;
-                       const T *q = lx + pr.p0;
-                       const T ro = own_odd<T, T, O>(own, q, s.lo_o + s.hi_o);
-                       xj[pr.p0 + 1] = (1 - a) * q[1] + a * (f[pr.p0 + 1] - ro) / own[1];
-                       if (pr.m < P - 1) {
-                         const T re = own_even<T, T, O>(own, q, s.lo_e + s.hi_e);
-                         xj[pr.p0 + 2] = (1 - a) * q[2] + a * (f[pr.p0 + 2] - re) / own[3 + O];
-                       }
-                     });
-      for (int i = threadIdx.x; i < N; i += kWgThreads) lx[i] = xj[i];
-      __syncthreads();
-    } else {
-      wg_sweep<T, O>(tb, red, lg, val, lx, f, omega, kind == 3);
-    }
-    res = wg_defect_norm<T, O>(tb, red, lg, val, lx, f, lred);
+    if (kind == 1) wg_jacobi<T, O>(lds, lv, lx, f, xj, omega);
+    else wg_sweeps<T, O>(lds, lv, lx, f, xj, omega, kind == 3, 1, false);
+    __syncthreads();
+    res = wg_defect_norm<T, O>(lds, lv, lx, f, lred);
   }
-  for (int i = threadIdx.x; i < N; i += kWgThreads) x[i] = lx[i];
+  for (int i = threadIdx.x; i < N; i += Wg<T, O>::kThreads) x[i] = lx[i];
 }
-
 // Row-scaled FP16 copy of the FP32 values: entry k of an active row holds
 // a_k / a_diag rounded to FP16 (saturated at +-65504, the largest finite FP16
 // value), and dinv[p] = 1 / a_diag in FP32.  A pair's slots of a group are
@@ -453,25 +1117,63 @@ __global__ __launch_bounds__(64) void k_scaled_values(LineSet set, int lg, const
   const UnitLines u = unit_lines<O>(set, M, lg, blockIdx.x / segs);
   const int t = threadIdx.x + 64 * (blockIdx.x % segs), m = t & (P - 1), y = u.y0 + L::S * (t >> lg);
   if (y > M - 2) return;
-  const GroupTable<O> &g = group_table<O>();
-  const int c = line_class<O>(u.y0, u.z), nlo = g.nlo[c], ng = g.ng[c];
-  const int64_t base = L::group_base(P, y, u.z);
-  const float *v = val + line_values<float, O>(P, base, m);
-  _Float16 *o = val16 + line_values<_Float16, O>(P, base, m);
-  const float *own = v + (int64_t)nlo * (L::VL * P);
+  const GroupOrder<O> g(u.y0, u.z);
+  const int nlo = g.before(), ng = g.groups();
+  const float *v = val + line_values<O>(P, y, u.z);
+  _Float16 *o = val16 + line_values<O>(P, y, u.z);
+  float own[L::VL];
+  load_group<float, O>(v + (int64_t)nlo * (L::VL * P), P, m, own);
   const int p0 = M * (y + M * u.z) + 2 * m;
   const bool even = m < P - 1;
-  const float ro = 1.0f / own[1 * P], re = even ? 1.0f / own[(3 + O) * P] : 0.0f;
+  const float ro = 1.0f / own[1], re = even ? 1.0f / own[3 + O] : 0.0f;
   dinv[p0 + 1] = ro;
   if (even) dinv[p0 + 2] = re;
   for (int k = 0; k < ng; k++) {
     float a[L::VL];
     _Float16 h[L::VL];
-    load_group<float, O>(v + (int64_t)k * (L::VL * P), P, a);
+    load_group<float, O>(v + (int64_t)k * (L::VL * P), P, m, a);
 #pragma unroll
     for (int s = 0; s < L::VL; s++)
       h[s] = (_Float16)fminf(fmaxf(a[s] * (s < 3 ? ro : re), -65504.0f), 65504.0f);
-    __builtin_memcpy(o + (int64_t)k * (L::VL * P), h, sizeof(h));
+    static_assert(Slots<_Float16, O>::W >= L::VL, "one chunk");
+    __builtin_memcpy(o + (int64_t)k * (L::VL * P) + Slots<_Float16, O>::at(P, m, 0), h, sizeof(h));
+  }
+}
+
+// The FP32 copy of FP64 values; with mass: val = mass (+ kk) + c a first
+// (MatAdd of Blas2.C:128-150).  One thread per row pair of a group, because
+// the two types hold their slots in different chunks.
+template <int O, bool SYSTEM>
+__global__ __launch_bounds__(kBlock) void k_values(int lg, int64_t npairs, double *__restrict__ val,
+                                                   float *__restrict__ val32, const double *__restrict__ mass,
+                                                   const double *__restrict__ kk, const double *__restrict__ a,
+                                                   double c) {
+  using S = Slots<double, O>;
+  const int P = 1 << lg;
+  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < npairs; i += (int64_t)gridDim.x * kBlock) {
+    const int m = (int)(i & (P - 1));
+    const int64_t g = (i >> lg) * (S::VL * P);
+    double v[S::VL];
+    if constexpr (SYSTEM) {
+      double ma[S::VL], aa[S::VL], ka[S::VL];
+      load_group<double, O>(mass + g, P, m, ma);
+      load_group<double, O>(a + g, P, m, aa);
+      if (kk) load_group<double, O>(kk + g, P, m, ka);
+#pragma unroll
+      for (int s = 0; s < S::VL; s++) v[s] = (kk ? ma[s] + ka[s] : ma[s]) + c * aa[s];
+#pragma unroll
+      for (int s = 0; s < S::VL; s += S::W) __builtin_memcpy(val + g + S::at(P, m, s), v + s, S::width(s) * sizeof(double));
+    } else {
+      load_group<double, O>(val + g, P, m, v);
+    }
+    if (val32) {
+      using F = Slots<float, O>;
+      float w[F::VL];
+#pragma unroll
+      for (int s = 0; s < F::VL; s++) w[s] = (float)v[s];
+#pragma unroll
+      for (int s = 0; s < F::VL; s += F::W) __builtin_memcpy(val32 + g + F::at(P, m, s), w + s, F::width(s) * sizeof(float));
+    }
   }
 }
 
@@ -508,15 +1210,19 @@ static void timer_events(hipEvent_t *e0, hipEvent_t *e1) {
   t.used++;
 }
 template <typename... KA, typename... A>
-static void launch(void (*k)(KA...), unsigned grid, unsigned block, hipStream_t st, A... a) {
+static void launch_lds(void (*k)(KA...), unsigned grid, unsigned block, size_t lds, hipStream_t st, A... a) {
   if (grid == 0) return;
   if (g_timer) {
     hipEvent_t e0, e1;
     timer_events(&e0, &e1);
-    hipExtLaunchKernelGGL(k, dim3(grid), dim3(block), 0, st, e0, e1, 0, a...);
+    hipExtLaunchKernelGGL(k, dim3(grid), dim3(block), lds, st, e0, e1, 0, a...);
   } else {
-    hipLaunchKernelGGL(k, dim3(grid), dim3(block), 0, st, a...);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, st, a...);
   }
+}
+template <typename... KA, typename... A>
+static void launch(void (*k)(KA...), unsigned grid, unsigned block, hipStream_t st, A... a) {
+  launch_lds(k, grid, block, 0, st, a...);
 }
 
 // lines of one class period per unit, planes of a set
@@ -603,9 +1309,86 @@ static void sweeps(const DevLayout &D, const V *val, const float *dinv, T *x, co
     }
   }
 }
+template <typename T> static WgLevel<T> wg_level(const DevLayout &D, const T *val) {
+  return WgLevel<T>{val, D.pairs, D.lg, D.pair_tiles};
+}
+int pair_tiles(const Layout &L) {
+  // the largest group: the residues with the most lines
+  const int C = L.order == 2 ? 3 : 2, n = (L.M - 3) / C + 1;
+  return (int)(((int64_t)n * n * ((L.M - 1) / 2) + kPairTile - 1) / kPairTile);
+}
+size_t pair_table_size(const DevLayout &D) {
+  // (and the offsets of the groups)
+  return D.order == 2 ? (size_t)9 * D.pair_tiles * kPairTile + (2 * Wg<float, 2>::kOffsets + 7) / 8
+                      : (size_t)4 * D.pair_tiles * kPairTile;
+}
+void pair_table(const DevLayout &D, int2 *pairs, hipStream_t st) {
+  if (D.lg > 5) throw std::logic_error("pair_table: level too large");
+  const int G = D.order == 2 ? 9 : 4;
+  using L2 = Lines<2>;
+  if (D.order == 2) {
+    hipLaunchKernelGGL(k_group_offsets<2>, dim3(L2::S * L2::S), dim3(L2::kMaxGroups), 0, st, D.lg,
+                       reinterpret_cast<short *>(pairs + G * D.pair_tiles * kPairTile));
+    hipLaunchKernelGGL(k_pair_table<2>, dim3(G * D.pair_tiles), dim3(kPairTile), 0, st, D.lg, D.pair_tiles, pairs);
+  } else {
+    hipLaunchKernelGGL(k_pair_table<1>, dim3(G * D.pair_tiles), dim3(kPairTile), 0, st, D.lg, D.pair_tiles, pairs);
+  }
+}
+// launch of a one-workgroup kernel with `lds` bytes of dynamic LDS
+template <typename... KA, typename... A>
+static void launch_wg_grid(void (*k)(KA...), int grid, int threads, size_t lds, hipStream_t st, A... a) {
+  // (beyond the default limit the kernel's own limit is raised)
+  if (lds > 48 * 1024)
+    check(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+          "LDS size");
+  launch_lds(k, (unsigned)grid, (unsigned)threads, lds, st, a...);
+}
+template <typename... KA, typename... A>
+static void launch_wg(void (*k)(KA...), int threads, size_t lds, hipStream_t st, A... a) {
+  launch_wg_grid(k, 1, threads, lds, st, a...);
+}
+// ... with a launch per plane colour where the row pairs of a plane's line
+// group fit one wavefront, M <= 17.  (Four wavefronts per split took 33^3 in
+// one tile as well: 67 / 99 us per sweep of Q2, 27.6 / 35 us of Q1, FP32 /
+// FP64, against 74 / 78 and 23 / 24 us by line groups: there a CU reads the
+// values of a plane no faster than the launches go by.)
+bool plane_sweeps_fit(const DevLayout &D) {
+  const int C = D.order == 2 ? 3 : 2;
+  return D.M >= 3 && (((D.M - 3) / C + 1) << D.lg) <= 64;
+}
+template <typename T, int O>
+static void plane_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n,
+                         bool zero, const int *bnd_set, hipStream_t st) {
+  constexpr int C = Lines<O>::C;
+  WgSweeps<O> it{n, ssor, zero};
+  WgStep step;
+  bool more = it.next(step);
+  while (more) {
+    // the steps up to the next plane colour
+    const int zr = step.g / C, z0 = zr ? zr : C;
+    const bool start = zero && it.s == 0;
+    uint64_t steps = 0, upper = 0;
+    int k = 0;
+    do {
+      steps |= (uint64_t)plane_step(step) << 12 * k;
+      if (zero && it.s == 0 && !(step.sums & (kSumHi | kSumKept)))
+        upper |= (uint64_t)plane_step(WgStep{0, 0, kSumHi}) << 12 * k;
+      k++;
+      more = it.next(step);
+    } while (more && step.g / C == zr && k < 5);
+    launch_wg_grid(k_plane_sweep<T, O>, (D.M - 2 - z0) / C + 1, Plane<T, O>::kThreads, Plane<T, O>::lds_bytes(D.M), st,
+                   wg_level(D, val), z0, steps, upper, x, f, ssor ? psum : (T *)nullptr, omega,
+                   start ? bnd_set : (const int *)nullptr);
+  }
+}
 template <typename T>
 void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n, bool zero,
-                const int *bnd_set, hipStream_t st) {
+                const int *bnd_set, bool planes, hipStream_t st) {
+  if (planes && plane_sweeps_fit(D) && D.lg >= 1) {  // (3^3: one row)
+    if (D.order == 2) plane_sweeps<T, 2>(D, val, x, f, psum, omega, ssor, n, zero, bnd_set, st);
+    else plane_sweeps<T, 1>(D, val, x, f, psum, omega, ssor, n, zero, bnd_set, st);
+    return;
+  }
   sweeps<T, T>(D, val, nullptr, x, f, psum, omega, ssor, n, zero, bnd_set, st);
 }
 void sor_sweeps_scaled(const DevLayout &D, const _Float16 *val16, const float *dinv, float *x, const float *f,
@@ -619,16 +1402,22 @@ void scaled_values(const DevLayout &D, const float *val, _Float16 *val16, float 
   if (D.order == 2) hipLaunchKernelGGL(k_scaled_values<2>, dim3(g), dim3(64), 0, st, s, D.lg, val, val16, dinv);
   else hipLaunchKernelGGL(k_scaled_values<1>, dim3(g), dim3(64), 0, st, s, D.lg, val, val16, dinv);
 }
-template <typename T>
-void sweep_wg(const DevLayout &D, const T *val, T *x, const T *f, double omega, int ssor, hipStream_t st) {
-  if (!sweep_wg_fits(D, sizeof(T))) throw std::logic_error("sweep_wg: level does not fit in LDS");
-  const size_t lds = (size_t)D.N * sizeof(T);
+template <bool SYSTEM>
+static void values(const DevLayout &D, double *val, float *val32, const double *mass, const double *k, const double *a,
+                   double c, hipStream_t st) {
+  const int64_t np = D.nvals / (D.order == 2 ? Lines<2>::VL : Lines<1>::VL);
+  const dim3 g((unsigned)std::min<int64_t>((np + kBlock - 1) / kBlock, 1 << 20));
   if (D.order == 2)
-    hipLaunchKernelGGL((k_sweep_wg<T, 2>), dim3(1), dim3(kWgThreads), lds, st, D.lg, val, x, f, omega, ssor, D.boundary,
-                       D.nboundary);
+    hipLaunchKernelGGL((k_values<2, SYSTEM>), g, dim3(kBlock), 0, st, D.lg, np, val, val32, mass, k, a, c);
   else
-    hipLaunchKernelGGL((k_sweep_wg<T, 1>), dim3(1), dim3(kWgThreads), lds, st, D.lg, val, x, f, omega, ssor, D.boundary,
-                       D.nboundary);
+    hipLaunchKernelGGL((k_values<1, SYSTEM>), g, dim3(kBlock), 0, st, D.lg, np, val, val32, mass, k, a, c);
+}
+void values32(const DevLayout &D, const double *val, float *val32, hipStream_t st) {
+  values<false>(D, const_cast<double *>(val), val32, nullptr, nullptr, nullptr, 0.0, st);
+}
+void system_matrix(const DevLayout &D, double *val, float *val32, const double *mass, const double *k, const double *a,
+                   double c, hipStream_t st) {
+  values<true>(D, val, val32, mass, k, a, c, st);
 }
 template <typename T>
 void coarse_wg(const DevLayout &D, const T *val, T *x, const T *f, double omega, int kind, int maxit, double red,
@@ -637,11 +1426,11 @@ void coarse_wg(const DevLayout &D, const T *val, T *x, const T *f, double omega,
   if (kind < 1 || kind > 3) throw std::invalid_argument("coarse_wg: smoother must be 1, 2 or 3");
   const size_t lds = (size_t)D.N * sizeof(T);
   if (D.order == 2)
-    hipLaunchKernelGGL((k_coarse_wg<T, 2>), dim3(1), dim3(kWgThreads), lds, st, D.lg, val, x, f, omega, kind, maxit, red,
-                       D.boundary, D.nboundary, xj);
+    launch_wg(k_coarse_wg<T, 2>, Wg<T, 2>::kThreads, Wg<T, 2>::kRedBytes + lds, st, wg_level(D, val), x, f, omega, kind, maxit,
+              red, (const int *)D.boundary, D.nboundary, xj);
   else
-    hipLaunchKernelGGL((k_coarse_wg<T, 1>), dim3(1), dim3(kWgThreads), lds, st, D.lg, val, x, f, omega, kind, maxit, red,
-                       D.boundary, D.nboundary, xj);
+    launch_wg(k_coarse_wg<T, 1>, Wg<T, 1>::kThreads, Wg<T, 1>::kRedBytes + lds, st, wg_level(D, val), x, f, omega, kind, maxit,
+              red, (const int *)D.boundary, D.nboundary, xj);
 }
 
 // Calibration kernels of the dispatch measurements: a dispatch that does
@@ -677,8 +1466,7 @@ void stream_read(const void *p, int64_t bytes, float *sink, hipStream_t st) {
   template void rows_apply<T>(const DevLayout &, int, const T *, const T *, const T *, T *, double, hipStream_t,  \
                               const T *);                                                                        \
   template void sor_sweeps<T>(const DevLayout &, const T *, T *, const T *, T *, double, bool, int, bool,        \
-                              const int *, hipStream_t);                                                         \
-  template void sweep_wg<T>(const DevLayout &, const T *, T *, const T *, double, int, hipStream_t);              \
+                              const int *, bool, hipStream_t);                                                   \
   template void coarse_wg<T>(const DevLayout &, const T *, T *, const T *, double, int, int, double, T *, hipStream_t);
 PMX_INST(double)
 PMX_INST(float)

@@ -10,63 +10,65 @@
 
 namespace pmx {
 
-// The (dy, dz) groups of a line in storage order, per class of lines (y mod S,
-// z mod S): first the groups whose lines come before the line in the sweep
-// order ((z mod C, y mod C), y fastest), then the line itself, then the
-// others; each part in (dz, dy) order.
-template <int O> struct GroupTable {
-  using L = Lines<O>;
-  int off[L::S * L::S][L::kMaxGroups];  // (dy + 8) + 16 (dz + 8)
-  int pos[L::S * L::S][25];             // storage position of (dy, dz) at (dy + 2) + 5 (dz + 2), -1 if absent
-  int nlo[L::S * L::S];                 // groups before the line itself
-  int ng[L::S * L::S];                  // all groups
+// The (dy, dz) groups of a line in storage order: the planes dz whose lattice
+// planes come before the line's in the sweep order (z mod C), then the line's
+// own plane, then the others; in a plane dz != 0 the lines dy = -ey .. ey, in
+// its own plane the lines before it (y mod C), itself, the lines after it.  An
+// axis gives its offsets in this order as nibbles (offset + 2) of a word,
+// computed and not read from memory: a sweep launch of a few microseconds
+// would wait for the table.
+struct AxisOrder {
+  unsigned seq;  // nibble i: i-th offset + 2
+  int e, lo;     // half extent, offsets before 0
 };
-template <int O> constexpr GroupTable<O> make_group_table() {
-  using L = Lines<O>;
-  GroupTable<O> t{};
-  for (int b = 0; b < L::S; b++)
-    for (int a = 0; a < L::S; a++) {
-      const int c = a + L::S * b, ey = L::ext(a), ez = L::ext(b), me = (b % L::C) * L::C + a % L::C;
-      for (int i = 0; i < 25; i++) t.pos[c][i] = -1;
-      int k = 0;
-      for (int part = 0; part < 3; part++) {
-        if (part == 1) t.nlo[c] = k;
-        for (int dz = -ez; dz <= ez; dz++)
-          for (int dy = -ey; dy <= ey; dy++) {
-            const int g = ((b + dz + L::S) % L::C) * L::C + (a + dy + L::S) % L::C;
-            const bool own = dy == 0 && dz == 0;
-            if (!((part == 0 && g < me) || (part == 1 && own) || (part == 2 && g > me))) continue;
-            t.pos[c][(dy + 2) + 5 * (dz + 2)] = k;
-            t.off[c][k++] = (dy + 8) + 16 * (dz + 8);
-          }
-      }
-      t.ng[c] = k;
-    }
-  return t;
+template <int O> __device__ __forceinline__ AxisOrder axis_order(int t) {
+  const int e = Lines<O>::ext(t);
+  if constexpr (O == 1) {
+    // (t mod 2) = 0: 0, -1, 1; 1: -1, 1, 0
+    const bool r = t & 1;
+    return AxisOrder{r ? 0x231u : 0x312u, 1, r ? 2 : 0};
+  } else {
+    // residues mod 3; the extent 2 offsets +-2 have the residue of -+1
+    const int r = t % 3;
+    const bool w = e == 2;
+    const unsigned q0 = w ? 0x43102u : 0x312u;  // 0 | -2 -1 1 2
+    const unsigned q1 = w ? 0x30241u : 0x321u;  // -1 2 | 0 | -2 1
+    const unsigned q2 = w ? 0x24310u : 0x231u;  // -2 -1 1 2 | 0
+    return AxisOrder{r == 0 ? q0 : r == 1 ? q1 : q2, e, r == 0 ? 0 : r == 1 ? (w ? 2 : 1) : (w ? 4 : 2)};
+  }
 }
-static __device__ constexpr GroupTable<1> kGroups1 = make_group_table<1>();
-static __device__ constexpr GroupTable<2> kGroups2 = make_group_table<2>();
-template <int O> __device__ __forceinline__ const GroupTable<O> &group_table() {
-  if constexpr (O == 1) return kGroups1;
-  else return kGroups2;
-}
-template <int O> __device__ __forceinline__ int line_class(int y, int z) {
-  return y % Lines<O>::S + Lines<O>::S * (z % Lines<O>::S);
-}
+template <int O> struct GroupOrder {
+  AxisOrder y, z;
+  __device__ __forceinline__ GroupOrder(int ly, int lz) : y(axis_order<O>(ly)), z(axis_order<O>(lz)) {}
+  __device__ __forceinline__ int wy() const { return 2 * y.e + 1; }
+  __device__ __forceinline__ int groups() const { return wy() * (2 * z.e + 1); }
+  __device__ __forceinline__ int before() const { return z.lo * wy() + y.lo; }
+  // offset of group k in the lattice: dy + M dz
+  __device__ __forceinline__ int line(int k, int M) const {
+    // k / 3 and k / 5 for k < 25
+    const int j = O == 1 || y.e == 1 ? (k * 11) >> 5 : (k * 13) >> 6, i = k - j * wy();
+    const int dz = (int)((z.seq >> (4 * j)) & 15) - 2;
+    const int dy = dz ? i - y.e : (int)((y.seq >> (4 * i)) & 15) - 2;
+    return dy + M * dz;
+  }
+  // storage position of (dy, dz)
+  __device__ __forceinline__ int position(int dy, int dz) const {
+    int j = 0, i = dy + y.e;
+    for (int q = 0; q < 5; q++)
+      if (((z.seq >> (4 * q)) & 15) == (unsigned)(dz + 2) && q <= 2 * z.e) j = q;
+    if (dz == 0)
+      for (int q = 0; q < 5; q++)
+        if (((y.seq >> (4 * q)) & 15) == (unsigned)(dy + 2) && q <= 2 * y.e) i = q;
+    return j * wy() + i;
+  }
+};
 
 // value of row (x, y, z) for the column at (dx, dy, dz)
-template <int O>
+template <typename V, int O>
 __device__ __forceinline__ int64_t value_index(int P, int x, int y, int z, int dx, int dy, int dz) {
   using L = Lines<O>;
-  const int k = group_table<O>().pos[line_class<O>(y, z)][(dy + 2) + 5 * (dz + 2)];
-  return ((L::group_base(P, y, z) + k) * L::VL + L::slot(x, dx)) * P + ((x - 1) >> 1);
-}
-// the same in the FP16 smoother values (a pair's slots of a group contiguous)
-template <int O>
-__device__ __forceinline__ int64_t value_index16(int P, int x, int y, int z, int dx, int dy, int dz) {
-  using L = Lines<O>;
-  const int k = group_table<O>().pos[line_class<O>(y, z)][(dy + 2) + 5 * (dz + 2)];
-  return ((L::group_base(P, y, z) + k) * P + ((x - 1) >> 1)) * L::VL + L::slot(x, dx);
+  const int k = GroupOrder<O>(y, z).position(dy, dz);
+  return (L::group_base(P, y, z) + k) * (L::VL * P) + Slots<V, O>::at(P, (x - 1) >> 1, L::slot(x, dx));
 }
 
 // MI355X dispatches consecutive workgroups round-robin over its 8 XCDs.  Remap
@@ -105,38 +107,30 @@ template <typename T, int W> __device__ __forceinline__ void load_run(const T *q
   __builtin_memcpy(r, q, W * sizeof(T));
 }
 
-// The stored values of a group for the row pair of a lane: element s at
-// v[s * P] (FP64, FP32), contiguous (FP16).
-template <typename V, int O> __device__ __forceinline__ void load_group(const V *v, int P, V *out) {
-  constexpr int VL = Lines<O>::VL;
-  if constexpr (sizeof(V) == 2) {
-    __builtin_memcpy(out, v, VL * sizeof(V));
-  } else {
+// The stored values of a group (at v) for row pair m.
+template <typename V, int O> __device__ __forceinline__ void load_group(const V *v, int P, int m, V *out) {
+  using S = Slots<V, O>;
 #pragma unroll
-    for (int s = 0; s < VL; s++) out[s] = v[s * P];
-  }
+  for (int c = 0; c < S::VL; c += S::W) __builtin_memcpy(out + c, v + S::at(P, m, c), S::width(c) * sizeof(V));
 }
-// offset of a lane's values in a line, and of consecutive groups
-template <typename V, int O> __device__ __forceinline__ int64_t line_values(int P, int64_t base, int m) {
-  constexpr int VL = Lines<O>::VL;
-  if constexpr (sizeof(V) == 2) return (base * P + m) * VL;
-  else return base * VL * P + m;
+// first value of a line
+template <int O> __device__ __forceinline__ int64_t line_values(int P, int y, int z) {
+  return Lines<O>::group_base(P, y, z) * (Lines<O>::VL * P);
 }
 
 // Adds groups k0, k0 + step, ... < k1 of a line to the sums of a lane's row
-// pair, x = 2m + 1 (so) and 2m + 2 (se).  v: the lane's values of group 0; x:
+// pair, x = 2m + 1 (so) and 2m + 2 (se).  v: the line's values; x:
 // lattice vector at (2m, y, z); d3: distance of the run's second part (3, or
 // less for the last pair, whose even row is the boundary node and has zero
 // values: its columns are clamped to the lattice).  The order of the sums is
 // that of k, whatever the unrolling.
 template <typename T, typename V, int O, int U>
-__device__ __forceinline__ void add_groups(const V *__restrict__ v, const T *x, const int *__restrict__ off, int k0,
-                                           int k1, int step, int P, int M, int d3, T &so, T &se) {
+__device__ __forceinline__ void add_groups(const V *__restrict__ v, const T *x, const GroupOrder<O> &g, int k0, int k1,
+                                           int step, int P, int M, int m, int d3, T &so, T &se) {
   constexpr int VL = Lines<O>::VL, NX = O == 2 ? 5 : 4;
   auto fetch = [&](int k, V *w, T *r) {
-    const int o = off[k];
-    const T *q = x + ((o & 15) - 8 + M * ((o >> 4) - 8)) * M;
-    load_group<V, O>(v + (int64_t)k * (VL * P), P, w);
+    const T *q = x + g.line(k, M) * M;
+    load_group<V, O>(v + (int64_t)k * (VL * P), P, m, w);
     load_run<T, 3>(q, r);
     load_run<T, NX - 3>(q + d3, r + 3);
   };
@@ -146,20 +140,16 @@ __device__ __forceinline__ void add_groups(const V *__restrict__ v, const T *x, 
 #pragma unroll
     for (int e = 0; e < 2 * O + 1; e++) se = fma((T)w[3 + e], r[e + 2 - O], se);
   };
-  int k = k0;
-  for (; k + (U - 1) * step < k1; k += U * step) {
+  // all loads of U groups are issued before the first sum (past the last group
+  // it is read again and not added)
+  for (int k = k0; k < k1; k += U * step) {
     V w[U][VL];
     T r[U][NX];
 #pragma unroll
-    for (int u = 0; u < U; u++) fetch(k + u * step, w[u], r[u]);
+    for (int u = 0; u < U; u++) fetch(k + u * step < k1 ? k + u * step : k, w[u], r[u]);
 #pragma unroll
-    for (int u = 0; u < U; u++) add(w[u], r[u]);
-  }
-  for (; k < k1; k += step) {
-    V w[VL];
-    T r[NX];
-    fetch(k, w, r);
-    add(w, r);
+    for (int u = 0; u < U; u++)
+      if (u == 0 || k + u * step < k1) add(w[u], r[u]);
   }
 }
 

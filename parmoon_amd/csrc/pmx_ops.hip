@@ -409,10 +409,11 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
   const double g = 2.0 * n;  // reference -> physical derivative factor 2/h
   // the row's entries: group position of (dy, dz), slot of dx
   const int P = (M - 1) / 2;
-  const int64_t v0 = line_values<double, ORDER>(P, Lines<ORDER>::group_base(P, py, pz), (px - 1) >> 1);
-  const int *pos = group_table<ORDER>().pos[__builtin_amdgcn_readfirstlane(line_class<ORDER>(py, pz))];
+  const int64_t v0 = line_values<ORDER>(P, py, pz);
+  const GroupOrder<ORDER> go(__builtin_amdgcn_readfirstlane(py), __builtin_amdgcn_readfirstlane(pz));
   auto at = [&](int dx, int dy, int dz) {
-    return v0 + (int64_t)(pos[(dy + 2) + 5 * (dz + 2)] * Lines<ORDER>::VL + Lines<ORDER>::slot(px, dx)) * P;
+    return v0 + go.position(dy, dz) * (Lines<ORDER>::VL * P) +
+           Slots<double, ORDER>::at(P, (px - 1) >> 1, Lines<ORDER>::slot(px, dx));
   };
   double frhs = 0;
   // Q1 rows of the one-matrix forms (27 slots) are accumulated in registers
@@ -610,8 +611,7 @@ __global__ void k_values_to_csr(const int *__restrict__ rowptr, const int *__res
   for (int n = b; n < e; n++) {
     const int q = dof2lat[kcol[n]];
     const int dx = q % M - x, dy = (q / M) % M - y, dz = q / (M * M) - z;
-    if constexpr (sizeof(T) == 2) out[n] = (double)val[value_index16<O>(P, x, y, z, dx, dy, dz)];
-    else out[n] = (double)val[value_index<O>(P, x, y, z, dx, dy, dz)];
+    out[n] = (double)val[value_index<T, O>(P, x, y, z, dx, dy, dz)];
   }
 }
 
@@ -629,7 +629,7 @@ __global__ void k_csr_to_values(const int *__restrict__ rowptr, const int *__res
   for (int n = b; n < e; n++) {
     const int q = dof2lat[kcol[n]];
     const int dx = q % M - x, dy = (q / M) % M - y, dz = q / (M * M) - z;
-    val[value_index<O>(P, x, y, z, dx, dy, dz)] = in[n];
+    val[value_index<double, O>(P, x, y, z, dx, dy, dz)] = in[n];
   }
 }
 
@@ -692,7 +692,7 @@ __global__ void k_values_to_aug(int M, const int *__restrict__ iidx, const int *
     for (int dy = -ey; dy <= ey; dy++)
       for (int dx = -ex; dx <= ex; dx++) {
         const int q = (x + dx) + M * ((y + dy) + M * (z + dz));
-        const double v = val[value_index<O>(P, x, y, z, dx, dy, dz)];
+        const double v = val[value_index<double, O>(P, x, y, z, dx, dy, dz)];
         const int cq = cidx[q];
         if (cq >= 0) row[cq] = v;
         else row[nI + q] = -v;
@@ -1313,8 +1313,9 @@ __device__ __forceinline__ void assemble_row_kc(double (*sh)[64 * kKcPad], bool 
       part[e] = reinterpret_cast<const double2 *>(kc + (cell * 27 + a) * kKcRow)[q];
     }
   };
-  const int *pos = group_table<2>().pos[__builtin_amdgcn_readfirstlane(line_class<2>(py, pz))];
-  double *v = val + line_values<double, 2>(P, Lines<2>::group_base(P, py, pz), (px - 1) >> 1);
+  const GroupOrder<2> go(y0, z0);
+  double *v = val + line_values<2>(P, py, pz);
+  const int m = (px - 1) >> 1;
   double frhs = 0;
   double acc[NS];
 #pragma unroll
@@ -1346,7 +1347,7 @@ __device__ __forceinline__ void assemble_row_kc(double (*sh)[64 * kKcPad], bool 
       const int lx = (NCX == 2 && dx >= 0) ? 1 : 0, ly = (NCY == 2 && dy >= 0) ? 1 : 0,
                 lz = (NCZ == 2 && dz >= 0) ? 1 : 0;
       if (lx == ix && ly == iy && lz == iz && ok)
-        v[(int64_t)(pos[(dy + 2) + 5 * (dz + 2)] * Lines<2>::VL + (EX == 1 ? dx + 1 : dx + 5)) * P] = acc[q];
+        v[go.position(dy, dz) * (Lines<2>::VL * P) + Slots<double, 2>::at(P, m, EX == 1 ? dx + 1 : dx + 5)] = acc[q];
     }
   }
   if (ok) rhs[px + M * (py + M * pz)] = frhs;
@@ -1586,19 +1587,6 @@ __global__ void k_tcd_rhs(int M, const double *__restrict__ oldrhs, const double
 }
 void interpolate(const DevLayout &D, const double *prm_dev, double *x, hipStream_t st) {
   hipLaunchKernelGGL(k_interpolate, dim3(grid_for(D.N)), dim3(kBlock), 0, st, prm_dev, D.M, x);
-}
-// val = mass (+ k) + c a (MatAdd of Blas2.C:128-150 on the stored stencil values)
-__global__ void k_system_matrix(double *__restrict__ val, float *__restrict__ val32, const double *__restrict__ mass,
-                                const double *__restrict__ k, const double *__restrict__ a, double c, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const double v = (k ? mass[i] + k[i] : mass[i]) + c * a[i];
-    val[i] = v;
-    if (val32) val32[i] = (float)v;
-  }
-}
-void system_matrix(double *val, float *val32, const double *mass, const double *k, const double *a, double c,
-                   int64_t n, hipStream_t st) {
-  hipLaunchKernelGGL(k_system_matrix, dim3(grid_for(n)), dim3(kBlock), 0, st, val, val32, mass, k, a, c, n);
 }
 void tcd_rhs(const DevLayout &D, const double *oldrhs, const double *rhs, const double *m_old, const double *a_old,
              const double *k_old, double t3, double t4, double t2, double *B, hipStream_t st) {

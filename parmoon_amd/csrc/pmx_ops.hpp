@@ -18,6 +18,9 @@ struct DevLayout {
   int nboundary = 0;
   int *boundary = nullptr;
   int64_t max_colour_rows = 0;    // rows of the largest colour
+  // the row pairs of each line group (M <= 33; k_pair_table)
+  const int2 *pairs = nullptr;
+  int pair_tiles = 0;
   int ncolours = 0;
 };
 
@@ -91,10 +94,13 @@ void rows_apply(const DevLayout &D, int mode, const T *val, const T *x, const T 
 // the Dirichlet entries of x are left as they are.  psum (SSOR): N entries of
 // scratch that hold the upper sums of the result's rows afterwards.  zero: the
 // interior of x is zero (its contribution is not read); bnd_set (optional,
-// with zero): a device flag that is not 0 if the boundary of x is not zero.
+// with zero): a device flag that is not 0 if the boundary of x is not zero;
+// planes: a launch per plane colour instead of one per line group where
+// plane_sweeps_fit (the same result bit for bit).
+bool plane_sweeps_fit(const DevLayout &D);
 template <typename T>
 void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n, bool zero,
-                const int *bnd_set, hipStream_t st);
+                const int *bnd_set, bool planes, hipStream_t st);
 // the same on the row-scaled FP16 values and the FP32 1/diag of scaled_values
 // (psum: sums of the scaled values)
 void sor_sweeps_scaled(const DevLayout &D, const _Float16 *val16, const float *dinv, float *x, const float *f,
@@ -109,14 +115,17 @@ void fe_errors(const DevLayout &D, const double *prm_dev, const double *qref, co
                const double *u, double *part, double *out, hipStream_t st);
 // a == b bit for bit (n doubles; flag: one device int of scratch; synchronises st)
 bool bits_equal(const double *a, const double *b, int64_t n, int *flag, hipStream_t st);
-// whole SOR (ssor 0) / SSOR (ssor 1) sweep with Dirichlet rows x = f, one
-// workgroup with the level's x in LDS (levels with M^3 * s <= kSweepLdsBytes)
+// x of the level fits the LDS of the one-workgroup kernel
 inline bool sweep_wg_fits(const DevLayout &D, size_t s) { return (int64_t)D.N * (int64_t)s <= kSweepLdsBytes; }
+// pair table of a small level: pair_tiles(L) tiles of kPairTile entries per
+// line group
+constexpr int kPairTile = 256;
+int pair_tiles(const Layout &L);
+size_t pair_table_size(const DevLayout &D);
+void pair_table(const DevLayout &D, int2 *pairs, hipStream_t st);
 // the row-scaled FP16 copy of the FP32 stencil values (a_ij / a_ii,
 // saturated to the finite FP16 range) and dinv = 1 / a_ii on the active rows
 void scaled_values(const DevLayout &D, const float *val, _Float16 *val16, float *dinv, hipStream_t st);
-template <typename T>
-void sweep_wg(const DevLayout &D, const T *val, T *x, const T *f, double omega, int ssor, hipStream_t st);
 // the coarse-level smoothing loop of TMultiGrid3D (MultiGrid3D.C:225-337) in
 // one workgroup (levels with sweep_wg_fits): sweeps of kind 1 Jacobi, 2 SOR,
 // 3 SSOR while ||f - A x|| > red ||f - A x_0|| and fewer than maxit were
@@ -191,8 +200,10 @@ constexpr int64_t kCellMatrixDoubles = 27 * 28;  // cell buffer entries per Q2 c
 // K oldsol, nullptr for the Galerkin forms)
 void interpolate(const DevLayout &D, const double *prm_dev, double *x, hipStream_t st);
 // val = mass (+ k) + c a; val32 (if not null) receives its FP32 rounding
-void system_matrix(double *val, float *val32, const double *mass, const double *k, const double *a, double c,
-                   int64_t n, hipStream_t st);
+void system_matrix(const DevLayout &D, double *val, float *val32, const double *mass, const double *k, const double *a,
+                   double c, hipStream_t st);
+// the FP32 copy of the level's values
+void values32(const DevLayout &D, const double *val, float *val32, hipStream_t st);
 void tcd_rhs(const DevLayout &D, const double *oldrhs, const double *rhs, const double *m_old, const double *a_old,
              const double *k_old, double t3, double t4, double t2, double *B, hipStream_t st);
 void givens(double *H, double *cs, double *sn, double *s, int i, int ld, double *res, hipStream_t st);
