@@ -41,12 +41,23 @@ __host__ __device__ inline double grf_field(const double *prm, double x, double 
   return s * 0.17677669529663688110021109052621;  // sqrt(2/64)
 }
 
+// the trigonometric factors of the example functions, evaluated where used
+struct PointTrig {
+  double x, y, z;
+  static constexpr double pi = 3.14159265358979323846;
+  __host__ __device__ double sx() const { return sin(pi * x); }
+  __host__ __device__ double sy() const { return sin(pi * y); }
+  __host__ __device__ double sz() const { return sin(pi * z); }
+  __host__ __device__ double cx() const { return cos(pi * x); }
+  __host__ __device__ double cy() const { return cos(pi * y); }
+  __host__ __device__ double cz() const { return cos(pi * z); }
+};
 // CHEAP = true: only the examples whose coefficients are evaluated inline
 // at every point (Laplace, sine, heat, rotating); the curl-Fourier and
 // lognormal branches, which kernels for the inline examples never take, are
 // left out of the code so they do not weigh on its registers
-template <bool CHEAP = false>
-__host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, double y, double z) {
+template <bool CHEAP, class Trig>
+__host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, double y, double z, const Trig &tr) {
   const double pi = 3.14159265358979323846;
   QpCoeffs k;
   const int ex = (int)prm[PMX_PRM_EXAMPLE];
@@ -61,10 +72,10 @@ __host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, 
   if (ex == PMX_EX_LAPLACE) {
     k.b0 = k.b1 = k.b2 = 0;
     k.c = 0;
-    k.f = 3 * pi * pi * eps * sin(pi * x) * sin(pi * y) * sin(pi * z);
+    k.f = 3 * pi * pi * eps * tr.sx() * tr.sy() * tr.sz();
   } else if (ex == PMX_EX_SINE_CD) {
-    const double sx = sin(pi * x), sy = sin(pi * y), sz = sin(pi * z);
-    const double cx = cos(pi * x), cy = cos(pi * y), cz = cos(pi * z);
+    const double sx = tr.sx(), sy = tr.sy(), sz = tr.sz();
+    const double cx = tr.cx(), cy = tr.cy(), cz = tr.cz();
     const double u = sx * sy * sz;
     k.f = 3 * pi * pi * eps * u + pi * (k.b0 * cx * sy * sz + k.b1 * sx * cy * sz + k.b2 * sx * sy * cz) + k.c * u;
   } else if (!CHEAP && ex == PMX_EX_CURL_FOURIER) {
@@ -81,7 +92,7 @@ __host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, 
     k.eps = 1.0;
     k.b0 = k.b1 = k.b2 = 0;
     k.c = 0;
-    k.f = (3. * pi * pi - 0.1) * exp(-0.1 * t) * sin(pi * x) * cos(pi * y) * cos(pi * z);
+    k.f = (3. * pi * pi - 0.1) * exp(-0.1 * t) * tr.sx() * tr.cy() * tr.cz();
   } else if (!CHEAP && ex == PMX_EX_LOGNORMAL) {
     if constexpr (!CHEAP) {
       k.eps = eps * exp(prm[PMX_PRM_GRF_SIGMA] * grf_field(prm, x, y, z));
@@ -95,6 +106,11 @@ __host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, 
     k.f = 0.0;
   }
   return k;
+}
+
+template <bool CHEAP = false>
+__host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, double y, double z) {
+  return example_coeffs<CHEAP>(prm, x, y, z, PointTrig{x, y, z});
 }
 
 __host__ __device__ inline double example_bound_value(const double *prm, double x, double y, double z) {

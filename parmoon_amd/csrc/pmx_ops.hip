@@ -395,6 +395,38 @@ __host__ __device__ inline bool coeffs_inline(int example) {
 // coordinate lies in one cell along it, every other node in two), so the
 // loops are uniform across the wavefront and the basis tables are read with
 // scalar loads; TWO selects the second matrix of the SUPG TCD form.
+struct RowPoint {
+  double u0, ux, uy, uz, k0, f;  // of K_ab, of the second matrix, of the rhs
+};
+// a quadrature point's factors of a row, with the row's basis function (value
+// fa and physical derivatives) there
+__device__ __forceinline__ RowPoint row_point(const double *Qq, double fa, double gax, double gay, double gaz, int form,
+                                              double g) {
+  const double w = Qq[0], eps = Qq[1], b0 = Qq[2], b1 = Qq[3], b2 = Qq[4];
+  const double cc = Qq[5], ff = Qq[6], dl = Qq[7];
+  const double bga = b0 * gax + b1 * gay + b2 * gaz;
+  RowPoint r;
+  // the rhs is f (phi_a + delta b.grad phi_a), with delta = 0 for the Galerkin
+  // rhs and for MatrixMRhsAssemble (TCD3D.C:64, 117)
+  const double sa = fa + dl * bga;
+  r.f = w * ff * sa;
+  if (form == PMX_FORM_MASS || form == PMX_FORM_MASS_SUPG) {
+    r.u0 = fa;
+    r.ux = r.uy = r.uz = r.k0 = 0;
+  } else {
+    r.u0 = cc * sa;
+    r.ux = eps * gax + b0 * sa;
+    r.uy = eps * gay + b1 * sa;
+    r.uz = eps * gaz + b2 * sa;
+    r.k0 = dl * bga;
+  }
+  r.u0 *= w;
+  r.ux *= w * g;
+  r.uy *= w * g;
+  r.uz *= w * g;
+  r.k0 *= w;
+  return r;
+}
 template <int ORDER, int EX, int EY, int EZ, bool TWO, bool INL, bool RONLY>
 __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int n, int nq, int form,
                                              const double *__restrict__ prm, const double *__restrict__ qref,
@@ -416,26 +448,14 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
            Slots<double, ORDER>::at(P, (px - 1) >> 1, Lines<ORDER>::slot(px, dx));
   };
   double frhs = 0;
-  // Q1 rows of the one-matrix forms (27 slots) are accumulated in registers
-  // over the 8 cells (loops unrolled, every slot a compile-time index) and
-  // stored once; Q2 rows and the two-matrix form (whose unrolled loops need
-  // too many registers) add each cell's contribution into the values (Q2:
-  // cleared beforehand; Q1: the first cell of a slot stores)
-  constexpr bool REG = ORDER == 1 && !TWO;
-  constexpr int UNR = REG ? 2 : 1;
-  double racc[REG ? 27 : 1];
-  if constexpr (REG) {
-#pragma unroll
-    for (int q = 0; q < 27; q++) racc[q] = 0.0;
-  }
   // incident cells per direction: lattice coordinate x lies in cells
   // floor((x-1)/ORDER) .. floor(x/ORDER) (two cells at a vertex plane)
   const int cx0 = (px - 1) / ORDER, cy0 = (py - 1) / ORDER, cz0 = (pz - 1) / ORDER;
-#pragma unroll UNR
+#pragma unroll 1
   for (int iz = 0; iz < NCZ; iz++)
-#pragma unroll UNR
+#pragma unroll 1
     for (int iy = 0; iy < NCY; iy++)
-#pragma unroll UNR
+#pragma unroll 1
       for (int ix = 0; ix < NCX; ix++) {
         const int cx = cx0 + ix, cy = cy0 + iy, cz = cz0 + iz;
         const int ax = px - ORDER * cx, ay = py - ORDER * cy, az = pz - ORDER * cz;
@@ -460,39 +480,16 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
 #pragma unroll
             for (int e = 0; e < 8; e++) Qq[e] = Q[8 * q + e];
           }
-          const double w = Qq[0], eps = Qq[1], b0 = Qq[2], b1 = Qq[3], b2 = Qq[4];
-          const double cc = Qq[5], ff = Qq[6], dl = Qq[7];
           const double *Ta = tab + (q * NB + a) * 4;
-          const double fa = Ta[0], gax = g * Ta[1], gay = g * Ta[2], gaz = g * Ta[3];
-          const double bga = b0 * gax + b1 * gay + b2 * gaz;
-          double u0, ux, uy, uz, k0 = 0;
-          if (RONLY) {
-            // RhsAssemble / RhsAssemble_SUPG: f (phi_a + delta b.grad phi_a)
-            // (delta = 0 for the Galerkin rhs)
-            frhs += w * ff * (fa + dl * bga);
-            continue;
-          }
-          if (form == PMX_FORM_MASS || form == PMX_FORM_MASS_SUPG) {
-            // the mass matrix; the rhs is f (phi_a + delta b.grad phi_a) with
-            // delta = 0 for MatrixMRhsAssemble (TCD3D.C:64, 117)
-            u0 = fa; ux = uy = uz = 0;
-            frhs += w * ff * (fa + dl * bga);
-          } else {
-            const double sa = fa + dl * bga;
-            u0 = cc * sa;
-            ux = eps * gax + b0 * sa;
-            uy = eps * gay + b1 * sa;
-            uz = eps * gaz + b2 * sa;
-            frhs += w * ff * sa;
-            k0 = dl * bga;
-          }
-          u0 *= w; ux *= w * g; uy *= w * g; uz *= w * g; k0 *= w;
+          const RowPoint r = row_point(Qq, Ta[0], g * Ta[1], g * Ta[2], g * Ta[3], form, g);
+          frhs += r.f;
+          if (RONLY) continue;
           const double *Tq = tab + q * NB * 4;
 #pragma unroll
           for (int b = 0; b < NB; b++) {
             const double *Tb = Tq + 4 * b;
-            acc[b] += u0 * Tb[0] + ux * Tb[1] + uy * Tb[2] + uz * Tb[3];
-            if (TWO) acc2[b] += k0 * Tb[0];
+            acc[b] += r.u0 * Tb[0] + r.ux * Tb[1] + r.uy * Tb[2] + r.uz * Tb[3];
+            if (TWO) acc2[b] += r.k0 * Tb[0];
           }
         }
         if (RONLY) continue;
@@ -501,25 +498,10 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
         for (int b = 0; b < NB; b++) {
           const int bx = b % K, by = (b / K) % K, bz = b / (K * K);
           const int dx = ORDER * cx + bx - px, dy = ORDER * cy + by - py, dz = ORDER * cz + bz - pz;
-          const int slot = (dx + EX) + (2 * EX + 1) * ((dy + EY) + (2 * EY + 1) * (dz + EZ));
-          if constexpr (REG) {
-            racc[slot] += acc[b];
-          } else if (ORDER == 1 && (ix == 0 || bx == 1) && (iy == 0 || by == 1) && (iz == 0 || bz == 1)) {
-            // Q1: the first of the row's cells (in loop order) that meets
-            // the slot, (max(0, dx), max(0, dy), max(0, dz)), stores; the
-            // later ones add, so the values need no clearing beforehand
-            val[at(dx, dy, dz)] = acc[b];
-            if (TWO) val2[at(dx, dy, dz)] = acc2[b];
-          } else {
-            val[at(dx, dy, dz)] += acc[b];
-            if (TWO) val2[at(dx, dy, dz)] += acc2[b];
-          }
+          val[at(dx, dy, dz)] += acc[b];
+          if (TWO) val2[at(dx, dy, dz)] += acc2[b];
         }
       }
-  if constexpr (REG && !RONLY) {
-#pragma unroll
-    for (int q = 0; q < 27; q++) val[at(q % 3 - 1, (q / 3) % 3 - 1, q / 9 - 1)] = racc[q];
-  }
   rhs[p] = frhs;
 }
 
@@ -528,11 +510,11 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
 // next, so that a wavefront's rows have one stencil shape and its stores of a
 // slot are contiguous.  False: no row.
 template <int O>
-__device__ __forceinline__ bool unit_row(const LineSet &set, int M, int lg, int *px, int *py, int *pz) {
+__device__ __forceinline__ bool unit_row(const LineSet &set, int M, int lg, int lane, int *px, int *py, int *pz) {
   const int b = xcd_remap(blockIdx.x, gridDim.x), P = 1 << lg, segs = lg > 6 ? P / 64 : 1;
   const int part = b % (2 * segs);
   const UnitLines u = unit_lines<O>(set, M, lg, b / (2 * segs));
-  const int t = threadIdx.x + 64 * (part >> 1), m = t & (P - 1);
+  const int t = lane + 64 * (part >> 1), m = t & (P - 1);
   *px = 2 * m + 1 + (part & 1);
   *py = u.y0 + Lines<O>::S * (t >> lg);
   *pz = u.z;
@@ -555,7 +537,7 @@ __global__ __launch_bounds__(kRowsPerBlock) void k_assemble(LineSet set, int lg,
                                                      double *__restrict__ val, double *__restrict__ val2,
                                                      double *__restrict__ rhs) {
   int px, py, pz;
-  const bool ok = unit_row<ORDER>(set, M, lg, &px, &py, &pz);
+  const bool ok = unit_row<ORDER>(set, M, lg, threadIdx.x, &px, &py, &pz);
   const int code = unit_shape<ORDER>(lg, set, M);
   if (!ok) return;
   const int form = (int)prm[PMX_PRM_FORM];
@@ -576,6 +558,181 @@ __global__ __launch_bounds__(kRowsPerBlock) void k_assemble(LineSet set, int lg,
     default: PMX_AROW(2, 2, 2, 2); break;
   }
 #undef PMX_AROW
+}
+// a value that is the same in all lanes, in scalar registers
+__device__ __forceinline__ double uniform(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)(unsigned)u), hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+// the factors of the example functions from those of the points' coordinates
+struct AxisPoint {
+  double x, s, c;  // coordinate, sin(pi x), cos(pi x)
+};
+struct AxisTrig {
+  const AxisPoint &X, &Y, &Z;
+  __device__ __forceinline__ double sx() const { return X.s; }
+  __device__ __forceinline__ double sy() const { return Y.s; }
+  __device__ __forceinline__ double sz() const { return Z.s; }
+  __device__ __forceinline__ double cx() const { return X.c; }
+  __device__ __forceinline__ double cy() const { return Y.c; }
+  __device__ __forceinline__ double cz() const { return Z.c; }
+};
+// Q1 rows with matrices: a workgroup takes the 64 rows of unit_row, its
+// wavefront j the j-th of the rows' 8 cells (ix + 2 iy + 4 iz); the cells'
+// rows of the local matrices meet in LDS and are added in the order of j, a
+// slot of the 64 rows per wavefront and turn.
+//
+// Bound by the FP64 operations of the points and, on small levels, by the
+// chain of a thread, which is 8 times shorter than with all cells of a row on
+// one thread.  The rule and the basis are tensor products (NP points per
+// axis), so a row is summed axis by axis (14 products per point instead of
+// 32, no table of basis values), and the trigonometric factors of the example
+// functions are those of the NP points of each axis.  Level of 8^3 cells,
+// 27 points, sine coefficients: 331 -> 17 us; 128^3, SUPG form of the rotating
+// flow (both matrices): 2.36 -> 1.88 ms.
+template <int NP, bool TWO, bool INL>
+__global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M, int n,
+                                                     const double *__restrict__ prm, const double *__restrict__ qref,
+                                                     const double *__restrict__ qp, double *__restrict__ val,
+                                                     double *__restrict__ val2, double *__restrict__ rhs) {
+  constexpr int NB = 8, R = kRowsPerBlock, NQ = NP * NP * NP;
+  __shared__ double sh[(TWO ? 2 : 1) * 8 * NB * R], sf[8 * R];
+  const int t = threadIdx.x & (R - 1), j = __builtin_amdgcn_readfirstlane(threadIdx.x / R);
+  int px, py, pz;
+  const bool ok = unit_row<1>(set, M, lg, t, &px, &py, &pz);
+  // (a row that exists for the lanes without one)
+  if (!ok) px = py = 1;
+  const int form = (int)prm[PMX_PRM_FORM];
+  {
+    const int ix = j & 1, iy = (j >> 1) & 1, iz = j >> 2;
+    const int cx = px - 1 + ix, cy = py - 1 + iy, cz = pz - 1 + iz;
+    const int64_t cell = cx + (int64_t)n * (cy + (int64_t)n * cz), ncell = (int64_t)n * n * n;
+    const double *Q = qp + cell * NQ * 8;
+    const double h = 1.0 / n, g = 2.0 * n;  // reference -> physical derivative factor 2/h
+    // basis functions of an axis at its points; the row's one along the axes
+    // and the derivatives -1/2, 1/2
+    double f0[NP], f1[NP], fz[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      const double xi = qref[4 * i];
+      f0[i] = uniform(0.5 * (1 - xi));
+      f1[i] = uniform(0.5 * (1 + xi));
+      fz[i] = iz ? f0[i] : f1[i];
+    }
+    const double gx = ix ? -0.5 * g : 0.5 * g, gy = iy ? -0.5 * g : 0.5 * g, gz = iz ? -0.5 * g : 0.5 * g;
+    const bool trig = INL && (int)prm[PMX_PRM_EXAMPLE] != PMX_EX_ROTATING;
+    auto axis_point = [&](int c, double xi) {
+      AxisPoint a{(c * h + 0.5 * h) + 0.5 * h * xi, 0, 0};
+      if (trig) sincospi(a.x, &a.s, &a.c);
+      return a;
+    };
+    AxisPoint Z[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) Z[i] = INL ? axis_point(cz, qref[4 * i]) : AxisPoint{0, 0, 0};
+    double acc[NB], acc2[NB], frhs = 0;
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[b] = acc2[b] = 0;
+    // inline coefficients: qp holds the per-point stabilisation parameters of
+    // k_qp_delta (nullptr for the forms without one)
+#pragma unroll 1
+    for (int qx = 0; qx < NP; qx++) {
+      const double xi = qref[4 * qx], x0 = uniform(0.5 * (1 - xi)), x1 = uniform(0.5 * (1 + xi)), fx = ix ? x0 : x1;
+      const AxisPoint X = INL ? axis_point(cx, xi) : AxisPoint{0, 0, 0};
+      double p[4] = {0, 0, 0, 0}, d[4] = {0, 0, 0, 0}, p2[4] = {0, 0, 0, 0};  // by + 2 bz
+#pragma unroll 1
+      for (int qy = 0; qy < NP; qy++) {
+        const double yi = qref[4 * qy], y0 = uniform(0.5 * (1 - yi)), y1 = uniform(0.5 * (1 + yi)), fy = iy ? y0 : y1;
+        const AxisPoint Y = INL ? axis_point(cy, yi) : AxisPoint{0, 0, 0};
+        const double gxy = gx * fy, gyx = gy * fx, gzxy = gz * (fx * fy), fxy = fx * fy;
+        double dl[NP];
+#pragma unroll
+        for (int qz = 0; qz < NP; qz++)
+          dl[qz] = (INL && qp) ? qp[(qx + NP * (qy + NP * qz)) * ncell + cell] : 0.0;
+        double a[2] = {0, 0}, ax[2] = {0, 0}, ay[2] = {0, 0}, a2[2] = {0, 0};  // bz
+#pragma unroll
+        for (int qz = 0; qz < NP; qz++) {
+          const int q = qx + NP * (qy + NP * qz);
+          double Qq[8];
+          if (INL) {
+            const QpCoeffs c = example_coeffs<true>(prm, X.x, Y.x, Z[qz].x, AxisTrig{X, Y, Z[qz]});
+            Qq[0] = qref[4 * q + 3] * (h * h * h / 8.0);
+            Qq[1] = c.eps; Qq[2] = c.b0; Qq[3] = c.b1; Qq[4] = c.b2; Qq[5] = c.c; Qq[6] = c.f;
+            Qq[7] = dl[qz];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++) Qq[e] = Q[8 * q + e];
+          }
+          const RowPoint r = row_point(Qq, fxy * fz[qz], gxy * fz[qz], gyx * fz[qz], gzxy, form, g);
+          frhs += r.f;
+          a[0] = fma(r.u0, f0[qz], fma(r.uz, -0.5, a[0]));
+          a[1] = fma(r.u0, f1[qz], fma(r.uz, 0.5, a[1]));
+          ax[0] = fma(r.ux, f0[qz], ax[0]);
+          ax[1] = fma(r.ux, f1[qz], ax[1]);
+          ay[0] = fma(r.uy, f0[qz], ay[0]);
+          ay[1] = fma(r.uy, f1[qz], ay[1]);
+          if (TWO) {
+            a2[0] = fma(r.k0, f0[qz], a2[0]);
+            a2[1] = fma(r.k0, f1[qz], a2[1]);
+          }
+        }
+#pragma unroll
+        for (int bz = 0; bz < 2; bz++) {
+          p[2 * bz] = fma(a[bz], y0, fma(ay[bz], -0.5, p[2 * bz]));
+          p[2 * bz + 1] = fma(a[bz], y1, fma(ay[bz], 0.5, p[2 * bz + 1]));
+          d[2 * bz] = fma(ax[bz], y0, d[2 * bz]);
+          d[2 * bz + 1] = fma(ax[bz], y1, d[2 * bz + 1]);
+          if (TWO) {
+            p2[2 * bz] = fma(a2[bz], y0, p2[2 * bz]);
+            p2[2 * bz + 1] = fma(a2[bz], y1, p2[2 * bz + 1]);
+          }
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        acc[2 * b] = fma(p[b], x0, fma(d[b], -0.5, acc[2 * b]));
+        acc[2 * b + 1] = fma(p[b], x1, fma(d[b], 0.5, acc[2 * b + 1]));
+        if (TWO) {
+          acc2[2 * b] = fma(p2[b], x0, acc2[2 * b]);
+          acc2[2 * b + 1] = fma(p2[b], x1, acc2[2 * b + 1]);
+        }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      sh[(j * NB + b) * R + t] = acc[b];
+      if (TWO) sh[((8 + j) * NB + b) * R + t] = acc2[b];
+    }
+    sf[j * R + t] = frhs;
+  }
+  __syncthreads();
+  if (!ok) return;
+  const int P = (M - 1) / 2;
+  const int64_t v0 = line_values<1>(P, py, pz);
+  const GroupOrder<1> go(__builtin_amdgcn_readfirstlane(py), __builtin_amdgcn_readfirstlane(pz));
+  for (int q = j; q < 27; q += 8) {
+    // column dx lies in the cells ix = 0 (dx <= 0) and 1 (dx >= 0) along x as
+    // their node dx + 1 - ix
+    const int dx = q % 3 - 1, dy = (q / 3) % 3 - 1, dz = q / 9 - 1;
+    double s = 0, s2 = 0;
+    for (int iz = dz > 0; iz <= (dz >= 0); iz++)
+      for (int iy = dy > 0; iy <= (dy >= 0); iy++)
+        for (int ix = dx > 0; ix <= (dx >= 0); ix++) {
+          const int c = ix + 2 * iy + 4 * iz, b = (dx + 1 - ix) + 2 * (dy + 1 - iy) + 4 * (dz + 1 - iz);
+          s += sh[(c * NB + b) * R + t];
+          if (TWO) s2 += sh[((8 + c) * NB + b) * R + t];
+        }
+    const int64_t at =
+        v0 + go.position(dy, dz) * (Lines<1>::VL * P) + Slots<double, 1>::at(P, (px - 1) >> 1, Lines<1>::slot(px, dx));
+    val[at] = s;
+    if (TWO) val2[at] = s2;
+  }
+  if (j == 3) {  // (the others have four slots)
+    double f = 0;
+#pragma unroll
+    for (int c = 0; c < 8; c++) f += sf[c * R + t];
+    rhs[px + M * (py + M * pz)] = f;
+  }
 }
 __global__ void k_scatter(double *__restrict__ y, const int *__restrict__ idx, const double *__restrict__ v, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1358,7 +1515,7 @@ __global__ __launch_bounds__(kRowsPerBlock) void k_assemble_kc(LineSet set, int 
   static_assert(kRowsPerBlock == 64, "one wavefront");
   __shared__ double sh[2][64 * kKcPad];
   int px, py, pz;
-  const bool ok = unit_row<2>(set, M, lg, &px, &py, &pz);
+  const bool ok = unit_row<2>(set, M, lg, threadIdx.x, &px, &py, &pz);
   const int code = unit_shape<2>(lg, set, M);
 #define PMX_KROW(EX, EY, EZ) assemble_row_kc<EX, EY, EZ>(sh, ok, px, py, pz, lg, M, n, kc, val, rhs)
   switch (code) {
@@ -1456,28 +1613,40 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
     return;
   }
   // the per-row evaluation of Q2 rows adds every cell's contribution into
-  // the cleared values (Q1 rows store each slot first; the padding rows of
-  // the slices are never written and keep the zeros of the allocation)
+  // the cleared values (Q1 rows store each slot; the slots of boundary nodes
+  // are never written and keep the zeros of the allocation)
   if (D.order == 2) {
     check(hipMemsetAsync(val, 0, sizeof(double) * D.nvals, st), "memset val");
     if (val2) check(hipMemsetAsync(val2, 0, sizeof(double) * D.nvals, st), "memset val2");
   }
-#define PMX_ASM(O, TW, IN)                                                                                   \
-  hipLaunchKernelGGL((k_assemble<O, TW, IN, false>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq, prm_dev, qref, qsrc, tab, val, val2, rhs)
-#define PMX_ASM2(O, TW) \
-  do {                   \
-    if (inl) PMX_ASM(O, TW, true); \
-    else PMX_ASM(O, TW, false);    \
+#define PMX_ASM2(TW)                                                                                               \
+  do {                                                                                                             \
+    if (inl) PMX_ASM(TW, true);                                                                                    \
+    else PMX_ASM(TW, false);                                                                                       \
   } while (0)
   if (D.order == 1) {
-    if (val2) PMX_ASM2(1, true);
-    else PMX_ASM2(1, false);
+#define PMX_ASM3(NP, TW, IN)                                                                                       \
+  hipLaunchKernelGGL((k_assemble_q1<NP, TW, IN>), gr, dim3(8 * kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, prm_dev, \
+                     qref, qsrc, val, val2, rhs)
+#define PMX_ASM(TW, IN)                                                                                            \
+  do {                                                                                                             \
+    if (nq == 8) PMX_ASM3(2, TW, IN);                                                                              \
+    else PMX_ASM3(3, TW, IN);                                                                                      \
+  } while (0)
+    if (nq != 8 && nq != 27) throw std::logic_error("assemble: no Q1 kernel for the rule");
+    if (val2) PMX_ASM2(true);
+    else PMX_ASM2(false);
+#undef PMX_ASM
+#undef PMX_ASM3
   } else {
-    if (val2) PMX_ASM2(2, true);
-    else PMX_ASM2(2, false);
+#define PMX_ASM(TW, IN)                                                                                            \
+  hipLaunchKernelGGL((k_assemble<2, TW, IN, false>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq,      \
+                     prm_dev, qref, qsrc, tab, val, val2, rhs)
+    if (val2) PMX_ASM2(true);
+    else PMX_ASM2(false);
+#undef PMX_ASM
   }
 #undef PMX_ASM2
-#undef PMX_ASM
   hipLaunchKernelGGL(k_boundary_rhs, dim3((D.nboundary + kBlock - 1) / kBlock), dim3(kBlock), 0, st, D.boundary,
                      D.nboundary, D.M, prm_dev, rhs);
 }
