@@ -781,7 +781,8 @@ __device__ __forceinline__ void wg_stage(T *lx, const T *x, const T *__restrict_
 // Sweeps of small levels with a workgroup per plane: planes of one colour do
 // not couple, so the C (at a turn 2C - 1) line groups of a plane follow each
 // other in LDS, and a launch does the steps of a plane colour instead of one
-// line group.
+// line group.  With ALL one workgroup takes the whole level and a launch does all
+// steps of the sweeps.
 //
 // On top of the launch a step is a chain: sums, barrier, the colours of the
 // lines, barrier.  Wavefronts 0 .. kSplits - 1 take the splits of the sums
@@ -791,59 +792,71 @@ __device__ __forceinline__ void wg_stage(T *lx, const T *x, const T *__restrict_
 // FP32 / FP64: Q2 39 / 49 us (5 launches), Q1 16 / 17 us (3); a launch per line
 // group 74 / 77 us (17 launches), 23 / 24 us (7); all of it in one workgroup
 // 59 / 98 and 32 / 37 us.  (Splits that sweep as well, with the loads before
-// the colours: 46 / 57 us.)
+// the colours: 46 / 57 us.)  With ALL, 9^3: Q2 28 / 37 us (17 steps), Q1 11 / 13 us
+// (7 steps), by planes 37 / 47 and 15 / 16 us.
 template <typename T, int O> struct Plane {
   static constexpr int C = Lines<O>::C, VL = Lines<O>::VL;
   static constexpr int kThreads = 64 * (kSplits + 1), kPlanes = 2 * O + 1;
   static constexpr int kParts = O == 2 ? 6 : 2;  // groups of a part per split
   static constexpr int kLoads = O == 2 ? 5 : 3;  // elements of x per thread and round
-  static size_t lds_bytes(int M) {
-    return 64 * kSplits * sizeof(PairSums<T>) + 2 * Wg<T, O>::kOffsets + sizeof(T) * (kPlanes + 2) * M * M;
+  static size_t lds_bytes(int M, bool all) {
+    return 64 * kSplits * sizeof(PairSums<T>) + 2 * Wg<T, O>::kOffsets +
+           sizeof(T) * (all ? 3 * M : kPlanes + 2) * M * M;
   }
 };
-// A step in 12 bits: line group, direction, sums
-__host__ __device__ inline unsigned plane_step(const WgStep &s) {
-  return (unsigned)(s.g | s.seq << 4 | s.sums << 6);
-}
+// The steps of a launch: line group (4 bits), direction (2), sums (6), upper
+// sums too where the boundary values are not zero (1)
+constexpr int kPlaneSteps = 40;
+struct PlaneSteps {
+  unsigned code[kPlaneSteps];
+  int n;
+};
 template <int O> struct PlaneStep {
   int g, seq, sums;
-  __device__ __forceinline__ explicit PlaneStep(uint64_t code)
-      : g((int)(code & 15)), seq((int)(code >> 4 & 3)), sums((int)(code >> 6 & 63)) {}
+  __device__ __forceinline__ PlaneStep(unsigned code, bool bnd)
+      : g((int)(code & 15)), seq((int)(code >> 4 & 3)), sums((int)(code >> 6 & 63)) {
+    if (bnd && (code >> 12 & 1)) sums |= kSumHi;
+  }
   __device__ __forceinline__ int zr() const { return O == 2 ? (g * 11) >> 5 : g >> 1; }
   __device__ __forceinline__ int yr() const { return g - Lines<O>::C * zr(); }
   // groups before a line of extent O, the most of the step
   __device__ __forceinline__ int lower() const { return O == 2 ? 10 * zr() + 2 * yr() : 6 * zr() + 2 * yr(); }
 };
-template <typename T, int O>
-__global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel<T> lv, int z0, uint64_t steps,
-                                                                         uint64_t upper, T *x,
+template <typename T, int O, bool ALL>
+__global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel<T> lv, int z0, PlaneSteps steps, T *x,
                                                                          const T *__restrict__ f, T *psum, double omega,
                                                                          const int *__restrict__ bnd_set) {
   using L = Lines<O>;
   using Q = Plane<T, O>;
   extern __shared__ __align__(16) unsigned char wg_lds[];
-  constexpr int C = Q::C, VL = L::VL, NP = Q::kParts, NX = O == 2 ? 5 : 4, ES = sizeof(T), H = NP > 2 ? NP / 2 : NP;
+  constexpr int C = Q::C, E = ALL ? C * C : C, VL = L::VL, NP = Q::kParts, NX = O == 2 ? 5 : 4, ES = sizeof(T), H = NP > 2 ? NP / 2 : NP;
   const int P = 1 << lv.lg, M = 2 * P + 1, MM = M * M, z = z0 + C * (int)blockIdx.x;
   const int t = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   PairSums<T> *red = reinterpret_cast<PairSums<T> *>(wg_lds);
   short *tab = reinterpret_cast<short *>(red + 64 * kSplits);
-  // x of the planes that the rows touch, the plane's f and kept sums; positions
-  // are relative to the first of those planes
-  T *lx = reinterpret_cast<T *>(tab + Wg<T, O>::kOffsets), *lf = lx + (Q::kPlanes - O) * MM, *lp = lf + MM;
-  // (a start from zero has upper sums where the boundary values are not zero)
-  if (bnd_set && *bnd_set) steps |= upper;
+  // x of the planes that the rows touch, f and kept sums of the planes of the
+  // rows; positions are relative to the first of those planes
+  const int px = ALL ? M : Q::kPlanes, nx = px * MM, x0 = ALL ? 0 : (z - O) * MM;
+  const int nf = ALL ? nx : MM, f0 = ALL ? 0 : O * MM;
+  T *lx = reinterpret_cast<T *>(tab + Wg<T, O>::kOffsets), *lf = lx + nx - f0, *lp = lf + nf;
+  const bool bnd = bnd_set && *bnd_set;
   const LevelBuffer<T> buf(lv.val, L::values(P));
   const __amdgpu_buffer_rsrc_t pbuf = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int2 *>(lv.pairs), 0, Wg<T, O>::kGroups * lv.tiles * kPairTile * (int)sizeof(int2), 0x00020000);
-  // the lane's pair in each of the plane's line groups (of the lanes past the
-  // last line a pair that exists, for its position)
-  int2 e[C];
+  // the lane's pair in each of the line groups (of the lanes past the last line
+  // a pair that exists, for its position); pairs of group i
+  auto pairs = [&](int i) {
+    const int yr = i % C, zr = ALL ? i / C : 0, ny = (M - 2 - (yr ? yr : C)) / C + 1;
+    return (ALL ? ny * ((M - 2 - (zr ? zr : C)) / C + 1) : ny) << lv.lg;
+  };
+  int2 e[E];
   {
-    const int zr = z % C;
+    const int zr = ALL ? 0 : z % C;
 #pragma unroll
-    for (int yr = 0; yr < C; yr++) {
-      const int n = ((M - 2 - (yr ? yr : C)) / C + 1) << lv.lg;
-      e[yr] = pair_entry(pbuf, (((yr + C * zr) * lv.tiles) * kPairTile + (z - (zr ? zr : C)) / C * n + (t < n ? t : 0)) * 8);
+    for (int i = 0; i < E; i++) {
+      const int n = pairs(i);
+      const int skip = ALL ? 0 : (z - (zr ? zr : C)) / C * n;
+      e[i] = pair_entry(pbuf, (((i + C * zr) * lv.tiles) * kPairTile + skip + (t < n ? t : 0)) * 8);
     }
   }
   const LevelBuffer<T> bx(x, (int64_t)M * MM), bf(f, (int64_t)M * MM), bp(psum, (int64_t)M * MM);
@@ -853,24 +866,23 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
   T vx[Q::kLoads], vf, vp;
   float vo[2];
   auto x_loads = [&](int i0) {
-    const int x0 = (z - O) * MM;
 #pragma unroll
     for (int u = 0; u < Q::kLoads; u++) {
       const int i = i0 + u * Q::kThreads;
       // (elements outside the lattice load zero: they are not read)
-      vx[u] = bx.one(i < Q::kPlanes * MM && x0 + i >= 0 ? (x0 + i) * ES : kNoOffset);
+      vx[u] = bx.one(i < nx && x0 + i >= 0 ? (x0 + i) * ES : kNoOffset);
     }
   };
   auto x_stores = [&](int i0) {
 #pragma unroll
     for (int u = 0; u < Q::kLoads; u++) {
       const int i = i0 + u * Q::kThreads;
-      if (i < Q::kPlanes * MM) lx[i] = vx[u];
+      if (i < nx) lx[i] = vx[u];
     }
   };
   x_loads(threadIdx.x);
   {
-    const int i = threadIdx.x, off = i < MM ? (z * MM + i) * ES : kNoOffset;
+    const int i = threadIdx.x, off = i < nf ? (x0 + f0 + i) * ES : kNoOffset;
     vf = bf.one(off);
     vp = bp.one(kept ? off : kNoOffset);
     if (Wg<T, O>::kOffsets) {
@@ -879,15 +891,15 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
     }
   }
 #pragma unroll
-  for (int yr = 0; yr < C; yr++) {
-    e[yr].x -= (z - O) * MM;
-    if (t >= ((M - 2 - (yr ? yr : C)) / C + 1) << lv.lg) e[yr].x |= 1 << 27;
+  for (int i = 0; i < E; i++) {
+    e[i].x -= x0;
+    if (t >= pairs(i)) e[i].x |= 1 << 27;
   }
   auto stage = [&] {
     x_stores(threadIdx.x);
-    if ((int)threadIdx.x < MM) {
-      lf[O * MM + threadIdx.x] = vf;
-      lp[O * MM + threadIdx.x] = vp;
+    if ((int)threadIdx.x < nf) {
+      lf[f0 + threadIdx.x] = vf;
+      lp[f0 + threadIdx.x] = vp;
     }
 #pragma unroll
     for (int u = 0; u < 2; u++) {
@@ -895,24 +907,29 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
       if (i < Wg<T, O>::kOffsets / 2) reinterpret_cast<float *>(tab)[i] = vo[u];
     }
     static_assert(Wg<T, O>::kOffsets / 2 <= 2 * Q::kThreads, "offsets per thread");
-    for (int i = threadIdx.x + Q::kLoads * Q::kThreads; i < Q::kPlanes * MM; i += Q::kLoads * Q::kThreads) {
+    for (int i = threadIdx.x + Q::kLoads * Q::kThreads; i < nx; i += Q::kLoads * Q::kThreads) {
       x_loads(i);
       x_stores(i);
     }
-    for (int i = threadIdx.x + Q::kThreads; i < MM; i += Q::kThreads) {
-      lf[O * MM + i] = bf.one((z * MM + i) * ES);
-      lp[O * MM + i] = bp.one(kept ? (z * MM + i) * ES : kNoOffset);
+    for (int i = threadIdx.x + Q::kThreads; i < nf; i += Q::kThreads) {
+      lf[f0 + i] = bf.one((x0 + f0 + i) * ES);
+      lp[f0 + i] = bp.one(kept ? (x0 + f0 + i) * ES : kNoOffset);
     }
   };
   auto pair_of = [&](const PlaneStep<O> &s) {
-    int2 r = e[0];
+    const int g = ALL ? s.g : s.yr();
+    int rx = e[0].x, ry = e[0].y;
 #pragma unroll
-    for (int yr = 1; yr < C; yr++)
-      if (s.yr() == yr) r = e[yr];
-    return WgPair(r);
+    for (int i = 1; i < E; i++) {
+      // (masks: an index computed from g would put the entries into memory)
+      const int k = -(int)(g == i);
+      rx ^= (rx ^ e[i].x) & k;
+      ry ^= (ry ^ e[i].y) & k;
+    }
+    return WgPair(int2{rx, ry});
   };
   if (w < kSplits) {
-    PlaneStep<O> s(steps);
+    PlaneStep<O> s(steps.code[0], bnd);
     WgPair pr = pair_of(s);
     T v[NP][VL];
     int at[NP];  // x of the groups
@@ -971,7 +988,9 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
     stage();
     __syncthreads();
     positions(s.sums & kSumLo);
-    while (true) {
+    for (int i = 1;; i++) {
+      const bool more = i < steps.n;
+      const PlaneStep<O> sn(steps.code[more ? i : 0], bnd);
       PairSums<T> p{0, 0, 0, 0};
       if (s.sums & kSumLo) {
         add(true);
@@ -989,18 +1008,17 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
       }
       red[64 * w + t] = p;
       lds_barrier();
-      steps >>= 12;
-      if (steps) {
-        s = PlaneStep<O>(steps);
+      if (more) {
+        s = sn;
         pr = pair_of(s);
         load(s.sums & kSumLo);
         positions(s.sums & kSumLo);
       }
       lds_barrier();
-      if (!steps) break;
+      if (!more) break;
     }
   } else {
-    PlaneStep<O> s(steps);
+    PlaneStep<O> s(steps.code[0], bnd);
     WgPair pr = pair_of(s);
     auto load = [&](const WgPair &q, bool any, T *own) {
       buf.template group<O>(any && q.ok ? (q.base() + q.before()) * (VL * P * ES) : kNoOffset, P, q.m, own);
@@ -1009,11 +1027,11 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
     load(pr, true, own);
     stage();
     __syncthreads();
-    while (true) {
-      steps >>= 12;
-      const PlaneStep<O> sn(steps);
+    for (int i = 1;; i++) {
+      const bool more = i < steps.n;
+      const PlaneStep<O> sn(steps.code[more ? i : 0], bnd);
       const WgPair pn = pair_of(sn);
-      load(pn, steps != 0, next);
+      load(pn, more, next);
       const int p = pr.p0;
       PairRow<T> r{lf[p + 1], lf[p + 2], T(0), T(0), own[1], own[3 + O], T(1) / own[1], T(1) / own[3 + O]};
       T xp[3] = {lx[p], lx[p + 1], lx[p + 2]};
@@ -1044,18 +1062,18 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
         }
       }
       lds_barrier();
-      if (!steps) break;
+      if (!more) break;
       s = sn;
       pr = pn;
 #pragma unroll
       for (int c = 0; c < VL; c++) own[c] = next[c];
     }
   }
-  for (int i = threadIdx.x; i < MM; i += Q::kThreads) {
-    const int px = i % M, py = i / M;
-    if (px < 1 || py < 1 || px > M - 2 || py > M - 2) continue;
-    x[z * MM + i] = lx[O * MM + i];
-    if (kept) psum[z * MM + i] = lp[O * MM + i];
+  for (int i = threadIdx.x; i < nf; i += Q::kThreads) {
+    const int ix = i % M, iy = (i / M) % M, iz = i / MM;
+    if (ix < 1 || iy < 1 || ix > M - 2 || iy > M - 2 || (ALL && (iz < 1 || iz > M - 2))) continue;
+    x[x0 + f0 + i] = lx[f0 + i];
+    if (kept) psum[x0 + f0 + i] = lp[f0 + i];
   }
 }
 // ||f - A x|| of the LDS iterate over all rows (Dirichlet rows: 0), the same
@@ -1356,29 +1374,35 @@ bool plane_sweeps_fit(const DevLayout &D) {
   const int C = D.order == 2 ? 3 : 2;
   return D.M >= 3 && (((D.M - 3) / C + 1) << D.lg) <= 64;
 }
+// ... in one workgroup where the pairs of a line group fit a wavefront, M <= 9
+static bool plane_sweeps_all(const DevLayout &D) {
+  const int C = D.order == 2 ? 3 : 2, n = (D.M - 3) / C + 1;
+  return (n * n << D.lg) <= 64;
+}
 template <typename T, int O>
 static void plane_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n,
                          bool zero, const int *bnd_set, hipStream_t st) {
   constexpr int C = Lines<O>::C;
+  const bool all = plane_sweeps_all(D);
+  const size_t lds = Plane<T, O>::lds_bytes(D.M, all);
+  T *ps = ssor ? psum : nullptr;
   WgSweeps<O> it{n, ssor, zero};
-  WgStep step;
-  bool more = it.next(step);
-  while (more) {
-    // the steps up to the next plane colour
-    const int zr = step.g / C, z0 = zr ? zr : C;
-    const bool start = zero && it.s == 0;
-    uint64_t steps = 0, upper = 0;
-    int k = 0;
+  WgStep s;
+  for (bool more = it.next(s); more;) {
+    // the steps up to the next plane colour, or all
+    const int zr = s.g / C, z0 = zr ? zr : C;
+    PlaneSteps steps{};
     do {
-      steps |= (uint64_t)plane_step(step) << 12 * k;
-      if (zero && it.s == 0 && !(step.sums & (kSumHi | kSumKept)))
-        upper |= (uint64_t)plane_step(WgStep{0, 0, kSumHi}) << 12 * k;
-      k++;
-      more = it.next(step);
-    } while (more && step.g / C == zr && k < 5);
-    launch_wg_grid(k_plane_sweep<T, O>, (D.M - 2 - z0) / C + 1, Plane<T, O>::kThreads, Plane<T, O>::lds_bytes(D.M), st,
-                   wg_level(D, val), z0, steps, upper, x, f, ssor ? psum : (T *)nullptr, omega,
-                   start ? bnd_set : (const int *)nullptr);
+      const bool upper = zero && it.s == 0 && !(s.sums & (kSumHi | kSumKept));
+      steps.code[steps.n++] = (unsigned)(s.g | s.seq << 4 | s.sums << 6 | (upper ? 1 : 0) << 12);
+      more = it.next(s);
+    } while (more && (all || s.g / C == zr) && steps.n < kPlaneSteps);
+    if (all)
+      launch_wg_grid(k_plane_sweep<T, O, true>, 1, Plane<T, O>::kThreads, lds, st, wg_level(D, val), 0, steps, x, f, ps,
+                     omega, bnd_set);
+    else
+      launch_wg_grid(k_plane_sweep<T, O, false>, (D.M - 2 - z0) / C + 1, Plane<T, O>::kThreads, lds, st,
+                     wg_level(D, val), z0, steps, x, f, ps, omega, bnd_set);
   }
 }
 template <typename T>
