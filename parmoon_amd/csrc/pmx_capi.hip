@@ -1871,8 +1871,7 @@ int pmx_defect_noalloc(pmx_system *sys, int level, const double *x, const double
     double *part = noalloc_scratch(*Y.ctx);
     hipStream_t st = Y.ctx->st;
     rows_apply<double>(lv.D, 1, lv.v64.val.p, x, b, r, 0.0, st);
-    boundary<double>(lv.D, 1, r, x, b, st);
-    dot_chunked(r, r, lv.L.N, part, res, 1, st);
+    defect_norm(lv.D, r, x, b, part, res, st);
     check(hipGetLastError(), "pmx_defect_noalloc launch");
   })
 }
