@@ -425,7 +425,8 @@ static void ensure_learned(System &Y) {
 // What is known of a level's x when its smoothing starts: nothing; zero in the
 // interior (x = f on the Dirichlet nodes, Y.bnd_set tells if those are zero);
 // zero everywhere, and f zero on the Dirichlet nodes.
-enum { kStartAny = 0, kStartInteriorZero = 1, kStartZero = 2 };
+// (all but kStartAny: the Dirichlet rows are x = f)
+enum { kStartAny = 0, kStartInteriorZero = 1, kStartZero = 2, kStartBoundary = 3 };
 // `sweeps` sweeps on v.x; true: v.psum holds the upper sums of the result
 template <typename T>
 static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweeps, int start = kStartAny) {
@@ -446,15 +447,15 @@ static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweep
   // Dirichlet rows x = f (no sweep changes them afterwards)
   if (start == kStartAny) boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
   const int *bs = start == kStartInteriorZero ? Y.bnd_set.p : nullptr;
+  const bool zero = start == kStartInteriorZero || start == kStartZero;
   if constexpr (std::is_same<T, float>::value) {
     if (Y.half_smoother && !planes) {
       if (!lv.have_val16) throw std::logic_error("level_smooth: FP16 smoother values missing");
-      sor_sweeps_scaled(lv.D, lv.val16.p, lv.sdinv.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps,
-                        start != kStartAny, bs, st);
+      sor_sweeps_scaled(lv.D, lv.val16.p, lv.sdinv.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps, zero, bs, st);
       return false;
     }
   }
-  sor_sweeps<T>(lv.D, v.val.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps, start != kStartAny, bs, planes, st);
+  sor_sweeps<T>(lv.D, v.val.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps, zero, bs, planes, st);
   return kind == 3;
 }
 // Learned post-smoothing of one level (replaces the post-sweeps of
@@ -526,7 +527,7 @@ static bool mg_cycle(System &Y, int i, bool post = true, int start = kStartAny) 
     const int cs = ((int)o[9] == 1 || (int)o[9] == 2 || (int)o[9] == 17) ? (int)o[9] : 3;
     if (cs == 17 && lv.ainv_n > 0) {
       gemv_coarse<T>(lv.ainv_n, (int)lv.L.N, lv.ainv.p, lv.iidx.p, v.f.p, v.x.p, st);
-      boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
+      if (start == kStartAny) boundary<T>(lv.D, 2, v.x.p, nullptr, v.f.p, st);
     } else if (cs >= 1 && cs <= 3 && sweep_wg_fits(lv.D, sizeof(T))) {
       // sweeps until the defect is reduced by SC_COARSE_RED_FACTOR_SCALAR
       // (opt[11]) or SC_COARSE_MAXIT_SCALAR (opt[10]) sweeps were made
@@ -568,8 +569,10 @@ static bool mg_cycle(System &Y, int i, bool post = true, int start = kStartAny) 
   // the first visit of the coarse level starts from its Reset (x = 0); the
   // learned pre-smoothing there takes d = f (restrict_ with zero_surface
   // leaves the coarse f zero on the Dirichlet surface, so the Dirichlet
-  // entries of that defect are the ones A x = 0 would give)
-  for (int j = 0; j < Y.rec[i]; j++) mg_cycle<T>(Y, i - 1, true, j == 0 && Y.x_zero_shortcut ? kStartZero : kStartAny);
+  // entries of that defect are the ones A x = 0 would give).  There x = f = 0
+  // on the Dirichlet rows from then on, as x = f on those of the finest level:
+  // no operation of the cycle changes them.
+  for (int j = 0; j < Y.rec[i]; j++) mg_cycle<T>(Y, i - 1, true, j == 0 && Y.x_zero_shortcut ? kStartZero : kStartBoundary);
   if ((int)o[12] < 1) Y.rec[i] = 1;
   // prolongation, CorrectNodes and x += SC_GMG_DAMP e
   prolongate_add<T>(cl.D, lv.D, cv.x.p, v.x.p, o[13], st);
@@ -581,7 +584,7 @@ static bool mg_cycle(System &Y, int i, bool post = true, int start = kStartAny) 
         post_done = true;
       }
     }
-    if (!post_done) upper = level_smooth<T>(Y, lv, kind, o[8], (int)o[7]);
+    if (!post_done) upper = level_smooth<T>(Y, lv, kind, o[8], (int)o[7], start == kStartAny ? kStartAny : kStartBoundary);
   }
   if (slc) {
     // TMGLevel3D::StepLengthControl (MGLevel3D.C:908-960), MultiGrid3D.C:671-679:
