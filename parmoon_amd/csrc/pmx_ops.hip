@@ -1366,7 +1366,7 @@ void values_to_csr(const DevLayout &D, const int *rowptr, const int *kcol, const
     hipLaunchKernelGGL((k_values_to_csr<T, 1>), g, dim3(kBlock), 0, st, rowptr, kcol, dof2lat, D.N, active, D.M, val, out);
 }
 
-// ---- Q2 one-matrix forms on MFMA: local matrices per cell, then a row gather.
+// ---- Q2 one-matrix forms: local matrices per cell, then a row gather.
 // With Phi_q the 4 x 27 table of (phi, dphi/dxi, dphi/deta, dphi/dzeta) at
 // point q, every form above is K = sum_q Phi_q^T D_q Phi_q (rows: test
 // functions a, columns: trial functions b) with, for the convection-diffusion
@@ -1374,139 +1374,187 @@ void values_to_csr(const DevLayout &D, const int *rowptr, const int *kcol, const
 //   D[0][0] = w c          D[0][d] = w g b_d
 //   D[e][0] = w g c s b_e  D[e][d] = w g^2 (eps [e == d] + s b_e b_d)
 // and the right-hand side f_a = sum_q r_q . Phi_q[:, a] with r = w f (1, g s b);
-// the mass form has D[0][0] = w and r = (w f, 0, 0, 0).  One wavefront
-// computes a cell as a 32 x 32 product (27 x 27 padded, column 27 carrying the
-// right-hand side) over K = 4 nq, one v_mfma_f64_16x16x4f64 per 16 x 16 tile
-// and quadrature point: lane l holds A = Phi_q[l/16][16R + l%16] and
-// B = (D_q Phi_q)[l/16][16C + l%16]; the result lane l, register r is entry
-// (16R + l/16 + 4r, 16C + l%16).  The tables sit in LDS ([q][comp][32]).
-typedef double doublex4 __attribute__((ext_vector_type(4)));
-// 8 wavefronts share one copy of the tables (64 KB for the 64-point rule)
-constexpr int kCellWaves = 8, kCellThreads = 64 * kCellWaves;
+// the mass form has D[0][0] = w and r = w f (1, g s b).
+//
+// The rule (NP points per axis) and the basis are tensor products, so the sum
+// is taken axis by axis: x, y, z one after the other, a pair of 1D basis
+// functions (of a and of b) at a time.  After the x sum the rows and columns
+// without a y or z derivative (phi and dphi/dxi) have the same y and z factors
+// and are one class (N), so 3 x 3 classes (N, Y, Z) remain of 4 x 4, after the
+// y sum 2 x 2.  For 64 points a cell takes 33 thousand products instead of the
+// 187 thousand of the plain sum (262 thousand on padded 16 x 16 x 4 matrix
+// instructions).  A workgroup takes kCells cells; a thread holds, of one cell,
+//   x: a line (y, z) of points and one basis function of a,
+//   y: a pair of x functions and one z,
+//   z: a pair of x and a pair of y functions,
+// and the sums between the axes go through LDS.  64^3 cells, 64 points: 3.75 ms by
+// the matrix instructions, 1.05 ms now (the cell buffer is 1.6 GB); 16^3 cells and
+// the levels below them, 27 points: 410 -> 64 us with the gather.
 constexpr int kKcRow = 28;  // doubles per local row in the cell buffer: 27 entries + rhs
-#ifndef PMX_CELLS_PER_PASS
-#define PMX_CELLS_PER_PASS 2
-#endif
-constexpr int kCellsPerPass = PMX_CELLS_PER_PASS;  // cells per wavefront pass of k_cell_mfma
-// CPC cells per wavefront pass: every quadrature point's table values are
-// read from LDS once for the CPC cells (10 LDS reads per lane and point
-// serve CPC x 4 MFMAs), with CPC independent accumulation chains per
-// wavefront.  Each cell's products and sums are those of one cell alone.
-template <bool INL, bool MASS, int CPC>
-__global__ __launch_bounds__(kCellThreads) void k_cell_mfma(int n, int nq, int form, const double *__restrict__ prm,
-                                                  const double *__restrict__ qref, const double *__restrict__ qp,
-                                                  const double *__restrict__ tab, double *__restrict__ kc) {
-  extern __shared__ __align__(16) unsigned char cell_lds[];
-  double *lt = reinterpret_cast<double *>(cell_lds);  // [nq][4][32]
+constexpr int kCells = 4, kCellThreads = 192;
+template <int NP, bool INL>
+__global__ __launch_bounds__(kCellThreads) void k_cell_sum(int n, int form, const double *__restrict__ prm,
+                                                           const double *__restrict__ qref,
+                                                           const double *__restrict__ qp, double *__restrict__ kc) {
+  constexpr int YZ = NP * NP, NQ = NP * YZ, XS = 81 * YZ, YS = 4 * 81 * NP, TS = XS > YS ? XS : YS;
+  static_assert(kCells * 3 * YZ <= kCellThreads && kCells * 12 * NP <= kCellThreads, "a thread per task");
+  __shared__ double tx[kCells * TS];  // x sums [class][pair][z][y], then y sums [class][pair][pair][z]
+  __shared__ double rx[kCells * 9 * YZ], ry[kCells * 18 * NP];  // those of the right-hand side
   const int tid = threadIdx.x;
-  for (int i = tid; i < nq * 128; i += kCellThreads) {
-    const int q = i >> 7, comp = (i >> 5) & 3, b = i & 31;
-    lt[i] = b < 27 ? tab[((int64_t)q * 27 + b) * 4 + comp] : 0.0;
+  const int64_t ncells = (int64_t)n * n * n, cell0 = (int64_t)blockIdx.x * kCells;
+  // 1D basis functions and derivatives at the points
+  double f[3][NP], d[3][NP];
+#pragma unroll
+  for (int i = 0; i < NP; i++) {
+    const double t = qref[4 * i];
+    f[0][i] = uniform(0.5 * t * (t - 1));
+    f[1][i] = uniform(1 - t * t);
+    f[2][i] = uniform(0.5 * t * (t + 1));
+    d[0][i] = uniform(t - 0.5);
+    d[1][i] = uniform(-2 * t);
+    d[2][i] = uniform(t + 0.5);
+  }
+  if (tid < kCells * 3 * YZ) {
+    const int c = tid / (3 * YZ), ax = (tid / YZ) % 3, yz = tid % YZ;
+    // (a cell past the last one repeats it and is not stored)
+    const int64_t cell = cell0 + c < ncells ? cell0 + c : ncells - 1;
+    const int cx = (int)(cell % n), cy = (int)((cell / n) % n), cz = (int)(cell / ((int64_t)n * n));
+    const bool mass = form == PMX_FORM_MASS || form == PMX_FORM_MASS_SUPG;
+    const double g = 2.0 * n;
+    double t[9][3], r[3] = {0, 0, 0};  // class (row, column), function of b
+#pragma unroll
+    for (int i = 0; i < 9; i++) t[i][0] = t[i][1] = t[i][2] = 0;
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      double Q[8];
+      if (INL) {
+        qp_coeffs<true>(prm, qref, n, cx, cy, cz, i + NP * yz, form, Q);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) Q[e] = qp[(cell * NQ + i + NP * yz) * 8 + e];
+      }
+      const double w = Q[0], xa = ax == 0 ? f[0][i] : ax == 1 ? f[1][i] : f[2][i],
+                   da = ax == 0 ? d[0][i] : ax == 1 ? d[1][i] : d[2][i];
+      const double wgs = w * g * Q[7], s1 = wgs * Q[2], s2 = wgs * Q[3], s3 = wgs * Q[4];
+      // D = s v^T + eps w g^2 on the diagonal of the derivatives, s = (w, s1, s2, s3)
+      const double rn = w * xa + s1 * da, rY = s2 * xa, rZ = s3 * xa;
+      r[0] += Q[6] * rn;
+      r[1] += Q[6] * rY;
+      r[2] += Q[6] * rZ;
+      const double sn = mass ? w * xa : rn, sY = mass ? 0.0 : rY, sZ = mass ? 0.0 : rZ;
+      const double v0 = mass ? 1.0 : Q[5], v1 = mass ? 0.0 : g * Q[2], v2 = mass ? 0.0 : g * Q[3],
+                   v3 = mass ? 0.0 : g * Q[4], ee = mass ? 0.0 : w * g * g * Q[1];
+      const double m[3][4] = {{sn * v0, sn * v1 + ee * da, sn * v2, sn * v3},
+                              {sY * v0, sY * v1, sY * v2 + ee * xa, sY * v3},
+                              {sZ * v0, sZ * v1, sZ * v2, sZ * v3 + ee * xa}};
+#pragma unroll
+      for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) {
+          t[3 * k][b] = fma(m[k][0], f[b][i], fma(m[k][1], d[b][i], t[3 * k][b]));
+          t[3 * k + 1][b] = fma(m[k][2], f[b][i], t[3 * k + 1][b]);
+          t[3 * k + 2][b] = fma(m[k][3], f[b][i], t[3 * k + 2][b]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+#pragma unroll
+      for (int b = 0; b < 3; b++) tx[c * TS + (k * 9 + 3 * ax + b) * YZ + yz] = t[k][b];
+#pragma unroll
+    for (int k = 0; k < 3; k++) rx[(c * 9 + 3 * k + ax) * YZ + yz] = r[k];
   }
   __syncthreads();
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l = tid & 63, comp = l >> 4, col = l & 15;
-  const double g = 2.0 * n;
-  // per-lane selectors of row `comp` of D (branch-free loop body keeps the
-  // accumulators in place across quadrature points)
-  const bool r0 = comp == 0;
-  const double s1 = comp == 1 ? 1.0 : 0.0, s2 = comp == 2 ? 1.0 : 0.0, s3 = comp == 3 ? 1.0 : 0.0;
-  const bool rhs_col = col == 11;  // column 27 = 16 + 11 of the second column tile
-  const int64_t ncells = (int64_t)n * n * n;
-  const int64_t ngroups = (ncells + CPC - 1) / CPC;
-  for (int64_t grp = (int64_t)blockIdx.x * kCellWaves + wave; grp < ngroups;
-       grp += (int64_t)gridDim.x * kCellWaves) {
-    // the cells of this pass (a pass past the last cell repeats the last
-    // one and does not store it)
-    int64_t cell[CPC];
-    int cx[CPC], cy[CPC], cz[CPC];
+  {
+    const int c = tid / (9 * NP), xp = (tid / NP) % 9, z = tid % NP;
+    const bool matrix = tid < kCells * 9 * NP;
+    double t[9][4];  // pair of y functions, class (row, column)
 #pragma unroll
-    for (int k = 0; k < CPC; k++) {
-      cell[k] = grp * CPC + k < ncells ? grp * CPC + k : ncells - 1;
-      cx[k] = (int)(cell[k] % n);
-      cy[k] = (int)((cell[k] / n) % n);
-      cz[k] = (int)(cell[k] / ((int64_t)n * n));
-    }
-    doublex4 a00[CPC], a01[CPC], a10[CPC], a11[CPC];
+    for (int i = 0; i < 9; i++) t[i][0] = t[i][1] = t[i][2] = t[i][3] = 0;
+    if (matrix) {
 #pragma unroll
-    for (int k = 0; k < CPC; k++) {
-      a00[k] = doublex4{0.0, 0.0, 0.0, 0.0};
-      a01[k] = a00[k];
-      a10[k] = a00[k];
-      a11[k] = a00[k];
-    }
-    // coefficients of the next quadrature point are loaded one step ahead
-    double Qn[CPC][8];
-    if (!INL) {
+      for (int y = 0; y < NP; y++) {
+        double v[9];
 #pragma unroll
-      for (int k = 0; k < CPC; k++)
+        for (int k = 0; k < 9; k++) v[k] = tx[c * TS + (k * 9 + xp) * YZ + z * NP + y];
 #pragma unroll
-        for (int e = 0; e < 8; e++) Qn[k][e] = qp[cell[k] * nq * 8 + e];
-    }
-    for (int q = 0; q < nq; q++) {
-      const double *T = lt + q * 128;
-      const double t0 = T[col], t1 = T[32 + col], t2 = T[64 + col], t3 = T[96 + col];
-      const double u0 = T[16 + col], u1 = T[48 + col], u2 = T[80 + col], u3 = T[112 + col];
-      const double av0 = T[comp * 32 + col], av1 = T[comp * 32 + 16 + col];
-      const int qn = q + 1 < nq ? q + 1 : q;
+        for (int a = 0; a < 3; a++) {
+          const double fa = f[a][y], da = d[a][y];
+          const double nn = v[0] * fa + v[3] * da, ny = v[1] * fa + v[4] * da, nz = v[2] * fa + v[5] * da;
+          const double zn = v[6] * fa, zy = v[7] * fa, zz = v[8] * fa;
 #pragma unroll
-      for (int k = 0; k < CPC; k++) {
-        double Qq[8];
-        if (INL) {
-          qp_coeffs<true>(prm, qref, n, cx[k], cy[k], cz[k], q, form, Qq);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; e++) Qq[e] = Qn[k][e];
-#pragma unroll
-          for (int e = 0; e < 8; e++) Qn[k][e] = qp[(cell[k] * nq + qn) * 8 + e];
-        }
-        const double w = Qq[0], eps = Qq[1], cc = Qq[5], ff = Qq[6], dl = Qq[7];
-        const double b0 = Qq[2], b1 = Qq[3], b2 = Qq[4];
-        // row comp of D = s v + t e_comp with v = (c, g b): s = w for row 0 and
-        // w g delta b_comp below it, t = w g^2 eps on the diagonal of rows 1-3;
-        // the right-hand-side weight is f s
-        double d0, d1, d2, d3, rr;
-        if (MASS) {
-          d0 = r0 ? w : 0.0;
-          d1 = d2 = d3 = 0.0;
-          // right-hand-side weights w f (1, g delta b): delta = 0 for
-          // MatrixMRhsAssemble, Compute_SDFEM_delta for MatrixMRhsAssemble_SUPG
-          const double be = s1 * b0 + s2 * b1 + s3 * b2;
-          rr = ff * (r0 ? w : w * g * dl * be);
-        } else {
-          const double be = s1 * b0 + s2 * b1 + s3 * b2;  // b_comp (0 for comp 0)
-          const double sc = r0 ? w : w * g * dl * be;
-          const double t = r0 ? 0.0 : w * g * g * eps;
-          const double gb0 = g * b0, gb1 = g * b1, gb2 = g * b2;
-          d0 = sc * cc;
-          d1 = sc * gb0 + s1 * t;
-          d2 = sc * gb1 + s2 * t;
-          d3 = sc * gb2 + s3 * t;
-          rr = ff * sc;
-        }
-        const double bv0 = d0 * t0 + d1 * t1 + d2 * t2 + d3 * t3;
-        double bv1 = d0 * u0 + d1 * u1 + d2 * u2 + d3 * u3;
-        bv1 = rhs_col ? rr : bv1;
-        a00[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(av0, bv0, a00[k], 0, 0, 0);
-        a01[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(av0, bv1, a01[k], 0, 0, 0);
-        a10[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(av1, bv0, a10[k], 0, 0, 0);
-        a11[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(av1, bv1, a11[k], 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < CPC; k++) {
-      if (grp * CPC + k >= ncells) continue;
-      double *K = kc + cell[k] * (27 * kKcRow);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int a0 = comp + 4 * r, a1 = 16 + comp + 4 * r, b0 = col, b1 = 16 + col;
-        K[a0 * kKcRow + b0] = a00[k][r];
-        if (b1 < kKcRow) K[a0 * kKcRow + b1] = a01[k][r];
-        if (a1 < 27) {
-          K[a1 * kKcRow + b0] = a10[k][r];
-          if (b1 < kKcRow) K[a1 * kKcRow + b1] = a11[k][r];
+          for (int b = 0; b < 3; b++) {
+            double *o = t[3 * a + b];
+            o[0] = fma(nn, f[b][y], fma(ny, d[b][y], o[0]));
+            o[1] = fma(nz, f[b][y], o[1]);
+            o[2] = fma(zn, f[b][y], fma(zy, d[b][y], o[2]));
+            o[3] = fma(zz, f[b][y], o[3]);
+          }
         }
       }
+    } else if (tid < kCells * 12 * NP) {
+      const int i = tid - kCells * 9 * NP, c = i / (3 * NP), ax = (i / NP) % 3, z = i % NP;
+      double o[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+#pragma unroll
+      for (int y = 0; y < NP; y++) {
+        const double v0 = rx[(c * 9 + ax) * YZ + z * NP + y], v1 = rx[(c * 9 + 3 + ax) * YZ + z * NP + y],
+                     v2 = rx[(c * 9 + 6 + ax) * YZ + z * NP + y];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+          o[a][0] = fma(v0, f[a][y], fma(v1, d[a][y], o[a][0]));
+          o[a][1] = fma(v2, f[a][y], o[a][1]);
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) ry[((c * 2 + k) * 9 + 3 * a + ax) * NP + z] = o[a][k];
+    }
+    __syncthreads();
+    if (matrix) {
+#pragma unroll
+      for (int y = 0; y < 9; y++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) tx[c * TS + ((k * 9 + xp) * 9 + y) * NP + z] = t[y][k];
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < kCells * 90; i += kCellThreads) {
+    const int c = i / 90, j = i % 90;
+    if (cell0 + c >= ncells) break;
+    double *K = kc + (cell0 + c) * (27 * kKcRow);
+    if (j < 81) {
+      // (x, y) functions of a, of b
+      const int a9 = j / 9, b9 = j % 9, xp = 3 * (a9 % 3) + b9 % 3, yp = 3 * (a9 / 3) + b9 / 3;
+      double o[9];
+#pragma unroll
+      for (int k = 0; k < 9; k++) o[k] = 0;
+#pragma unroll
+      for (int z = 0; z < NP; z++) {
+        double v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = tx[c * TS + ((k * 9 + xp) * 9 + yp) * NP + z];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+          const double nn = v[0] * f[a][z] + v[2] * d[a][z], nz = v[1] * f[a][z] + v[3] * d[a][z];
+#pragma unroll
+          for (int b = 0; b < 3; b++) o[3 * a + b] = fma(nn, f[b][z], fma(nz, d[b][z], o[3 * a + b]));
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) K[(a9 + 9 * a) * kKcRow + b9 + 9 * b] = o[3 * a + b];
+    } else {
+      const int a9 = j - 81;
+      double o[3] = {0, 0, 0};
+#pragma unroll
+      for (int z = 0; z < NP; z++) {
+        const double v0 = ry[((c * 2) * 9 + a9) * NP + z], v1 = ry[((c * 2 + 1) * 9 + a9) * NP + z];
+#pragma unroll
+        for (int a = 0; a < 3; a++) o[a] = fma(v0, f[a][z], fma(v1, d[a][z], o[a]));
+      }
+#pragma unroll
+      for (int a = 0; a < 3; a++) K[(a9 + 9 * a) * kKcRow + 27] = o[a];
     }
   }
 }
@@ -1676,21 +1724,17 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
     return;
   }
   if (kc && D.order == 2 && !val2) {
-    // local matrices on MFMA, then the row gather from the cell buffer
-    const int64_t ngroups = (ncells + kCellsPerPass - 1) / kCellsPerPass;
-    const unsigned grid = (unsigned)std::min<int64_t>((ngroups + kCellWaves - 1) / kCellWaves, 4096);
-    const size_t lds = (size_t)nq * 128 * sizeof(double);
-#define PMX_CELL(IN, MS)                                                                                   \
-  hipLaunchKernelGGL((k_cell_mfma<IN, MS, kCellsPerPass>), dim3(grid), dim3(kCellThreads), lds, st, D.n, nq, form,   \
-                     prm_dev, qref, qpbuf, tab, kc)
-    const bool ms = form == PMX_FORM_MASS || form == PMX_FORM_MASS_SUPG;
-    if (inl) {
-      if (ms) PMX_CELL(true, true);
-      else PMX_CELL(true, false);
-    } else {
-      if (ms) PMX_CELL(false, true);
-      else PMX_CELL(false, false);
-    }
+    // local matrices, then the row gather from the cell buffer
+#define PMX_CELL(NP, IN)                                                                                               \
+  hipLaunchKernelGGL((k_cell_sum<NP, IN>), dim3((unsigned)((ncells + kCells - 1) / kCells)), dim3(kCellThreads), 0, st, \
+                     D.n, form, prm_dev, qref, qpbuf, kc)
+    if (nq == 27) {
+      if (inl) PMX_CELL(3, true);
+      else PMX_CELL(3, false);
+    } else if (nq == 64) {
+      if (inl) PMX_CELL(4, true);
+      else PMX_CELL(4, false);
+    } else throw std::logic_error("assemble: no Q2 kernel for the rule");
 #undef PMX_CELL
     hipLaunchKernelGGL(k_assemble_kc, gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, kc, val, rhs);
     hipLaunchKernelGGL(k_boundary_rhs, dim3((D.nboundary + kBlock - 1) / kBlock), dim3(kBlock), 0, st, D.boundary,
