@@ -55,6 +55,10 @@ struct DevBuf {
     alloc(m);
     if (p) check(hipMemsetAsync(p, 0, sizeof(T) * m, st), "clear");
   }
+  // room for m elements at least
+  void reserve(size_t m) {
+    if (m > n) alloc(m);
+  }
   void upload(const T *h, size_t m, hipStream_t st) {
     alloc(m);
     check(hipMemcpyAsync(p, h, sizeof(T) * m, hipMemcpyHostToDevice, st), "upload");
@@ -127,6 +131,12 @@ struct System {
   DevBuf<double> kc;                  // Q2 cell matrices (finest level's cells x 27 x 28)
   // Krylov workspace
   DevBuf<double> sol, b, r64;         // finest level, FP64 (lattice)
+  // a host vector in the reference numbering on its way to or from a level
+  // (at most the finest level's size; the calls that use it end with the
+  // stream idle)
+  DevBuf<double> io;
+  // input, target and loss of a gradient call, kept up to kKeepGradient
+  DevBuf<float> gin, gtarget, gloss;
   DevBuf<double> sol_try, r_try;      // FP32 form: the corrected iterate and its defect before acceptance
   // a caller's finest-level CSR matrix (lattice-permuted) as the FP64 Krylov
   // operator of pmx_iterate; the MG cycle keeps the system's own levels
@@ -1213,29 +1223,19 @@ static void ensure_csr_host(System &Y, Level &lv) {
 // host (reference numbering) <-> device lattice vector
 template <typename T>
 static void to_lattice(System &Y, Level &lv, const double *host, T *dev) {
-  DevBuf<double> tmp;
-  tmp.upload(host, lv.L.N, Y.ctx->st);
-  DevBuf<double> lat;
-  lat.alloc(lv.L.N);
-  gather<double, double>(lat.p, tmp.p, lv.lat2dof.p, lv.L.N, Y.ctx->st);
-  if (std::is_same<T, double>::value)
-    check(hipMemcpyAsync(dev, lat.p, sizeof(double) * lv.L.N, hipMemcpyDeviceToDevice, Y.ctx->st), "copy");
-  else
-    convert<float, double>((float *)dev, lat.p, lv.L.N, Y.ctx->st);
-  check(hipStreamSynchronize(Y.ctx->st), "sync");
+  hipStream_t st = Y.ctx->st;
+  Y.io.reserve(lv.L.N);
+  check(hipMemcpyAsync(Y.io.p, host, sizeof(double) * lv.L.N, hipMemcpyHostToDevice, st), "h2d");
+  gather<T, double>(dev, Y.io.p, lv.lat2dof.p, lv.L.N, st);
+  check(hipStreamSynchronize(st), "sync");
 }
 template <typename T>
 static void from_lattice(System &Y, Level &lv, const T *dev, double *host) {
-  DevBuf<double> lat, tmp;
-  lat.alloc(lv.L.N);
-  tmp.alloc(lv.L.N);
-  if (std::is_same<T, double>::value)
-    check(hipMemcpyAsync(lat.p, dev, sizeof(double) * lv.L.N, hipMemcpyDeviceToDevice, Y.ctx->st), "copy");
-  else
-    convert<double, float>(lat.p, (const float *)dev, lv.L.N, Y.ctx->st);
-  gather<double, double>(tmp.p, lat.p, lv.dof2lat.p, lv.L.N, Y.ctx->st);
-  check(hipMemcpyAsync(host, tmp.p, sizeof(double) * lv.L.N, hipMemcpyDeviceToHost, Y.ctx->st), "d2h");
-  check(hipStreamSynchronize(Y.ctx->st), "sync");
+  hipStream_t st = Y.ctx->st;
+  Y.io.reserve(lv.L.N);
+  gather<double, T>(Y.io.p, dev, lv.dof2lat.p, lv.L.N, st);
+  check(hipMemcpyAsync(host, Y.io.p, sizeof(double) * lv.L.N, hipMemcpyDeviceToHost, st), "d2h");
+  check(hipStreamSynchronize(st), "sync");
 }
 
 }  // namespace pmx
@@ -2226,6 +2226,8 @@ int pmx_learned_forward(pmx_system *sys, int M, const float *in, float *out) {
     check(hipStreamSynchronize(st), "sync");
   })
 }
+// elements of the largest gradient input that stays allocated (128 MB)
+constexpr size_t kKeepGradient = (size_t)1 << 25;
 int pmx_learned_gradient(pmx_system *sys, int M, const float *in, const float *target, float *grads,
                          double *loss) {
   PMX_TRY({
@@ -2236,19 +2238,24 @@ int pmx_learned_gradient(pmx_system *sys, int M, const float *in, const float *t
     hipStream_t st = Y.ctx->st;
     const int64_t N = (int64_t)M * M * M;
     if (net_reserve(net, N, true)) Y.invalidate_graphs();
-    DevBuf<float> din, dtg, dl;
-    din.upload(in, (size_t)N * kNetIn, st);
-    dtg.upload(target, N, st);
-    dl.alloc(1);
+    Y.gin.reserve((size_t)N * kNetIn);
+    Y.gtarget.reserve(N);
+    Y.gloss.alloc(1);
+    check(hipMemcpyAsync(Y.gin.p, in, sizeof(float) * N * kNetIn, hipMemcpyHostToDevice, st), "h2d input");
+    check(hipMemcpyAsync(Y.gtarget.p, target, sizeof(float) * N, hipMemcpyHostToDevice, st), "h2d target");
     net_zero_grads(net, st);
-    net_forward(net, M, din.p, true, st);
-    net_backward(net, M, dtg.p, dl.p, st);
+    net_forward(net, M, Y.gin.p, true, st);
+    net_backward(net, M, Y.gtarget.p, Y.gloss.p, st);
     if (grads)
       check(hipMemcpyAsync(grads, net.grads, sizeof(float) * net_total_params(), hipMemcpyDeviceToHost, st),
             "d2h grads");
     float l = 0;
-    check(hipMemcpyAsync(&l, dl.p, sizeof(float), hipMemcpyDeviceToHost, st), "d2h loss");
+    check(hipMemcpyAsync(&l, Y.gloss.p, sizeof(float), hipMemcpyDeviceToHost, st), "d2h loss");
     check(hipStreamSynchronize(st), "sync");
+    if (Y.gin.n > kKeepGradient) {
+      Y.gin.release();
+      Y.gtarget.release();
+    }
     if (loss) *loss = l;
   })
 }

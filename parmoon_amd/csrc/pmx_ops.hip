@@ -1938,6 +1938,8 @@ template void convert<double, float>(double *, const float *, int64_t, hipStream
 template void add_convert<double, float>(double *, const float *, int64_t, hipStream_t);
 template void add_convert<double, double>(double *, const double *, int64_t, hipStream_t);
 template void gather<double, double>(double *, const double *, const int *, int64_t, hipStream_t);
+template void gather<float, double>(float *, const double *, const int *, int64_t, hipStream_t);
+template void gather<double, float>(double *, const float *, const int *, int64_t, hipStream_t);
 template void gather<float, float>(float *, const float *, const int *, int64_t, hipStream_t);
 template void multi_axpy<double, double>(double *, const double *, const double *, int, int64_t, int64_t, hipStream_t);
 template void multi_axpy<float, float>(float *, const float *, const double *, int, int64_t, int64_t, hipStream_t);
