@@ -353,7 +353,7 @@ static void coarse_inverse(System &Y, Level &lv) {
   const int64_t nv = lv.L.nstored;
   lv.flag.alloc(1);
   if (lv.ainv_n == nI && lv.ainv_src.p && bits_equal(lv.v64.val.p, lv.ainv_src.p, nv, lv.flag.p, st)) return;
-  lv.aug.alloc((size_t)nI * (nI + N));
+  lv.aug.alloc((size_t)coarse_inverse_scratch(nI, N));
   lv.piv.alloc(nI);
   lv.ainv.alloc((size_t)nI * N);
   lv.ainv_n = 0;

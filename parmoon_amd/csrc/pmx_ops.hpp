@@ -156,7 +156,9 @@ template <typename T> void start_boundary(const DevLayout &D, T *x, const T *f, 
 template <typename T>
 void gemv_coarse(int nI, int N, const double *W, const int *iidx, const T *x, T *y, hipStream_t st);
 // W of the level by Gauss-Jordan with partial pivoting (cidx: lattice node ->
-// interior row or -1; aug: n_I x (n_I + N) workspace; piv: n_I ints)
+// interior row or -1; aug: workspace of coarse_inverse_scratch doubles; piv: n_I
+// ints)
+int64_t coarse_inverse_scratch(int nI, int N);
 void coarse_inverse_dense(const DevLayout &D, const double *val, const int *iidx, const int *cidx, int nI, double *aug,
                           int *piv, double *W, hipStream_t st);
 template <typename T, typename U> void gather(T *out, const U *in, const int *map, int64_t n, hipStream_t st);
