@@ -121,7 +121,7 @@ struct System {
   bool assembled = false;
   bool two_matrices = false;
   DevBuf<double> prm, qref, tab, qpbuf;
-  int64_t qp_tab_off = 0;  // offset of the curl-Fourier phase tables in qpbuf
+  int64_t qp_tab_off = 0;  // offset of the phase tables in qpbuf
   int cell_measure = 0;    // prm[PMX_PRM_CELL_MEASURE] of the last assembly
   int nq = 0;
   int tab_key = -1;                   // rule of the uploaded tables
@@ -317,7 +317,7 @@ static void ensure_tables(System &Y, bool linear) {
   // the qp records of the finest level, then room for the curl-Fourier
   // phase tables of any level
   Y.qp_tab_off = (int64_t)Y.lev.back()->Nb.ncells * nq * 8;
-  Y.qpbuf.alloc((size_t)(Y.qp_tab_off + fourier_tab_len(Y.lev.back()->L.n, nq)));
+  Y.qpbuf.alloc((size_t)(Y.qp_tab_off + phase_tab_len(Y.lev.back()->L.n, nq)));
   Y.tab_key = key;
 }
 

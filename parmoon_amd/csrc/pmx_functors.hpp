@@ -34,11 +34,12 @@ __host__ __device__ inline void fourier_b(const double *prm, double x, double y,
   b[2] = s * (dA[1][0] - dA[0][1]);
 }
 
+constexpr double kGrfScale = 0.17677669529663688110021109052621;  // sqrt(2/64)
 __host__ __device__ inline double grf_field(const double *prm, double x, double y, double z) {
   const double *G = prm + PMX_PRM_GRF;
   double s = 0;
   for (int k = 0; k < 64; k++) s += cos(G[4 * k] * x + G[4 * k + 1] * y + G[4 * k + 2] * z + G[4 * k + 3]);
-  return s * 0.17677669529663688110021109052621;  // sqrt(2/64)
+  return s * kGrfScale;
 }
 
 // the trigonometric factors of the example functions, evaluated where used

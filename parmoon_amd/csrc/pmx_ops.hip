@@ -248,21 +248,22 @@ __host__ __device__ inline bool form_has_delta(int form) {
 // two complex products per mode instead of a cosine, and the three loads of
 // a mode touch one cache line per wavefront.  The values differ from the
 // direct evaluation by rounding only.
-__device__ __forceinline__ int rule_points_1d(int nq) { return nq <= 8 ? 2 : (nq <= 27 ? 3 : 4); }
-__global__ __launch_bounds__(kBlock) void k_fourier_tables(const double *__restrict__ prm,
+__host__ __device__ inline int rule_points_1d(int nq) { return nq <= 8 ? 2 : (nq <= 27 ? 3 : 4); }
+template <bool GRF>
+__global__ __launch_bounds__(kBlock) void k_phase_tables(const double *__restrict__ prm,
                                                            const double *__restrict__ qref, int nq, int n,
                                                            double *__restrict__ tab) {
   const int np = rule_points_1d(nq);
   const int id = blockIdx.x * kBlock + threadIdx.x;
-  if (id >= kFourierModes * 3 * n * np) return;
+  if (id >= (GRF ? kGrfModes : kFourierModes) * 3 * n * np) return;
   const int ci = id % (n * np), d = (id / (n * np)) % 3, m = id / (3 * n * np);
   const int c = ci / np, i = ci % np;
   const double twopi = 6.283185307179586476925286766559;
   const double h = 1.0 / n;
-  const double *t = prm + PMX_PRM_FOURIER + m * 5;
+  const double *t = GRF ? prm + PMX_PRM_GRF + m * 4 : prm + PMX_PRM_FOURIER + m * 5;
   // point i of the 1D rule is the first coordinate of point q = i
   const double X = (c * h + 0.5 * h) + 0.5 * h * qref[4 * i];
-  const double a = twopi * t[1 + d] * X + (d == 0 ? t[4] : 0.0);
+  const double a = GRF ? t[d] * X + (d == 0 ? t[3] : 0.0) : twopi * t[1 + d] * X + (d == 0 ? t[4] : 0.0);
   tab[2 * id] = cos(a);
   tab[2 * id + 1] = sin(a);
 }
@@ -376,6 +377,57 @@ __global__ __launch_bounds__(kBlock) void k_qp_data_fourier(const double *__rest
     if (cm4) qp_record(prm, (int)prm[PMX_PRM_FORM], 1.0 / n, qref[4 * q + 3], k, o, &k0);
     else qp_record(prm, (int)prm[PMX_PRM_FORM], 1.0 / n, qref[4 * q + 3], k, o);
   }
+}
+// ... and for the log-normal example, eps exp(sigma g) with the field g of
+// grf_field, a sum of cosines at 64 frequencies: a cosine of the sum of three
+// phases is the real part of the product of the tables' factors, 2 operations per
+// point and mode behind the product of a line's y and z factors.  (Evaluating the
+// cosines was all of an assembly: 13.2 ms of 15.5 at 128^3 cells, 27 points.)
+// 64^3 cells and the levels below: 1.37 -> 0.34 ms.
+template <int NQ>
+__global__ __launch_bounds__(kBlock) void k_qp_data_grf(const double *__restrict__ prm,
+                                                        const double *__restrict__ qref, int n,
+                                                        const double *__restrict__ tab, double *__restrict__ out) {
+  constexpr int np = NQ == 8 ? 2 : (NQ == 27 ? 3 : 4);
+  // a thread takes the np x np points of a cell with one z
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t >= n * np) return;
+  const int cx = t / np, iz = t % np;
+  const int cy = blockIdx.y % n, cz = blockIdx.y / n;
+  const int64_t L = (int64_t)n * np;  // entries per (mode, axis)
+  double s[np][np];
+#pragma unroll
+  for (int i = 0; i < np * np; i++) s[i / np][i % np] = 0;
+#pragma unroll 2
+  for (int m = 0; m < kGrfModes; m++) {
+    const double *fx = tab + 2 * ((m * 3 + 0) * L + cx * np);
+    const double *fy = tab + 2 * ((m * 3 + 1) * L + cy * np);
+    const double *fz = tab + 2 * ((m * 3 + 2) * L + cz * np + iz);
+#pragma unroll
+    for (int y = 0; y < np; y++) {
+      const double pr = fy[2 * y] * fz[0] - fy[2 * y + 1] * fz[1], pi = fy[2 * y] * fz[1] + fy[2 * y + 1] * fz[0];
+#pragma unroll
+      for (int i = 0; i < np; i++) s[y][i] += fx[2 * i] * pr - fx[2 * i + 1] * pi;
+    }
+  }
+  const int64_t cell = cx + (int64_t)n * blockIdx.y;
+  QpCoeffs k;
+  k.c = prm[PMX_PRM_C];
+  k.b0 = prm[PMX_PRM_B0];
+  k.b1 = prm[PMX_PRM_B1];
+  k.b2 = prm[PMX_PRM_B2];
+  k.f = 1.0;
+#pragma unroll 1
+  for (int y = 0; y < np; y++)
+#pragma unroll
+    for (int i = 0; i < np; i++) {
+      double g = s[0][i];
+#pragma unroll
+      for (int c = 1; c < np; c++) g = y == c ? s[c][i] : g;
+      k.eps = prm[PMX_PRM_EPS] * exp(prm[PMX_PRM_GRF_SIGMA] * (g * kGrfScale));
+      const int q = i + np * (y + np * iz);
+      qp_record(prm, (int)prm[PMX_PRM_FORM], 1.0 / n, qref[4 * q + 3], k, out + (cell * NQ + q) * 8);
+    }
 }
 // examples whose coefficients are cheaper to evaluate again than to read back
 __host__ __device__ inline bool coeffs_inline(int example) {
@@ -1785,19 +1837,24 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
   const bool inl = !qp_given && coeffs_inline(example) && !corner;
   if (!inl && !qp_given) {
     // (grid y = n^2 lines of cells: up to 255 cells per direction)
-    if (example == PMX_EX_CURL_FOURIER && ftab && (int64_t)D.n * D.n <= 65535) {
-      const int64_t nt = fourier_tab_len(D.n, nq) / 2;  // complex entries
-      hipLaunchKernelGGL(k_fourier_tables, dim3((unsigned)((nt + kBlock - 1) / kBlock)), dim3(kBlock), 0, st,
-                         prm_dev, qref, nq, D.n, ftab);
+    const bool grf = example == PMX_EX_LOGNORMAL && !corner;
+    if ((example == PMX_EX_CURL_FOURIER || grf) && ftab && (int64_t)D.n * D.n <= 65535) {
       const int nl = nq == 8 ? 4 : (nq == 27 ? 9 : 16);  // x-lines of points per cell
-      const dim3 g((unsigned)((D.n * nl + kBlock - 1) / kBlock), (unsigned)(D.n * D.n));
-      if (nq == 8)
-        hipLaunchKernelGGL(k_qp_data_fourier<8>, g, dim3(kBlock), 0, st, prm_dev, qref, D.n, ftab, qpbuf, corner);
-      else if (nq == 27)
-        hipLaunchKernelGGL(k_qp_data_fourier<27>, g, dim3(kBlock), 0, st, prm_dev, qref, D.n, ftab, qpbuf, corner);
-      else if (nq == 64)
-        hipLaunchKernelGGL(k_qp_data_fourier<64>, g, dim3(kBlock), 0, st, prm_dev, qref, D.n, ftab, qpbuf, corner);
-      else throw std::logic_error("assemble: rule without the curl-Fourier kernel");
+      if (nq != 8 && nq != 27 && nq != 64) throw std::logic_error("assemble: rule without phase tables");
+      // complex entries
+      const int64_t nt = (int64_t)(grf ? kGrfModes : kFourierModes) * 3 * D.n * rule_points_1d(nq);
+      const dim3 gt((unsigned)((nt + kBlock - 1) / kBlock));
+      const int per = grf ? rule_points_1d(nq) : nl;  // threads per cell
+      const dim3 g((unsigned)((D.n * per + kBlock - 1) / kBlock), (unsigned)(D.n * D.n));
+      if (grf) {
+        hipLaunchKernelGGL(k_phase_tables<true>, gt, dim3(kBlock), 0, st, prm_dev, qref, nq, D.n, ftab);
+        auto *k = nq == 8 ? k_qp_data_grf<8> : nq == 27 ? k_qp_data_grf<27> : k_qp_data_grf<64>;
+        hipLaunchKernelGGL(k, g, dim3(kBlock), 0, st, prm_dev, qref, D.n, ftab, qpbuf);
+      } else {
+        hipLaunchKernelGGL(k_phase_tables<false>, gt, dim3(kBlock), 0, st, prm_dev, qref, nq, D.n, ftab);
+        auto *k = nq == 8 ? k_qp_data_fourier<8> : nq == 27 ? k_qp_data_fourier<27> : k_qp_data_fourier<64>;
+        hipLaunchKernelGGL(k, g, dim3(kBlock), 0, st, prm_dev, qref, D.n, ftab, qpbuf, corner);
+      }
     } else {
       hipLaunchKernelGGL(k_qp_data, dim3((unsigned)((ncq + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, prm_dev,
                          qref, nq, D.n, qpbuf, corner);

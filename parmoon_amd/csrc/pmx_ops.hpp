@@ -179,20 +179,20 @@ void values_to_csr(const DevLayout &D, const int *rowptr, const int *kcol, const
 // buffer of n^3 x 27 x 28 doubles for the Q2 one-matrix forms on MFMA
 // (nullptr: the per-row evaluation); qp_given: qpbuf already holds the
 // quadrature-point records (coefficients from host callbacks)
-// ftab (optional): room for fourier_tab_len(n, nq) doubles; with it the
+// ftab (optional): room for phase_tab_len(n, nq) doubles; with it the
 // curl-Fourier example's coefficients come from per-level phase tables.
 // corner (required for CELL_MEASURE 4, else unused): the per-cell frame codes
 // of Numbering::corner on the device.
 void assemble(const DevLayout &D, const double *prm_dev, int example, int form, const double *qref, int nq,
               const double *tab, double *qpbuf, double *kc, double *val, double *val2, double *rhs, hipStream_t st,
               bool qp_given = false, double *ftab = nullptr, const uint8_t *corner = nullptr);
-// doubles of the curl-Fourier phase table of a level with n cells per
-// direction and an nq-point tensor rule (complex factors of the 3 x 8 modes
-// of PMX_PRM_FOURIER per axis, cell index and 1D point)
-constexpr int kFourierModes = 24;
-inline int64_t fourier_tab_len(int n, int nq) {
+// doubles of the phase tables of a level with n cells per direction and an
+// nq-point tensor rule: complex factors per mode, axis, cell index and 1D point
+// of the 3 x 8 modes of PMX_PRM_FOURIER or the 64 of PMX_PRM_GRF
+constexpr int kFourierModes = 24, kGrfModes = 64;
+inline int64_t phase_tab_len(int n, int nq) {
   const int np = nq <= 8 ? 2 : (nq <= 27 ? 3 : 4);
-  return 2 * (int64_t)kFourierModes * 3 * n * np;
+  return 2 * (int64_t)kGrfModes * 3 * n * np;
 }
 // y[idx[i]] = v[i]
 void scatter(double *y, const int *idx, const double *v, int n, hipStream_t st);
