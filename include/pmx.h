@@ -183,7 +183,7 @@ int pmx_csr_matvec(pmx_ctx *ctx, int n, const int *rowptr, const int *kcol, cons
  *  [19] precision 2: number of finest levels with the learned post-smoother
  *       (0 = the levels it was trained for)
  *  [20] precision 2: learned steps per post-smoothing (default 1)
- *  [21] SOR/SSOR sweeps of small levels (at most 17^3 lattice nodes) whose
+ *  [21] SOR/SSOR sweeps of small levels (at most 17^3 lattice nodes, Q2 33^3) whose
  *       largest colour has at most this many rows run plane by plane (same
  *       iterate, fewer launches); 0 = all of them, < 0 = never
  *  [22] precision 2: the finest [22] of the [19] levels keep the plain smoother

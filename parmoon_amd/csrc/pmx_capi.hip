@@ -444,7 +444,7 @@ static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweep
   Vecs<T> &v = vecs<T>(lv);
   // small levels sweep by planes, with FP32 values also where the larger ones
   // take FP16 values (there is no traffic to save); opt[21] as in pmx.h
-  const bool planes = plane_sweeps_fit(lv.D) && (Y.opt[21] == 0 || lv.D.max_colour_rows <= (int64_t)Y.opt[21]);
+  const bool planes = plane_sweeps_used(lv.D) && (Y.opt[21] == 0 || lv.D.max_colour_rows <= (int64_t)Y.opt[21]);
   if (kind == 1) {
     for (int s = 0; s < sweeps; s++) {
       copy<T>(v.aux.p, v.x.p, lv.L.N, st);
@@ -459,7 +459,7 @@ static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweep
   const int *bs = start == kStartInteriorZero ? Y.bnd_set.p : nullptr;
   const bool zero = start == kStartInteriorZero || start == kStartZero;
   if constexpr (std::is_same<T, float>::value) {
-    if (Y.half_smoother && !planes) {
+    if (Y.half_smoother && !(planes && plane_sweeps_fit(lv.D))) {
       if (!lv.have_val16) throw std::logic_error("level_smooth: FP16 smoother values missing");
       sor_sweeps_scaled(lv.D, lv.val16.p, lv.sdinv.p, v.x.p, v.f.p, v.psum.p, omega, kind == 3, sweeps, zero, bs, st);
       return false;

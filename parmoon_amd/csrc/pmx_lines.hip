@@ -794,13 +794,15 @@ __device__ __forceinline__ void wg_stage(T *lx, const T *x, const T *__restrict_
 // 59 / 98 and 32 / 37 us.  (Splits that sweep as well, with the loads before
 // the colours: 46 / 57 us.)  With ALL, 9^3: Q2 28 / 37 us (17 steps), Q1 11 / 13 us
 // (7 steps), by planes 37 / 47 and 15 / 16 us.
-template <typename T, int O> struct Plane {
+// SL: wavefronts of row pairs (each has kSplits + 1 of the workgroup)
+template <typename T, int O, int SL> struct Plane {
   static constexpr int C = Lines<O>::C, VL = Lines<O>::VL;
-  static constexpr int kThreads = 64 * (kSplits + 1), kPlanes = 2 * O + 1;
-  static constexpr int kParts = O == 2 ? 6 : 2;  // groups of a part per split
+  static constexpr int kThreads = 64 * (kSplits + 1) * SL, kPlanes = 2 * O + 1;
+  // groups of a part per split and batch: all of them if the registers allow
+  static constexpr int kParts = O == 1 ? 2 : SL == 1 ? 6 : sizeof(T) == 4 ? 3 : 2;
   static constexpr int kLoads = O == 2 ? 5 : 3;  // elements of x per thread and round
   static size_t lds_bytes(int M, bool all) {
-    return 64 * kSplits * sizeof(PairSums<T>) + 2 * Wg<T, O>::kOffsets +
+    return 64 * kSplits * SL * sizeof(PairSums<T>) + 2 * Wg<T, O>::kOffsets +
            sizeof(T) * (all ? 3 * M : kPlanes + 2) * M * M;
   }
 };
@@ -822,18 +824,23 @@ template <int O> struct PlaneStep {
   // groups before a line of extent O, the most of the step
   __device__ __forceinline__ int lower() const { return O == 2 ? 10 * zr() + 2 * yr() : 6 * zr() + 2 * yr(); }
 };
-template <typename T, int O, bool ALL>
-__global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel<T> lv, int z0, PlaneSteps steps, T *x,
+template <typename T, int O, bool ALL, int SL>
+__global__ __launch_bounds__((Plane<T, O, SL>::kThreads)) void k_plane_sweep(WgLevel<T> lv, int z0, PlaneSteps steps, T *x,
                                                                          const T *__restrict__ f, T *psum, double omega,
                                                                          const int *__restrict__ bnd_set) {
   using L = Lines<O>;
-  using Q = Plane<T, O>;
+  using Q = Plane<T, O, SL>;
   extern __shared__ __align__(16) unsigned char wg_lds[];
-  constexpr int C = Q::C, E = ALL ? C * C : C, VL = L::VL, NP = Q::kParts, NX = O == 2 ? 5 : 4, ES = sizeof(T), H = NP > 2 ? NP / 2 : NP;
+  constexpr int C = Q::C, E = ALL ? C * C : C, VL = L::VL, NP = Q::kParts, NX = O == 2 ? 5 : 4, ES = sizeof(T),
+                H = NP == 6 ? 3 : NP;
+  constexpr bool kBatches = O == 2 && NP < 6;
   const int P = 1 << lv.lg, M = 2 * P + 1, MM = M * M, z = z0 + C * (int)blockIdx.x;
   const int t = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  PairSums<T> *red = reinterpret_cast<PairSums<T> *>(wg_lds);
-  short *tab = reinterpret_cast<short *>(red + 64 * kSplits);
+  // wavefronts of the splits, then those of the rows
+  const bool rows = w >= kSplits * SL;
+  const int slot = rows ? w - kSplits * SL : w / kSplits, split = w % kSplits;
+  PairSums<T> *const sums = reinterpret_cast<PairSums<T> *>(wg_lds), *const red = sums + 64 * kSplits * slot;
+  short *tab = reinterpret_cast<short *>(sums + 64 * kSplits * SL);
   // x of the planes that the rows touch, f and kept sums of the planes of the
   // rows; positions are relative to the first of those planes
   const int px = ALL ? M : Q::kPlanes, nx = px * MM, x0 = ALL ? 0 : (z - O) * MM;
@@ -856,7 +863,8 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
     for (int i = 0; i < E; i++) {
       const int n = pairs(i);
       const int skip = ALL ? 0 : (z - (zr ? zr : C)) / C * n;
-      e[i] = pair_entry(pbuf, (((i + C * zr) * lv.tiles) * kPairTile + skip + (t < n ? t : 0)) * 8);
+      const int q = 64 * slot + t;
+      e[i] = pair_entry(pbuf, (((i + C * zr) * lv.tiles) * kPairTile + skip + (q < n ? q : 0)) * 8);
     }
   }
   const LevelBuffer<T> bx(x, (int64_t)M * MM), bf(f, (int64_t)M * MM), bp(psum, (int64_t)M * MM);
@@ -893,7 +901,7 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
 #pragma unroll
   for (int i = 0; i < E; i++) {
     e[i].x -= x0;
-    if (t >= pairs(i)) e[i].x |= 1 << 27;
+    if (64 * slot + t >= pairs(i)) e[i].x |= 1 << 27;
   }
   auto stage = [&] {
     x_stores(threadIdx.x);
@@ -928,16 +936,19 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
     }
     return WgPair(int2{rx, ry});
   };
-  if (w < kSplits) {
+  if (!rows) {
     PlaneStep<O> s(steps.code[0], bnd);
     WgPair pr = pair_of(s);
     T v[NP][VL];
     int at[NP];  // x of the groups
-    // the values of one part; the second half of them only where a row of the
-    // step has so many groups
-    auto many = [&](bool lo) { return NP > 2 && (lo ? s.lower() : L::kMaxGroups - 1 - s.lower()) > kSplits * H; };
-    auto load = [&](bool lo) {
-      const int k0 = lo ? w : pr.before() + 1 + w, k1 = !pr.ok ? 0 : lo ? pr.before() : pr.groups();
+    // groups of a part, the most of a row of the step
+    auto count = [&](bool lo) { return lo ? s.lower() : L::kMaxGroups - 1 - s.lower(); };
+    // the values of one part (batch b of it); the second half of them only where
+    // a row of the step has so many groups
+    auto many = [&](bool lo) { return NP == 6 && count(lo) > kSplits * H; };
+    auto load = [&](bool lo, int b) {
+      const int k0 = (lo ? 0 : pr.before() + 1) + split + kSplits * NP * b,
+                k1 = !pr.ok ? 0 : lo ? pr.before() : pr.groups();
       const int off = (pr.base() + k0) * (VL * P * ES);
       auto one = [&](int i) {
         buf.template group<O>(k0 + kSplits * i < k1 ? off + i * (kSplits * VL * P * ES) : kNoOffset, P, pr.m, v[i]);
@@ -949,8 +960,8 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
         for (int i = H; i < NP; i++) one(i);
       }
     };
-    auto positions = [&](bool lo) {
-      const int k0 = lo ? w : pr.before() + 1 + w, k1 = lo ? pr.before() : pr.groups();
+    auto positions = [&](bool lo, int b) {
+      const int k0 = (lo ? 0 : pr.before() + 1) + split + kSplits * NP * b, k1 = lo ? pr.before() : pr.groups();
       const GroupOrder<1> o((s.g & 1) + 2, (s.g >> 1) + 2);
 #pragma unroll
       for (int i = 0; i < NP; i++) {
@@ -964,7 +975,6 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
     T so, se;
     auto add = [&](bool lo) {
       const int d3 = pr.last ? (O == 2 ? 1 : 2) : 3;
-      so = se = 0;
       auto one = [&](int i) {
         const T *q = lx + at[i];
         T r[NX];
@@ -984,35 +994,47 @@ __global__ __launch_bounds__((Plane<T, O>::kThreads)) void k_plane_sweep(WgLevel
         for (int i = H; i < NP; i++) one(i);
       }
     };
-    load(s.sums & kSumLo);
+    // a part whose first batch is loaded
+    auto part = [&](bool lo) {
+      so = se = 0;
+      add(lo);
+      if constexpr (kBatches) {
+        for (int b = 1; kSplits * NP * b < count(lo); b++) {
+          load(lo, b);
+          positions(lo, b);
+          add(lo);
+        }
+      }
+    };
+    load(s.sums & kSumLo, 0);
     stage();
     __syncthreads();
-    positions(s.sums & kSumLo);
+    positions(s.sums & kSumLo, 0);
     for (int i = 1;; i++) {
       const bool more = i < steps.n;
       const PlaneStep<O> sn(steps.code[more ? i : 0], bnd);
       PairSums<T> p{0, 0, 0, 0};
       if (s.sums & kSumLo) {
-        add(true);
+        part(true);
         p.lo_o = so;
         p.lo_e = se;
         if (s.sums & kSumHi) {
-          load(false);
-          positions(false);
+          load(false, 0);
+          positions(false, 0);
         }
       }
       if (s.sums & kSumHi) {
-        add(false);
+        part(false);
         p.hi_o = so;
         p.hi_e = se;
       }
-      red[64 * w + t] = p;
+      red[64 * split + t] = p;
       lds_barrier();
       if (more) {
         s = sn;
         pr = pair_of(s);
-        load(s.sums & kSumLo);
-        positions(s.sums & kSumLo);
+        load(s.sums & kSumLo, 0);
+        positions(s.sums & kSumLo, 0);
       }
       lds_barrier();
       if (!more) break;
@@ -1366,25 +1388,30 @@ static void launch_wg(void (*k)(KA...), int threads, size_t lds, hipStream_t st,
   launch_wg_grid(k, 1, threads, lds, st, a...);
 }
 // ... with a launch per plane colour where the row pairs of a plane's line
-// group fit one wavefront, M <= 17.  (Four wavefronts per split took 33^3 in
-// one tile as well: 67 / 99 us per sweep of Q2, 27.6 / 35 us of Q1, FP32 /
-// FP64, against 74 / 78 and 23 / 24 us by line groups: there a CU reads the
-// values of a plane no faster than the launches go by.)
+// group fit one wavefront, M <= 17
 bool plane_sweeps_fit(const DevLayout &D) {
   const int C = D.order == 2 ? 3 : 2;
   return D.M >= 3 && (((D.M - 3) / C + 1) << D.lg) <= 64;
 }
+// ... with three wavefronts of pairs per plane: Q2, M = 33.  An SSOR sweep takes 54
+// / 76 us (FP32 / FP64) against 74 / 78 us by line groups.  (All groups of a part in
+// flight at once, as at M = 17, does not fit the registers of 15 wavefronts: 63 /
+// 96 us.)  A Q1 sweep has 7 launches by line groups, not 17, and is faster so.
+static bool plane_sweeps_three(const DevLayout &D) {
+  return D.order == 2 && !plane_sweeps_fit(D) && (((D.M - 3) / 3 + 1) << D.lg) <= 192;
+}
+bool plane_sweeps_used(const DevLayout &D) { return plane_sweeps_fit(D) || plane_sweeps_three(D); }
 // ... in one workgroup where the pairs of a line group fit a wavefront, M <= 9
 static bool plane_sweeps_all(const DevLayout &D) {
   const int C = D.order == 2 ? 3 : 2, n = (D.M - 3) / C + 1;
   return (n * n << D.lg) <= 64;
 }
-template <typename T, int O>
+template <typename T, int O, int SL>
 static void plane_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n,
                          bool zero, const int *bnd_set, hipStream_t st) {
   constexpr int C = Lines<O>::C;
-  const bool all = plane_sweeps_all(D);
-  const size_t lds = Plane<T, O>::lds_bytes(D.M, all);
+  const bool all = SL == 1 && plane_sweeps_all(D);
+  const size_t lds = Plane<T, O, SL>::lds_bytes(D.M, all);
   T *ps = ssor ? psum : nullptr;
   WgSweeps<O> it{n, ssor, zero};
   WgStep s;
@@ -1398,19 +1425,20 @@ static void plane_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *
       more = it.next(s);
     } while (more && (all || s.g / C == zr) && steps.n < kPlaneSteps);
     if (all)
-      launch_wg_grid(k_plane_sweep<T, O, true>, 1, Plane<T, O>::kThreads, lds, st, wg_level(D, val), 0, steps, x, f, ps,
+      launch_wg_grid(k_plane_sweep<T, O, true, 1>, 1, Plane<T, O, 1>::kThreads, lds, st, wg_level(D, val), 0, steps, x, f, ps,
                      omega, bnd_set);
     else
-      launch_wg_grid(k_plane_sweep<T, O, false>, (D.M - 2 - z0) / C + 1, Plane<T, O>::kThreads, lds, st,
+      launch_wg_grid(k_plane_sweep<T, O, false, SL>, (D.M - 2 - z0) / C + 1, Plane<T, O, SL>::kThreads, lds, st,
                      wg_level(D, val), z0, steps, x, f, ps, omega, bnd_set);
   }
 }
 template <typename T>
 void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n, bool zero,
                 const int *bnd_set, bool planes, hipStream_t st) {
-  if (planes && plane_sweeps_fit(D) && D.lg >= 1) {  // (3^3: one row)
-    if (D.order == 2) plane_sweeps<T, 2>(D, val, x, f, psum, omega, ssor, n, zero, bnd_set, st);
-    else plane_sweeps<T, 1>(D, val, x, f, psum, omega, ssor, n, zero, bnd_set, st);
+  if (planes && plane_sweeps_used(D) && D.lg >= 1) {  // (3^3: one row)
+    if (D.order == 1) plane_sweeps<T, 1, 1>(D, val, x, f, psum, omega, ssor, n, zero, bnd_set, st);
+    else if (plane_sweeps_fit(D)) plane_sweeps<T, 2, 1>(D, val, x, f, psum, omega, ssor, n, zero, bnd_set, st);
+    else plane_sweeps<T, 2, 3>(D, val, x, f, psum, omega, ssor, n, zero, bnd_set, st);
     return;
   }
   sweeps<T, T>(D, val, nullptr, x, f, psum, omega, ssor, n, zero, bnd_set, st);

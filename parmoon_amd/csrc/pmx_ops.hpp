@@ -97,8 +97,9 @@ void rows_apply(const DevLayout &D, int mode, const T *val, const T *x, const T 
 // interior of x is zero (its contribution is not read); bnd_set (optional,
 // with zero): a device flag that is not 0 if the boundary of x is not zero;
 // planes: a launch per plane colour instead of one per line group where
-// plane_sweeps_fit (the same result bit for bit).
-bool plane_sweeps_fit(const DevLayout &D);
+// plane_sweeps_used (the same result bit for bit).
+bool plane_sweeps_fit(const DevLayout &D);   // M <= 17
+bool plane_sweeps_used(const DevLayout &D);  // and Q2 levels with M = 33
 template <typename T>
 void sor_sweeps(const DevLayout &D, const T *val, T *x, const T *f, T *psum, double omega, bool ssor, int n, bool zero,
                 const int *bnd_set, bool planes, hipStream_t st);

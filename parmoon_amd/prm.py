@@ -135,7 +135,7 @@ def solver_opt(solver=16, restart=20, maxit=200, res_norm_min=1e-10, red_factor=
                bicg_flexible=1, precision=0, rel_target=0.0, inner_red=1e-4, eager=0, learned_levels=0,
                learned_steps=1, wg_sweep_rows=0, learned_skip=0, learned_pre=0):
     """The 24-entry solver option vector; entries 0-15 are shared with the oracle.
-    wg_sweep_rows: small levels (at most 17^3 lattice nodes) whose largest
+    wg_sweep_rows: small levels (at most 17^3 lattice nodes, Q2 33^3) whose largest
     colour has at most this many rows sweep with a workgroup per plane
     (0 = all of them, < 0 = never).
     learned_skip: the finest levels of the learned ones that keep the plain
