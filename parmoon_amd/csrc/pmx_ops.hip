@@ -1402,8 +1402,7 @@ __global__ __launch_bounds__(kMgsWg) void k_mgs_wg(T *__restrict__ w, const T *_
 template <typename T>
 void mgs_arnoldi(T *w, const T *V, int64_t n, int k1, double *h, T *vnext, double *part, hipStream_t st) {
   if (n <= kMgsWgMax) {
-    auto *k = n <= kMgsWg ? k_mgs_wg<T, 1> : n <= 2 * kMgsWg ? k_mgs_wg<T, 2>
-            : n <= 4 * kMgsWg ? k_mgs_wg<T, 4> : k_mgs_wg<T, 8>;
+    auto *k = n <= kMgsWg ? k_mgs_wg<T, 1> : k_mgs_wg<T, 8>;  // (levels have 729 nodes or less, or 4913)
     hipLaunchKernelGGL(k, dim3(1), dim3(kMgsWg), 0, st, w, V, n, k1, h, vnext);
     return;
   }
