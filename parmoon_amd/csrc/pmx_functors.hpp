@@ -42,6 +42,9 @@ __host__ __device__ inline double grf_field(const double *prm, double x, double 
   return s * kGrfScale;
 }
 
+__host__ __device__ inline QpCoeffs rotating_coeffs(double eps, double x, double y) {
+  return QpCoeffs{eps, -(y - 0.5), x - 0.5, 0.2, 0.0, 0.0};
+}
 // the trigonometric factors of the example functions, evaluated where used
 struct PointTrig {
   double x, y, z;
@@ -100,11 +103,7 @@ __host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, 
       k.f = 1.0;
     }
   } else if (ex == PMX_EX_ROTATING) {
-    k.b0 = -(y - 0.5);
-    k.b1 = x - 0.5;
-    k.b2 = 0.2;
-    k.c = 0;
-    k.f = 0.0;
+    k = rotating_coeffs(eps, x, y);
   }
   return k;
 }

@@ -642,13 +642,17 @@ struct AxisTrig {
 // 32, no table of basis values), and the trigonometric factors of the example
 // functions are those of the NP points of each axis.  Level of 8^3 cells,
 // 27 points, sine coefficients: 331 -> 17 us; 128^3, SUPG form of the rotating
-// flow (both matrices): 2.36 -> 1.88 ms.
-template <int NP, bool TWO, bool INL>
+// flow (both matrices): 2.36 -> 1.88 ms (1.65 below).
+// SRC: where the coefficients come from; the rotating flow apart, whose kernel
+// then has no sines and fits more wavefronts (128^3, both matrices: 1.88 -> 1.65 ms)
+enum { kRecords = 0, kInline = 1, kRotating = 2 };
+template <int NP, bool TWO, int SRC>
 __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M, int n,
                                                      const double *__restrict__ prm, const double *__restrict__ qref,
                                                      const double *__restrict__ qp, double *__restrict__ val,
                                                      double *__restrict__ val2, double *__restrict__ rhs) {
   constexpr int NB = 8, R = kRowsPerBlock, NQ = NP * NP * NP;
+  constexpr bool INL = SRC != kRecords;
   __shared__ double sh[(TWO ? 2 : 1) * 8 * NB * R], sf[8 * R];
   const int t = threadIdx.x & (R - 1), j = __builtin_amdgcn_readfirstlane(threadIdx.x / R);
   int px, py, pz;
@@ -673,10 +677,9 @@ __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M,
       fz[i] = iz ? f0[i] : f1[i];
     }
     const double gx = ix ? -0.5 * g : 0.5 * g, gy = iy ? -0.5 * g : 0.5 * g, gz = iz ? -0.5 * g : 0.5 * g;
-    const bool trig = INL && (int)prm[PMX_PRM_EXAMPLE] != PMX_EX_ROTATING;
     auto axis_point = [&](int c, double xi) {
       AxisPoint a{(c * h + 0.5 * h) + 0.5 * h * xi, 0, 0};
-      if (trig) sincospi(a.x, &a.s, &a.c);
+      if (SRC == kInline) sincospi(a.x, &a.s, &a.c);
       return a;
     };
     AxisPoint Z[NP];
@@ -707,7 +710,9 @@ __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M,
           const int q = qx + NP * (qy + NP * qz);
           double Qq[8];
           if (INL) {
-            const QpCoeffs c = example_coeffs<true>(prm, X.x, Y.x, Z[qz].x, AxisTrig{X, Y, Z[qz]});
+            const QpCoeffs c = SRC == kRotating
+                                   ? rotating_coeffs(prm[PMX_PRM_EPS], X.x, Y.x)
+                                   : example_coeffs<true>(prm, X.x, Y.x, Z[qz].x, AxisTrig{X, Y, Z[qz]});
             Qq[0] = qref[4 * q + 3] * (h * h * h / 8.0);
             Qq[1] = c.eps; Qq[2] = c.b0; Qq[3] = c.b1; Qq[4] = c.b2; Qq[5] = c.c; Qq[6] = c.f;
             Qq[7] = dl[qz];
@@ -1156,11 +1161,11 @@ void scale_inv(T *y, const T *x, const double *nrm, int64_t n, hipStream_t st) {
 }
 // The end of a defect r = f - A x: its Dirichlet rows, f - x on the lattice
 // surface, and the norm, one workgroup of BLOCK threads per kDotChunk (up to
-// kDefectSmall: all) elements without a grid-stride loop, so that the number of
+// kDefectSmall, 17^3: all) elements without a grid-stride loop, so that the number of
 // partial sums grows with n; a single workgroup writes the norm itself.
 // Bound by the launches: the surface, the sum and its last step as launches of
 // their own took 5.6 us more at 9^3 (13.6 us per call).
-constexpr int64_t kDefectSmall = 16384;
+constexpr int64_t kDefectSmall = 8 * 1024;
 template <int BLOCK, int PER>
 __global__ __launch_bounds__(BLOCK) void k_defect_norm(int M, double *r, const double *x, const double *f,
                                                        double *__restrict__ part, int64_t n, int last) {
@@ -1170,7 +1175,7 @@ __global__ __launch_bounds__(BLOCK) void k_defect_norm(int M, double *r, const d
 #pragma unroll
   for (int k = 0; k < PER; k++) {
     const int64_t i = base + k * BLOCK + threadIdx.x;
-    if (i >= n) break;
+    if (i >= n) continue;
     const unsigned yz = (unsigned)i / (unsigned)M;
     const int ix = (int)((unsigned)i - yz * M), iy = (int)(yz % (unsigned)M), iz = (int)(yz / (unsigned)M);
     double v;
@@ -1191,7 +1196,8 @@ void defect_norm(const DevLayout &D, double *r, const double *x, const double *f
                  hipStream_t st) {
   const int64_t n = D.N, nb = (n + kDotChunk - 1) / kDotChunk;
   if (n <= kDefectSmall) {
-    hipLaunchKernelGGL((k_defect_norm<1024, kDefectSmall / 1024>), dim3(1), dim3(1024), 0, st, D.M, r, x, f, out, n, 1);
+    auto *k = n <= 1024 ? k_defect_norm<1024, 1> : k_defect_norm<1024, kDefectSmall / 1024>;
+    hipLaunchKernelGGL(k, dim3(1), dim3(1024), 0, st, D.M, r, x, f, out, n, 1);
     return;
   }
   hipLaunchKernelGGL((k_defect_norm<kBlock, kDotChunk / kBlock>), dim3((unsigned)nb), dim3(kBlock), 0, st, D.M, r, x, f,
@@ -1912,34 +1918,33 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
     check(hipMemsetAsync(val, 0, sizeof(double) * D.nvals, st), "memset val");
     if (val2) check(hipMemsetAsync(val2, 0, sizeof(double) * D.nvals, st), "memset val2");
   }
-#define PMX_ASM2(TW)                                                                                               \
-  do {                                                                                                             \
-    if (inl) PMX_ASM(TW, true);                                                                                    \
-    else PMX_ASM(TW, false);                                                                                       \
-  } while (0)
   if (D.order == 1) {
-#define PMX_ASM3(NP, TW, IN)                                                                                       \
-  hipLaunchKernelGGL((k_assemble_q1<NP, TW, IN>), gr, dim3(8 * kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, prm_dev, \
+#define PMX_ASM3(NP, TW, SRC)                                                                                      \
+  hipLaunchKernelGGL((k_assemble_q1<NP, TW, SRC>), gr, dim3(8 * kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, prm_dev, \
                      qref, qsrc, val, val2, rhs)
-#define PMX_ASM(TW, IN)                                                                                            \
+#define PMX_ASM(NP, TW)                                                                                            \
   do {                                                                                                             \
-    if (nq == 8) PMX_ASM3(2, TW, IN);                                                                              \
-    else PMX_ASM3(3, TW, IN);                                                                                      \
+    if (!inl) PMX_ASM3(NP, TW, kRecords);                                                                          \
+    else if (example == PMX_EX_ROTATING) PMX_ASM3(NP, TW, kRotating);                                              \
+    else PMX_ASM3(NP, TW, kInline);                                                                                \
   } while (0)
     if (nq != 8 && nq != 27) throw std::logic_error("assemble: no Q1 kernel for the rule");
-    if (val2) PMX_ASM2(true);
-    else PMX_ASM2(false);
+    if (nq == 8 && val2) PMX_ASM(2, true);
+    else if (nq == 8) PMX_ASM(2, false);
+    else if (val2) PMX_ASM(3, true);
+    else PMX_ASM(3, false);
 #undef PMX_ASM
 #undef PMX_ASM3
   } else {
 #define PMX_ASM(TW, IN)                                                                                            \
   hipLaunchKernelGGL((k_assemble<2, TW, IN, false>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq,      \
                      prm_dev, qref, qsrc, tab, val, val2, rhs)
-    if (val2) PMX_ASM2(true);
-    else PMX_ASM2(false);
+    if (val2 && inl) PMX_ASM(true, true);
+    else if (val2) PMX_ASM(true, false);
+    else if (inl) PMX_ASM(false, true);
+    else PMX_ASM(false, false);
 #undef PMX_ASM
   }
-#undef PMX_ASM2
   hipLaunchKernelGGL(k_boundary_rhs, dim3((D.nboundary + kBlock - 1) / kBlock), dim3(kBlock), 0, st, D.boundary,
                      D.nboundary, D.M, prm_dev, rhs);
 }
