@@ -43,10 +43,9 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0      # MI355X HBM3E, GB/s
 FP64_PEAK_TFLOPS = 78.6    # MI355X FP64 (vector = MFMA), TFLOP/s
 BF16_PEAK_TFLOPS = 2500.0  # MI355X dense BF16 MFMA, TFLOP/s
-# HBM bytes per dispatch at 64^3 Q2 from hardware counters (None: not counted
-# for the current kernels)
-TRAFFIC_SSOR_LAUNCH = None  # k_line_sweep<float, float, 2>, one line group (average over the sweeps)
-TRAFFIC_SPMV = None  # k_line_rows<float, 2, 0>
+# HBM bytes per dispatch at 64^3 Q2 from hardware counters (tests/cpp/kernel_probe)
+TRAFFIC_SSOR_LAUNCH = 58661990  # k_line_sweep<float, float, 2>, one line group (average over the sweeps)
+TRAFFIC_SPMV = 547418214  # k_line_rows<float, 2, 0>
 
 
 def cpu_info():
@@ -391,14 +390,15 @@ def main():
                      "rel_res": float(infos[-1][1] / infos[-1][2]), "rc": int(rc)}
 
     # Rooflines on the finest level.  Algorithmic bytes are the bytes the
-    # colour-sliced stencil format has to move (values are stored without
-    # column indices; x counted once per launch, every launch gathers from
-    # all of it):
+    # line layout has to move (values are stored without column indices; x
+    # counted once per launch, every launch gathers from all of it):
     #   SpMV:                 stored values s_v + x (N s_v) + y of the active rows
-    #   SSOR group launch:    the group's values + x (N s_v) + f read and x
-    #                         written for the group's rows; one launch = one of
-    #                         the 9 line groups (3 colours each), forward or
-    #                         backward
+    #   SSOR group launch:    average over the 2 * 9 - 1 launches of a sweep of
+    #                         the 9 line groups (3 colours each): all values once
+    #                         forward, the half after a line and its own group (1
+    #                         of 16) backward, x (N s_v), and of the rows f, x and
+    #                         the kept sums written forward, f, x and the sums read
+    #                         and written backward
     # Durations are those of the single dispatches (events recorded by the
     # dispatch, pmx_time_kernel 10 / 11), not of back-to-back launch sequences.
     nvals = int(d[6])
@@ -410,7 +410,7 @@ def main():
         ms_spmv = S.time_kernel(11, -1, prec, reps=20)
         ms_col = S.time_kernel(10, -1, prec, reps=4)
         b_spmv = nvals * sv + N * sv + nact * sv
-        b_col = nvals * sv / ngrp + N * sv + 2 * nact * sv / ngrp
+        b_col = (nvals * (1.5 + 0.5 / 16) + 7 * nact) * sv / (2 * ngrp - 1) + N * sv
         roof[prec] = {"spmv_ms": ms_spmv, "spmv_bytes": b_spmv, "col_ms": ms_col, "col_bytes": b_col}
     # calibration of the group launch on the same level and with the same
     # dispatch events: a dispatch that does nothing (its workgroup counts) and
@@ -539,9 +539,10 @@ def main():
                           "frac": round(spmv_gbs / HBM_PEAK_GBS, 4), "traffic": TRAFFIC_SPMV,
                           "algorithmic_bytes": int(r32["spmv_bytes"]), "dispatch_ms": round(r32["spmv_ms"], 5),
                           "fp64_GBs": round(roof[0]["spmv_bytes"] / (roof[0]["spmv_ms"] * 1e-3) / 1e9, 1)},
-        # Q2 assembly of the finest level against the FP64 peak (B^T D B model:
-        # 47.4 GFLOP with the 27-point rule, 112.3 GFLOP with the 64-point rule)
-        "roofline_assembly": {"bound": "mfma", "kernel": "k_qp_data + k_cell_mfma + k_assemble_kc (finest level)",
+        # Q2 assembly of the finest level against the FP64 peak (operations of the
+        # plain sum B^T D B: 47.4 GFLOP with the 27-point rule, 112.3 GFLOP with the
+        # 64-point rule; k_cell_sum takes a fifth of them)
+        "roofline_assembly": {"bound": "fp64", "kernel": "k_qp_data + k_cell_sum + k_assemble_kc (finest level)",
                               "achieved": round(asm_tf, 2), "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                               "frac": round(asm_tf / FP64_PEAK_TFLOPS, 4),
                               "gauss4_achieved": round(asm4_tf, 2),

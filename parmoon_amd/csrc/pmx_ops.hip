@@ -440,7 +440,7 @@ __host__ __device__ inline bool coeffs_inline(int example) {
 //   K_ab = sum_q w [ u0 phi_b + u . grad phi_b ]
 // with s_a = phi_a + delta b.grad phi_a, u0 = c s_a, u = eps grad phi_a + b s_a
 // (BilinearAssemble / _SD, ConvDiff3D.C:118-145,182-213; mass and TCD forms,
-// TCD3D.C:37-322), and adds it into its own CSS row.  No two threads write
+// TCD3D.C:37-322), and adds it into its own row of values.  No two threads write
 // the same row, so no atomics and no colouring of cells are needed, and the
 // writes of a wavefront are coalesced.
 // The incident cells per direction are compile-time (a Q2 node with an odd
@@ -545,7 +545,7 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
           }
         }
         if (RONLY) continue;
-        // add the row into the CSS slots of node p
+        // add the row into the value slots of node p
 #pragma unroll
         for (int b = 0; b < NB; b++) {
           const int bx = b % K, by = (b / K) % K, bz = b / (K * K);
@@ -1724,7 +1724,7 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_sum(int n, int form, cons
   }
 }
 // Row gather from the cell buffer: the thread of active node p adds row a of
-// each incident cell's local matrix into its CSS row and sums the rhs column.
+// each incident cell's local matrix into its row of values and sums the rhs column.
 // The row's stencil slots are accumulated in registers over its incident
 // cells (in the order (iz, iy, ix)) and every slot is stored once, after the
 // last cell that touches it (a slot (dx, dy, dz) gets its last contribution
