@@ -159,6 +159,12 @@ __host__ __device__ inline void example_exact_grad(const double *prm, double x, 
   }
 }
 
+// coth(a) as 1 / tanh(a), whose tanh rounds to 1 in FP64 from a = 19.1 on (1 -
+// tanh a < 2 exp(-2 a) < 2^-54): the same bits without the hyperbolic tangent
+// and its reciprocal where convection dominates, which is where a
+// stabilisation parameter is used
+__host__ __device__ inline double coth_fp64(double a) { return a > 20.0 ? 1.0 : 1 / tanh(a); }
+
 // Compute_SDFEM_delta for SDFEM_TYPE 0/1/2 with CELL_MEASURE 0
 __host__ __device__ inline double sdfem_delta(const double *prm, double hK, double eps, double b1, double b2,
                                               double b3) {
@@ -174,7 +180,7 @@ __host__ __device__ inline double sdfem_delta(const double *prm, double hK, doub
     const double nu = 1.0 / pd;
     if (nb > 0) {
       const double alpha = nu * nb * hK / (2 * eps);
-      delta = nu * hK * (1 / tanh(alpha) - 1 / alpha) / (2 * nb);
+      delta = nu * hK * (coth_fp64(alpha) - 1 / alpha) / (2 * nb);
     }
     delta *= delta0;
   }
@@ -190,7 +196,7 @@ __host__ __device__ inline double rhs_supg_tau(double hK, double eps, double b1,
   const double bb = sqrt(b1 * b1 + b2 * b2 + b3 * b3);
   if (!(bb > 0)) return 0.0;
   const double pe = hK * bb / (2 * eps);
-  const double tau = pe < 1e-2 ? pe / (6 * bb) : (1 / tanh(pe) - 1 / pe) / (2 * bb);
+  const double tau = pe < 1e-2 ? pe / (6 * bb) : (coth_fp64(pe) - 1 / pe) / (2 * bb);
   return tau * hK;
 }
 

@@ -107,6 +107,23 @@ def test_entries_match_the_oracle(ctx, order, nref, example, linear):
     S.close()
 
 
+@pytest.mark.parametrize("order,alpha", [(1, 0.02), (1, 19.0), (1, 20.0 - 1e-9), (1, 20.0 + 1e-9), (2, 22.0),
+                                         (1, 1e9)])
+def test_streamline_parameter_around_its_limit(ctx, order, alpha):
+    """delta = (coth a - 1/a) hK / (2 |b|) with the local Peclet number a on both
+    sides of the value from which coth a is 1 in FP64."""
+    print(f"[case] streamline parameter, order {order} alpha {alpha}", flush=True)
+    blk = P.config1b()
+    nu = 1.0 / (blk[P.POLYDEG] if blk[P.POLYDEG] > 0 else 1.0)
+    blk[P.EPS] = nu * np.linalg.norm(blk[P.B0:P.B2 + 1]) * np.sqrt(3.0) / 8 / (2 * alpha)
+    S, O = pa.System(ctx, 3, 1, order), orc.System(3, 1, order)
+    S.assemble(blk)
+    O.assemble(blk)
+    assert rel(S.entries(), O.entries()) < 1e-12
+    assert rel(S.rhs(), O.rhs()) < 1e-12
+    S.close()
+
+
 @pytest.mark.parametrize("order,nref", [(1, 1), (1, 2), (1, 3), (2, 2), (1, 4)])
 def test_exact_coarse_solve(ctx, order, nref):
     """One level: the cycle is the explicit inverse (1, 27, 343, 343 and 3375
