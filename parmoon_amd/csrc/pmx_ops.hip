@@ -645,6 +645,11 @@ struct AxisTrig {
 // flow (both matrices): 2.36 -> 1.88 ms (1.65 below).
 // SRC: where the coefficients come from; the rotating flow apart, whose kernel
 // then has no sines and fits more wavefronts (128^3, both matrices: 1.88 -> 1.65 ms)
+// A workgroup has two wavefronts per SIMD, so a second one on the CU (68 KB of
+// LDS with both matrices) needs at most 128 registers: a thread's sums over the
+// points along x are kept in LDS, where they are needed at the end, and the
+// points along z are a loop (174 -> 118 registers; three steps of the rotating
+// transient at 128^3 together with the cheaper parameter of k_qp_delta 66.1 -> 63.6 ms).
 enum { kRecords = 0, kInline = 1, kRotating = 2 };
 template <int NP, bool TWO, int SRC>
 __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M, int n,
@@ -653,6 +658,7 @@ __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M,
                                                      double *__restrict__ val2, double *__restrict__ rhs) {
   constexpr int NB = 8, R = kRowsPerBlock, NQ = NP * NP * NP;
   constexpr bool INL = SRC != kRecords;
+  constexpr int kUnrollZ = SRC == kInline ? NP : 1;
   __shared__ double sh[(TWO ? 2 : 1) * 8 * NB * R], sf[8 * R];
   const int t = threadIdx.x & (R - 1), j = __builtin_amdgcn_readfirstlane(threadIdx.x / R);
   int px, py, pz;
@@ -666,28 +672,21 @@ __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M,
     const int64_t cell = cx + (int64_t)n * (cy + (int64_t)n * cz), ncell = (int64_t)n * n * n;
     const double *Q = qp + cell * NQ * 8;
     const double h = 1.0 / n, g = 2.0 * n;  // reference -> physical derivative factor 2/h
-    // basis functions of an axis at its points; the row's one along the axes
-    // and the derivatives -1/2, 1/2
-    double f0[NP], f1[NP], fz[NP];
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-      const double xi = qref[4 * i];
-      f0[i] = uniform(0.5 * (1 - xi));
-      f1[i] = uniform(0.5 * (1 + xi));
-      fz[i] = iz ? f0[i] : f1[i];
-    }
+    // (the basis functions of an axis have the derivatives -1/2, 1/2)
     const double gx = ix ? -0.5 * g : 0.5 * g, gy = iy ? -0.5 * g : 0.5 * g, gz = iz ? -0.5 * g : 0.5 * g;
     auto axis_point = [&](int c, double xi) {
       AxisPoint a{(c * h + 0.5 * h) + 0.5 * h * xi, 0, 0};
       if (SRC == kInline) sincospi(a.x, &a.s, &a.c);
       return a;
     };
-    AxisPoint Z[NP];
+    AxisPoint Z[SRC == kInline ? NP : 1];
+    if constexpr (SRC == kInline) {
 #pragma unroll
-    for (int i = 0; i < NP; i++) Z[i] = INL ? axis_point(cz, qref[4 * i]) : AxisPoint{0, 0, 0};
-    double acc[NB], acc2[NB], frhs = 0;
-#pragma unroll
-    for (int b = 0; b < NB; b++) acc[b] = acc2[b] = 0;
+      for (int i = 0; i < NP; i++) Z[i] = axis_point(cz, qref[4 * i]);
+    } else {
+      Z[0] = AxisPoint{0, 0, 0};  // (not read)
+    }
+    double *acc = sh + j * NB * R + t, *acc2 = acc + 8 * NB * R, frhs = 0;  // this thread's: no barrier
     // inline coefficients: qp holds the per-point stabilisation parameters of
     // k_qp_delta (nullptr for the forms without one)
 #pragma unroll 1
@@ -705,32 +704,36 @@ __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M,
         for (int qz = 0; qz < NP; qz++)
           dl[qz] = (INL && qp) ? qp[(qx + NP * (qy + NP * qz)) * ncell + cell] : 0.0;
         double a[2] = {0, 0}, ax[2] = {0, 0}, ay[2] = {0, 0}, a2[2] = {0, 0};  // bz
-#pragma unroll
+#pragma unroll kUnrollZ
         for (int qz = 0; qz < NP; qz++) {
           const int q = qx + NP * (qy + NP * qz);
+          const double zi = qref[4 * qz], z0 = uniform(0.5 * (1 - zi)), z1 = uniform(0.5 * (1 + zi)), fz = iz ? z0 : z1;
           double Qq[8];
           if (INL) {
             const QpCoeffs c = SRC == kRotating
                                    ? rotating_coeffs(prm[PMX_PRM_EPS], X.x, Y.x)
-                                   : example_coeffs<true>(prm, X.x, Y.x, Z[qz].x, AxisTrig{X, Y, Z[qz]});
+                                   : example_coeffs<true>(prm, X.x, Y.x, Z[SRC == kInline ? qz : 0].x,
+                                                          AxisTrig{X, Y, Z[SRC == kInline ? qz : 0]});
             Qq[0] = qref[4 * q + 3] * (h * h * h / 8.0);
             Qq[1] = c.eps; Qq[2] = c.b0; Qq[3] = c.b1; Qq[4] = c.b2; Qq[5] = c.c; Qq[6] = c.f;
-            Qq[7] = dl[qz];
+            Qq[7] = dl[0];
+#pragma unroll
+            for (int i = 0; i + 1 < NP; i++) dl[i] = dl[i + 1];
           } else {
 #pragma unroll
             for (int e = 0; e < 8; e++) Qq[e] = Q[8 * q + e];
           }
-          const RowPoint r = row_point(Qq, fxy * fz[qz], gxy * fz[qz], gyx * fz[qz], gzxy, form, g);
+          const RowPoint r = row_point(Qq, fxy * fz, gxy * fz, gyx * fz, gzxy, form, g);
           frhs += r.f;
-          a[0] = fma(r.u0, f0[qz], fma(r.uz, -0.5, a[0]));
-          a[1] = fma(r.u0, f1[qz], fma(r.uz, 0.5, a[1]));
-          ax[0] = fma(r.ux, f0[qz], ax[0]);
-          ax[1] = fma(r.ux, f1[qz], ax[1]);
-          ay[0] = fma(r.uy, f0[qz], ay[0]);
-          ay[1] = fma(r.uy, f1[qz], ay[1]);
+          a[0] = fma(r.u0, z0, fma(r.uz, -0.5, a[0]));
+          a[1] = fma(r.u0, z1, fma(r.uz, 0.5, a[1]));
+          ax[0] = fma(r.ux, z0, ax[0]);
+          ax[1] = fma(r.ux, z1, ax[1]);
+          ay[0] = fma(r.uy, z0, ay[0]);
+          ay[1] = fma(r.uy, z1, ay[1]);
           if (TWO) {
-            a2[0] = fma(r.k0, f0[qz], a2[0]);
-            a2[1] = fma(r.k0, f1[qz], a2[1]);
+            a2[0] = fma(r.k0, z0, a2[0]);
+            a2[1] = fma(r.k0, z1, a2[1]);
           }
         }
 #pragma unroll
@@ -747,18 +750,15 @@ __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M,
       }
 #pragma unroll
       for (int b = 0; b < 4; b++) {
-        acc[2 * b] = fma(p[b], x0, fma(d[b], -0.5, acc[2 * b]));
-        acc[2 * b + 1] = fma(p[b], x1, fma(d[b], 0.5, acc[2 * b + 1]));
+        double *o = acc + 2 * b * R, *o2 = acc2 + 2 * b * R;
+        o[0] = fma(p[b], x0, fma(d[b], -0.5, qx ? o[0] : 0.0));
+        o[R] = fma(p[b], x1, fma(d[b], 0.5, qx ? o[R] : 0.0));
         if (TWO) {
-          acc2[2 * b] = fma(p2[b], x0, acc2[2 * b]);
-          acc2[2 * b + 1] = fma(p2[b], x1, acc2[2 * b + 1]);
+          o2[0] = fma(p2[b], x0, qx ? o2[0] : 0.0);
+          o2[R] = fma(p2[b], x1, qx ? o2[R] : 0.0);
         }
       }
-    }
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-      sh[(j * NB + b) * R + t] = acc[b];
-      if (TWO) sh[((8 + j) * NB + b) * R + t] = acc2[b];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the compiler would keep the sums in registers)
     }
     sf[j * R + t] = frhs;
   }
