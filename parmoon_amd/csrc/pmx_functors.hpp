@@ -45,23 +45,39 @@ __host__ __device__ inline double grf_field(const double *prm, double x, double 
 __host__ __device__ inline QpCoeffs rotating_coeffs(double eps, double x, double y) {
   return QpCoeffs{eps, -(y - 0.5), x - 0.5, 0.2, 0.0, 0.0};
 }
-// the trigonometric factors of the example functions, evaluated where used
-struct PointTrig {
-  double x, y, z;
-  static constexpr double pi = 3.14159265358979323846;
-  __host__ __device__ double sx() const { return sin(pi * x); }
-  __host__ __device__ double sy() const { return sin(pi * y); }
-  __host__ __device__ double sz() const { return sin(pi * z); }
-  __host__ __device__ double cx() const { return cos(pi * x); }
-  __host__ __device__ double cy() const { return cos(pi * y); }
-  __host__ __device__ double cz() const { return cos(pi * z); }
+// The examples with constant eps, b and c, whose source is a sum of products of
+// sin(pi x) (s) and cos(pi x) (c) of the three coordinates: the factors of the
+// products, in the order x, y, z.  The same functions as in example_coeffs.
+struct SineCoeffs {
+  double eps, b0, b1, b2, c;
+  double sss, css, scs, ssc, scc;
 };
+__host__ __device__ inline SineCoeffs sine_coeffs(const double *prm) {
+  const double pi = 3.14159265358979323846;
+  const int ex = (int)prm[PMX_PRM_EXAMPLE];
+  SineCoeffs k{prm[PMX_PRM_EPS], prm[PMX_PRM_B0], prm[PMX_PRM_B1], prm[PMX_PRM_B2], prm[PMX_PRM_C], 0, 0, 0, 0, 0};
+  if (ex == PMX_EX_SINE_CD) {
+    k.sss = 3 * pi * pi * k.eps + k.c;
+    k.css = pi * k.b0;
+    k.scs = pi * k.b1;
+    k.ssc = pi * k.b2;
+  } else if (ex == PMX_EX_LAPLACE || ex == PMX_EX_HEAT_AMC) {
+    k.b0 = k.b1 = k.b2 = k.c = 0;
+    if (ex == PMX_EX_LAPLACE) {
+      k.sss = 3 * pi * pi * k.eps;
+    } else {
+      k.eps = 1.0;
+      k.scc = (3. * pi * pi - 0.1) * exp(-0.1 * prm[PMX_PRM_TIME]);
+    }
+  }
+  return k;
+}
 // CHEAP = true: only the examples whose coefficients are evaluated inline
 // at every point (Laplace, sine, heat, rotating); the curl-Fourier and
 // lognormal branches, which kernels for the inline examples never take, are
 // left out of the code so they do not weigh on its registers
-template <bool CHEAP, class Trig>
-__host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, double y, double z, const Trig &tr) {
+template <bool CHEAP = false>
+__host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, double y, double z) {
   const double pi = 3.14159265358979323846;
   QpCoeffs k;
   const int ex = (int)prm[PMX_PRM_EXAMPLE];
@@ -76,10 +92,10 @@ __host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, 
   if (ex == PMX_EX_LAPLACE) {
     k.b0 = k.b1 = k.b2 = 0;
     k.c = 0;
-    k.f = 3 * pi * pi * eps * tr.sx() * tr.sy() * tr.sz();
+    k.f = 3 * pi * pi * eps * sin(pi * x) * sin(pi * y) * sin(pi * z);
   } else if (ex == PMX_EX_SINE_CD) {
-    const double sx = tr.sx(), sy = tr.sy(), sz = tr.sz();
-    const double cx = tr.cx(), cy = tr.cy(), cz = tr.cz();
+    const double sx = sin(pi * x), sy = sin(pi * y), sz = sin(pi * z);
+    const double cx = cos(pi * x), cy = cos(pi * y), cz = cos(pi * z);
     const double u = sx * sy * sz;
     k.f = 3 * pi * pi * eps * u + pi * (k.b0 * cx * sy * sz + k.b1 * sx * cy * sz + k.b2 * sx * sy * cz) + k.c * u;
   } else if (!CHEAP && ex == PMX_EX_CURL_FOURIER) {
@@ -96,7 +112,7 @@ __host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, 
     k.eps = 1.0;
     k.b0 = k.b1 = k.b2 = 0;
     k.c = 0;
-    k.f = (3. * pi * pi - 0.1) * exp(-0.1 * t) * tr.sx() * tr.cy() * tr.cz();
+    k.f = (3. * pi * pi - 0.1) * exp(-0.1 * t) * sin(pi * x) * cos(pi * y) * cos(pi * z);
   } else if (!CHEAP && ex == PMX_EX_LOGNORMAL) {
     if constexpr (!CHEAP) {
       k.eps = eps * exp(prm[PMX_PRM_GRF_SIGMA] * grf_field(prm, x, y, z));
@@ -106,11 +122,6 @@ __host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, 
     k = rotating_coeffs(eps, x, y);
   }
   return k;
-}
-
-template <bool CHEAP = false>
-__host__ __device__ inline QpCoeffs example_coeffs(const double *prm, double x, double y, double z) {
-  return example_coeffs<CHEAP>(prm, x, y, z, PointTrig{x, y, z});
 }
 
 __host__ __device__ inline double example_bound_value(const double *prm, double x, double y, double z) {

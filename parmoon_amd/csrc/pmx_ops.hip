@@ -617,18 +617,8 @@ __device__ __forceinline__ double uniform(double v) {
   const unsigned lo = __builtin_amdgcn_readfirstlane((int)(unsigned)u), hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
   return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
-// the factors of the example functions from those of the points' coordinates
 struct AxisPoint {
   double x, s, c;  // coordinate, sin(pi x), cos(pi x)
-};
-struct AxisTrig {
-  const AxisPoint &X, &Y, &Z;
-  __device__ __forceinline__ double sx() const { return X.s; }
-  __device__ __forceinline__ double sy() const { return Y.s; }
-  __device__ __forceinline__ double sz() const { return Z.s; }
-  __device__ __forceinline__ double cx() const { return X.c; }
-  __device__ __forceinline__ double cy() const { return Y.c; }
-  __device__ __forceinline__ double cz() const { return Z.c; }
 };
 // Q1 rows with matrices: a workgroup takes the 64 rows of unit_row, its
 // wavefront j the j-th of the rows' 8 cells (ix + 2 iy + 4 iz); the cells'
@@ -638,27 +628,27 @@ struct AxisTrig {
 // Bound by the FP64 operations of the points and, on small levels, by the
 // chain of a thread, which is 8 times shorter than with all cells of a row on
 // one thread.  The rule and the basis are tensor products (NP points per
-// axis), so a row is summed axis by axis (14 products per point instead of
-// 32, no table of basis values), and the trigonometric factors of the example
-// functions are those of the NP points of each axis.  Level of 8^3 cells,
-// 27 points, sine coefficients: 331 -> 17 us; 128^3, SUPG form of the rotating
-// flow (both matrices): 2.36 -> 1.88 ms (1.65 below).
-// SRC: where the coefficients come from; the rotating flow apart, whose kernel
-// then has no sines and fits more wavefronts (128^3, both matrices: 1.88 -> 1.65 ms)
+// axis), so a row is summed axis by axis (14 products per point instead of 32,
+// no table of basis values).
+// SRC: where the coefficients come from.  kInline: constant coefficients and a
+// source of sines and cosines, two products per point from the factors of the
+// axes (sine_coeffs); the rotating flow has a kernel without them.
 // A workgroup has two wavefronts per SIMD, so a second one on the CU (68 KB of
 // LDS with both matrices) needs at most 128 registers: a thread's sums over the
 // points along x are kept in LDS, where they are needed at the end, and the
-// points along z are a loop (174 -> 118 registers; three steps of the rotating
-// transient at 128^3 together with the cheaper parameter of k_qp_delta 66.1 -> 63.6 ms).
+// points along z are a loop (rotating flow, both matrices 174 -> 118 registers;
+// inline source 223 -> 126; both matrices with it take 148 and stay at one).
+// 128^3, rotating flow: both matrices 2.36 -> 1.70 -> 1.29 ms (a row per thread,
+// axis by axis, two workgroups), one 1.43 -> 1.10 ms.  8^3 and 16^3 cells, inline
+// source: 331 -> 19.9 -> 17.2 us.
 enum { kRecords = 0, kInline = 1, kRotating = 2 };
 template <int NP, bool TWO, int SRC>
-__global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M, int n,
-                                                     const double *__restrict__ prm, const double *__restrict__ qref,
-                                                     const double *__restrict__ qp, double *__restrict__ val,
-                                                     double *__restrict__ val2, double *__restrict__ rhs) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TWO && SRC == kInline ? 2 : 4)))
+void k_assemble_q1(LineSet set, int lg, int M, int n, const double *__restrict__ prm, const double *__restrict__ qref,
+                   const double *__restrict__ qp, double *__restrict__ val, double *__restrict__ val2,
+                   double *__restrict__ rhs) {
   constexpr int NB = 8, R = kRowsPerBlock, NQ = NP * NP * NP;
   constexpr bool INL = SRC != kRecords;
-  constexpr int kUnrollZ = SRC == kInline ? NP : 1;
   __shared__ double sh[(TWO ? 2 : 1) * 8 * NB * R], sf[8 * R];
   const int t = threadIdx.x & (R - 1), j = __builtin_amdgcn_readfirstlane(threadIdx.x / R);
   int px, py, pz;
@@ -679,12 +669,19 @@ __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M,
       if (SRC == kInline) sincospi(a.x, &a.s, &a.c);
       return a;
     };
-    AxisPoint Z[SRC == kInline ? NP : 1];
-    if constexpr (SRC == kInline) {
+    // kInline: constant coefficients and the factors of the source's terms; the
+    // lines of a workgroup lie in one plane, so all of this is uniform
+    SineCoeffs sc{};
+    double zs[NP], zc[NP];
+    if (SRC == kInline) {
+      sc = sine_coeffs(prm);
+      for (double *v : {&sc.sss, &sc.css, &sc.scs, &sc.ssc, &sc.scc}) *v = uniform(*v);
+    }
 #pragma unroll
-      for (int i = 0; i < NP; i++) Z[i] = axis_point(cz, qref[4 * i]);
-    } else {
-      Z[0] = AxisPoint{0, 0, 0};  // (not read)
+    for (int i = 0; i < NP; i++) {
+      const AxisPoint Z = SRC == kInline ? axis_point(cz, qref[4 * i]) : AxisPoint{0, 0, 0};
+      zs[i] = uniform(Z.s);
+      zc[i] = uniform(Z.c);
     }
     double *acc = sh + j * NB * R + t, *acc2 = acc + 8 * NB * R, frhs = 0;  // this thread's: no barrier
     // inline coefficients: qp holds the per-point stabilisation parameters of
@@ -698,22 +695,30 @@ __global__ __launch_bounds__(512) void k_assemble_q1(LineSet set, int lg, int M,
       for (int qy = 0; qy < NP; qy++) {
         const double yi = qref[4 * qy], y0 = uniform(0.5 * (1 - yi)), y1 = uniform(0.5 * (1 + yi)), fy = iy ? y0 : y1;
         const AxisPoint Y = INL ? axis_point(cy, yi) : AxisPoint{0, 0, 0};
+        const double fs = (sc.sss * X.s + sc.css * X.c) * Y.s + sc.scs * X.s * Y.c;
+        const double fc = X.s * (sc.ssc * Y.s + sc.scc * Y.c);
         const double gxy = gx * fy, gyx = gy * fx, gzxy = gz * (fx * fy), fxy = fx * fy;
         double dl[NP];
 #pragma unroll
         for (int qz = 0; qz < NP; qz++)
           dl[qz] = (INL && qp) ? qp[(qx + NP * (qy + NP * qz)) * ncell + cell] : 0.0;
         double a[2] = {0, 0}, ax[2] = {0, 0}, ay[2] = {0, 0}, a2[2] = {0, 0};  // bz
-#pragma unroll kUnrollZ
+#pragma unroll 1
         for (int qz = 0; qz < NP; qz++) {
           const int q = qx + NP * (qy + NP * qz);
           const double zi = qref[4 * qz], z0 = uniform(0.5 * (1 - zi)), z1 = uniform(0.5 * (1 + zi)), fz = iz ? z0 : z1;
           double Qq[8];
           if (INL) {
-            const QpCoeffs c = SRC == kRotating
-                                   ? rotating_coeffs(prm[PMX_PRM_EPS], X.x, Y.x)
-                                   : example_coeffs<true>(prm, X.x, Y.x, Z[SRC == kInline ? qz : 0].x,
-                                                          AxisTrig{X, Y, Z[SRC == kInline ? qz : 0]});
+            QpCoeffs c;
+            if constexpr (SRC == kRotating) c = rotating_coeffs(prm[PMX_PRM_EPS], X.x, Y.x);
+            else c = QpCoeffs{sc.eps, sc.b0, sc.b1, sc.b2, sc.c, fs * zs[0] + fc * zc[0]};
+            // (the next point's to the front; back in order after NP turns)
+            const double zs0 = zs[0], zc0 = zc[0];
+#pragma unroll
+            for (int i = 0; i < NP; i++) {
+              zs[i] = i + 1 < NP ? zs[i + 1] : zs0;
+              zc[i] = i + 1 < NP ? zc[i + 1] : zc0;
+            }
             Qq[0] = qref[4 * q + 3] * (h * h * h / 8.0);
             Qq[1] = c.eps; Qq[2] = c.b0; Qq[3] = c.b1; Qq[4] = c.b2; Qq[5] = c.c; Qq[6] = c.f;
             Qq[7] = dl[0];
@@ -1171,16 +1176,27 @@ __global__ __launch_bounds__(BLOCK) void k_defect_norm(int M, double *r, const d
                                                        double *__restrict__ part, int64_t n, int last) {
   __shared__ double sh[BLOCK / 64];
   const int64_t base = (int64_t)blockIdx.x * (BLOCK * PER);
+  // all loads are issued before the first is used (a branch around each would
+  // wait for it): a lane of an interior row reads r in the place of f and x
+  double a[PER], b[PER];
+  bool surface[PER];
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    const int64_t j = base + k * BLOCK + threadIdx.x, i = j < n ? j : n - 1;
+    const unsigned yz = (unsigned)i / (unsigned)M;
+    const int ix = (int)((unsigned)i - yz * M), iy = (int)(yz % (unsigned)M), iz = (int)(yz / (unsigned)M);
+    surface[k] = ix == 0 || iy == 0 || iz == 0 || ix == M - 1 || iy == M - 1 || iz == M - 1;
+    const double *pa = surface[k] ? f : r, *pb = surface[k] ? x : r;
+    a[k] = pa[i];
+    b[k] = pb[i];
+  }
   double s = 0;
 #pragma unroll
   for (int k = 0; k < PER; k++) {
     const int64_t i = base + k * BLOCK + threadIdx.x;
+    const double v = surface[k] ? a[k] - b[k] : a[k];
     if (i >= n) continue;
-    const unsigned yz = (unsigned)i / (unsigned)M;
-    const int ix = (int)((unsigned)i - yz * M), iy = (int)(yz % (unsigned)M), iz = (int)(yz / (unsigned)M);
-    double v;
-    if (ix == 0 || iy == 0 || iz == 0 || ix == M - 1 || iy == M - 1 || iz == M - 1) r[i] = v = f[i] - x[i];
-    else v = r[i];
+    if (surface[k]) r[i] = v;
     s += v * v;
   }
   for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);

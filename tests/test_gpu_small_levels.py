@@ -107,6 +107,45 @@ def test_entries_match_the_oracle(ctx, order, nref, example, linear):
     S.close()
 
 
+@pytest.mark.parametrize("nref", [1, 3, 5])
+@pytest.mark.parametrize("example,linear", [("laplace", True), ("laplace", False), ("sine", True), ("sine", False),
+                                            ("heat", False)])
+def test_q1_rows_of_constant_coefficients(ctx, nref, example, linear):
+    """Rows and right-hand sides with a reaction and a time, 8 and 27 points."""
+    print(f"[case] Q1 rows nref {nref} {example} linear {linear}", flush=True)
+    if example == "heat":
+        blk = P.heat_amc(0.3)
+    elif example == "laplace":
+        blk = P.base(P.EX_LAPLACE, eps=0.7)
+    else:
+        blk = P.base(P.EX_SINE_CD, eps=1e-2, form=P.FORM_SDFEM, b=(0.3, -1.0, 0.5), c=0.7)
+    blk[P.LINEAR] = 1.0 if linear else 0.0
+    S, O = pa.System(ctx, nref, 1, 1), orc.System(nref, 1, 1)
+    S.assemble(blk)
+    O.assemble(blk)
+    assert rel(S.entries(), O.entries()) < 1e-12
+    assert rel(S.rhs(), O.rhs()) < 1e-12
+    S.close()
+
+
+def test_two_matrices_of_constant_coefficients(ctx):
+    """A step of the SUPG time form with the sine coefficients: solution against
+    the oracle's, both solved to 1e-10 of the residual or better."""
+    print("[case] TCD SUPG step, sine coefficients, 8^3 Q1", flush=True)
+    from test_gpu_tcd_supg import supg_opt
+    prm = P.base(P.EX_SINE_CD, eps=1e-2, form=P.FORM_TCD_SUPG_AK, b=(0.3, -1.0, 0.5))
+    S, O = pa.System(ctx, 1, 3, 1), orc.System(1, 3, 1)
+    u0 = orc.Space(3, 1).interpolate(prm)
+    S.tcd_init(prm, u0)
+    p = prm.copy()
+    p[P.TIME] = 1e-2
+    S.tcd_step(p, [1e-2, .5, .5, .5, .5], supg_opt(0))
+    O.set_multicolour()
+    ref, _ = O.tcd3d(prm, [1e-2, 1.5e-2, .5, .5, .5, .5], supg_opt(), u0, max_steps=1)
+    assert rel(S.solution(), ref) < 1e-9
+    S.close()
+
+
 @pytest.mark.parametrize("order,alpha", [(1, 0.02), (1, 19.0), (1, 20.0 - 1e-9), (1, 20.0 + 1e-9), (2, 22.0),
                                          (1, 1e9)])
 def test_streamline_parameter_around_its_limit(ctx, order, alpha):
