@@ -632,8 +632,9 @@ static bool mg_cycle_from_zero(System &Y) {
 // The cycle is captured once into a HIP graph and replayed, so the GPU is not
 // left waiting on launches.  True: the finest level's psum holds the upper
 // sums of z.
+// surface: z's Dirichlet entries go to it too (fine_matvec's, y = A z).
 template <typename T>
-static bool mg_prec(System &Y, T *z, const T *vin) {
+static bool mg_prec(System &Y, T *z, const T *vin, T *surface = nullptr) {
   hipStream_t st = Y.ctx->st;
   Level &lv = *Y.lev.back();
   Vecs<T> &v = vecs<T>(lv);
@@ -669,15 +670,17 @@ static bool mg_prec(System &Y, T *z, const T *vin) {
   } else {
     upper = mg_cycle_from_zero<T>(Y);
   }
-  copy<T>(z, v.x.p, lv.L.N, st);
+  if (surface) copy_surface<T>(lv.D, z, v.x.p, surface, st);
+  else copy<T>(z, v.x.p, lv.L.N, st);
   return upper;
 }
 
 // y = A x on the finest level (stencil + Dirichlet identity rows); in FP64
 // the caller's CSR matrix instead while pmx_iterate runs
-// (upper: x is the result that mg_prec has just left, with its upper sums)
+// (upper: x is the result that mg_prec has just left, with its upper sums;
+// surface: it has set y's Dirichlet rows)
 template <typename T>
-static void fine_matvec(System &Y, const T *x, T *y, bool upper = false) {
+static void fine_matvec(System &Y, const T *x, T *y, bool upper = false, bool surface = false) {
   Level &lv = *Y.lev.back();
   if constexpr (std::is_same<T, double>::value) {
     if (Y.use_ucsr) {
@@ -686,7 +689,7 @@ static void fine_matvec(System &Y, const T *x, T *y, bool upper = false) {
     }
   }
   rows_apply<T>(lv.D, 0, vecs<T>(lv).val.p, x, nullptr, y, 0.0, Y.ctx->st, upper ? vecs<T>(lv).psum.p : nullptr);
-  boundary<T>(lv.D, 0, y, x, nullptr, Y.ctx->st);
+  if (!surface) boundary<T>(lv.D, 0, y, x, nullptr, Y.ctx->st);
 }
 template <typename T>
 static void fine_defect(System &Y, const T *x, const T *b, T *r) {
@@ -740,8 +743,8 @@ static int fgmres(System &Y, T *x, const T *b, int m, int maxit, double rmin, do
     int i;
     for (i = 0; i < m && j <= maxit; i++, j++) {
       T *vi = V + (size_t)i * N, *zi = Z + (size_t)i * N;
-      const bool upper = mg_prec<T>(Y, zi, vi);
-      fine_matvec<T>(Y, zi, w, upper);
+      const bool upper = mg_prec<T>(Y, zi, vi, w);
+      fine_matvec<T>(Y, zi, w, upper, true);
       mgs_arnoldi<T>(w, V, N, i + 1, H + (size_t)i * ld, V + (size_t)(i + 1) * N, part, st);
       givens(H, cs, sn, s, i, ld, res, st);
       const double r_prev = r;
@@ -849,8 +852,8 @@ static int bicgstab(System &Y, T *x, const T *b, int maxit, double rmin, double 
       check(hipMemcpyAsync(p, t, sizeof(T) * N, hipMemcpyDeviceToDevice, st), "copy");
     }
     rho_last = rho;
-    bool upper = mg_prec<T>(Y, yv, p);
-    if (flexible) fine_matvec<T>(Y, yv, v, upper);
+    bool upper = mg_prec<T>(Y, yv, p, flexible ? v : nullptr);
+    if (flexible) fine_matvec<T>(Y, yv, v, upper, true);
     else check(hipMemcpyAsync(v, yv, sizeof(T) * N, hipMemcpyDeviceToDevice, st), "copy");
     dot<T>(rt, v, N, part, sc + 1, 0, st);
     double delta = read_scalar(Y, sc + 1);
@@ -861,8 +864,8 @@ static int bicgstab(System &Y, T *x, const T *b, int maxit, double rmin, double 
     dot<T>(r, r, N, part, sc + 2, 1, st);
     dn = read_scalar(Y, sc + 2);
     if (dn < dn0 * red || dn < rmin) break;
-    upper = mg_prec<T>(Y, yv, r);
-    if (flexible) fine_matvec<T>(Y, yv, t, upper);
+    upper = mg_prec<T>(Y, yv, r, flexible ? t : nullptr);
+    if (flexible) fine_matvec<T>(Y, yv, t, upper, true);
     else check(hipMemcpyAsync(t, yv, sizeof(T) * N, hipMemcpyDeviceToDevice, st), "copy");
     dot<T>(t, t, N, part, sc + 3, 0, st);
     double tt = read_scalar(Y, sc + 3);

@@ -58,6 +58,8 @@ void stream_read(const void *p, int64_t bytes, float *sink, hipStream_t st);
 
 template <typename T> void fill(T *x, T v, int64_t n, hipStream_t st);
 template <typename T> void copy(T *y, const T *x, int64_t n, hipStream_t st);
+// z = x, and y = x on the Dirichlet nodes
+template <typename T> void copy_surface(const DevLayout &D, T *z, const T *x, T *y, hipStream_t st);
 template <typename T>
 void axpy(T *y, const T *x, const double *alpha_dev, double sgn, double ac, int64_t n, hipStream_t st);
 template <typename T, typename U> void convert(T *y, const U *x, int64_t n, hipStream_t st);
