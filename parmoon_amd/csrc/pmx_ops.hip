@@ -880,16 +880,31 @@ __global__ __launch_bounds__(kBlock) void k_csr_spmv(int n, const int *__restric
 // rows B identity), so A^-1 f = [A_II^-1 (f_I - A_IB f_B); f_B].  The device
 // keeps W = A_II^-1 [I_I, -A_IB] as an n_I x N matrix in lattice column order:
 // y_I = W f (one wavefront per row, FP64), y_B = f_B.
+// Bound by latency: a row of 729 columns is 12 loads of a lane.  kGemvLoads of
+// them are in flight at a time (past the end the last column again, not added),
+// and a workgroup has one row, so that the rows of a few hundred spread over the CUs.  343 rows of 729
+// columns: FP32 vectors 8.4 -> 3.4 us, FP64 8.4 -> 3.0 us (four rows per workgroup,
+// one load waited for after another).
+constexpr int kGemvLoads = 8;
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_gemv_coarse(int nI, int N, const double *__restrict__ W,
-                                                        const int *__restrict__ iidx, const T *__restrict__ x,
-                                                        T *__restrict__ y) {
-  const int lane = threadIdx.x & 63;
-  const int row = (blockIdx.x * kBlock + threadIdx.x) >> 6;
-  if (row >= nI) return;
+__global__ __launch_bounds__(64) void k_gemv_coarse(int N, const double *__restrict__ W, const int *__restrict__ iidx,
+                                                    const T *__restrict__ x, T *__restrict__ y) {
+  const int lane = threadIdx.x, row = blockIdx.x;
   double s = 0;
   const double *a = W + (int64_t)row * N;
-  for (int j = lane; j < N; j += 64) s += a[j] * (double)x[j];
+  for (int j0 = lane; j0 < N; j0 += 64 * kGemvLoads) {
+    double av[kGemvLoads];
+    T xv[kGemvLoads];
+#pragma unroll
+    for (int u = 0; u < kGemvLoads; u++) {
+      const int j = j0 + 64 * u < N ? j0 + 64 * u : N - 1;
+      av[u] = a[j];
+      xv[u] = x[j];
+    }
+#pragma unroll
+    for (int u = 0; u < kGemvLoads; u++)
+      if (j0 + 64 * u < N) s += av[u] * (double)xv[u];
+  }
   for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
   if (lane == 0) y[iidx[row]] = (T)s;
 }
@@ -1145,7 +1160,8 @@ bool bits_equal(const double *a, const double *b, int64_t n, int *flag, hipStrea
   return h == 0;
 }
 // z = x and, on the lattice surface, y = x: the Dirichlet rows of y = A z in
-// the copy that leaves z, a launch less per Krylov step (2 to 5 us whatever the size)
+// the copy that leaves z, a launch less per Krylov step (129^3 FP32: 6.5 us, in two
+// launches 5.5 + 5.1)
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_copy_surface(int M, T *__restrict__ z, const T *__restrict__ x,
                                                          T *__restrict__ y, unsigned n) {
@@ -1497,8 +1513,7 @@ void restrict_(const DevLayout &C, const DevLayout &F, T *rc, const T *rf, hipSt
 }
 template <typename T>
 void gemv_coarse(int nI, int N, const double *W, const int *iidx, const T *x, T *y, hipStream_t st) {
-  const unsigned g = (unsigned)((nI * 64 + kBlock - 1) / kBlock);
-  hipLaunchKernelGGL(k_gemv_coarse<T>, dim3(g), dim3(kBlock), 0, st, nI, N, W, iidx, x, y);
+  hipLaunchKernelGGL(k_gemv_coarse<T>, dim3((unsigned)nI), dim3(64), 0, st, N, W, iidx, x, y);
 }
 // (k_gj_panel has a thread per row)
 static bool gj_by_panels(int nI) { return nI <= kGjRows; }
