@@ -132,9 +132,11 @@ struct System {
   // Krylov workspace
   DevBuf<double> sol, b, r64;         // finest level, FP64 (lattice)
   // a host vector in the reference numbering on its way to or from a level
-  // (at most the finest level's size; the calls that use it end with the
-  // stream idle)
+  // (at most the finest level's size).  io_lock is held from its reservation
+  // until the stream is idle: two threads may be in calls on one system (a
+  // download beside a solve), and the launches of both go to one stream
   DevBuf<double> io;
+  std::mutex io_lock;
   // input, target and loss of a gradient call, kept up to kKeepGradient
   DevBuf<float> gin, gtarget, gloss;
   DevBuf<double> sol_try, r_try;      // FP32 form: the corrected iterate and its defect before acceptance
@@ -1227,6 +1229,7 @@ static void ensure_csr_host(System &Y, Level &lv) {
 template <typename T>
 static void to_lattice(System &Y, Level &lv, const double *host, T *dev) {
   hipStream_t st = Y.ctx->st;
+  std::lock_guard<std::mutex> lock(Y.io_lock);
   Y.io.reserve(lv.L.N);
   check(hipMemcpyAsync(Y.io.p, host, sizeof(double) * lv.L.N, hipMemcpyHostToDevice, st), "h2d");
   gather<T, double>(dev, Y.io.p, lv.lat2dof.p, lv.L.N, st);
@@ -1235,6 +1238,7 @@ static void to_lattice(System &Y, Level &lv, const double *host, T *dev) {
 template <typename T>
 static void from_lattice(System &Y, Level &lv, const T *dev, double *host) {
   hipStream_t st = Y.ctx->st;
+  std::lock_guard<std::mutex> lock(Y.io_lock);
   Y.io.reserve(lv.L.N);
   gather<double, T>(Y.io.p, dev, lv.dof2lat.p, lv.L.N, st);
   check(hipMemcpyAsync(host, Y.io.p, sizeof(double) * lv.L.N, hipMemcpyDeviceToHost, st), "d2h");
