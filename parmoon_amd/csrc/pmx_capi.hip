@@ -137,8 +137,11 @@ struct System {
   // download beside a solve), and the launches of both go to one stream
   DevBuf<double> io;
   std::mutex io_lock;
-  // input, target and loss of a gradient call, kept up to kKeepGradient
+  // input, target and loss of a gradient call, kept up to kKeepGradient;
+  // grad_lock is held for the whole call (another thread's call may replace or
+  // release the buffers, and sums into the same gradient)
   DevBuf<float> gin, gtarget, gloss;
+  std::mutex grad_lock;
   DevBuf<double> sol_try, r_try;      // FP32 form: the corrected iterate and its defect before acceptance
   // a caller's finest-level CSR matrix (lattice-permuted) as the FP64 Krylov
   // operator of pmx_iterate; the MG cycle keeps the system's own levels
@@ -2244,6 +2247,7 @@ int pmx_learned_gradient(pmx_system *sys, int M, const float *in, const float *t
     if (!net.ready) throw std::logic_error("learned smoother: no parameters");
     hipStream_t st = Y.ctx->st;
     const int64_t N = (int64_t)M * M * M;
+    std::lock_guard<std::mutex> lock(Y.grad_lock);
     if (net_reserve(net, N, true)) Y.invalidate_graphs();
     Y.gin.reserve((size_t)N * kNetIn);
     Y.gtarget.reserve(N);

@@ -1,6 +1,7 @@
 """Calls on one system from several threads: downloads beside each other and
-beside a solve return what they return alone, bit for bit (the vectors pass
-through one buffer of the system)."""
+beside a solve, and gradients of several lattices, return what they return
+alone, bit for bit (vectors and gradient inputs pass through kept buffers of
+the system)."""
 import threading
 
 import numpy as np
@@ -58,4 +59,20 @@ def test_downloads_beside_each_other_and_a_solve(ctx):
     assert all(np.array_equal(alone, a) for a in got[0])
     assert all(np.array_equal(want[0], a) for a in got[1])
     assert all(np.array_equal(S.rhs(level=1), a) for a in got[2])
+    S.close()
+
+
+def test_gradients_of_several_lattices(ctx):
+    """129^3 is beyond the size whose buffers stay allocated."""
+    print("[case] network gradients on 129^3, 33^3 and 5^3 in three threads", flush=True)
+    S = pa.System(ctx, 1, 2, 1)
+    S.assemble(P.config1b())
+    S.learned_init(11)
+    rng = np.random.default_rng(4)
+    data = [(rng.standard_normal((M, M, M, 16), np.float32), rng.standard_normal((M, M, M), np.float32))
+            for M in (129, 33, 5)]
+    want = [S.learned_gradient(u, t) for u, t in data]
+    got = run_threads([lambda u=u, t=t: S.learned_gradient(u, t) for u, t in data], 6)
+    for (g, l), res in zip(want, got):
+        assert all(np.array_equal(g, a) and l == b for a, b in res)
     S.close()
