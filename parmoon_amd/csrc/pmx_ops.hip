@@ -502,12 +502,13 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
   double frhs = 0;
   // incident cells per direction: lattice coordinate x lies in cells
   // floor((x-1)/ORDER) .. floor(x/ORDER) (two cells at a vertex plane)
+  constexpr int UNR = ORDER == 1 ? 2 : 1;  // (right-hand sides of Q1: the 8 cells; 4.7 -> 4.4 ms there)
   const int cx0 = (px - 1) / ORDER, cy0 = (py - 1) / ORDER, cz0 = (pz - 1) / ORDER;
-#pragma unroll 1
+#pragma unroll UNR
   for (int iz = 0; iz < NCZ; iz++)
-#pragma unroll 1
+#pragma unroll UNR
     for (int iy = 0; iy < NCY; iy++)
-#pragma unroll 1
+#pragma unroll UNR
       for (int ix = 0; ix < NCX; ix++) {
         const int cx = cx0 + ix, cy = cy0 + iy, cz = cz0 + iz;
         const int ax = px - ORDER * cx, ay = py - ORDER * cy, az = pz - ORDER * cz;
@@ -558,25 +559,48 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
 }
 
 // Rows of the one-thread-per-row assembly kernels: 64 row pairs of a unit's
-// lines (unit_lines), the odd rows in one workgroup and the even rows in the
-// next, so that a wavefront's rows have one stencil shape and its stores of a
-// slot are contiguous.  False: no row.
+// lines (unit_lines), the odd rows in one workgroup and the even rows in
+// another, so that a wavefront's rows have one stencil shape and its stores of a
+// slot are contiguous.
+// Q2: a row has 1, 2, 4 or 8 cells, by the parities of its coordinates.
+// Workgroups go to the shader engines in turn, so that shapes which alternate
+// with a short period put all the long rows on the same ones.  Units therefore
+// come in runs of kShapeRun, and a run's workgroups part by part and (one line
+// per unit) parity of y by parity of y.  Two-matrix form of the sine example, 64
+// points, 64^3 / 32^3: parts alternating 34.5 / 4.2 ms, runs of 8 22.1 / 3.6 ms,
+// of 16 22.5 / 3.6 ms, of 64 23.7 / 3.6 ms.
+struct RowBlock {
+  int part;  // parity of x, segment of the line
+  UnitLines u;
+};
+constexpr int kShapeRun = 8;
+template <int O> __device__ __forceinline__ RowBlock row_block(const LineSet &set, int M, int lg) {
+  const int b = xcd_remap(blockIdx.x, gridDim.x), parts = lg > 6 ? (1 << lg) / 32 : 2;
+  if (O == 1) return RowBlock{b % parts, unit_lines<O>(set, M, lg, b / parts)};
+  const int kz = b / (parts * set.upz), r = b - kz * (parts * set.upz);
+  const int first = r / (parts * kShapeRun) * kShapeRun, i = r - parts * first;
+  const int n = set.upz - first < kShapeRun ? set.upz - first : kShapeRun;
+  const int part = i / n;
+  int j = i - part * n;
+  if (lg >= 6) {
+    const int h = (n + 1) >> 1;
+    j = j < h ? 2 * j : 2 * (j - h) + 1;
+  }
+  return RowBlock{part, unit_lines<O>(set, M, lg, kz * set.upz + first + j)};
+}
+// False: no row.
 template <int O>
-__device__ __forceinline__ bool unit_row(const LineSet &set, int M, int lg, int lane, int *px, int *py, int *pz) {
-  const int b = xcd_remap(blockIdx.x, gridDim.x), P = 1 << lg, segs = lg > 6 ? P / 64 : 1;
-  const int part = b % (2 * segs);
-  const UnitLines u = unit_lines<O>(set, M, lg, b / (2 * segs));
-  const int t = lane + 64 * (part >> 1), m = t & (P - 1);
-  *px = 2 * m + 1 + (part & 1);
-  *py = u.y0 + Lines<O>::S * (t >> lg);
-  *pz = u.z;
+__device__ __forceinline__ bool unit_row(const RowBlock &b, int M, int lg, int lane, int *px, int *py, int *pz) {
+  const int P = 1 << lg, t = lane + 64 * (b.part >> 1), m = t & (P - 1);
+  *px = 2 * m + 1 + (b.part & 1);
+  *py = b.u.y0 + Lines<O>::S * (t >> lg);
+  *pz = b.u.z;
   return *py <= M - 2 && *px <= M - 2;
 }
 // the same shape for the whole wavefront
-template <int O> __device__ __forceinline__ int unit_shape(int lg, const LineSet &set, int M) {
-  const int b = xcd_remap(blockIdx.x, gridDim.x), segs = lg > 6 ? (1 << lg) / 64 : 1;
-  const UnitLines u = unit_lines<O>(set, M, lg, b / (2 * segs));
-  return __builtin_amdgcn_readfirstlane(Lines<O>::ext(1 + (b & 1)) * 100 + Lines<O>::ext(u.y0) * 10 + Lines<O>::ext(u.z));
+template <int O> __device__ __forceinline__ int unit_shape(const RowBlock &b) {
+  return __builtin_amdgcn_readfirstlane(Lines<O>::ext(1 + (b.part & 1)) * 100 + Lines<O>::ext(b.u.y0) * 10 +
+                                        Lines<O>::ext(b.u.z));
 }
 static unsigned row_blocks(const DevLayout &D, int units) {
   return (unsigned)units * 2 * (D.lg > 6 ? (1u << D.lg) / 64 : 1);
@@ -589,9 +613,14 @@ __global__ __launch_bounds__(kRowsPerBlock) void k_assemble(LineSet set, int lg,
                                                      double *__restrict__ val, double *__restrict__ val2,
                                                      double *__restrict__ rhs) {
   int px, py, pz;
-  const bool ok = unit_row<ORDER>(set, M, lg, threadIdx.x, &px, &py, &pz);
-  const int code = unit_shape<ORDER>(lg, set, M);
+  const RowBlock rb = row_block<ORDER>(set, M, lg);
+  const bool ok = unit_row<ORDER>(rb, M, lg, threadIdx.x, &px, &py, &pz);
+  const int code = unit_shape<ORDER>(rb);
   if (!ok) return;
+  // (known to be uniform, they and what follows from them take the scalar
+  // registers that the coefficients' constants need in the loop over the points;
+  // right-hand side of the sine example at 128^3 Q1 4.41 -> 4.24 ms)
+  asm volatile("" : "+v"(py), "+v"(pz));
   const int form = (int)prm[PMX_PRM_FORM];
 #define PMX_AROW(O, EX, EY, EZ) \
   assemble_row<O, EX, EY, EZ, TWO, INL, RONLY>(px, py, pz, M, n, nq, form, prm, qref, qp, tab, val, val2, rhs)
@@ -652,7 +681,7 @@ void k_assemble_q1(LineSet set, int lg, int M, int n, const double *__restrict__
   __shared__ double sh[(TWO ? 2 : 1) * 8 * NB * R], sf[8 * R];
   const int t = threadIdx.x & (R - 1), j = __builtin_amdgcn_readfirstlane(threadIdx.x / R);
   int px, py, pz;
-  const bool ok = unit_row<1>(set, M, lg, t, &px, &py, &pz);
+  const bool ok = unit_row<1>(row_block<1>(set, M, lg), M, lg, t, &px, &py, &pz);
   // (a row that exists for the lanes without one)
   if (!ok) px = py = 1;
   const int form = (int)prm[PMX_PRM_FORM];
@@ -1864,8 +1893,9 @@ __global__ __launch_bounds__(kRowsPerBlock) void k_assemble_kc(LineSet set, int 
   static_assert(kRowsPerBlock == 64, "one wavefront");
   __shared__ double sh[2][64 * kKcPad];
   int px, py, pz;
-  const bool ok = unit_row<2>(set, M, lg, threadIdx.x, &px, &py, &pz);
-  const int code = unit_shape<2>(lg, set, M);
+  const RowBlock rb = row_block<2>(set, M, lg);
+  const bool ok = unit_row<2>(rb, M, lg, threadIdx.x, &px, &py, &pz);
+  const int code = unit_shape<2>(rb);
 #define PMX_KROW(EX, EY, EZ) assemble_row_kc<EX, EY, EZ>(sh, ok, px, py, pz, lg, M, n, kc, val, rhs)
   switch (code) {
     case 111: PMX_KROW(1, 1, 1); break;

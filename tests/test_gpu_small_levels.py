@@ -228,3 +228,27 @@ def test_arnoldi_at_small_sizes(ctx, nref, restart, precision):
     r, _ = O.levels[-1].defect(O.entries(), x, rhs)
     assert float(np.linalg.norm(r)) <= 1.1e-11 * info[2]
     S.close()
+
+
+@pytest.mark.parametrize("nref", [1, 2, 3, 5, 6, 7])
+@pytest.mark.parametrize("example", ["sine", "curl"])
+def test_q2_rows_match_cell_matrices(ctx, nref, example):
+    """The two-matrix form without stabilisation and the form of the right-hand
+    side alone (a row per thread) against the one-matrix form (cell matrices):
+    lines of 2 to 128 row pairs, several lines or a half of one per workgroup."""
+    print(f"[case] Q2 rows against cell matrices nref {nref} {example}", flush=True)
+    blk = (P.config2(nref=min(nref, 5)) if example == "curl" else
+           P.base(P.EX_SINE_CD, eps=1e-2, b=(0.3, -1.0, 0.5), c=0.7, linear=True))
+    blk[P.DELTA0] = 0.0
+    S = pa.System(ctx, nref, 1, 2)
+    x = np.random.default_rng(8).standard_normal(int(S.dims()[0]))
+    out = {}
+    for form in (P.FORM_TCD_A, P.FORM_TCD_SUPG_AK, P.FORM_RHS):
+        b = blk.copy()
+        b[P.FORM] = form
+        S.assemble(b)
+        out[form] = (S.matvec(x), S.rhs())
+    assert rel(out[P.FORM_TCD_SUPG_AK][0], out[P.FORM_TCD_A][0]) < 1e-12
+    assert rel(out[P.FORM_TCD_SUPG_AK][1], out[P.FORM_TCD_A][1]) < 1e-12
+    assert rel(out[P.FORM_RHS][1], out[P.FORM_TCD_A][1]) < 1e-12
+    S.close()
