@@ -360,6 +360,11 @@ template <typename T, int O> struct Wg {
   static constexpr int kGroups = Lines<O>::C * Lines<O>::C;
   static constexpr int kParts = O == 2 && sizeof(T) == 4 ? 3 : 2;  // groups of a row per split and batch
   static constexpr int kOffsets = O == 2 ? Lines<2>::S * Lines<2>::S * Lines<2>::kMaxGroups : 0;
+  // the pairs of a line group fit a wavefront (M <= 9)
+  __device__ static bool small(int lg) {
+    const int n = (2 * (1 << lg) - 2) / Lines<O>::C + 1;
+    return (n * n << lg) <= 64;
+  }
   // LDS of a slot: the partial sums of its splits, a row pair's own group and
   // the reciprocals of its diagonals
   static constexpr int kRow = Lines<O>::VL + 2;
@@ -484,6 +489,8 @@ template <typename T, int O> struct WgLds {
 // indices.  A tile's groups come in batches of kSplits * kParts, the next one
 // in flight while one is added.  The own group is loaded by split 1, which
 // hands it over with the sums (split 0 still uses the one of the tile before).
+// it.alone: each slot has a line group of its own, of at most 64 pairs (none if
+// step.g is past the last one).
 template <typename T, int O, class It, class Pre, class F>
 __device__ __forceinline__ void wg_run(const WgLds<T, O> &lds, const WgLevel<T> &lv, const T *lx, It it,
                                        Pre before_sums, F fn) {
@@ -498,10 +505,15 @@ __device__ __forceinline__ void wg_run(const WgLds<T, O> &lds, const WgLevel<T> 
     WgStep st;
     int tile, nlo, n;  // batches of the lower part, of both
     __device__ __forceinline__ void start() {
+      tile = 0;
+      if (st.g >= W::kGroups) {
+        nlo = 0;
+        n = 1;
+        return;
+      }
       // (lines of extent 2 have the most groups)
       const int zr = O == 2 ? (st.g * 11) >> 5 : st.g >> 1, yr = st.g - L::C * zr;
       const int lo = O == 2 ? 10 * zr + 2 * yr : 6 * zr + 2 * yr, hi = L::kMaxGroups - 1 - lo;
-      tile = 0;
       nlo = (st.sums & kSumLo) ? (lo + B - 1) / B : 0;
       n = nlo + ((st.sums & kSumHi) ? (hi + B - 1) / B : 0);
       if (n == 0) n = 1;
@@ -515,8 +527,13 @@ __device__ __forceinline__ void wg_run(const WgLds<T, O> &lds, const WgLevel<T> 
   };
   const __amdgpu_buffer_rsrc_t pbuf = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int2 *>(lv.pairs), 0, W::kGroups * lv.tiles * kPairTile * (int)sizeof(int2), 0x00020000);
+  const int first = it.alone ? 0 : 64 * slot;  // a slot's pairs of a tile
   auto entry = [&](const At &a, bool any) {
-    return pair_entry(pbuf, any ? ((a.st.g * lv.tiles + a.tile) * kPairTile + 64 * slot + t) * 8 : kNoOffset);
+    const bool none = !any || a.st.g >= W::kGroups;
+    int2 e = pair_entry(
+        pbuf, none ? kNoOffset : ((a.st.g * lv.tiles + a.tile) * kPairTile + first + t) * 8);
+    if (none) e.x = 1 << 27;
+    return e;
   };
   // line offset of group k of the lane's pair (class of the line group for Q1)
   auto line_offset = [&](const At &a, const WgPair &pr, int k) {
@@ -674,6 +691,7 @@ __device__ __forceinline__ void wg_sweep_pair(const WgStep &st, const WgPair &pr
 template <int O> struct WgSweeps {
   int n;
   bool ssor, zero;
+  static constexpr bool alone = false;
   int s = 0, j = -1;  // sweep, position in it (forward 0 .. G-1, backward G .. 2G-2)
   __host__ __device__ bool next(WgStep &st) {
     constexpr int G = Lines<O>::C * Lines<O>::C;
@@ -699,13 +717,24 @@ template <int O> struct WgSweeps {
     return true;
   }
 };
-// every row once, in the order of the groups
-template <int O> struct WgAll {
+// Every row once, in the order of the groups.  No row waits for another, so on
+// levels whose groups fit a wavefront each slot takes a group of its own: a step
+// costs its barriers and the latency of its loads whatever it holds, and 9 (4)
+// groups take 3 (1) steps.  10 coarse solves of up to 10 Jacobi sweeps with their
+// norms, FP64 / FP32, 5^3 Q2: 9.3 / 6.6 ms a group per step, 3.4 / 2.7 ms now; a
+// lane per row without barriers between the colours took 6.6 / 6.5 ms.
+template <typename T, int O> struct WgAll {
   int sums;
-  int g = -1;
+  bool alone;
+  int slot;
+  int s = -1;
+  __device__ __forceinline__ WgAll(int sums, int lg)
+      : sums(sums), alone(Wg<T, O>::small(lg)),
+        slot(alone ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kSplits : 0) {}
   __device__ __forceinline__ bool next(WgStep &st) {
-    st = WgStep{++g, 0, sums};
-    return g < Lines<O>::C * Lines<O>::C;
+    const int first = ++s * (alone ? Wg<T, O>::kSlots : 1);
+    st = WgStep{first + slot, 0, sums};
+    return first < Wg<T, O>::kGroups;
   }
 };
 template <typename T, int O>
@@ -734,7 +763,7 @@ template <typename T, int O, class F>
 __device__ __forceinline__ void wg_defect(const WgLds<T, O> &lds, const WgLevel<T> &lv, const T *lx, const T *f, const T *psum,
                                           bool half, F fn) {
   wg_run<T, O>(
-      lds, lv, lx, WgAll<O>{half ? kSumLo : kSumLo | kSumHi},
+      lds, lv, lx, WgAll<T, O>(half ? kSumLo : kSumLo | kSumHi, lv.lg),
       [](const WgStep &, const WgPair &) { return WgNothing{}; },
       [&](const WgStep &, const WgPair &pr, PairSums<T> s, const T *own, WgNothing) {
         if (half) {
@@ -753,7 +782,7 @@ __device__ __forceinline__ void wg_jacobi(const WgLds<T, O> &lds, const WgLevel<
   const int M = 2 * (1 << lv.lg) + 1;
   const T a = (T)omega;
   wg_run<T, O>(
-      lds, lv, lx, WgAll<O>{kSumLo | kSumHi}, [](const WgStep &, const WgPair &) { return WgNothing{}; },
+      lds, lv, lx, WgAll<T, O>(kSumLo | kSumHi, lv.lg), [](const WgStep &, const WgPair &) { return WgNothing{}; },
       [&](const WgStep &, const WgPair &pr, const PairSums<T> &s, const T *own, WgNothing) {
         T ro, re;
         wg_off_diagonal<T, O>(pr, s, own, lx, ro, re);

@@ -252,3 +252,28 @@ def test_q2_rows_match_cell_matrices(ctx, nref, example):
     assert rel(out[P.FORM_TCD_SUPG_AK][1], out[P.FORM_TCD_A][1]) < 1e-12
     assert rel(out[P.FORM_RHS][1], out[P.FORM_TCD_A][1]) < 1e-12
     S.close()
+
+
+@pytest.mark.parametrize("order,nref", [(1, 1), (1, 2), (1, 3), (1, 4), (2, 1), (2, 2), (2, 3)])
+@pytest.mark.parametrize("coarse", [1, 3])
+def test_coarse_loop_matches_the_oracle(ctx, order, nref, coarse):
+    """One level of 3^3 .. 17^3 nodes: the cycle is the coarse loop, three sweeps
+    (reduction 0) or as many as its norms ask for."""
+    print(f"[case] coarse loop order {order} nref {nref} coarse {coarse}", flush=True)
+    S, O = pa.System(ctx, nref, 1, order), orc.System(nref, 1, order)
+    blk = P.config1b() if order == 1 else P.config2(nref=nref)
+    S.assemble(blk)
+    O.assemble(blk)
+    if coarse == 3:
+        O.set_multicolour()
+    sp = O.levels[-1]
+    rng = np.random.default_rng(6)
+    rhs, sol0 = rng.standard_normal(sp.N), rng.standard_normal(sp.N)
+    sol0[sp.active:] = rhs[sp.active:]
+    for sweeps, red in [(3, 0.0), (10, 0.3)]:
+        opt = P.solver_opt(solver=11, maxit=2, res_norm_min=0.0, red_factor=0.0, omega=0.6, coarse=coarse,
+                           coarse_sweeps=sweeps, coarse_red=red)
+        ref, _ = O.solve(opt, rhs, sol0)
+        got, _, _ = S.solve(opt, rhs, sol0, check=False)
+        assert rel(got, ref) < 1e-12, (sweeps, red)
+    S.close()
