@@ -172,7 +172,7 @@ int pmx_csr_matvec(pmx_ctx *ctx, int n, const int *rowptr, const int *kcol, cons
  *  [14] BiCGStab flexible branch (1 = v = A y)
  *  [15] precision: 0 FP64 throughout, 1 FP32 operator/MG/Krylov vectors
  *       inside an FP64 defect correction, 2 = 1 plus the learned post-smoother;
- *       3 / 4 = 1 / 2 with the launched SOR/SSOR sweeps
+ *       3 / 4 = 1 / 2 with the SOR/SSOR sweeps by line groups
  *       reading row-scaled FP16 values (a_ij / a_ii, saturated to the finite
  *       FP16 range) and 1 / a_ii in FP32: half the value bytes of the sweeps,
  *       which only precondition (defects, transfers and Krylov vectors keep
@@ -185,7 +185,8 @@ int pmx_csr_matvec(pmx_ctx *ctx, int n, const int *rowptr, const int *kcol, cons
  *  [20] precision 2: learned steps per post-smoothing (default 1)
  *  [21] SOR/SSOR sweeps of small levels (at most 17^3 lattice nodes, Q2 33^3) whose
  *       largest colour has at most this many rows run plane by plane (same
- *       iterate, fewer launches); 0 = all of them, < 0 = never
+ *       iterate, fewer launches); 0 = all of them, < 0 = never.  Precision 3 / 4:
+ *       17^3 at most, a Q2 level of 33^3 sweeps by line groups
  *  [22] precision 2: the finest [22] of the [19] levels keep the plain smoother
  *  [23] precision 2: 1 = the learned steps also replace the pre-smoothing
  * info (out, 8 doubles): [0] iterations (Krylov steps summed) [1] final FP64
@@ -283,7 +284,7 @@ int pmx_tcd_restore_massmat(pmx_system *sys);
  * same level, also per dispatch: 12 a dispatch that does nothing with the
  * workgroup count of each group launch, 13 a plain streaming read of a group's
  * share of the stored values in the precision's storage.  precision 0 FP64,
- * 1 FP32, 3 FP32 with the launched SOR/SSOR sweeps on row-scaled FP16 values
+ * 1 FP32, 3 FP32 with the SOR/SSOR sweeps by line groups on row-scaled FP16 values
  * (opt[15] = 3).  out: ms. */
 int pmx_time_kernel(pmx_system *sys, int kernel, int level, int precision, int reps, double *ms);
 

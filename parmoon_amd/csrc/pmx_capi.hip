@@ -127,7 +127,6 @@ struct System {
   int tab_key = -1;                   // rule of the uploaded tables
   int example = 0;                    // prm[PMX_PRM_EXAMPLE] of the last assembly
   int form = 0;                       // prm[PMX_PRM_FORM] of the last assembly
-  bool mfma_assembly = true;          // Q2 one-matrix forms through the cell buffer
   DevBuf<double> kc;                  // Q2 cell matrices (finest level's cells x 27 x 28)
   // Krylov workspace
   DevBuf<double> sol, b, r64;         // finest level, FP64 (lattice)
@@ -184,8 +183,8 @@ struct System {
   bool learn_active = false;
   bool x_zero_shortcut = true;  // see mg_cycle
   int fallbacks = 0;
-  // FP32 forms: SOR/SSOR sweeps launched per colour read row-scaled FP16
-  // values (opt[15] = 3 / 4)
+  // FP32 forms: the SOR/SSOR sweeps by line groups read row-scaled FP16 values
+  // (opt[15] = 3 / 4)
   bool half_smoother = false;
   DevBuf<double> lscal;               // norm, (d, Ac), (Ac, Ac)
   DevBuf<int> bnd_set;                // start_zero / start_boundary
@@ -326,9 +325,9 @@ static void ensure_tables(System &Y, bool linear) {
   Y.tab_key = key;
 }
 
-// the cell buffer of the MFMA assembly (Q2 only; sized for the finest level)
+// the cell buffer of the Q2 one-matrix forms (sized for the finest level)
 static double *cell_buffer(System &Y) {
-  if (Y.order != 2 || !Y.mfma_assembly) return nullptr;
+  if (Y.order != 2) return nullptr;
   const int64_t n = Y.lev.back()->L.n;
   Y.kc.alloc((size_t)(n * n * n * kCellMatrixDoubles));
   return Y.kc.p;
@@ -447,8 +446,10 @@ template <typename T>
 static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweeps, int start = kStartAny) {
   hipStream_t st = Y.ctx->st;
   Vecs<T> &v = vecs<T>(lv);
-  // small levels sweep by planes, with FP32 values also where the larger ones
-  // take FP16 values (there is no traffic to save); opt[21] as in pmx.h
+  // small levels sweep by planes, up to 17^3 nodes with FP32 values also where the
+  // larger ones take FP16 values (there is no traffic to save); opt[21] as in pmx.h.
+  // 33^3 Q2 takes the FP16 values by line groups (SSOR sweep 71 us; FP32 by planes
+  // 54 us, by line groups 74 us)
   const bool planes = plane_sweeps_used(lv.D) && (Y.opt[21] == 0 || lv.D.max_colour_rows <= (int64_t)Y.opt[21]);
   if (kind == 1) {
     for (int s = 0; s < sweeps; s++) {
@@ -2061,7 +2062,7 @@ int pmx_time_kernel(pmx_system *sys, int kernel, int level, int precision, int r
     std::memcpy(Y.opt, PMX_DEFAULT_VCYCLE, sizeof(Y.opt));
     hipStream_t st = Y.ctx->st;
     if (precision < 0 || precision > 3 || precision == 2) throw std::invalid_argument("precision must be 0, 1 or 3");
-    // 3: FP32 with the SOR/SSOR colour launches on row-scaled FP16 values
+    // 3: FP32 with the SOR/SSOR sweeps by line groups on row-scaled FP16 values
     Y.half_smoother = precision == 3;
     if (precision == 3) precision = 1;
     if (precision) ensure_val32(Y);

@@ -409,8 +409,7 @@ struct WgPair {
   __device__ __forceinline__ int groups() const { return (int)(line >> 21 & 31); }
   __device__ __forceinline__ int cls() const { return (int)(line >> 26); }
 };
-// What a step needs of a level; plane: of one plane of it, x in LDS from the
-// first plane that the rows touch
+// what a step needs of a level
 template <typename T> struct WgLevel {
   const T *val;
   const int2 *pairs;
@@ -724,24 +723,24 @@ template <int O> struct WgSweeps {
 // norms, FP64 / FP32, 5^3 Q2: 9.3 / 6.6 ms a group per step, 3.4 / 2.7 ms now; a
 // lane per row without barriers between the colours took 6.6 / 6.5 ms.
 template <typename T, int O> struct WgAll {
-  int sums;
   bool alone;
   int slot;
   int s = -1;
-  __device__ __forceinline__ WgAll(int sums, int lg)
-      : sums(sums), alone(Wg<T, O>::small(lg)),
+  __device__ __forceinline__ explicit WgAll(int lg)
+      : alone(Wg<T, O>::small(lg)),
         slot(alone ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kSplits : 0) {}
   __device__ __forceinline__ bool next(WgStep &st) {
     const int first = ++s * (alone ? Wg<T, O>::kSlots : 1);
-    st = WgStep{first + slot, 0, sums};
+    st = WgStep{first + slot, 0, kSumLo | kSumHi};
     return first < Wg<T, O>::kGroups;
   }
 };
+// one SOR / SSOR sweep; psum: scratch of N entries
 template <typename T, int O>
-__device__ __forceinline__ void wg_sweeps(const WgLds<T, O> &lds, const WgLevel<T> &lv, T *lx, const T *f, T *psum,
-                                          double omega, bool ssor, int n, bool zero) {
+__device__ __forceinline__ void wg_sweep(const WgLds<T, O> &lds, const WgLevel<T> &lv, T *lx, const T *f, T *psum,
+                                          double omega, bool ssor) {
   wg_run<T, O>(
-      lds, lv, lx, WgSweeps<O>{n, ssor, zero},
+      lds, lv, lx, WgSweeps<O>{1, ssor, false},
       [&](const WgStep &st, const WgPair &pr) { return wg_sweep_row<T, O>(st, pr, lx, f, psum); },
       [&](const WgStep &st, const WgPair &pr, const PairSums<T> &s, const T *own, const WgSweepRow<T> &row) {
         wg_sweep_pair<T, O>(st, pr, s, own, row, lx, psum, 1 << lv.lg, omega);
@@ -758,18 +757,12 @@ __device__ __forceinline__ void wg_off_diagonal(const WgPair &pr, const PairSums
   ro = own_odd<T, T, O>(own, xe, s.lo_o + s.hi_o);
   re = own_even<T, T, O>(own, xe, s.lo_e + s.hi_e);
 }
-// fn(pair, odd, even): f - A x of every row pair; half: psum holds the upper sums
+// fn(pair, odd, even): f - A x of every row pair
 template <typename T, int O, class F>
-__device__ __forceinline__ void wg_defect(const WgLds<T, O> &lds, const WgLevel<T> &lv, const T *lx, const T *f, const T *psum,
-                                          bool half, F fn) {
+__device__ __forceinline__ void wg_defect(const WgLds<T, O> &lds, const WgLevel<T> &lv, const T *lx, const T *f, F fn) {
   wg_run<T, O>(
-      lds, lv, lx, WgAll<T, O>(half ? kSumLo : kSumLo | kSumHi, lv.lg),
-      [](const WgStep &, const WgPair &) { return WgNothing{}; },
-      [&](const WgStep &, const WgPair &pr, PairSums<T> s, const T *own, WgNothing) {
-        if (half) {
-          s.hi_o = psum[pr.p0 + 1];
-          s.hi_e = psum[pr.p0 + 2];
-        }
+      lds, lv, lx, WgAll<T, O>(lv.lg), [](const WgStep &, const WgPair &) { return WgNothing{}; },
+      [&](const WgStep &, const WgPair &pr, const PairSums<T> &s, const T *own, WgNothing) {
         T ro, re;
         wg_off_diagonal<T, O>(pr, s, own, lx, ro, re);
         fn(pr, f[pr.p0 + 1] - fma(own[1], lx[pr.p0 + 1], ro), f[pr.p0 + 2] - fma(own[3 + O], lx[pr.p0 + 2], re));
@@ -782,7 +775,7 @@ __device__ __forceinline__ void wg_jacobi(const WgLds<T, O> &lds, const WgLevel<
   const int M = 2 * (1 << lv.lg) + 1;
   const T a = (T)omega;
   wg_run<T, O>(
-      lds, lv, lx, WgAll<T, O>(kSumLo | kSumHi, lv.lg), [](const WgStep &, const WgPair &) { return WgNothing{}; },
+      lds, lv, lx, WgAll<T, O>(lv.lg), [](const WgStep &, const WgPair &) { return WgNothing{}; },
       [&](const WgStep &, const WgPair &pr, const PairSums<T> &s, const T *own, WgNothing) {
         T ro, re;
         wg_off_diagonal<T, O>(pr, s, own, lx, ro, re);
@@ -1133,7 +1126,7 @@ template <typename T, int O>
 __device__ double wg_defect_norm(const WgLds<T, O> &lds, const WgLevel<T> &lv, const T *lx, const T *f, double *lred) {
   constexpr int NT = Wg<T, O>::kThreads;
   double sum = 0;
-  wg_defect<T, O>(lds, lv, lx, f, nullptr, false, [&](const WgPair &pr, T d, T e) {
+  wg_defect<T, O>(lds, lv, lx, f, [&](const WgPair &pr, T d, T e) {
     if (!pr.ok) return;
     sum += (double)d * (double)d;
     if (!pr.last) sum += (double)e * (double)e;
@@ -1168,7 +1161,7 @@ __global__ __launch_bounds__((Wg<T, O>::kThreads)) void k_coarse_wg(WgLevel<T> l
   const double reduction = red_factor * res;
   for (int it = 0; res > reduction && it < maxit; it++) {
     if (kind == 1) wg_jacobi<T, O>(lds, lv, lx, f, xj, omega);
-    else wg_sweeps<T, O>(lds, lv, lx, f, xj, omega, kind == 3, 1, false);
+    else wg_sweep<T, O>(lds, lv, lx, f, xj, omega, kind == 3);
     __syncthreads();
     res = wg_defect_norm<T, O>(lds, lv, lx, f, lred);
   }

@@ -446,7 +446,7 @@ __host__ __device__ inline bool coeffs_inline(int example) {
 // The incident cells per direction are compile-time (a Q2 node with an odd
 // coordinate lies in one cell along it, every other node in two), so the
 // loops are uniform across the wavefront and the basis tables are read with
-// scalar loads; TWO selects the second matrix of the SUPG TCD form.
+// scalar loads; val2 is the second matrix of the SUPG TCD form.
 struct RowPoint {
   double u0, ux, uy, uz, k0, f;  // of K_ab, of the second matrix, of the rhs
 };
@@ -479,7 +479,7 @@ __device__ __forceinline__ RowPoint row_point(const double *Qq, double fa, doubl
   r.k0 *= w;
   return r;
 }
-template <int ORDER, int EX, int EY, int EZ, bool TWO, bool INL, bool RONLY>
+template <int ORDER, int EX, int EY, int EZ, bool INL, bool RONLY>
 __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int n, int nq, int form,
                                              const double *__restrict__ prm, const double *__restrict__ qref,
                                              const double *__restrict__ qp, const double *__restrict__ tab,
@@ -542,7 +542,7 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
           for (int b = 0; b < NB; b++) {
             const double *Tb = Tq + 4 * b;
             acc[b] += r.u0 * Tb[0] + r.ux * Tb[1] + r.uy * Tb[2] + r.uz * Tb[3];
-            if (TWO) acc2[b] += r.k0 * Tb[0];
+            acc2[b] += r.k0 * Tb[0];
           }
         }
         if (RONLY) continue;
@@ -552,7 +552,7 @@ __device__ __forceinline__ void assemble_row(int px, int py, int pz, int M, int 
           const int bx = b % K, by = (b / K) % K, bz = b / (K * K);
           const int dx = ORDER * cx + bx - px, dy = ORDER * cy + by - py, dz = ORDER * cz + bz - pz;
           val[at(dx, dy, dz)] += acc[b];
-          if (TWO) val2[at(dx, dy, dz)] += acc2[b];
+          val2[at(dx, dy, dz)] += acc2[b];
         }
       }
   rhs[p] = frhs;
@@ -606,7 +606,7 @@ static unsigned row_blocks(const DevLayout &D, int units) {
   return (unsigned)units * 2 * (D.lg > 6 ? (1u << D.lg) / 64 : 1);
 }
 
-template <int ORDER, bool TWO, bool INL, bool RONLY>
+template <int ORDER, bool INL, bool RONLY>
 __global__ __launch_bounds__(kRowsPerBlock) void k_assemble(LineSet set, int lg, int M, int n, int nq,
                                                      const double *__restrict__ prm, const double *__restrict__ qref,
                                                      const double *__restrict__ qp, const double *__restrict__ tab,
@@ -623,7 +623,7 @@ __global__ __launch_bounds__(kRowsPerBlock) void k_assemble(LineSet set, int lg,
   asm volatile("" : "+v"(py), "+v"(pz));
   const int form = (int)prm[PMX_PRM_FORM];
 #define PMX_AROW(O, EX, EY, EZ) \
-  assemble_row<O, EX, EY, EZ, TWO, INL, RONLY>(px, py, pz, M, n, nq, form, prm, qref, qp, tab, val, val2, rhs)
+  assemble_row<O, EX, EY, EZ, INL, RONLY>(px, py, pz, M, n, nq, form, prm, qref, qp, tab, val, val2, rhs)
   if (ORDER == 1) {
     PMX_AROW(1, 1, 1, 1);
     return;
@@ -1961,7 +1961,7 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
   if (form == PMX_FORM_RHS || form == PMX_FORM_RHS_SUPG) {
     // right-hand-side forms (no local matrices): the matrices are left as they are
 #define PMX_RHS(O, IN)                                                                                     \
-  hipLaunchKernelGGL((k_assemble<O, false, IN, true>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq, prm_dev, qref, qsrc, tab, nullptr, nullptr, rhs)
+  hipLaunchKernelGGL((k_assemble<O, IN, true>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq, prm_dev, qref, qsrc, tab, nullptr, nullptr, rhs)
     if (D.order == 1) {
       if (inl) PMX_RHS(1, true);
       else PMX_RHS(1, false);
@@ -1992,14 +1992,9 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
                        D.nboundary, D.M, prm_dev, rhs);
     return;
   }
-  // the per-row evaluation of Q2 rows adds every cell's contribution into
-  // the cleared values (Q1 rows store each slot; the slots of boundary nodes
-  // are never written and keep the zeros of the allocation)
-  if (D.order == 2) {
-    check(hipMemsetAsync(val, 0, sizeof(double) * D.nvals, st), "memset val");
-    if (val2) check(hipMemsetAsync(val2, 0, sizeof(double) * D.nvals, st), "memset val2");
-  }
   if (D.order == 1) {
+    // (every slot is stored; those of boundary nodes are never written and keep
+    // the zeros of the allocation)
 #define PMX_ASM3(NP, TW, SRC)                                                                                      \
   hipLaunchKernelGGL((k_assemble_q1<NP, TW, SRC>), gr, dim3(8 * kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, prm_dev, \
                      qref, qsrc, val, val2, rhs)
@@ -2017,13 +2012,16 @@ void assemble(const DevLayout &D, const double *prm_dev, int example, int form, 
 #undef PMX_ASM
 #undef PMX_ASM3
   } else {
-#define PMX_ASM(TW, IN)                                                                                            \
-  hipLaunchKernelGGL((k_assemble<2, TW, IN, false>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq,      \
-                     prm_dev, qref, qsrc, tab, val, val2, rhs)
-    if (val2 && inl) PMX_ASM(true, true);
-    else if (val2) PMX_ASM(true, false);
-    else if (inl) PMX_ASM(false, true);
-    else PMX_ASM(false, false);
+    // Q2, two matrices: a row per thread adds every cell's contribution into the
+    // cleared values
+    if (!val2) throw std::logic_error("assemble: Q2 without a cell buffer");
+    check(hipMemsetAsync(val, 0, sizeof(double) * D.nvals, st), "memset val");
+    check(hipMemsetAsync(val2, 0, sizeof(double) * D.nvals, st), "memset val2");
+#define PMX_ASM(IN)                                                                                             \
+  hipLaunchKernelGGL((k_assemble<2, IN, false>), gr, dim3(kRowsPerBlock), 0, st, set, D.lg, D.M, D.n, nq, prm_dev, \
+                     qref, qsrc, tab, val, val2, rhs)
+    if (inl) PMX_ASM(true);
+    else PMX_ASM(false);
 #undef PMX_ASM
   }
   hipLaunchKernelGGL(k_boundary_rhs, dim3((D.nboundary + kBlock - 1) / kBlock), dim3(kBlock), 0, st, D.boundary,
@@ -2185,13 +2183,10 @@ template void values_to_csr<_Float16>(const DevLayout &, const int *, const int 
 template void fill<uint16_t>(uint16_t *, uint16_t, int64_t, hipStream_t);
 template void fill<int>(int *, int, int64_t, hipStream_t);
 template void convert<float, double>(float *, const double *, int64_t, hipStream_t);
-template void convert<double, float>(double *, const float *, int64_t, hipStream_t);
 template void add_convert<double, float>(double *, const float *, int64_t, hipStream_t);
-template void add_convert<double, double>(double *, const double *, int64_t, hipStream_t);
 template void gather<double, double>(double *, const double *, const int *, int64_t, hipStream_t);
 template void gather<float, double>(float *, const double *, const int *, int64_t, hipStream_t);
 template void gather<double, float>(double *, const float *, const int *, int64_t, hipStream_t);
-template void gather<float, float>(float *, const float *, const int *, int64_t, hipStream_t);
 template void multi_axpy<double, double>(double *, const double *, const double *, int, int64_t, int64_t, hipStream_t);
 template void multi_axpy<float, float>(float *, const float *, const double *, int, int64_t, int64_t, hipStream_t);
 

@@ -179,8 +179,7 @@ void values_to_csr(const DevLayout &D, const int *rowptr, const int *kcol, const
                 const T *val, double *out, hipStream_t st);
 // example: prm[PMX_PRM_EXAMPLE] (selects evaluating the coefficients inline or
 // through the quadrature-point buffer); form: prm[PMX_PRM_FORM]; kc: cell
-// buffer of n^3 x 27 x 28 doubles for the Q2 one-matrix forms on MFMA
-// (nullptr: the per-row evaluation); qp_given: qpbuf already holds the
+// buffer of n^3 x 27 x 28 doubles for the Q2 one-matrix forms; qp_given: qpbuf already holds the
 // quadrature-point records (coefficients from host callbacks)
 // ftab (optional): room for phase_tab_len(n, nq) doubles; with it the
 // curl-Fourier example's coefficients come from per-level phase tables.
