@@ -44,8 +44,40 @@ HBM_PEAK_GBS = 8000.0      # MI355X HBM3E, GB/s
 FP64_PEAK_TFLOPS = 78.6    # MI355X FP64 (vector = MFMA), TFLOP/s
 BF16_PEAK_TFLOPS = 2500.0  # MI355X dense BF16 MFMA, TFLOP/s
 # HBM bytes per dispatch at 64^3 Q2 from hardware counters (tests/cpp/kernel_probe)
-TRAFFIC_SSOR_LAUNCH = 58661990  # k_line_sweep<float, float, 2>, one line group (average over the sweeps)
-TRAFFIC_SPMV = 547418214  # k_line_rows<float, 2, 0>
+TRAFFIC_SSOR_LAUNCH = 47511111  # k_line_sweep<float, float, 2>, one line group (average over a V(2,2) cycle's sweeps)
+TRAFFIC_SPMV = 547236757  # k_line_rows<float, 2, 0>
+
+
+def group_launch_bytes(nvals, N, nact, sv):
+    """Bytes of a line-group launch, average over the SSOR smoothing of a Q2
+    V(2,2) cycle: two sweeps from zero, two from an iterate, each forward over the
+    9 groups and back (a group at a turn takes part in one launch).  Group 3 zr +
+    yr has on average 16 (dy, dz) groups per line, 6 zr + 1.5 yr of them before
+    the line.  Per launch: the groups it adds and the line's own of the group's
+    values, x of those lines and the line, and of the rows f, x written, the kept
+    sums read (but in a smoothing's first pass) and written."""
+    total, launches = 0.0, 0
+    for first_hi in (False, True):  # from zero there is nothing after a line
+        for groups, lo, hi, kept in ((range(9), True, first_hi, False), (range(7, -1, -1), False, True, True),
+                                     (range(1, 9), True, False, True), (range(7, -1, -1), False, True, True)):
+            for g in groups:
+                before = 6.0 * (g // 3) + 1.5 * (g % 3)
+                values = 1.0 + (before if lo else 0.0) + (15.0 - before if hi else 0.0)
+                lines = 1.0 + (g if lo else 0.0) + (8.0 - g if hi else 0.0)
+                total += (nvals * values / 16 + N * lines + nact * (4.0 if kept else 3.0)) / 9 * sv
+                launches += 1
+    return total / launches
+
+
+def assembly_work(n, points, nvals):
+    """(bytes, operations) of the Q2 assembly of n^3 cells with points^3 quadrature
+    points: records and cell buffer written and read, values written; products and
+    sums of k_cell_sum axis by axis (x with the 66 of a point and basis function, y,
+    z)."""
+    p = points
+    by = 8 * (2 * 8 * p ** 3 * n ** 3 + 2 * 27 * 28 * n ** 3 + nvals)
+    fma = 3 * p ** 3 * 66 + 9 * p * p * 81 + 81 * p * 30
+    return by, 2.0 * fma * n ** 3
 
 
 def cpu_info():
@@ -330,7 +362,7 @@ def main():
     nref = args.nref
     prm = P.config2(nref=nref)
     ctx = pa.Context(0)
-    # host set-up of the five levels (numbering, stencil layout, block tables)
+    # set-up of the five levels (numbering, layout, pair tables)
     # and their device buffers: once per mesh, outside the steps
     t0 = time.perf_counter()
     S = pa.System(ctx, nref - 4, 5, 2)
@@ -390,27 +422,20 @@ def main():
                      "rel_res": float(infos[-1][1] / infos[-1][2]), "rc": int(rc)}
 
     # Rooflines on the finest level.  Algorithmic bytes are the bytes the
-    # line layout has to move (values are stored without column indices; x
-    # counted once per launch, every launch gathers from all of it):
+    # line layout has to move (values are stored without column indices):
     #   SpMV:                 stored values s_v + x (N s_v) + y of the active rows
-    #   SSOR group launch:    average over the 2 * 9 - 1 launches of a sweep of
-    #                         the 9 line groups (3 colours each): all values once
-    #                         forward, the half after a line and its own group (1
-    #                         of 16) backward, x (N s_v), and of the rows f, x and
-    #                         the kept sums written forward, f, x and the sums read
-    #                         and written backward
+    #   SSOR group launch:    group_launch_bytes
     # Durations are those of the single dispatches (events recorded by the
     # dispatch, pmx_time_kernel 10 / 11), not of back-to-back launch sequences.
     nvals = int(d[6])
     nact = int(d[1])
-    ngrp = int(round(int(d[7]) ** (2 / 3)))  # line groups: colours per axis squared
     kern = {}
     roof = {}
     for prec, sv in ((1, 4), (0, 8)):
         ms_spmv = S.time_kernel(11, -1, prec, reps=20)
         ms_col = S.time_kernel(10, -1, prec, reps=4)
         b_spmv = nvals * sv + N * sv + nact * sv
-        b_col = (nvals * (1.5 + 0.5 / 16) + 7 * nact) * sv / (2 * ngrp - 1) + N * sv
+        b_col = group_launch_bytes(nvals, N, nact, sv)
         roof[prec] = {"spmv_ms": ms_spmv, "spmv_bytes": b_spmv, "col_ms": ms_col, "col_bytes": b_col}
     # calibration of the group launch on the same level and with the same
     # dispatch events: a dispatch that does nothing (its workgroup counts) and
@@ -446,7 +471,6 @@ def main():
     S.assemble(prm4)
     asm4_finest_ms = S.time_kernel(4, -1, 0, reps=3)
     t_asm4 = sum(S.time_kernel(4, lvl, 0, reps=3) for lvl in range(5)) * 1e-3
-    flops_asm4 = 428544.0 * (2 ** nref) ** 3  # Q2, 64-point rule, B^T D B model per cell
 
     offop = None
     if train is not None and not args.no_offop:
@@ -478,12 +502,12 @@ def main():
     t_asm_call = res[main_form]["t_asm"]
     steps_ms = (res[main_form]["t_asm"] + res[main_form]["t_solve"]) * 1e3  # assemble call + solve
     t64 = res.get("fp64", {}).get("t_solve")
-    flops_asm = 180792.0 * (2 ** nref) ** 3  # Q2, 27-point rule, B^T D B model per cell
     r32 = roof[1]
     col_gbs = r32["col_bytes"] / (r32["col_ms"] * 1e-3) / 1e9
     spmv_gbs = r32["spmv_bytes"] / (r32["spmv_ms"] * 1e-3) / 1e9
-    asm_tf = flops_asm / (kern["assembly_finest_ms"] * 1e-3) / 1e12
-    asm4_tf = flops_asm4 / (asm4_finest_ms * 1e-3) / 1e12
+    b_asm, f_asm = assembly_work(2 ** nref, 3, nvals)
+    b_asm4, f_asm4 = assembly_work(2 ** nref, 4, nvals)
+    t_fin, t_fin4 = kern["assembly_finest_ms"] * 1e-3, asm4_finest_ms * 1e-3
     out = {
         "metric": "time-to-1e-10 FP64 residual (s), learned+FP32 vs plain FP64 GMG; assembly DOF/s",
         "value": round(t_main, 5),
@@ -525,8 +549,9 @@ def main():
                        "ssor_group_fp64_dispatch": round(roof[0]["col_ms"], 4),
                        **{k: round(v, 4) for k, v in kern.items()}},
         # the dominant kernel of the timed solve: the line-group launches of the
-        # finest level's FP32 SSOR sweeps
-        "roofline": {"bound": "hbm", "kernel": "k_line_sweep<float,float,2> (one SSOR group launch, finest level)",
+        # finest level's FP32 SSOR sweeps, average over the 66 of a cycle
+        "roofline": {"bound": "hbm", "kernel": "k_line_sweep<float,float,2> (one SSOR group launch of a V(2,2) "
+                                               "cycle, finest level)",
                      "achieved": round(col_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(col_gbs / HBM_PEAK_GBS, 4), "traffic": TRAFFIC_SSOR_LAUNCH,
                      "algorithmic_bytes": int(r32["col_bytes"]), "dispatch_ms": round(r32["col_ms"], 5),
@@ -539,14 +564,16 @@ def main():
                           "frac": round(spmv_gbs / HBM_PEAK_GBS, 4), "traffic": TRAFFIC_SPMV,
                           "algorithmic_bytes": int(r32["spmv_bytes"]), "dispatch_ms": round(r32["spmv_ms"], 5),
                           "fp64_GBs": round(roof[0]["spmv_bytes"] / (roof[0]["spmv_ms"] * 1e-3) / 1e9, 1)},
-        # Q2 assembly of the finest level against the FP64 peak (operations of the
-        # plain sum B^T D B: 47.4 GFLOP with the 27-point rule, 112.3 GFLOP with the
-        # 64-point rule; k_cell_sum takes a fifth of them)
-        "roofline_assembly": {"bound": "fp64", "kernel": "k_qp_data + k_cell_sum + k_assemble_kc (finest level)",
-                              "achieved": round(asm_tf, 2), "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                              "frac": round(asm_tf / FP64_PEAK_TFLOPS, 4),
-                              "gauss4_achieved": round(asm4_tf, 2),
-                              "gauss4_frac": round(asm4_tf / FP64_PEAK_TFLOPS, 4)},
+        # Q2 assembly of the finest level (assembly_work), 27- and 64-point rule
+        "roofline_assembly": {"bound": "hbm",
+                              "kernel": "k_qp_data_fourier + k_cell_sum + k_assemble_kc (finest level)",
+                              "achieved": round(b_asm / t_fin / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                              "frac": round(b_asm / t_fin / 1e9 / HBM_PEAK_GBS, 4), "bytes": b_asm,
+                              "fp64_tflops": round(f_asm / t_fin / 1e12, 2),
+                              "fp64_frac": round(f_asm / t_fin / 1e12 / FP64_PEAK_TFLOPS, 4),
+                              "gauss4_achieved": round(b_asm4 / t_fin4 / 1e9, 1),
+                              "gauss4_frac": round(b_asm4 / t_fin4 / 1e9 / HBM_PEAK_GBS, 4), "gauss4_bytes": b_asm4,
+                              "gauss4_fp64_tflops": round(f_asm4 / t_fin4 / 1e12, 2)},
         "roofline_conv": conv,
     }
     if not args.no_cpu:

@@ -279,8 +279,9 @@ int pmx_tcd_restore_massmat(pmx_system *sys);
  * timed with two events around the `reps` repetitions (ms per repetition).
  * 10 and 11 give the average duration of a single dispatch, from events
  * recorded by the dispatch itself (hipExtLaunchKernelGGL), without the gaps
- * between dispatches: 10 one launch of an SSOR sweep (a line group: the
- * colours of equal (y, z) residues), 11 one SpMV; calibration of 10 on the
+ * between dispatches: 10 one launch (a line group: the colours of equal (y, z)
+ * residues) of the SSOR smoothing of a V(2,2) cycle on the level, two sweeps
+ * from zero and two from the iterate they leave, 11 one SpMV; calibration of 10 on the
  * same level, also per dispatch: 12 a dispatch that does nothing with the
  * workgroup count of each group launch, 13 a plain streaming read of a group's
  * share of the stored values in the precision's storage.  precision 0 FP64,

@@ -11,6 +11,7 @@
 #include <stdexcept>
 #include <string>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/pmx.h"
@@ -2102,16 +2103,26 @@ int pmx_time_kernel(pmx_system *sys, int kernel, int level, int precision, int r
     };
     if (kernel == 10 || kernel == 11) {
       // durations of the individual dispatches (not the gaps between them):
-      // 10 the group launches of SSOR sweeps (launches forced), 11 SpMV
+      // 10 the group launches of a V(2,2) cycle's SSOR smoothing (launches
+      // forced): two sweeps from zero and two from the iterate they leave, with
+      // f = 1 in the interior, 11 SpMV
       Y.opt[21] = -1;
-      auto run = [&]() {
-        if (kernel == 10) {
-          if (precision) level_smooth<float>(Y, lv, 3, 1.0, 1);
-          else level_smooth<double>(Y, lv, 3, 1.0, 1);
-        } else {
-          if (precision) rows_apply<float>(lv.D, 0, lv.v32.val.p, lv.v32.x.p, nullptr, lv.v32.d.p, 0.0, st);
-          else rows_apply<double>(lv.D, 0, lv.v64.val.p, lv.v64.x.p, nullptr, lv.v64.d.p, 0.0, st);
+      auto run_t = [&](auto &v) {
+        using T = std::remove_pointer_t<decltype(v.x.p)>;
+        if (kernel == 11) {
+          rows_apply<T>(lv.D, 0, v.val.p, v.x.p, nullptr, v.d.p, 0.0, st);
+          return;
         }
+        fill<T>(v.f.p, T(1), lv.L.N, st);
+        boundary<T>(lv.D, 3, v.f.p, nullptr, nullptr, st);
+        fill<T>(v.x.p, T(0), lv.L.N, st);
+        fill<int>(Y.bnd_set.p, 0, 1, st);
+        level_smooth<T>(Y, lv, 3, 1.0, 2, kStartInteriorZero);
+        level_smooth<T>(Y, lv, 3, 1.0, 2, kStartBoundary);
+      };
+      auto run = [&]() {
+        if (precision) run_t(lv.v32);
+        else run_t(lv.v64);
       };
       run();
       DispatchTimer tm;
