@@ -277,3 +277,49 @@ def test_coarse_loop_matches_the_oracle(ctx, order, nref, coarse):
         got, _, _ = S.solve(opt, rhs, sol0, check=False)
         assert rel(got, ref) < 1e-12, (sweeps, red)
     S.close()
+
+
+def test_relaxed_sweeps_of_long_lines(ctx):
+    """257^3 Q1, two SSOR sweeps with omega 0.7: the turns within and between the
+    sweeps, with the sums kept there, against the definition by residuals."""
+    S = pa.System(ctx, 7, 2, 1)
+    S.assemble(P.config1b())
+    n, na = int(S.dims()[0]), int(S.dims()[1])
+    col = S.colours()[:na]
+    rng = np.random.default_rng(9)
+    x, b = rng.standard_normal(n), rng.standard_normal(n)
+    diag, ref = np.zeros(na), x.copy()
+    ref[na:] = b[na:]
+    for c in range(8):
+        e = np.zeros(n)
+        e[:na][col == c] = 1.0
+        diag += np.where(col == c, S.matvec(e)[:na], 0.0)
+    for c in 2 * (list(range(8)) + list(range(7, -1, -1))):
+        r, _ = S.defect(ref, b)
+        ref[:na] += np.where(col == c, 0.7 * r[:na] / diag, 0.0)
+        print(f"[case] residual before colour {c}", flush=True)
+    assert rel(S.smooth(3, 0.7, 2, x, b), ref) < 1e-12
+    S.close()
+
+
+def test_solves_on_long_lines(ctx):
+    """257^3 Q1, five levels: sweeps from zero, kept sums in the defects and in A z,
+    in FP64, FP32 and with FP16 values.  The residual that the solve reports is
+    that of its solution, and the FP32 forms, which restart the Krylov space with
+    every outer correction, take at most twice the iterations."""
+    S = pa.System(ctx, 4, 5, 1)
+    S.assemble(P.config1b())
+    rhs = S.rhs()
+    its = {}
+    for prec in (0, 1, 3):
+        print(f"[case] 257^3 Q1 solve, precision {prec}", flush=True)
+        opt = P.solver_opt(solver=16, restart=30, maxit=200, res_norm_min=0.0, red_factor=0.0, rel_target=1e-8,
+                           smoother=3, omega=1.0, precision=prec)
+        info, rc = S.solve_resident(opt, check=False)
+        assert rc == 0 and info[1] <= 1e-8 * info[2] * 1.0001, (prec, rc, info)
+        _, res = S.defect(S.solution(), rhs)
+        assert abs(res - info[1]) <= 1e-5 * res, (prec, res, info)
+        its[prec] = int(info[0])
+    print(f"iterations {its}", flush=True)
+    assert max(its[1], its[3]) <= 2 * its[0]
+    S.close()
