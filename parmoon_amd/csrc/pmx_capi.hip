@@ -449,7 +449,7 @@ static bool level_smooth(System &Y, Level &lv, int kind, double omega, int sweep
   Vecs<T> &v = vecs<T>(lv);
   // small levels sweep by planes, up to 17^3 nodes with FP32 values also where the
   // larger ones take FP16 values (there is no traffic to save); opt[21] as in pmx.h.
-  // 33^3 Q2 takes the FP16 values by line groups (SSOR sweep 71 us; FP32 by planes
+  // 33^3 Q2 takes the FP16 values by line groups (SSOR sweep 71 - 75 us; FP32 by planes
   // 54 us, by line groups 74 us)
   const bool planes = plane_sweeps_used(lv.D) && (Y.opt[21] == 0 || lv.D.max_colour_rows <= (int64_t)Y.opt[21]);
   if (kind == 1) {
